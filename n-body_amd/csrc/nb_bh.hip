@@ -19,18 +19,20 @@
 //                  scan, and a stable scatter whose per-wave ranks come from
 //                  64-bit ballots (8 ballots give each lane the mask of lanes
 //                  holding the same digit). Stable => sorted by (code, index).
-//   4. permute     gather (x, y, z, m) into sorted order.
-//   5. prefix      FP64 exclusive prefix of (m, m x, m y, m z) over sorted bodies:
-//                  any node's mass and centre of mass is a difference of two
-//                  prefix entries (cells are contiguous code ranges).
-//   6. octree      breadth-first, one level per round: a node with more than
-//                  leaf_size bodies (and level < 10) splits into its non-empty
-//                  Morton-digit children, found by binary search in its code
-//                  range; children get consecutive indices from a scan of child
-//                  counts, so numbering is deterministic. Ropes (`next`) point to
+//   4. mark        gather (x, y, z, m) into sorted order; per body the levels at
+//                  which a node starts there; per tile the node counts of every
+//                  level and the FP64 sums of (m, m x, m y, m z).
+//   5. scan        of the tiles' counts and sums.
+//   6. emit        per body the nodes that start or end there, and the FP64
+//                  prefix: any node's mass and centre of mass is a difference of
+//                  two prefix entries (cells are contiguous code ranges). The
+//                  octree is breadth-first: a node with more than leaf_size bodies
+//                  (and level < 10) splits into its non-empty Morton-digit
+//                  children, which get consecutive indices. Ropes (`next`) point to
 //                  the next sibling, or the parent's rope for the last child —
 //                  the firstChild/next contract of Octree.cpp:264-294.
 //   7. com         per node from the prefix; single-body nodes copy the body.
+//                  Also the wave ranges of the traversal.
 //   8. traverse    one lane per sorted body, stackless rope walk with the
 //                  reference's opening test s^2 < theta^2 d^2 (Octree.cpp:320);
 //                  a leaf that is not accepted is evaluated body by body.
@@ -48,6 +50,7 @@ namespace {
 // tiles of 2048 keys (8 per lane) measured 40 us faster per 4M-body sort than
 // 4096 (more tiles in flight) and than 1024 (larger histograms).
 constexpr int kScanThreads = 256;
+constexpr int kScanWaves = kScanThreads / 64;
 // Traversal groups: each wave of the traversal takes one "wave range" of at
 // most kWaveBodies consecutive sorted bodies. Ranges are cut along the tree: the
 // children of a node holding more than kWaveBodies bodies are packed in order
@@ -233,29 +236,17 @@ __global__ __launch_bounds__(256) void k_morton(const float4* __restrict__ pm, i
   vals[i] = (uint32_t)i;
 }
 
-// ---- generic reduce-then-scan (int32 and FP64x4) ----------------------------
-// The element count is either a constant or the size of one octree level,
-// read on the device: count = level_off[l + 1] - level_off[l].
-// The count is clamped to the launch bound `cap`, so a bad level table can
-// never send the scan past its buffers.
-__device__ __forceinline__ int scan_count(const int* level_off, int l, int n_const, int cap) {
-  const int c = level_off ? level_off[l + 1] - level_off[l] : n_const;
-  return c < 0 ? 0 : (c > cap ? cap : c);
-}
-
-// Pass 1 of an exclusive int scan: the sum of every kScanTile-element tile.
-__global__ __launch_bounds__(kScanThreads) void k_iscan_reduce(const int* __restrict__ in,
-                                                               const int* level_off, int l,
-                                                               int n_const, int cap,
+// ---- exclusive int scan -------------------------------------------------------
+// Pass 1: the sum of every kScanTile-element tile.
+__global__ __launch_bounds__(kScanThreads) void k_iscan_reduce(const int* __restrict__ in, int n,
                                                                int* __restrict__ part) {
-  const int n = scan_count(level_off, l, n_const, cap);
   const int base = blockIdx.x * kScanTile;
   int s = 0;
   for (int k = threadIdx.x; k < kScanTile; k += kScanThreads) {
     const int e = base + k;
     if (e < n) s += in[e];
   }
-  __shared__ int wsum[kScanThreads / 64];
+  __shared__ int wsum[kScanWaves];
   int tile = 0;
   (void)block_excl_scan(s, wsum, tile);
   if (threadIdx.x == 0) part[blockIdx.x] = tile;
@@ -264,29 +255,12 @@ __global__ __launch_bounds__(kScanThreads) void k_iscan_reduce(const int* __rest
 // Pass 2: every tile adds up the tile sums before it (a few KB of L2 reads per
 // tile, which replaces a separate one-block scan of the sums and its launch),
 // then rescans its own elements from there (8 consecutive elements per thread,
-// one block scan of the thread sums). Block 0 also adds up all nparts tile sums
-// into part[nparts] and, for a level, publishes the next level's end:
-// level_off[l + 2] = level_off[l + 1] + total.
-__global__ __launch_bounds__(kScanThreads) void k_iscan_final(const int* __restrict__ in,
-                                                              const int* level_off, int l,
-                                                              int n_const, int cap,
-                                                              int* __restrict__ part, int nparts,
-                                                              int* level_off_mut,
+// one block scan of the thread sums).
+__global__ __launch_bounds__(kScanThreads) void k_iscan_final(const int* __restrict__ in, int n,
+                                                              const int* __restrict__ part,
                                                               int* __restrict__ out) {
-  const int n = scan_count(level_off, l, n_const, cap);
   const int base = blockIdx.x * kScanTile;
-  __shared__ int wsum[kScanThreads / 64];
-  if (blockIdx.x == 0) {
-    int all = 0;
-    for (int b = threadIdx.x; b < nparts; b += kScanThreads) all += part[b];
-    int total = 0;
-    (void)block_excl_scan(all, wsum, total);
-    if (threadIdx.x == 0) {
-      part[nparts] = total;
-      if (level_off_mut) level_off_mut[l + 2] = level_off[l + 1] + total;
-    }
-  }
-  if (base >= n) return;
+  __shared__ int wsum[kScanWaves];
   int pre = 0;
   for (int b = threadIdx.x; b < (int)blockIdx.x; b += kScanThreads) pre += part[b];
   int start = 0;
@@ -311,14 +285,10 @@ __global__ __launch_bounds__(kScanThreads) void k_iscan_final(const int* __restr
 }
 
 // Exclusive scan of at most kSingleScan elements by one workgroup (8 consecutive
-// elements per thread), for the small scans: one launch instead of two. Writes
-// level_off[l + 2] like k_iscan_final.
+// elements per thread), for the small scans: one launch instead of two.
 constexpr int kSingleScan = 8192;
-__global__ __launch_bounds__(1024) void k_iscan_single(const int* __restrict__ in,
-                                                       const int* level_off, int l, int n_const,
-                                                       int cap, int* __restrict__ out,
-                                                       int* level_off_mut) {
-  const int n = scan_count(level_off, l, n_const, cap);
+__global__ __launch_bounds__(1024) void k_iscan_single(const int* __restrict__ in, int n,
+                                                       int* __restrict__ out) {
   constexpr int kPer = kSingleScan / 1024;
   const int base = threadIdx.x * kPer;
   int v[kPer];
@@ -333,18 +303,14 @@ __global__ __launch_bounds__(1024) void k_iscan_single(const int* __restrict__ i
   __shared__ int wsum[16];
   if (lane == 63) wsum[wave] = incl;
   __syncthreads();
-  int before = 0, total = 0;
-  for (int w = 0; w < 16; ++w) {  // fixed order
-    before += w < wave ? wsum[w] : 0;
-    total += wsum[w];
-  }
+  int before = 0;
+  for (int w = 0; w < wave; ++w) before += wsum[w];
   int run = before + incl - sum;
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     if (base + k < n) out[base + k] = run;
     run += v[k];
   }
-  if (threadIdx.x == 0 && level_off_mut) level_off_mut[l + 2] = level_off[l + 1] + total;
 }
 
 // FP64 prefix of (m, m x, m y, m z): prefix[k] = sum over sorted bodies < k.
@@ -356,29 +322,6 @@ __device__ __forceinline__ double4 add4(double4 a, double4 b) {
   return make_double4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
 }
 
-// Tiles of kScanTile = 8 rows x 256 bodies: thread t holds the bodies t, 256 + t,
-// ..., so every wave load and store is one contiguous 1 KB (float4) or 2 KB
-// (double4) run.
-__global__ __launch_bounds__(kScanThreads) void k_mscan_reduce(const float4* __restrict__ pms,
-                                                               int n, double4* __restrict__ part) {
-  constexpr int kRows = kScanTile / kScanThreads;
-  const int base = blockIdx.x * kScanTile;
-  double4 s = make_double4(0, 0, 0, 0);
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const int e = base + r * kScanThreads + threadIdx.x;
-    if (e < n) s = add4(s, body_moments(pms[e]));
-  }
-  __shared__ double4 sh[kScanThreads];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = kScanThreads / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) sh[threadIdx.x] = add4(sh[threadIdx.x], sh[threadIdx.x + w]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-
 __device__ __forceinline__ double4 shfl_up4(double4 v, int off) {
   return make_double4(__shfl_up(v.x, off), __shfl_up(v.y, off), __shfl_up(v.z, off),
                       __shfl_up(v.w, off));
@@ -386,74 +329,6 @@ __device__ __forceinline__ double4 shfl_up4(double4 v, int off) {
 __device__ __forceinline__ double4 wave_incl_scan4(double4 v) {
   return make_double4(wave_incl_scan(v.x), wave_incl_scan(v.y), wave_incl_scan(v.z),
                       wave_incl_scan(v.w));
-}
-
-// Exclusive scan of the block sums by one block, in a fixed order: each thread
-// folds a contiguous run of partials, the 256 run totals are scanned (wave DPP
-// prefixes, then the 4 wave totals in wave order), then each thread rewrites its
-// run. part[nparts] receives the total.
-__global__ __launch_bounds__(kScanThreads) void k_mscan_partials(double4* __restrict__ part,
-                                                                 int nparts) {
-  const int per = (nparts + kScanThreads - 1) / kScanThreads;
-  const int b0 = min((int)threadIdx.x * per, nparts);
-  const int b1 = min(b0 + per, nparts);
-  double4 tot = make_double4(0, 0, 0, 0);
-  for (int b = b0; b < b1; ++b) tot = add4(tot, part[b]);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const double4 incl = wave_incl_scan4(tot);
-  __shared__ double4 wtot[kScanThreads / 64];
-  if (lane == 63) wtot[wave] = incl;
-  __syncthreads();
-  double4 run = make_double4(0, 0, 0, 0), grand = make_double4(0, 0, 0, 0);
-  for (int w = 0; w < kScanThreads / 64; ++w) {
-    if (w < wave) run = add4(run, wtot[w]);
-    grand = add4(grand, wtot[w]);
-  }
-  const double4 below = shfl_up4(incl, 1);  // inclusive value of the lane below
-  if (lane > 0) run = add4(run, below);
-  for (int b = b0; b < b1; ++b) {
-    const double4 v = part[b];
-    part[b] = run;
-    run = add4(run, v);
-  }
-  if (threadIdx.x == 0) part[nparts] = grand;
-}
-
-// Exclusive prefix of each tile, row by row: a row of 256 bodies is scanned by
-// wave DPP prefixes and a fixed-order combine of the 4 wave totals; rows follow
-// each other in order. Deterministic (no atomics, fixed association).
-__global__ __launch_bounds__(kScanThreads) void k_mscan_final(const float4* __restrict__ pms,
-                                                              int n,
-                                                              const double4* __restrict__ part,
-                                                              double4* __restrict__ prefix) {
-  constexpr int kRows = kScanTile / kScanThreads;
-  constexpr int kWaves = kScanThreads / 64;
-  const int base = blockIdx.x * kScanTile;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __shared__ double4 wtot[kRows][kWaves];
-  double4 incl[kRows];
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const int e = base + r * kScanThreads + threadIdx.x;
-    const double4 x0 = e < n ? body_moments(pms[e]) : make_double4(0, 0, 0, 0);
-    const double4 x = wave_incl_scan4(x0);
-    if (lane == 63) wtot[r][wave] = x;
-    const double4 below = shfl_up4(x, 1);  // inclusive value of the lane below
-    incl[r] = lane > 0 ? below : make_double4(0, 0, 0, 0);
-  }
-  __syncthreads();
-  double4 run = part[blockIdx.x];  // exclusive start of this tile
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    double4 before = run;  // tile start + earlier rows + earlier waves of this row
-    for (int w = 0; w < kWaves; ++w) {
-      if (w < wave) before = add4(before, wtot[r][w]);
-      run = add4(run, wtot[r][w]);
-    }
-    const int e = base + r * kScanThreads + threadIdx.x;
-    if (e < n) prefix[e] = add4(before, incl[r]);  // incl[r]: exclusive within the wave
-  }
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) prefix[n] = part[gridDim.x];
 }
 
 // ---- 3. radix sort ------------------------------------------------------------
@@ -575,17 +450,6 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(
   }
 }
 
-// ---- 4. permute -------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_gather(const float4* __restrict__ pm,
-                                                const uint32_t* __restrict__ perm, int n,
-                                                float4* __restrict__ pms) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) {
-    const uint32_t p = perm[i];
-    pms[i] = p < (uint32_t)n ? pm[p] : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-}
-
 // Morton reordering of the resident state: dst[k] = src[perm[k]] per component.
 __global__ __launch_bounds__(256) void k_permute_d3(const double* __restrict__ src,
                                                     const uint32_t* __restrict__ perm, int n,
@@ -615,83 +479,261 @@ __global__ __launch_bounds__(256) void k_permute_f32(const float* __restrict__ s
 __device__ __forceinline__ int link_count(int w) { return w >> 4; }
 __device__ __forceinline__ int link_level(int w) { return w & 15; }
 
-// First index in [lo, hi) whose digit (codes >> shift) & 7 is >= d (digits are sorted).
-__device__ __forceinline__ int digit_lower_bound(const uint32_t* __restrict__ codes, int lo,
-                                                 int hi, int shift, uint32_t d) {
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (((codes[mid] >> shift) & 7u) < d) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
+// Octal digits that two 30-bit codes share from the top (0..10).
+__device__ __forceinline__ int common_level(uint32_t a, uint32_t b) {
+  const uint32_t x = a ^ b;
+  return x ? (29 - (31 - __clz((int)x))) / 3 : kMaxLevel;
 }
 
-// Boundaries of the 8 digit cells of the sorted range [s, e): bound[d] = first
-// index whose digit is >= d (bound[0] = s, bound[8] = e). The seven binary
-// searches run in lockstep, so each step issues seven independent loads and the
-// latency is log2(e - s) loads rather than seven times that (dense nodes near
-// the disc centres hold 10^5 bodies). Counting the digits of short ranges with
-// independent loads instead was measured slower.
-__device__ __forceinline__ void digit_bounds(const uint32_t* __restrict__ codes, int s, int e,
-                                             int shift, int (&bound)[9]) {
-  int lo[7], hi[7];
-#pragma unroll
-  for (int d = 0; d < 7; ++d) {
-    lo[d] = s;
-    hi[d] = e;
+constexpr int kTreeWaves = kTreeTile / 64;  // one body per thread
+constexpr int kMaxLeaf = 64;  // bodies per leaf that nb_create accepts
+
+// The octree without a loop over its levels. In the sorted codes every cell is a
+// run of bodies, so a body i can start one cell per level, from the level d(i) at
+// which it parts from the body before it (d = digits in common + 1) downwards;
+// such a cell is a node if it is the root or its parent holds more than `leaf`
+// bodies. The cell of level l around i does so exactly when some leaf + 1
+// consecutive bodies, i among them, share l digits. With
+//   c(k) = digits in common of the codes k and k + leaf,
+//   depth(i) = max of c(k) over k = i - leaf .. i,
+// the nodes that start at i are therefore those of the levels d(i) .. D(i),
+// D(i) = min(depth(i) + 1, 10), and a node of level l there has children exactly
+// when l < D(i). A node's index is the number of nodes of the levels above plus
+// the number of nodes of its level that start before i: a count per tile and
+// level (here), a scan of the counts (k_tree_scan), and a rank inside the tile
+// (k_tree_emit). Three launches of one coalesced pass each take the place of a
+// count, a scan and an emission for each of the ten levels with their binary
+// searches (gather to centres of mass at 65,536 bodies: 31 launches, 175 us -> 4
+// launches, 30 us; at 2^22: 508 -> 260 us).
+//
+// This kernel also brings the bodies into sorted order and sums the moments of
+// its tile for the FP64 prefix: it reads the permutation and the codes anyway.
+// Tiles of 1024 bodies, one per thread: at 65,536 bodies these kernels are chains
+// of latencies, and eight bodies per thread took 17 + 28 us where one takes 7 + 7 us.
+__global__ __launch_bounds__(kTreeTile) void k_tree_mark(
+    const uint32_t* __restrict__ codes, const uint32_t* __restrict__ perm,
+    const float4* __restrict__ pm, int n, int leaf, float4* __restrict__ pms,
+    double4* __restrict__ part, unsigned char* __restrict__ marks, int* __restrict__ level_cnt) {
+  __shared__ uint32_t s_code[kTreeTile + 2 * kMaxLeaf];  // the tile and kMaxLeaf on either side
+  __shared__ signed char s_win[2][kTreeTile + kMaxLeaf];
+  __shared__ int s_cnt[kLevels][kTreeWaves];
+  __shared__ double4 s_mom[kTreeWaves];
+  const int base = blockIdx.x * kTreeTile;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int i = base + threadIdx.x;
+  float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (i < n) {
+    const uint32_t p = perm[i];
+    if (p < (uint32_t)n) q = pm[p];
   }
-  for (int len = e - s; len > 0; len >>= 1) {  // ceil(log2) + 1 rounds cover every search
-    uint32_t v[7];
+  for (int x = threadIdx.x; x < kTreeTile + 2 * kMaxLeaf; x += kTreeTile) {
+    const int k = base - kMaxLeaf + x;
+    s_code[x] = k >= 0 && k < n ? codes[k] : 0u;
+  }
+  __syncthreads();
+  // c(k) at s_win[0][k - (base - kMaxLeaf)]; leaf <= kMaxLeaf, so k + leaf is staged
+  for (int x = threadIdx.x; x < kTreeTile + kMaxLeaf; x += kTreeTile) {
+    const int k = base - kMaxLeaf + x;
+    s_win[0][x] = k >= 0 && k + leaf < n ? (signed char)common_level(s_code[x], s_code[x + leaf]) : -1;
+  }
+  // windows of 2, 4, ... entries ending at x, up to the largest power of two
+  // that leaf + 1 holds: two of those cover a window of leaf + 1
+  int buf = 0, span = 1;
+  for (; 2 * span <= leaf + 1; span *= 2, buf ^= 1) {
+    __syncthreads();
+    for (int x = threadIdx.x; x < kTreeTile + kMaxLeaf; x += kTreeTile) {
+      const signed char v = s_win[buf][x];
+      s_win[buf ^ 1][x] = x >= span ? max(v, s_win[buf][x - span]) : v;
+    }
+  }
+  __syncthreads();
+  int d = kLevels, D = 0;  // no node
+  if (i < n) {
+    const int x = kMaxLeaf + threadIdx.x;
+    const int depth = max(s_win[buf][x], s_win[buf][x - (leaf + 1 - span)]);
+    D = min(depth + 1, kMaxLevel);
+    d = i == 0 ? 0 : common_level(s_code[x - 1], s_code[x]) + 1;
+    marks[i] = (unsigned char)(d << 4 | D);
+    pms[i] = q;
+  }
+  int cnt = 0;  // lane l: this wave's nodes of level l
 #pragma unroll
-    for (int d = 0; d < 7; ++d) v[d] = lo[d] < hi[d] ? codes[(lo[d] + hi[d]) >> 1] : 0u;
-#pragma unroll
-    for (int d = 0; d < 7; ++d)
-      if (lo[d] < hi[d]) {
-        const int mid = (lo[d] + hi[d]) >> 1;
-        if (((v[d] >> shift) & 7u) < (uint32_t)(d + 1)) lo[d] = mid + 1;
-        else hi[d] = mid;
+  for (int l = 0; l < kLevels; ++l) {
+    const int c = __popcll(__ballot(d <= l && l <= D));
+    cnt = lane == l ? c : cnt;
+  }
+  const double4 mom = wave_incl_scan4(body_moments(q));
+  if (lane < kLevels) s_cnt[lane][wave] = cnt;
+  if (lane == 63) s_mom[wave] = mom;
+  __syncthreads();
+  if (threadIdx.x < kLevels) {
+    int c = 0;
+    for (int w = 0; w < kTreeWaves; ++w) c += s_cnt[threadIdx.x][w];
+    level_cnt[threadIdx.x * gridDim.x + blockIdx.x] = c;
+  } else if (threadIdx.x == 64) {
+    double4 m = s_mom[0];
+    for (int w = 1; w < kTreeWaves; ++w) m = add4(m, s_mom[w]);
+    part[blockIdx.x] = m;
+  }
+}
+
+// Block 0: exclusive scan of the tiles' moments in a fixed order: each thread
+// folds a contiguous run of tiles, the 256 run totals are scanned (wave DPP
+// prefixes, then the 4 wave totals in wave order), then each thread rewrites its
+// run; part[tiles] receives the total. Block 1 + l: the same for the tiles' node
+// counts of level l, whose total goes to counters[2 + l]. Block 1 also resets the
+// traversal's work items and ticket, and lists the ranges of a system that no
+// node packs.
+__global__ __launch_bounds__(kScanThreads) void k_tree_scan(double4* __restrict__ part,
+                                                            int* __restrict__ level_cnt,
+                                                            int tiles, int n, int leaf, int pairs,
+                                                            int* __restrict__ counters,
+                                                            int4* __restrict__ waves,
+                                                            int* __restrict__ rec_hist) {
+  const int per = (tiles + kScanThreads - 1) / kScanThreads;
+  const int b0 = min((int)threadIdx.x * per, tiles);
+  const int b1 = min(b0 + per, tiles);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (blockIdx.x == 0) {
+    double4 tot = make_double4(0, 0, 0, 0);
+    for (int b = b0; b < b1; ++b) tot = add4(tot, part[b]);
+    const double4 incl = wave_incl_scan4(tot);
+    __shared__ double4 wtot[kScanWaves];
+    if (lane == 63) wtot[wave] = incl;
+    __syncthreads();
+    double4 run = make_double4(0, 0, 0, 0), grand = make_double4(0, 0, 0, 0);
+    for (int w = 0; w < kScanWaves; ++w) {
+      if (w < wave) run = add4(run, wtot[w]);
+      grand = add4(grand, wtot[w]);
+    }
+    const double4 below = shfl_up4(incl, 1);  // inclusive value of the lane below
+    if (lane > 0) run = add4(run, below);
+    for (int b = b0; b < b1; ++b) {
+      const double4 v = part[b];
+      part[b] = run;
+      run = add4(run, v);
+    }
+    if (threadIdx.x == 0) part[tiles] = grand;
+    return;
+  }
+  int* cnt = level_cnt + (blockIdx.x - 1) * tiles;
+  __shared__ int wsum[kScanWaves];
+  int sum = 0, total = 0;
+  for (int b = b0; b < b1; ++b) sum += cnt[b];
+  int run = block_excl_scan(sum, wsum, total);
+  for (int b = b0; b < b1; ++b) {
+    const int v = cnt[b];
+    cnt[b] = run;
+    run += v;
+  }
+  if (threadIdx.x == 0) counters[1 + blockIdx.x] = total;
+  if (blockIdx.x != 1) return;
+  if (threadIdx.x < kCostBuckets) rec_hist[threadIdx.x] = 0;  // this pass's traversal order starts empty
+  if (threadIdx.x == 0) {
+    int r = 0;
+    if (n <= kWaveBodies) {
+      waves[r++] = make_int4(0, n, 0, 0);
+    } else if (n <= leaf) {
+      // the root is itself a leaf, so no node packs ranges below it: chunk it,
+      // two full chunks per record, a shorter last chunk on its own
+      for (int o = 0; o < n; o += kWaveBodies) {
+        const int k = min(kWaveBodies, n - o), o2 = o + kWaveBodies;
+        if (pairs && k == kWaveBodies && n - o2 >= kWaveBodies) {
+          waves[r++] = make_int4(o, k, o2, kWaveBodies);
+          o = o2;
+        } else {
+          waves[r++] = make_int4(o, k, 0, 0);
+        }
       }
-  }
-  // a search whose interval is not empty yet (at most one more halving) finishes here
-#pragma unroll
-  for (int d = 0; d < 7; ++d)
-    while (lo[d] < hi[d]) {
-      const int mid = (lo[d] + hi[d]) >> 1;
-      if (((codes[mid] >> shift) & 7u) < (uint32_t)(d + 1)) lo[d] = mid + 1;
-      else hi[d] = mid;
     }
-  bound[0] = s;
-  bound[8] = e;
-#pragma unroll
-  for (int d = 0; d < 7; ++d) bound[d + 1] = lo[d];
+    counters[0] = r;
+    counters[1] = 0;  // traversal ticket
+  }
 }
 
-// Counts the non-empty children of every internal node of level l and keeps
-// their boundaries (bound[1..7]; bound[0] and bound[8] are the node's own range)
-// for k_tree_emit, which would otherwise repeat the seven binary searches.
-__global__ __launch_bounds__(256) void k_tree_count(const uint32_t* __restrict__ codes, int n,
-                                                    const int4* __restrict__ link,
-                                                    const int* __restrict__ level_off, int l,
-                                                    int leaf, int cap,
-                                                    int* __restrict__ child_cnt,
-                                                    int* __restrict__ child_bounds) {
-  const int lo = level_off[l];
-  const int hi = min(level_off[l + 1], lo + cap);  // cap = launch bound of this level
-  const int shift = 27 - 3 * l;
-  for (int k = lo + blockIdx.x * 256 + threadIdx.x; k < hi; k += gridDim.x * 256) {
-    const int4 nd = link[k];
-    const int cnt = link_count(nd.w);
-    int nc = 0;
-    if (cnt > leaf && nd.z >= 0 && nd.z + cnt <= n) {
-      int bound[9];
-      digit_bounds(codes, nd.z, nd.z + cnt, shift, bound);
+// Per tile: the exclusive FP64 prefix of the moments (wave DPP prefixes, then a
+// DPP prefix of the 16 wave totals: a fixed association, no atomics) and the
+// nodes that start or end in it. The body i that starts a node writes its first
+// child (which starts at i too), its start and its level; the last body i of a
+// node writes its end and its rope: the node of the lowest level that starts at
+// i + 1, which is a sibling of it or of the closest ancestor that has one. Few
+// levels are active in 64 neighbouring bodies, so the others are branched over
+// (at 2^22 bodies 141 us without that, 94 us with it).
+__global__ __launch_bounds__(kTreeTile) void k_tree_emit(
+    const float4* __restrict__ pms, int n, const double4* __restrict__ part,
+    const unsigned char* __restrict__ marks, const int* __restrict__ level_cnt,
+    const int* __restrict__ counters, int64_t max_nodes, double4* __restrict__ prefix,
+    int4* __restrict__ link, int* __restrict__ node_end, int* __restrict__ level_off,
+    int* __restrict__ flags) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t lt = (uint64_t(1) << lane) - 1;
+  const int e = blockIdx.x * kTreeTile + threadIdx.x;
+  __shared__ double4 s_mom[kTreeWaves];
+  __shared__ int s_off[kLevels][kTreeWaves];  // node starts per wave, then their first index
+  const double4 x0 = e < n ? body_moments(pms[e]) : make_double4(0, 0, 0, 0);
+  const int mark = e < n ? marks[e] : kLevels << 4;
+  const int dn = e + 1 < n ? marks[e + 1] >> 4 : 0;  // after the last body every node ends
+  const int d = mark >> 4, D = e < n ? mark & 15 : -1;
+  const double4 x = wave_incl_scan4(x0);
+  int cnt = 0;
 #pragma unroll
-      for (int d = 0; d < 8; ++d) nc += bound[d + 1] > bound[d] ? 1 : 0;
-#pragma unroll
-      for (int d = 1; d < 8; ++d) child_bounds[8 * (k - lo) + d] = bound[d];
-    }
-    child_cnt[k - lo] = nc;
+  for (int l = 0; l < kLevels; ++l) {
+    const int c = __popcll(__ballot(d <= l && l <= D));
+    cnt = lane == l ? c : cnt;
   }
+  if (lane == 63) s_mom[wave] = x;
+  if (lane < kLevels) s_off[lane][wave] = cnt;
+  __syncthreads();
+  if (wave < kLevels) {  // wave l: level l's node index at the start of every wave
+    const int l = wave;
+    int lo = 0;
+    for (int k = 0; k < l; ++k) lo += counters[2 + k];
+    const int v = lane < kTreeWaves ? s_off[l][lane] : 0;
+    const int at = wave_incl_scan(v) - v;
+    if (lane < kTreeWaves) s_off[l][lane] = lo + level_cnt[l * gridDim.x + blockIdx.x] + at;
+    if (blockIdx.x == 0 && lane == 0) {
+      level_off[l] = lo;
+      if (l == kMaxLevel) level_off[l + 1] = lo + counters[2 + l];
+    }
+  } else if (wave == kLevels) {
+    const double4 v = lane < kTreeWaves ? s_mom[lane] : make_double4(0, 0, 0, 0);
+    const double4 below = shfl_up4(wave_incl_scan4(v), 1);
+    const double4 run = part[blockIdx.x];  // exclusive start of this tile
+    if (lane < kTreeWaves) s_mom[lane] = lane > 0 ? add4(run, below) : run;
+  }
+  __syncthreads();
+  const double4 below = shfl_up4(x, 1);  // inclusive value of the lane below
+  const double4 start = s_mom[wave];
+  if (e < n) prefix[e] = lane > 0 ? add4(start, below) : start;
+  int* words = reinterpret_cast<int*>(link);
+  // idx[l]: index of a node of level l that starts at e
+  int idx[kLevels + 1], rope = -1;
+#pragma unroll
+  for (int l = 0; l < kLevels; ++l) {
+    const bool starts = d <= l && l <= D;
+    idx[l] = s_off[l][wave] + __popcll(__ballot(starts) & lt);
+    if (l == dn && e + 1 < n) rope = idx[l] + (starts ? 1 : 0);
+  }
+  idx[kLevels] = -1;
+  bool over = false;
+#pragma unroll
+  for (int l = 0; l < kLevels; ++l) {
+    const bool starts = d <= l && l <= D, ends = dn <= l && l <= D;
+    if (__ballot(starts || ends) == 0) continue;
+    const int64_t at = idx[l];
+    if (starts && at < max_nodes) {
+      words[4 * at] = l < D ? idx[l + 1] : -1;
+      *reinterpret_cast<int2*>(words + 4 * at + 2) = make_int2(e, l);
+    }
+    const int64_t in = at - (starts ? 0 : 1);  // the node of level l around e
+    if (ends && in >= 0 && in < max_nodes) {
+      words[4 * in + 1] = rope;
+      node_end[in] = e + 1;
+    }
+    over = over || (starts && at >= max_nodes);
+  }
+  if (over) atomicOr(flags, 2);
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) prefix[n] = part[gridDim.x];
 }
 
 // Wave ranges of one node's children (see kWaveBodies): calls out(start, count)
@@ -778,234 +820,6 @@ __device__ __forceinline__ void emit_records(int4* __restrict__ waves, int first
     if (wait[j].y > 0) put(make_int4(wait[j].x, wait[j].y, 0, 0));
 }
 
-__global__ __launch_bounds__(256) void k_tree_emit(const uint32_t* __restrict__ codes, int n,
-                                                   int4* __restrict__ link,
-                                                   const int* __restrict__ level_off, int l,
-                                                   int leaf, int cap,
-                                                   const int* __restrict__ child_off,
-                                                   const int* __restrict__ child_bounds,
-                                                   int64_t max_nodes, int* __restrict__ flags,
-                                                   int4* __restrict__ waves,
-                                                   int* __restrict__ wctl, int pairs) {
-  const int lo = level_off[l];
-  const int hi = min(level_off[l + 1], lo + cap);
-  const int next_lo = level_off[l + 1];
-  const int lane = threadIdx.x & 63;
-  // Rounds are uniform across the block, so every lane of a wave reaches the
-  // wave-wide range allocation below.
-  for (int base = lo + blockIdx.x * 256; base < hi; base += gridDim.x * 256) {
-    const int k = base + threadIdx.x;
-    int starts[8], ends[8], nc = 0;
-    int4 nd = make_int4(-1, -1, -1, 0);
-    bool internal = false;
-    if (k < hi) {
-      nd = link[k];
-      const int cnt = link_count(nd.w);
-      internal = cnt > leaf && nd.z >= 0 && nd.z + cnt <= n;
-    }
-    if (internal) {
-      int bound[9];  // as k_tree_count found them
-      bound[0] = nd.z;
-      bound[8] = nd.z + link_count(nd.w);
-#pragma unroll
-      for (int d = 1; d < 8; ++d) bound[d] = child_bounds[8 * (k - lo) + d];
-#pragma unroll
-      for (int d = 0; d < 8; ++d)
-        if (bound[d + 1] > bound[d]) {
-          starts[nc] = bound[d];
-          ends[nc] = bound[d + 1];
-          ++nc;
-        }
-      const int first = next_lo + child_off[k - lo];
-      if ((int64_t)first + nc > max_nodes) {
-        atomicOr(flags, 2);
-        internal = false;
-      } else {
-        for (int q = 0; q < nc; ++q) {
-          const int idx = first + q;
-          const int nxt = q + 1 < nc ? idx + 1 : nd.y;
-          link[idx] = make_int4(-1, nxt, starts[q], ((ends[q] - starts[q]) << 4) | (l + 1));
-        }
-        link[k].x = first;
-      }
-    }
-    // wave ranges of the children of nodes holding more than kWaveBodies bodies,
-    // in records of two: one atomic per wave reserves the records of all its lanes
-    const bool packs = internal && link_count(nd.w) > kWaveBodies;
-    const int nrec = packs ? count_records(starts, ends, nc, l, leaf, pairs) : 0;
-    const int incl = wave_incl_scan(nrec);
-    const int total = __shfl(incl, 63);
-    int wbase = 0;
-    if (lane == 63 && total > 0) wbase = atomicAdd(&wctl[0], total);
-    wbase = __shfl(wbase, 63);
-    if (nrec > 0) emit_records(waves, wbase + incl - nrec, n, starts, ends, nc, l, leaf, pairs);
-  }
-}
-
-// ---- 6a. the top levels from per-cell searches ---------------------------------------
-// Levels 0..kTopLevels are built without the level loop: a cell of level l is a
-// Morton prefix of 3l bits, so its body range in the sorted codes is found by a
-// lower-bound search for its smallest code, independently for every cell.
-// A cell is a node when it is the root, or it holds bodies and its parent holds
-// more than leaf_size; nodes are numbered breadth-first with children in digit
-// order, exactly as the level loop numbers them. The loop then continues from
-// level kTopLevels.
-
-__host__ __device__ constexpr int top_cell_base(int l) {  // first cell of level l
-  return l == 0 ? 0 : top_cell_base(l - 1) + (1 << (3 * (l - 1)));
-}
-__host__ __device__ constexpr int top_entry_base(int l) {  // first entry of level l
-  return top_cell_base(l) + l;
-}
-
-// top_start[top_entry_base(l) + c] = first sorted body of cell c of level l
-// (c = 8^l gives n).
-__global__ __launch_bounds__(256) void k_top_bounds(const uint32_t* __restrict__ codes, int n,
-                                                    int* __restrict__ top_start) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= kTopEntries) return;
-  int l = 0;
-  while (l < kTopLevels && e >= top_entry_base(l + 1)) ++l;
-  const uint32_t c = (uint32_t)(e - top_entry_base(l));
-  if (c == (1u << (3 * l))) {
-    top_start[e] = n;
-    return;
-  }
-  const uint32_t key = c << (30 - 3 * l);
-  int lo = 0, hi = n;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (codes[mid] < key) lo = mid + 1;
-    else hi = mid;
-  }
-  top_start[e] = lo;
-}
-
-// One workgroup: node links of levels 0..kTopLevels, level offsets, the wave
-// ranges of the nodes above kTopLevels, and the range counter / traversal ticket.
-__global__ __launch_bounds__(1024) void k_top_build(const int* __restrict__ top_start, int n,
-                                                    int leaf, int4* __restrict__ link,
-                                                    int* __restrict__ level_off,
-                                                    int4* __restrict__ waves,
-                                                    int* __restrict__ wctl,
-                                                    int* __restrict__ rec_hist, int pairs) {
-  __shared__ int s_idx[kTopCells];   // exclusive scan of existence, then node index
-  __shared__ int s_next[kTopCells];  // rope of each node
-  __shared__ int s_part[1024];
-  __shared__ int s_ranges;
-  const int tid = threadIdx.x;
-  auto cell_count = [&](int l, int c) {
-    const int e = top_entry_base(l) + c;
-    return top_start[e + 1] - top_start[e];
-  };
-  auto exists = [&](int l, int c) {
-    return l == 0 || (cell_count(l, c) > 0 && cell_count(l - 1, c >> 3) > leaf);
-  };
-  // 1. existence flags and their exclusive scan (cells in level order)
-  constexpr int kPer = (kTopCells + 1023) / 1024;
-  int flag[kPer];
-  int sum = 0;
-#pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const int g = tid * kPer + q;
-    int f = 0;
-    if (g < kTopCells) {
-      int l = 0;
-      while (l < kTopLevels && g >= top_cell_base(l + 1)) ++l;
-      f = exists(l, g - top_cell_base(l)) ? 1 : 0;
-    }
-    flag[q] = f;
-    sum += f;
-  }
-  s_part[tid] = sum;
-  if (tid == 0) s_ranges = 0;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {  // inclusive scan of the per-thread sums
-    const int v = tid >= off ? s_part[tid - off] : 0;
-    __syncthreads();
-    s_part[tid] += v;
-    __syncthreads();
-  }
-  int run = s_part[tid] - sum;
-#pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const int g = tid * kPer + q;
-    if (g < kTopCells) s_idx[g] = flag[q] ? run : -1;
-#pragma unroll
-    for (int l = 0; l <= kTopLevels; ++l)  // level_off[l] = nodes in the levels above l
-      if (g == top_cell_base(l)) level_off[l] = run;
-    run += flag[q];
-  }
-  if (tid == 1023) level_off[kTopLevels + 1] = s_part[1023];
-  __syncthreads();
-  if (tid < kCostBuckets) rec_hist[tid] = 0;  // this pass's traversal order starts empty
-  if (tid == 0) {
-    wctl[1] = 0;  // traversal ticket
-    if (n <= kWaveBodies) {
-      waves[0] = make_int4(0, n, 0, 0);
-      s_ranges = 1;
-    } else if (n <= leaf) {
-      // the root is itself a leaf, so no node packs ranges below it: chunk it,
-      // two full chunks per record, a shorter last chunk on its own
-      int r = 0;
-      for (int o = 0; o < n; o += kWaveBodies) {
-        const int k = min(kWaveBodies, n - o), o2 = o + kWaveBodies;
-        if (pairs && k == kWaveBodies && n - o2 >= kWaveBodies) {
-          waves[r++] = make_int4(o, k, o2, kWaveBodies);
-          o = o2;
-        } else {
-          waves[r++] = make_int4(o, k, 0, 0);
-        }
-      }
-      s_ranges = r;
-    }
-  }
-  // 2. links, level by level (a node's rope falls back to its parent's)
-  for (int l = 0; l <= kTopLevels; ++l) {
-    const int base = top_cell_base(l), cells = 1 << (3 * l);
-    for (int c = tid; c < cells; c += 1024) {
-      const int i = s_idx[base + c];
-      if (i < 0) continue;
-      const int cnt = cell_count(l, c);
-      const int start = top_start[top_entry_base(l) + c];
-      int nxt = l == 0 ? -1 : s_next[top_cell_base(l - 1) + (c >> 3)];
-      for (int sib = c + 1; sib < (c | 7) + 1 && l > 0; ++sib)
-        if (s_idx[base + sib] >= 0) {
-          nxt = s_idx[base + sib];
-          break;
-        }
-      s_next[base + c] = nxt;
-      int first = -1;
-      const bool internal = cnt > leaf && l < kMaxLevel;
-      if (internal && l < kTopLevels) {
-        const int cb = top_cell_base(l + 1) + 8 * c;
-        for (int d = 0; d < 8; ++d)
-          if (s_idx[cb + d] >= 0) {
-            first = s_idx[cb + d];
-            break;
-          }
-      }
-      link[i] = make_int4(first, nxt, start, (cnt << 4) | l);
-      // wave ranges of the children of a node above kTopLevels holding more
-      // than kWaveBodies bodies (level kTopLevels is done by the level loop)
-      if (internal && l < kTopLevels && cnt > kWaveBodies) {
-        int starts[8], ends[8], nc = 0;
-        const int eb = top_entry_base(l + 1) + 8 * c;
-        for (int d = 0; d < 8; ++d)
-          if (top_start[eb + d + 1] > top_start[eb + d]) {
-            starts[nc] = top_start[eb + d];
-            ends[nc] = top_start[eb + d + 1];
-            ++nc;
-          }
-        const int nrec = count_records(starts, ends, nc, l, leaf, pairs);
-        emit_records(waves, atomicAdd(&s_ranges, nrec), n, starts, ends, nc, l, leaf, pairs);
-      }
-    }
-    __syncthreads();
-  }
-  if (tid == 0) wctl[0] = s_ranges;
-}
-
 // ---- 7. centre of mass and opening radius -------------------------------------------
 // Squared opening radius of the default traversal: r = s_l / theta + delta, where
 // s_l is the cell side of the reference's test (Octree.cpp:311-320) and delta the
@@ -1042,36 +856,77 @@ __device__ __forceinline__ float open_radius2(float4 cm, uint32_t code, int l,
   return rc * rc;
 }
 
-__global__ __launch_bounds__(256) void k_tree_com(const int4* __restrict__ link, int n,
+// One thread per node: its centre of mass from the prefix, its opening radius,
+// its link's last word (count << 4 | level), and the wave ranges of the children
+// of nodes holding more than kWaveBodies bodies, in records of one or two: one
+// atomic per wave reserves the records of all its lanes.
+__global__ __launch_bounds__(256) void k_tree_com(int4* __restrict__ link,
+                                                  const int* __restrict__ node_end, int n,
                                                   int64_t max_nodes,
                                                   const int* __restrict__ level_off,
                                                   const double4* __restrict__ prefix,
                                                   const float4* __restrict__ pms,
                                                   const uint32_t* __restrict__ codes,
                                                   const float* __restrict__ geom, int cubic,
-                                                  float theta, float4* __restrict__ com,
+                                                  float theta, int leaf, int pairs,
+                                                  int4* __restrict__ waves,
+                                                  int* __restrict__ wctl,
+                                                  float4* __restrict__ com,
                                                   float* __restrict__ r2) {
   const int total = (int)min((int64_t)level_off[kMaxLevel + 1], max_nodes);
-  for (int k = blockIdx.x * 256 + threadIdx.x; k < total; k += gridDim.x * 256) {
-    const int4 nd = link[k];
-    const int cnt = link_count(nd.w);
-    if (nd.z < 0 || cnt < 1 || nd.z + cnt > n) {
-      com[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-      r2[k] = -1.f;
-      continue;
+  const int lane = threadIdx.x & 63;
+  int* words = reinterpret_cast<int*>(link);
+  // Rounds are uniform across the block, so every lane of a wave reaches the
+  // wave-wide record reservation.
+  for (int k0 = blockIdx.x * 256; k0 < total; k0 += gridDim.x * 256) {
+    const int k = k0 + threadIdx.x;
+    int starts[8], ends[8], nc = 0, nrec = 0, l = 0;
+    if (k < total) {
+      const int4 nd = link[k];
+      const int first = nd.x, start = nd.z;
+      l = nd.w & 15;
+      const int end = node_end[k], cnt = end - start;
+      words[4 * (int64_t)k + 3] = cnt << 4 | l;
+      float4 cm;
+      if (start < 0 || cnt < 1 || end > n) {
+        com[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+        r2[k] = -1.f;
+      } else {
+        if (cnt == 1) {
+          cm = pms[start];
+        } else {
+          const double4 a = prefix[start], b = prefix[end];
+          const double m = b.x - a.x;
+          const double inv = m > 0.0 ? 1.0 / m : 0.0;
+          cm = make_float4((float)((b.y - a.y) * inv), (float)((b.z - a.z) * inv),
+                           (float)((b.w - a.w) * inv), (float)m);
+        }
+        com[k] = cm;
+        r2[k] = open_radius2(cm, codes[start], l, geom, cubic, theta);
+        if (cnt > kWaveBodies && first >= 0 && l < kMaxLevel) {
+          // the children are consecutive nodes of the next level and tile the range
+          const int last = min(level_off[l + 2], total);
+          int s[8];  // eight independent loads; past the last child: >= end
+#pragma unroll
+          for (int q = 0; q < 8; ++q)
+            s[q] = first + q < last ? words[4 * (int64_t)(first + q) + 2] : end;
+#pragma unroll
+          for (int q = 0; q < 8; ++q)
+            if (s[q] < end) {
+              starts[q] = s[q];
+              ends[q] = q < 7 ? min(s[q < 7 ? q + 1 : 7], end) : end;
+              nc = q + 1;
+            }
+          nrec = count_records(starts, ends, nc, l, leaf, pairs);
+        }
+      }
     }
-    float4 cm;
-    if (cnt == 1) {
-      cm = pms[nd.z];
-    } else {
-      const double4 a = prefix[nd.z], b = prefix[nd.z + cnt];
-      const double m = b.x - a.x;
-      const double inv = m > 0.0 ? 1.0 / m : 0.0;
-      cm = make_float4((float)((b.y - a.y) * inv), (float)((b.z - a.z) * inv),
-                       (float)((b.w - a.w) * inv), (float)m);
-    }
-    com[k] = cm;
-    r2[k] = open_radius2(cm, codes[nd.z], link_level(nd.w), geom, cubic, theta);
+    const int incl = wave_incl_scan(nrec);
+    const int all = __shfl(incl, 63);
+    int wbase = 0;
+    if (lane == 63 && all > 0) wbase = atomicAdd(&wctl[0], all);
+    wbase = __shfl(wbase, 63);
+    if (nrec > 0) emit_records(waves, wbase + incl - nrec, n, starts, ends, nc, l, leaf, pairs);
   }
 }
 
@@ -1713,26 +1568,15 @@ __global__ void k_zero_u64(unsigned long long* p) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *p = 0ull;
 }
 
-int level_bound(int n, int l) {
-  int64_t w = 1;
-  for (int k = 0; k < l && w < n; ++k) w *= 8;
-  return (int)(w < n ? w : n);
-}
-
-// Enqueue an exclusive int scan: out[0..count) from in, count constant or per level.
-hipError_t iscan(const int* in, int* out, int* part, const int* level_off, int l, int n_const,
-                 int bound, int* level_off_mut, hipStream_t s) {
-  const int blocks = (bound + kScanTile - 1) / kScanTile;
-  if (blocks < 1) return hipSuccess;
-  if (bound <= kSingleScan) {
-    hipLaunchKernelGGL(k_iscan_single, dim3(1), dim3(1024), 0, s, in, level_off, l, n_const, bound,
-                       out, level_off_mut);
+// Enqueue an exclusive int scan: out[0..n) from in.
+hipError_t iscan(const int* in, int* out, int* part, int n, hipStream_t s) {
+  if (n <= kSingleScan) {
+    hipLaunchKernelGGL(k_iscan_single, dim3(1), dim3(1024), 0, s, in, n, out);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL(k_iscan_reduce, dim3(blocks), dim3(kScanThreads), 0, s, in, level_off, l,
-                     n_const, bound, part);
-  hipLaunchKernelGGL(k_iscan_final, dim3(blocks), dim3(kScanThreads), 0, s, in, level_off, l,
-                     n_const, bound, part, blocks, level_off_mut, out);
+  const int blocks = (n + kScanTile - 1) / kScanTile;
+  hipLaunchKernelGGL(k_iscan_reduce, dim3(blocks), dim3(kScanThreads), 0, s, in, n, part);
+  hipLaunchKernelGGL(k_iscan_final, dim3(blocks), dim3(kScanThreads), 0, s, in, n, part, out);
   return hipGetLastError();
 }
 
@@ -1758,11 +1602,10 @@ void nb_bh_carve(nb_ctx* c, char* base, int upto) {
   b.node_r2 = (float*)at(kBhR2);
   b.node_link = (int4*)at(kBhLink);
   b.level_off = (int*)at(kBhLevel);
-  b.child_cnt = (int*)at(kBhChildCnt);
-  b.child_off = (int*)at(kBhChildOff);
-  b.child_bounds = (int*)at(kBhChildBounds);
+  b.marks = (unsigned char*)at(kBhMarks);
+  b.node_end = (int*)at(kBhNodeEnd);
+  b.level_cnt = (int*)at(kBhLevelCnt);
   b.counters = (int*)at(kBhCounters);
-  b.top_start = (int*)at(kBhTopStart);
   b.waves = (int4*)at(kBhWaves);
   b.inter = (unsigned long long*)at(kBhInter);
   b.rec_cost = (float*)at(kBhRecCost);
@@ -1838,7 +1681,7 @@ hipError_t nb_morton_sort(nb_ctx* c) {
     const int in = pass & 1, out = in ^ 1;
     hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(kSortThreads), 0, s, b.keys[in], n, 8 * pass,
                        nb, b.digit_hist);
-    hipError_t e = iscan(b.digit_hist, offs, b.iscan_part, nullptr, 0, hist, hist, nullptr, s);
+    hipError_t e = iscan(b.digit_hist, offs, b.iscan_part, hist, s);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(kSortThreads), 0, s, b.keys[in],
                        b.vals[in], n, 8 * pass, nb, offs, b.keys[out], b.vals[out]);
@@ -1868,44 +1711,27 @@ hipError_t nb_bh_build(nb_ctx* c) {
   nb_bh_state& b = c->bh;
   const int n = c->n;
   hipStream_t s = c->stream;
-  const int g256 = (n + 255) / 256;
   hipError_t es = nb_morton_sort(c);
   if (es != hipSuccess) return es;
   const uint32_t* codes_sorted = b.keys[0];
   const uint32_t* perm = b.vals[0];
-  // 4. permute
-  hipLaunchKernelGGL(k_gather, dim3(g256), dim3(256), 0, s, c->pm, perm, n, b.pms);
-  // 5. FP64 prefix of mass moments
-  const int mblocks = (n + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL(k_mscan_reduce, dim3(mblocks), dim3(kScanThreads), 0, s, b.pms, n, b.scan_part);
-  hipLaunchKernelGGL(k_mscan_partials, dim3(1), dim3(kScanThreads), 0, s, b.scan_part, mblocks);
-  hipLaunchKernelGGL(k_mscan_final, dim3(mblocks), dim3(kScanThreads), 0, s, b.pms, n, b.scan_part,
-                     b.prefix);
-  // 6. octree: the top levels from per-cell searches, then level by level
+  const int tiles = (n + kTreeTile - 1) / kTreeTile;
   const int leaf = c->cfg.leaf_size;
-  hipLaunchKernelGGL(k_top_bounds, dim3((kTopEntries + 255) / 256), dim3(256), 0, s, codes_sorted,
-                     n, b.top_start);
   const int pairs = nb_bh_pairs(n, c->cfg.flags) ? 1 : 0;
-  hipLaunchKernelGGL(k_top_build, dim3(1), dim3(1024), 0, s, b.top_start, n, leaf, b.node_link,
-                     b.level_off, b.waves, b.counters, b.rec_hist, pairs);
-  for (int l = kTopLevels; l < kMaxLevel; ++l) {
-    const int bound = level_bound(n, l);
-    const int grid = std::max(1, std::min((bound + 255) / 256, 4096));
-    hipLaunchKernelGGL(k_tree_count, dim3(grid), dim3(256), 0, s, codes_sorted, n, b.node_link,
-                       b.level_off, l, leaf, bound, b.child_cnt, b.child_bounds);
-    hipError_t e = iscan(b.child_cnt, b.child_off, b.iscan_part, b.level_off, l, 0, bound,
-                         b.level_off, s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_tree_emit, dim3(grid), dim3(256), 0, s, codes_sorted, n, b.node_link,
-                       b.level_off, l, leaf, bound, b.child_off, b.child_bounds, b.max_nodes,
-                       c->flags, b.waves, b.counters, pairs);
-  }
-  // 7. centre of mass
+  // 4-6. bodies in sorted order, FP64 moment prefix, octree
+  hipLaunchKernelGGL(k_tree_mark, dim3(tiles), dim3(kTreeTile), 0, s, codes_sorted, perm, c->pm,
+                     n, leaf, b.pms, b.scan_part, b.marks, b.level_cnt);
+  hipLaunchKernelGGL(k_tree_scan, dim3(1 + kLevels), dim3(kScanThreads), 0, s, b.scan_part,
+                     b.level_cnt, tiles, n, leaf, pairs, b.counters, b.waves, b.rec_hist);
+  hipLaunchKernelGGL(k_tree_emit, dim3(tiles), dim3(kTreeTile), 0, s, b.pms, n, b.scan_part,
+                     b.marks, b.level_cnt, b.counters, b.max_nodes, b.prefix, b.node_link,
+                     b.node_end, b.level_off, c->flags);
+  // 7. centre of mass, wave ranges
   const int cgrid = (int)std::max<int64_t>(1, std::min<int64_t>((b.max_nodes + 255) / 256, 8192));
   const int cubic = (c->cfg.flags & NB_F_BH_AXIS_BOX) ? 0 : 1;
-  hipLaunchKernelGGL(k_tree_com, dim3(cgrid), dim3(256), 0, s, b.node_link, n, b.max_nodes,
-                     b.level_off, b.prefix, b.pms, codes_sorted, b.geom, cubic, c->cfg.theta,
-                     b.node_com, b.node_r2);
+  hipLaunchKernelGGL(k_tree_com, dim3(cgrid), dim3(256), 0, s, b.node_link, b.node_end, n,
+                     b.max_nodes, b.level_off, b.prefix, b.pms, codes_sorted, b.geom, cubic,
+                     c->cfg.theta, leaf, pairs, b.waves, b.counters, b.node_com, b.node_r2);
   return hipGetLastError();
 }
 

@@ -77,11 +77,10 @@ constexpr int kBboxBlocks = 1024;                     // bbox partial blocks
 constexpr int kSortThreads = 256;                     // 4 waves
 constexpr int kSortItems = 8;                         // keys per lane per radix pass
 constexpr int kSortTile = kSortThreads * kSortItems;  // 2048 keys per block
-constexpr int kScanTile = 2048;                       // elements per block in the scans
+constexpr int kScanTile = 2048;                       // elements per block in the int scan
+constexpr int kTreeTile = 1024;                       // bodies per block in the tree build
 constexpr int kSpare = 4;                             // zero-mass bodies after the sorted bodies
-constexpr int kTopLevels = 4;                         // levels built from per-cell searches
-constexpr int kTopCells = 1 + 8 + 64 + 512 + 4096;    // cells of levels 0..kTopLevels
-constexpr int kTopEntries = kTopCells + kTopLevels + 1;  // plus an end sentinel per level
+constexpr int kLevels = kMaxLevel + 1;                // levels a node can have
 constexpr int kCostBuckets = 64;  // half-octaves of estimated record time
 // Whether the Barnes-Hut build pairs sibling ranges (and the traversal orders
 // its work): by size unless a flag forces it either way.
@@ -92,8 +91,8 @@ inline bool nb_bh_pairs(int64_t n, int flags) {
 
 enum nb_bh_buf {
   kBhBbox, kBhGeom, kBhKey0, kBhKey1, kBhVal0, kBhVal1, kBhCodes, kBhHist, kBhIscan,
-  kBhPms, kBhPrefix, kBhScanPart, kBhCom, kBhR2, kBhLink, kBhLevel, kBhChildCnt,
-  kBhChildOff, kBhChildBounds, kBhCounters, kBhTopStart, kBhWaves, kBhInter, kBhFlags,
+  kBhPms, kBhPrefix, kBhScanPart, kBhCom, kBhR2, kBhLink, kBhLevel, kBhMarks,
+  kBhNodeEnd, kBhLevelCnt, kBhCounters, kBhWaves, kBhInter, kBhFlags,
   kBhRecCost, kBhRecBucket, kBhRecOrder, kBhRecHist, kBhBufCount
 };
 
@@ -126,15 +125,15 @@ constexpr nb_bh_layout nb_bh_layout_for(int64_t n) {
   bytes[kBhIscan] = 4 * scan_parts;
   bytes[kBhPms] = 16 * (n + kSpare);
   bytes[kBhPrefix] = 32 * (n + 1);
-  bytes[kBhScanPart] = 32 * ((n + kScanTile - 1) / kScanTile + 2);
+  bytes[kBhScanPart] = 32 * ((n + kTreeTile - 1) / kTreeTile + 1);
   bytes[kBhCom] = 16 * bound;
   bytes[kBhR2] = 4 * bound;
   bytes[kBhLink] = 16 * bound;
   bytes[kBhLevel] = 4 * (kMaxLevel + 2);
-  bytes[kBhChildCnt] = bytes[kBhChildOff] = 4 * n;
-  bytes[kBhChildBounds] = 4 * 8 * n;
+  bytes[kBhMarks] = n;
+  bytes[kBhNodeEnd] = 4 * bound;
+  bytes[kBhLevelCnt] = 4 * kLevels * ((n + kTreeTile - 1) / kTreeTile);
   bytes[kBhCounters] = 4 * 16;
-  bytes[kBhTopStart] = 4 * kTopEntries;
   bytes[kBhWaves] = 16 * n;
   bytes[kBhInter] = 8 * 2;
   bytes[kBhFlags] = 4 * 4;
@@ -177,13 +176,12 @@ struct nb_bh_state {
   float* node_r2 = nullptr;     // squared opening radius (s / theta + |COM - cell centre|)^2
   int4* node_link = nullptr;    // (first_child, next, start, count << 4 | level)
   int* level_off = nullptr;     // [kMaxLevel + 2] node index where each level begins
-  int* child_cnt = nullptr;     // per node of the current level: non-empty children
-  int* child_off = nullptr;     // exclusive scan of child_cnt
-  int* child_bounds = nullptr;  // per node of the current level: its 7 inner child boundaries [8 n]
+  unsigned char* marks = nullptr;  // per sorted body: levels at which a node starts there
+  int* node_end = nullptr;      // end of each node's body range
+  int* level_cnt = nullptr;     // [kLevels][tiles] node starts per tile, then their exclusive scan
   int* iscan_part = nullptr;    // int scan block partials
-  int* counters = nullptr;      // [0] wave ranges, [1] traversal ticket
+  int* counters = nullptr;      // [0] wave ranges, [1] traversal ticket, [2 + l] nodes of level l
   int4* waves = nullptr;        // records of one or two sibling wave ranges (start, count, start, count)
-  int* top_start = nullptr;     // first sorted body of every cell of the top levels
   // traversal order: records by the device time their bodies took in the last pass
   float* rec_cost = nullptr;    // per body (original index): last pass's time of its record / its bodies
   int* rec_bucket = nullptr;    // per record: cost bucket of this pass

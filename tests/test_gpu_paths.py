@@ -1,0 +1,43 @@
+"""Kernel variants and dispatch rules at the sizes where they can go wrong: tile
+edges, remainders, the smallest and largest of a range."""
+import numpy as np
+import pytest
+
+from helpers import rel_err
+
+pytestmark = pytest.mark.gpu
+
+EPS2, DT = 40.0, 0.0035
+
+
+@pytest.mark.parametrize("n", [1, 33, 1023, 1024, 1025, 3073])
+@pytest.mark.parametrize("leaf", [1, 31, 64])
+def test_tree_build_at_tile_edges(nb, ora, n, leaf):
+    """The build marks bodies in tiles of 1024 with a window of leaf + 1 bodies
+    across their edges: topology bit-exact, with runs of equal codes in it."""
+    rng = np.random.default_rng(1000 * n + leaf)
+    pos = rng.normal(size=(n, 3)) * rng.choice([1.0, 0.01], size=(n, 1))
+    pos[n // 2:] = pos[: n - n // 2] if n % 2 else pos[n // 2:]  # coincident bodies
+    m = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    with nb.Simulation(n, EPS2, DT, solver=nb.SOLVER_BH, leaf_size=leaf) as sim:
+        sim.upload(pos, np.zeros_like(pos), m)
+        f = sim.forces()
+        codes, perm = sim.debug_morton()
+        nodes, _ = sim.debug_tree()
+    p4 = np.zeros((n, 4), np.float32)
+    p4[:, :3], p4[:, 3] = pos, m
+    mn, mx = ora.bbox(p4)
+    ccodes = ora.morton(p4, mn, mx, cubic=True)
+    cperm, srt = ora.sort_codes(ccodes)
+    tree = ora.build_tree(srt, leaf)
+    np.testing.assert_array_equal(codes, ccodes)
+    np.testing.assert_array_equal(perm, cperm)
+    for mine, theirs in (("first_child", "first_child"), ("next", "next"), ("body_start", "start"),
+                         ("body_count", "count"), ("level", "level")):
+        np.testing.assert_array_equal(nodes[mine], tree[theirs])
+    com = ora.tree_com(tree, p4[cperm])
+    fc, _ = ora.bh_forces_group(p4[cperm], cperm, mn, mx, tree, com, EPS2, group=nb.BH_WAVE_BODIES,
+                                codes_sorted=srt)
+    # FP32 sums of at most n terms in another order: n / 2 rounding steps at worst
+    scale = np.abs(fc[:, :3]).max() + 1e-30
+    assert np.abs(f[:, :3] - fc[:, :3]).max() <= max(n, 64) * 2.0 ** -24 * scale
