@@ -1476,6 +1476,185 @@ __global__ __launch_bounds__(64 * kListWaves, kCount ? 5 : kListBlocksPerCU) voi
   }
 }
 
+// ---- 8b. one workgroup per range ------------------------------------------------------
+// The walk of one range by kWaves waves: what k_traverse_list does with one wave,
+// for systems with fewer ranges than the chip has waves, whose pass lasts as long
+// as its slowest walk (a range of far-out bodies in a large cell opens most of the
+// tree). The waves share the stack: an iteration pops up to 8 * kWaves nodes,
+// eight per wave, and every wave lists what it accepts in its own list. Opened
+// children go back in wave and lane order, so the stack's content, the lists and
+// with them every sum are the same in each run. A wave's list is summed when any
+// wave's is full, at the same point for all, so that no wave waits at a barrier
+// for another's arithmetic.
+// Stack bound: its entries' levels never decrease from bottom to top (children
+// are pushed in the order of their parents), and nodes of level l are pushed only
+// when all entries of that level or deeper are popped in the same iteration, so at
+// most 64 * kWaves entries of each of the levels 1 to 10 are ever held, and a
+// level that has a deeper one above it has lost 8 * kWaves of them:
+// (9 * 56 + 64) * kWaves entries.
+constexpr int block_stack(int waves) { return (9 * 56 + 64) * waves; }
+constexpr int kBlockListCap = 256;  // source indices per wave
+// Waves per range by the system's size. Measured Barnes-Hut steps in us (Plummer
+// sphere / uniform ball, leaf size 8), one, two, four and eight waves per range:
+//     4,000 bodies  333/269  243/204  198/164  169/140
+//    20,000         448/294  337/234  253/196  212/180
+//    65,536         404/342  339/279  330/267  333/272
+//   131,072         494/399  440/354  456/371  483/395
+//   262,144         662/522  661/534  742/596  812/647
+// Sixteen were 3% faster than eight at 4,000 bodies and 27% slower at 20,000; four
+// would be the best in a narrow band, by 3%. From 262,144 bodies on there are
+// enough ranges for every wave and the barriers only cost.
+constexpr int kBlock8Bodies = 5 << 14;    // below: eight waves per range
+constexpr int kBlockMaxBodies = 1 << 18;  // below: two; from here on k_traverse_list
+constexpr int kBlockWavesPerCU = 24;      // by LDS and 80 VGPRs, as k_traverse_list
+
+template <bool kGuard, int kWaves>
+__global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_block(
+    const float4* __restrict__ pms, const uint32_t* __restrict__ perm, int n,
+    const float4* __restrict__ com, const int4* __restrict__ link,
+    const int* __restrict__ level_off, int64_t max_nodes, const float* __restrict__ r2,
+    float eps2, double G, double* __restrict__ force, int* __restrict__ flags,
+    const int4* __restrict__ waves, int* __restrict__ wctl, const int* __restrict__ order,
+    float* __restrict__ cost, int stack_cap) {
+  __shared__ int2 stack[block_stack(kWaves)];
+  __shared__ uint32_t s_list[kWaves][kBlockListCap];
+  __shared__ float4 s_stage[kWaves][64];
+  __shared__ int2 s_cnt[kWaves];  // (opened children, list length) of each wave
+  __shared__ int s_lvl[kMaxLevel + 2];
+  __shared__ int s_rec;
+  static_assert(sizeof(s_stage[0]) >= 3 * kWaveBodies * sizeof(double), "a wave's sums fit its stage");
+  if (threadIdx.x < kMaxLevel + 2)
+    s_lvl[threadIdx.x] = (int)min((int64_t)level_off[threadIdx.x], max_nodes);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint64_t lt = (uint64_t(1) << lane) - 1;
+  uint32_t* list = s_list[wave];
+  float4* stage = s_stage[wave];
+  const int cap = stack_cap > 0 && stack_cap < block_stack(kWaves) ? stack_cap : block_stack(kWaves);
+  const int nrec = min(wctl[0], n);
+  unsigned long long unused = 0;
+  for (;;) {
+    if (threadIdx.x == 0) s_rec = atomicAdd(&wctl[1], 1);
+    __syncthreads();
+    const int w = __builtin_amdgcn_readfirstlane(s_rec);
+    if (w >= nrec) break;
+    const uint64_t t_start = wall_clock64();
+    const int ri = order ? order[w] : w;
+    const int4 rec = waves[(unsigned)ri < (unsigned)nrec ? ri : w];
+    const int P = copy_lanes(rec.y);
+    const int log2S = 6 - (31 - __clz(P)), slice = lane / P, slot = lane & (P - 1);
+    const bool valid = slot < rec.y;
+    const int t = min(rec.x + (valid ? slot : 0), n - 1);  // lanes past the range copy its first body
+    const float4 me = pms[t];
+    Box A, B;
+    lane_boxes(me, 0, 0, 0, A, B);
+    float ax = 0.f, ay = 0.f, az = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
+    int lc = 0, sp = 1;
+    auto flush = [&]() {
+      list_flush<false, kGuard>(list, lc, stage, lane, slice, log2S, pms, com, me, eps2, ax, ay, az,
+                                cx, cy, cz, unused);
+      lc = 0;
+    };
+    // a virtual parent whose only child is the root
+    if (threadIdx.x == 0) stack[0] = make_int2(0, (int)((1u << 27) | (uint32_t)n));
+    __syncthreads();
+    for (int iter = 0; sp > 0; ++iter) {  // sp is the same in every wave
+      if (iter > s_lvl[kMaxLevel + 1]) {  // every node is examined at most once
+        if (threadIdx.x == 0) atomicOr(flags, 4);
+        break;
+      }
+      const int k = min(sp, 8 * kWaves);
+      sp -= k;
+      const int q = 8 * wave + (lane >> 3), ci = lane & 7;
+      int child = -1;
+      int4 cl = make_int4(-1, -1, 0, 0);
+      float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
+      float rr = 0.f;
+      if (q < k) {  // entries and their candidates as in walk()
+        const int2 e = stack[sp + q];
+        const uint32_t ew = (uint32_t)e.y;
+        if (ci < (int)(ew >> 27)) {
+          const int cand = e.x + ci;
+          cl = link[cand];
+          c = com[cand];
+          rr = r2[cand];
+          if (cl.z < (int)(ew & ((1u << 27) - 1))) child = cand;
+        }
+      }
+      bool accept = false, leaf = false, open = false;
+      if (child >= 0) {
+        accept = rr < box_dist2(A, c);
+        leaf = !accept && cl.x < 0;
+        open = !accept && cl.x >= 0;
+      }
+      const bool acc = accept && c.w > 0.f;
+      const uint64_t ba = __ballot(acc);
+      if (acc) list[lc + __popcll(ba & lt)] = (uint32_t)child | kCellBit;
+      lc += __popcll(ba);
+      uint64_t bl = __ballot(leaf);
+      while (bl) {  // the bodies of leaves that are not accepted
+        const int src = __ffsll((unsigned long long)bl) - 1;
+        bl &= bl - 1;
+        const int ls = __builtin_amdgcn_readlane(cl.z, src);
+        const int lcount = __builtin_amdgcn_readlane(link_count(cl.w), src);
+        for (int off = 0; off < lcount; off += 64) {
+          const int m = min(64, lcount - off);
+          if (lc + 64 > kBlockListCap) flush();
+          if (lane < m) list[lc + lane] = (uint32_t)min(ls + off + lane, n - 1);
+          lc += m;
+        }
+      }
+      const uint64_t bo = __ballot(open);
+      if (lane == 0) s_cnt[wave] = make_int2(__popcll(bo), lc);
+      __syncthreads();  // counts are in, and every wave has read its entries
+      int before = 0, opened = 0, longest = 0;
+#pragma unroll
+      for (int v = 0; v < kWaves; ++v) {
+        const int2 o = s_cnt[v];
+        before += v < wave ? o.x : 0;
+        opened += o.x;
+        longest = max(longest, o.y);
+      }
+      opened = __builtin_amdgcn_readfirstlane(opened);
+      if (sp + opened > cap) {  // the same in every wave
+        if (threadIdx.x == 0) atomicOr(flags, 8);
+        break;
+      }
+      if (open) {
+        const uint32_t pend = (uint32_t)(cl.z + link_count(cl.w));
+        const int slots = max(0, min(8, s_lvl[link_level(cl.w) + 2] - cl.x));
+        stack[sp + before + __popcll(bo & lt)] = make_int2(cl.x, (int)(((uint32_t)slots << 27) | pend));
+      }
+      sp += opened;
+      // room for the next iteration's accepted cells (at most 64 per wave)
+      if (__builtin_amdgcn_readfirstlane(longest) + 64 > kBlockListCap) flush();
+      __syncthreads();
+    }
+    if (lc > 0) flush();
+    // each slice's compensated sum in FP64, the slices added (butterfly over the
+    // slice bits, fixed order), then the waves in order
+    double f[3] = {(double)ax + (double)cx, (double)ay + (double)cy, (double)az + (double)cz};
+    double* sums = reinterpret_cast<double*>(stage);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      for (int off = P; off < 64; off <<= 1) f[a] += __shfl_xor(f[a], off);
+      if (lane < P) sums[a * kWaveBodies + lane] = f[a];
+    }
+    __syncthreads();
+    const uint32_t o = perm[t];
+    if (wave == 0 && valid && lane < P && o < (uint32_t)n) {
+      for (int a = 0; a < 3; ++a) {
+        double all = f[a];
+        for (int v = 1; v < kWaves; ++v)
+          all += reinterpret_cast<const double*>(s_stage[v])[a * kWaveBodies + lane];
+        force[(int64_t)a * n + o] = G * all;
+      }
+      // the range's device time, shared out over its bodies for the next pass's order
+      if (cost) cost[o] = (float)(wall_clock64() - t_start) / (float)rec.y;
+    }
+  }
+}
+
 // ---- 8. traversal order ---------------------------------------------------------------
 // A persistent launch ends when its last wave finishes its last record, so the
 // records are taken costliest first: each record's estimate is the device time
@@ -1768,7 +1947,20 @@ hipError_t nb_bh_traverse(nb_ctx* c, bool count_interactions) {
   else if (group && count_interactions)
     hipLaunchKernelGGL((k_traverse_list<true, false>), dim3(gl), dim3(64 * kListWaves), 0, c->stream,
                        NB_LIST_ARGS);
-  else if (group && guard)
+  else if (group && n < kBlockMaxBodies && !nb_bh_pairs(n, c->cfg.flags)) {
+    const auto launch = [&](auto kernel, int waves) {
+      const int blocks = b.persist_blocks / kListBlocksPerCU * (kBlockWavesPerCU / waves);
+      hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * waves), 0, c->stream, b.pms, b.vals[0], n,
+                         b.node_com, b.node_link, b.level_off, b.max_nodes, b.node_r2, c->cfg.eps2,
+                         c->G, c->force, c->flags, b.waves, b.counters,
+                         ordered ? b.rec_order : nullptr, ordered ? b.rec_cost : nullptr,
+                         c->walk_stack);
+    };
+    if (n < kBlock8Bodies)
+      guard ? launch(k_traverse_block<true, 8>, 8) : launch(k_traverse_block<false, 8>, 8);
+    else
+      guard ? launch(k_traverse_block<true, 2>, 2) : launch(k_traverse_block<false, 2>, 2);
+  } else if (group && guard)
     hipLaunchKernelGGL((k_traverse_list<false, true>), dim3(gl), dim3(64 * kListWaves), 0, c->stream,
                        NB_LIST_ARGS);
   else if (group)

@@ -41,3 +41,24 @@ def test_tree_build_at_tile_edges(nb, ora, n, leaf):
     # FP32 sums of at most n terms in another order: n / 2 rounding steps at worst
     scale = np.abs(fc[:, :3]).max() + 1e-30
     assert np.abs(f[:, :3] - fc[:, :3]).max() <= max(n, 64) * 2.0 ** -24 * scale
+
+
+@pytest.mark.parametrize("n, leaf, eps2", [(3, 8, EPS2), (300, 64, EPS2), (5001, 1, 0.0), (20011, 64, EPS2),
+                                           (81919, 8, EPS2), (81920, 8, 0.0), (262143, 8, EPS2)])
+def test_workgroup_walk_equals_pair_walk(nb, n, leaf, eps2):
+    """Eight, then two waves per range, against the walk that one wave does for a
+    pair of ranges: the same interactions, summed in another order. A level-10
+    cell with more bodies than a wave's list holds is among them."""
+    pos, _, m = nb.ic_plummer(77 + n, n, 50.0, 1e4)
+    pos[: min(n // 2, 700)] = pos[0]
+    f = []
+    for flags in (0, nb.F_BH_PAIRS):
+        with nb.Simulation(n, eps2, DT, solver=nb.SOLVER_BH, leaf_size=leaf, flags=flags) as sim:
+            sim.upload(pos, np.zeros_like(pos), m)
+            f.append(sim.forces())
+            again = sim.forces()
+        np.testing.assert_array_equal(f[-1], again)
+    # FP32 partial sums of at most 192 terms, folded with compensation
+    assert np.percentile(rel_err(f[0], f[1]), 99) < 1e-5
+    scale = np.linalg.norm(f[1][:, :3], axis=1).max()
+    assert np.abs(f[0] - f[1]).max() <= 192 * 2.0 ** -24 * scale
