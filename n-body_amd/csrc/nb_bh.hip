@@ -10,13 +10,13 @@
 //
 // Pipeline per force pass (all on one stream, no host synchronisation, so the
 // whole step can be captured into a hipGraph):
-//   1. bbox        per-block min/max, then one block folds the partials and
-//                  writes the root box and the cell side^2 of each level.
+//   1. bbox        per-block min/max; every block of the next kernel folds them.
 //   2. encode      30-bit Morton code per body (bit-exact restatement of
 //                  morton.glsl: IEEE divide, clamp, 10-bit quantisation).
 //   3. sort        LSD radix sort of (code, body index), 4 passes of 8 bits.
-//                  Each pass: block digit histograms, a device-wide exclusive
-//                  scan, and a stable scatter whose per-wave ranks come from
+//                  Each pass: block digit histograms (the first one in 2.) and
+//                  a stable scatter, whose blocks add up the counts before
+//                  theirs themselves and whose per-wave ranks come from
 //                  64-bit ballots (8 ballots give each lane the mask of lanes
 //                  holding the same digit). Stable => sorted by (code, index).
 //   4. mark        gather (x, y, z, m) into sorted order; per body the levels at
@@ -46,9 +46,7 @@
 
 namespace {
 
-// Block and tile sizes shared with the buffer layout are in nb_internal.h. Sort
-// tiles of 2048 keys (8 per lane) measured 40 us faster per 4M-body sort than
-// 4096 (more tiles in flight) and than 1024 (larger histograms).
+// Block and tile sizes shared with the buffer layout are in nb_internal.h.
 constexpr int kScanThreads = 256;
 constexpr int kScanWaves = kScanThreads / 64;
 // Traversal groups: each wave of the traversal takes one "wave range" of at
@@ -118,70 +116,57 @@ __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int& total) {
 }
 
 // ---- 1. bounding box --------------------------------------------------------
-__global__ __launch_bounds__(256) void k_bbox_partial(const float4* __restrict__ pm, int n,
-                                                      float* __restrict__ part) {
+// Minimum and maximum per axis over a workgroup's threads; every thread gets them.
+// red: 6 floats of LDS per wave.
+template <int kWaves>
+__device__ __forceinline__ void block_bounds(float (&mn)[3], float (&mx)[3], float (*red)[6]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      mn[a] = fminf(mn[a], __shfl_xor(mn[a], off));
+      mx[a] = fmaxf(mx[a], __shfl_xor(mx[a], off));
+    }
+  if (lane == 0)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      red[wave][a] = mn[a];
+      red[wave][3 + a] = mx[a];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      mn[a] = fminf(mn[a], red[w][a]);
+      mx[a] = fmaxf(mx[a], red[w][3 + a]);
+    }
+}
+
+// Partial bounds per block, folded by every block of k_morton. Also clears the
+// radix passes' group counts.
+__global__ __launch_bounds__(1024) void k_bbox_partial(const float4* __restrict__ pm, int n,
+                                                       float* __restrict__ part,
+                                                       int* __restrict__ group_hist, int counts) {
+  __shared__ float red[16][6];
+  const int step = gridDim.x * 1024;
   float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX};
   float mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+  for (int i = blockIdx.x * 1024 + threadIdx.x; i < counts; i += step) group_hist[i] = 0;
+#pragma unroll 4
+  for (int i = blockIdx.x * 1024 + threadIdx.x; i < n; i += step) {
     const float4 p = pm[i];
     mn[0] = fminf(mn[0], p.x); mx[0] = fmaxf(mx[0], p.x);
     mn[1] = fminf(mn[1], p.y); mx[1] = fmaxf(mx[1], p.y);
     mn[2] = fminf(mn[2], p.z); mx[2] = fmaxf(mx[2], p.z);
   }
-  __shared__ float red[6][256];
-  for (int a = 0; a < 3; ++a) {
-    red[a][threadIdx.x] = mn[a];
-    red[3 + a][threadIdx.x] = mx[a];
-  }
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s)
-      for (int a = 0; a < 3; ++a) {
-        red[a][threadIdx.x] = fminf(red[a][threadIdx.x], red[a][threadIdx.x + s]);
-        red[3 + a][threadIdx.x] = fmaxf(red[3 + a][threadIdx.x], red[3 + a][threadIdx.x + s]);
-      }
-    __syncthreads();
-  }
-  if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
-}
-
-__global__ __launch_bounds__(256) void k_bbox_final(const float* __restrict__ part, int nparts,
-                                                    float* __restrict__ geom) {
-  float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX};
-  float mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-  for (int b = threadIdx.x; b < nparts; b += 256)
+  block_bounds<16>(mn, mx, red);
+  if (threadIdx.x == 0)
     for (int a = 0; a < 3; ++a) {
-      mn[a] = fminf(mn[a], part[6 * b + a]);
-      mx[a] = fmaxf(mx[a], part[6 * b + 3 + a]);
+      part[6 * blockIdx.x + a] = mn[a];
+      part[6 * blockIdx.x + 3 + a] = mx[a];
     }
-  __shared__ float red[6][256];
-  for (int a = 0; a < 3; ++a) {
-    red[a][threadIdx.x] = mn[a];
-    red[3 + a][threadIdx.x] = mx[a];
-  }
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s)
-      for (int a = 0; a < 3; ++a) {
-        red[a][threadIdx.x] = fminf(red[a][threadIdx.x], red[a][threadIdx.x + s]);
-        red[3 + a][threadIdx.x] = fmaxf(red[3 + a][threadIdx.x], red[3 + a][threadIdx.x + s]);
-      }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    float side = 0.f;
-    for (int a = 0; a < 3; ++a) {
-      geom[a] = red[a][0];
-      geom[3 + a] = red[3 + a][0];
-      const float ext = fmaxf(__fsub_rn(red[3 + a][0], red[a][0]), 1e-6f);
-      side = fmaxf(side, ext);
-    }
-    for (int l = 0; l <= kMaxLevel; ++l) {
-      const float s = ldexpf(side, -l);
-      geom[6 + l] = __fmul_rn(s, s);
-    }
-    geom[6 + kMaxLevel + 1] = side;  // cubic root extent
-  }
 }
 
 // ---- 2. Morton encode (morton.glsl:37-98) ------------------------------------
@@ -212,105 +197,71 @@ __device__ __forceinline__ uint32_t quantize(float p, float lo, float ext) {
   return (uint32_t)g;
 }
 
+// Digit counts of one tile (kSortTile keys, 1024 threads) from the LDS histogram
+// h: to the tile's row and, added up, to its group's.
+__device__ __forceinline__ void publish_counts(const int* h, int* __restrict__ hist,
+                                               int* __restrict__ group_hist) {
+  if (threadIdx.x < 256) {
+    const int c = h[threadIdx.x];
+    hist[blockIdx.x * 256 + threadIdx.x] = c;
+    if (c) atomicAdd(&group_hist[blockIdx.x / kSortGroup * 256 + threadIdx.x], c);
+  }
+}
+
+// Codes, and the digit counts of the first radix pass. Every block folds the
+// partial bounds itself (6 KB of L2 reads), which spares a launch of one block.
 // cubic = 1: one extent E = max_a max(max_a - min_a, 1e-6) on every axis (a cubic
 // root cell, so every cell is a cube of side E / 2^level); cubic = 0: each axis
 // over its own extent max(max_a - min_a, 1e-6), exactly morton.glsl's inputs.
-__global__ __launch_bounds__(256) void k_morton(const float4* __restrict__ pm, int n, int cubic,
-                                                const float* __restrict__ geom,
-                                                uint32_t* __restrict__ codes,
-                                                uint32_t* __restrict__ keys,
-                                                uint32_t* __restrict__ vals) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const float4 p = pm[i];
-  const float E = geom[6 + kMaxLevel + 1];
-  const float ex = cubic ? E : fmaxf(__fsub_rn(geom[3], geom[0]), 1e-6f);
-  const float ey = cubic ? E : fmaxf(__fsub_rn(geom[4], geom[1]), 1e-6f);
-  const float ez = cubic ? E : fmaxf(__fsub_rn(geom[5], geom[2]), 1e-6f);
-  const uint32_t qx = quantize(p.x, geom[0], ex);
-  const uint32_t qy = quantize(p.y, geom[1], ey);
-  const uint32_t qz = quantize(p.z, geom[2], ez);
-  const uint32_t code = expand_bits(qx) * 4u + expand_bits(qy) * 2u + expand_bits(qz);
-  codes[i] = code;
-  keys[i] = code;
-  vals[i] = (uint32_t)i;
-}
-
-// ---- exclusive int scan -------------------------------------------------------
-// Pass 1: the sum of every kScanTile-element tile.
-__global__ __launch_bounds__(kScanThreads) void k_iscan_reduce(const int* __restrict__ in, int n,
-                                                               int* __restrict__ part) {
-  const int base = blockIdx.x * kScanTile;
-  int s = 0;
-  for (int k = threadIdx.x; k < kScanTile; k += kScanThreads) {
-    const int e = base + k;
-    if (e < n) s += in[e];
-  }
-  __shared__ int wsum[kScanWaves];
-  int tile = 0;
-  (void)block_excl_scan(s, wsum, tile);
-  if (threadIdx.x == 0) part[blockIdx.x] = tile;
-}
-
-// Pass 2: every tile adds up the tile sums before it (a few KB of L2 reads per
-// tile, which replaces a separate one-block scan of the sums and its launch),
-// then rescans its own elements from there (8 consecutive elements per thread,
-// one block scan of the thread sums).
-__global__ __launch_bounds__(kScanThreads) void k_iscan_final(const int* __restrict__ in, int n,
-                                                              const int* __restrict__ part,
-                                                              int* __restrict__ out) {
-  const int base = blockIdx.x * kScanTile;
-  __shared__ int wsum[kScanWaves];
-  int pre = 0;
-  for (int b = threadIdx.x; b < (int)blockIdx.x; b += kScanThreads) pre += part[b];
-  int start = 0;
-  (void)block_excl_scan(pre, wsum, start);
-  constexpr int kPer = kScanTile / kScanThreads;  // 8 consecutive elements per thread
-  int v[kPer];
-  int s = 0;
+__global__ __launch_bounds__(1024) void k_morton(const float4* __restrict__ pm, int n, int cubic,
+                                                 const float* __restrict__ part, int nparts,
+                                                 float* __restrict__ geom,
+                                                 uint32_t* __restrict__ codes,
+                                                 int* __restrict__ hist,
+                                                 int* __restrict__ group_hist) {
+  __shared__ float red[16][6];
+  __shared__ int h[256];
+  if (threadIdx.x < 256) h[threadIdx.x] = 0;
+  float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX};
+  float mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+  if ((int)threadIdx.x < nparts)  // nparts <= kBboxBlocks
+    for (int a = 0; a < 3; ++a) {
+      mn[a] = part[6 * threadIdx.x + a];
+      mx[a] = part[6 * threadIdx.x + 3 + a];
+    }
+  block_bounds<16>(mn, mx, red);  // ends behind a barrier: h is clear
+  float ext[3], E = 0.f;
 #pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const int e = base + threadIdx.x * kPer + k;
-    v[k] = e < n ? in[e] : 0;
-    s += v[k];
+  for (int a = 0; a < 3; ++a) {
+    ext[a] = fmaxf(__fsub_rn(mx[a], mn[a]), 1e-6f);
+    E = fmaxf(E, ext[a]);
   }
-  int total = 0;
-  int run = start + block_excl_scan(s, wsum, total);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    for (int a = 0; a < 3; ++a) {
+      geom[a] = mn[a];
+      geom[3 + a] = mx[a];
+    }
+    for (int l = 0; l <= kMaxLevel; ++l) {
+      const float s = ldexpf(E, -l);
+      geom[6 + l] = __fmul_rn(s, s);
+    }
+    geom[6 + kMaxLevel + 1] = E;  // cubic root extent
+  }
 #pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const int e = base + threadIdx.x * kPer + k;
-    if (e < n) out[e] = run;
-    run += v[k];
+  for (int r = 0; r < kSortTile / 1024; ++r) {
+    const int i = blockIdx.x * kSortTile + r * 1024 + threadIdx.x;
+    if (i < n) {
+      const float4 p = pm[i];
+      const uint32_t qx = quantize(p.x, mn[0], cubic ? E : ext[0]);
+      const uint32_t qy = quantize(p.y, mn[1], cubic ? E : ext[1]);
+      const uint32_t qz = quantize(p.z, mn[2], cubic ? E : ext[2]);
+      const uint32_t code = expand_bits(qx) * 4u + expand_bits(qy) * 2u + expand_bits(qz);
+      codes[i] = code;
+      atomicAdd(&h[code & 255u], 1);
+    }
   }
-}
-
-// Exclusive scan of at most kSingleScan elements by one workgroup (8 consecutive
-// elements per thread), for the small scans: one launch instead of two.
-constexpr int kSingleScan = 8192;
-__global__ __launch_bounds__(1024) void k_iscan_single(const int* __restrict__ in, int n,
-                                                       int* __restrict__ out) {
-  constexpr int kPer = kSingleScan / 1024;
-  const int base = threadIdx.x * kPer;
-  int v[kPer];
-  int sum = 0;
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    v[k] = base + k < n ? in[base + k] : 0;
-    sum += v[k];
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int incl = wave_incl_scan(sum);
-  __shared__ int wsum[16];
-  if (lane == 63) wsum[wave] = incl;
   __syncthreads();
-  int before = 0;
-  for (int w = 0; w < wave; ++w) before += wsum[w];
-  int run = before + incl - sum;
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    if (base + k < n) out[base + k] = run;
-    run += v[k];
-  }
+  publish_counts(h, hist, group_hist);
 }
 
 // FP64 prefix of (m, m x, m y, m z): prefix[k] = sum over sorted bodies < k.
@@ -332,20 +283,19 @@ __device__ __forceinline__ double4 wave_incl_scan4(double4 v) {
 }
 
 // ---- 3. radix sort ------------------------------------------------------------
-__global__ __launch_bounds__(kSortThreads) void k_radix_hist(const uint32_t* __restrict__ keys,
-                                                             int n, int shift, int nblocks,
-                                                             int* __restrict__ hist) {
+__global__ __launch_bounds__(1024) void k_radix_hist(const uint32_t* __restrict__ keys, int n,
+                                                     int shift, int* __restrict__ hist,
+                                                     int* __restrict__ group_hist) {
   __shared__ int h[256];
-  h[threadIdx.x] = 0;
+  if (threadIdx.x < 256) h[threadIdx.x] = 0;
   __syncthreads();
-  const int base = blockIdx.x * kSortTile;
-#pragma unroll 4
-  for (int r = 0; r < kSortItems; ++r) {
-    const int e = base + r * kSortThreads + threadIdx.x;
+#pragma unroll
+  for (int r = 0; r < kSortTile / 1024; ++r) {
+    const int e = blockIdx.x * kSortTile + r * 1024 + threadIdx.x;
     if (e < n) atomicAdd(&h[(keys[e] >> shift) & 255u], 1);
   }
   __syncthreads();
-  hist[threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
+  publish_counts(h, hist, group_hist);
 }
 
 // Mask of the active lanes whose 8-bit digit equals this lane's digit.
@@ -360,96 +310,128 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, uint64_t active) {
   return m;
 }
 
-// Stable scatter of one 8-bit digit pass. The tile is first reordered in LDS by
-// digit (stable ranks from per-wave ballots, waves and rounds in element
-// order), then written out in LDS order: consecutive threads write the runs of
-// equal digits to consecutive global addresses instead of 64 scattered lines
-// per wave store.
-__global__ __launch_bounds__(kSortThreads) void k_radix_scatter(
+// Stable scatter of one 8-bit digit pass. A tile's first output index of a digit
+// is the number of smaller digits anywhere plus the number of its own digit in
+// earlier tiles: each block adds these up itself from the groups' counts and the
+// counts of the tiles before it in its group (four threads per digit; at 2^22
+// keys 32 groups and at most 63 tiles), so a pass is two launches without a scan
+// between them. The tile is first reordered in LDS by digit (stable ranks from
+// per-wave ballots, waves and rounds in element order), then written out in LDS
+// order: consecutive threads write the runs of equal digits to consecutive global
+// addresses instead of 64 scattered lines per wave store. Two keys per thread: a
+// pass over a small system is a chain of latencies (65,536 keys, counts and scatter:
+// 27 us in four launches with eight keys per thread, 11 us now; 2^22 keys 56 and 53).
+// kFirst: the values are the indices themselves.
+template <bool kFirst>
+__global__ __launch_bounds__(1024) void k_radix_scatter(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, int n, int shift,
-    int nblocks, const int* __restrict__ offsets, uint32_t* __restrict__ keys_out,
-    uint32_t* __restrict__ vals_out) {
-  __shared__ int whist[4][256];
-  __shared__ int wrun[4][256];
-  __shared__ int local_start[256];  // first tile slot of each digit
-  __shared__ int global_start[256];  // first output index of each digit for this tile
+    const int* __restrict__ hist, const int* __restrict__ group_hist, int groups,
+    uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out) {
+  constexpr int kRounds = kSortTile / 1024;
+  __shared__ int whist[16][256];  // per wave: digit counts, then first tile slots
+  __shared__ int s_part[2][4][256];
+  __shared__ int s_to_global[256];  // a digit's first output index minus its first tile slot
   __shared__ uint32_t sk[kSortTile], sv[kSortTile];
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  for (int w = 0; w < 4; ++w) whist[w][threadIdx.x] = 0;
-  __syncthreads();
-
-  // Wave w owns tile elements [w*kSortTile/4, (w+1)*kSortTile/4), 64 consecutive per round.
-  const int tile0 = blockIdx.x * kSortTile;
-  const int base = tile0 + wave * (kSortTile / 4);
+  __shared__ int wsum[2][4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint64_t lt = (uint64_t(1) << lane) - 1;
-  // The rounds read their keys again in phase 2 (coalesced, 4 B per key)
-  // instead of holding 16 keys and values per lane: the kernel then needs a few
-  // dozen VGPRs instead of hundreds, and many waves per SIMD hide the latency.
-  // phase 1: per-wave digit counts
-#pragma unroll 1
-  for (int r = 0; r < kSortItems; ++r) {
-    const int e = base + r * 64 + lane;
-    const uint64_t active = __ballot(e < n);
-    const uint32_t d = ((e < n ? keys_in[e] : 0u) >> shift) & 255u;
-    const uint64_t m = match_digit(d, active);
-    if (e < n && (m & lt) == 0) whist[wave][d] += __popcll(m);
+  const int tile0 = blockIdx.x * kSortTile;
+  // Wave w owns the tile elements [w * kSortTile / 16, (w + 1) * kSortTile / 16)
+  const int base = tile0 + wave * (kSortTile / 16) + lane;
+  uint32_t key[kRounds], val[kRounds];
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int e = base + 64 * r;
+    key[r] = e < n ? keys_in[e] : 0u;
+    val[r] = kFirst ? (uint32_t)e : e < n ? vals_in[e] : 0u;
   }
-  __syncthreads();
   {
-    // tile-local digit starts: exclusive scan of the tile's digit counts
+    const int d = threadIdx.x & 255, q = threadIdx.x >> 8;
+    const int mine = blockIdx.x / kSortGroup;
+    int total = 0, before = 0;
+    for (int g = q; g < groups; g += 4) {
+      const int c = group_hist[g * 256 + d];
+      total += c;
+      before += g < mine ? c : 0;
+    }
+    for (int t = mine * kSortGroup + q; t < (int)blockIdx.x; t += 4) before += hist[t * 256 + d];
+    s_part[0][q][d] = total;
+    s_part[1][q][d] = before;
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) whist[wave][64 * k + lane] = 0;  // the wave's own row
+  __builtin_amdgcn_wave_barrier();
+  int rank[kRounds];
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const bool in = base + 64 * r < n;
+    const uint32_t d = (key[r] >> shift) & 255u;
+    const uint64_t m = match_digit(d, __ballot(in));
+    rank[r] = whist[wave][d] + __popcll(m & lt);
+    __builtin_amdgcn_wave_barrier();
+    if (in && (m & lt) == 0) whist[wave][d] += __popcll(m);
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  int cnt = 0, total = 0, before = 0, incl_c = 0, incl_t = 0;
+  if (threadIdx.x < 256) {
     const int d = threadIdx.x;
-    const int cnt = whist[0][d] + whist[1][d] + whist[2][d] + whist[3][d];
-    const int incl = wave_incl_scan(cnt);
-    __shared__ int wsum[4];
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    int start = incl - cnt;
-    for (int w = 0; w < wave; ++w) start += wsum[w];
-    local_start[d] = start;
-    global_start[d] = offsets[d * nblocks + blockIdx.x];
-    int run = start;
-    for (int w = 0; w < 4; ++w) {
-      wrun[w][d] = run;
-      run += whist[w][d];
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      const int c = whist[w][d];
+      whist[w][d] = cnt;
+      cnt += c;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      total += s_part[0][q][d];
+      before += s_part[1][q][d];
+    }
+    incl_c = wave_incl_scan(cnt);
+    incl_t = wave_incl_scan(total);
+    if (lane == 63) {
+      wsum[0][wave] = incl_c;
+      wsum[1][wave] = incl_t;
     }
   }
   __syncthreads();
-  // phase 2: stable tile-local ranks, reorder in LDS
-#pragma unroll 1
-  for (int r = 0; r < kSortItems; ++r) {
-    const int e = base + r * 64 + lane;
-    const uint64_t active = __ballot(e < n);
-    const uint32_t key = e < n ? keys_in[e] : 0u;
-    const uint32_t val = e < n ? vals_in[e] : 0u;
-    const uint32_t d = (key >> shift) & 255u;
-    const uint64_t m = match_digit(d, active);
-    if (e < n) {
-      const int slot = wrun[wave][d] + __popcll(m & lt);
-      if (slot >= 0 && slot < kSortTile) {  // always true for a consistent histogram
-        sk[slot] = key;
-        sv[slot] = val;
-      }
+  if (threadIdx.x < 256) {
+    const int d = threadIdx.x;
+    int local = incl_c - cnt, global = incl_t - total + before;
+    for (int w = 0; w < wave; ++w) {
+      local += wsum[0][w];
+      global += wsum[1][w];
     }
-    __builtin_amdgcn_wave_barrier();
-    if (e < n && (m & lt) == 0) wrun[wave][d] += __popcll(m);
-    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int w = 0; w < 16; ++w) whist[w][d] += local;
+    s_to_global[d] = global - local;
   }
   __syncthreads();
-  // phase 3: write out in tile order
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int slot = whist[wave][(key[r] >> shift) & 255u] + rank[r];
+    if (base + 64 * r < n && slot >= 0 && slot < kSortTile) {  // always, for consistent counts
+      sk[slot] = key[r];
+      sv[slot] = val[r];
+    }
+  }
+  __syncthreads();
   const int count = min(kSortTile, n - tile0);
-#pragma unroll 4
-  for (int i = threadIdx.x; i < count; i += kSortThreads) {
-    const uint32_t key = sk[i];
-    const uint32_t d = (key >> shift) & 255u;
-    const int dst = global_start[d] + (i - local_start[d]);
-    if (dst >= 0 && dst < n) {
-      keys_out[dst] = key;
-      vals_out[dst] = sv[i];
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int i = r * 1024 + threadIdx.x;
+    if (i < count) {
+      const uint32_t k = sk[i];
+      const int dst = i + s_to_global[(k >> shift) & 255u];
+      if (dst >= 0 && dst < n) {
+        keys_out[dst] = k;
+        vals_out[dst] = sv[i];
+      }
     }
   }
 }
 
+// ---- 4. bodies in sorted order ------------------------------------------------
 // Morton reordering of the resident state: dst[k] = src[perm[k]] per component.
 __global__ __launch_bounds__(256) void k_permute_d3(const double* __restrict__ src,
                                                     const uint32_t* __restrict__ perm, int n,
@@ -1747,18 +1729,6 @@ __global__ void k_zero_u64(unsigned long long* p) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *p = 0ull;
 }
 
-// Enqueue an exclusive int scan: out[0..n) from in.
-hipError_t iscan(const int* in, int* out, int* part, int n, hipStream_t s) {
-  if (n <= kSingleScan) {
-    hipLaunchKernelGGL(k_iscan_single, dim3(1), dim3(1024), 0, s, in, n, out);
-    return hipGetLastError();
-  }
-  const int blocks = (n + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL(k_iscan_reduce, dim3(blocks), dim3(kScanThreads), 0, s, in, n, part);
-  hipLaunchKernelGGL(k_iscan_final, dim3(blocks), dim3(kScanThreads), 0, s, in, n, part, out);
-  return hipGetLastError();
-}
-
 }  // namespace
 
 void nb_bh_carve(nb_ctx* c, char* base, int upto) {
@@ -1773,7 +1743,7 @@ void nb_bh_carve(nb_ctx* c, char* base, int upto) {
   b.vals[1] = (uint32_t*)at(kBhVal1);
   b.codes = (uint32_t*)at(kBhCodes);
   b.digit_hist = (int*)at(kBhHist);
-  b.iscan_part = (int*)at(kBhIscan);
+  b.group_hist = (int*)at(kBhGroupHist);
   b.pms = (float4*)at(kBhPms);
   b.prefix = (double4*)at(kBhPrefix);
   b.scan_part = (double4*)at(kBhScanPart);
@@ -1844,26 +1814,26 @@ hipError_t nb_morton_sort(nb_ctx* c) {
   nb_bh_state& b = c->bh;
   const int n = c->n;
   hipStream_t s = c->stream;
-  const int g256 = (n + 255) / 256;
+  const int tiles = b.sort_blocks, groups = (tiles + kSortGroup - 1) / kSortGroup;
   // 1. bbox
-  hipLaunchKernelGGL(k_bbox_partial, dim3(b.bbox_blocks), dim3(256), 0, s, c->pm, n, b.bbox_part);
-  hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(256), 0, s, b.bbox_part, b.bbox_blocks, b.geom);
+  const int parts = std::min(b.bbox_blocks, (n + 1023) / 1024);
+  hipLaunchKernelGGL(k_bbox_partial, dim3(parts), dim3(1024), 0, s, c->pm, n, b.bbox_part,
+                     b.group_hist, 4 * 256 * groups);
   // 2. encode
   const int cubic = (c->cfg.flags & NB_F_BH_AXIS_BOX) ? 0 : 1;
-  hipLaunchKernelGGL(k_morton, dim3(g256), dim3(256), 0, s, c->pm, n, cubic, b.geom, b.codes, b.keys[0],
-                     b.vals[0]);
-  // 3. sort: 4 passes of 8 bits, ping-pong 0 -> 1 -> 0 -> 1 -> 0
-  const int nb = b.sort_blocks;
-  const int hist = 256 * nb;
-  int* offs = b.digit_hist + hist;
-  for (int pass = 0; pass < 4; ++pass) {
+  hipLaunchKernelGGL(k_morton, dim3(tiles), dim3(1024), 0, s, c->pm, n, cubic, b.bbox_part, parts,
+                     b.geom, b.codes, b.digit_hist, b.group_hist);
+  // 3. sort: 4 passes of 8 bits, codes -> 1 -> 0 -> 1 -> 0
+  hipLaunchKernelGGL((k_radix_scatter<true>), dim3(tiles), dim3(1024), 0, s, b.codes, nullptr, n, 0,
+                     b.digit_hist, b.group_hist, groups, b.keys[1], b.vals[1]);
+  for (int pass = 1; pass < 4; ++pass) {
     const int in = pass & 1, out = in ^ 1;
-    hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(kSortThreads), 0, s, b.keys[in], n, 8 * pass,
-                       nb, b.digit_hist);
-    hipError_t e = iscan(b.digit_hist, offs, b.iscan_part, hist, s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(kSortThreads), 0, s, b.keys[in],
-                       b.vals[in], n, 8 * pass, nb, offs, b.keys[out], b.vals[out]);
+    int* gh = b.group_hist + pass * groups * 256;
+    hipLaunchKernelGGL(k_radix_hist, dim3(tiles), dim3(1024), 0, s, b.keys[in], n, 8 * pass,
+                       b.digit_hist, gh);
+    hipLaunchKernelGGL((k_radix_scatter<false>), dim3(tiles), dim3(1024), 0, s, b.keys[in],
+                       b.vals[in], n, 8 * pass, b.digit_hist, gh, groups, b.keys[out],
+                       b.vals[out]);
   }
   b.sorted_buf = 0;
   return hipGetLastError();

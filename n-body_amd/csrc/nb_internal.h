@@ -73,11 +73,9 @@ constexpr int kMaxLevel = 10;
 // same layout out of a static device array. The Morton-sort buffers come first,
 // so a direct-sum context that only reorders (nb_sort_alloc) allocates the
 // prefix [0, off[kBhPms]).
-constexpr int kBboxBlocks = 1024;                     // bbox partial blocks
-constexpr int kSortThreads = 256;                     // 4 waves
-constexpr int kSortItems = 8;                         // keys per lane per radix pass
-constexpr int kSortTile = kSortThreads * kSortItems;  // 2048 keys per block
-constexpr int kScanTile = 2048;                       // elements per block in the int scan
+constexpr int kBboxBlocks = 256;                      // bbox partial blocks
+constexpr int kSortTile = 2048;                       // keys per block in the radix passes
+constexpr int kSortGroup = 64;                        // tiles whose digit counts are also added up
 constexpr int kTreeTile = 1024;                       // bodies per block in the tree build
 constexpr int kSpare = 4;                             // zero-mass bodies after the sorted bodies
 constexpr int kLevels = kMaxLevel + 1;                // levels a node can have
@@ -90,7 +88,7 @@ inline bool nb_bh_pairs(int64_t n, int flags) {
 }
 
 enum nb_bh_buf {
-  kBhBbox, kBhGeom, kBhKey0, kBhKey1, kBhVal0, kBhVal1, kBhCodes, kBhHist, kBhIscan,
+  kBhBbox, kBhGeom, kBhKey0, kBhKey1, kBhVal0, kBhVal1, kBhCodes, kBhHist, kBhGroupHist,
   kBhPms, kBhPrefix, kBhScanPart, kBhCom, kBhR2, kBhLink, kBhLevel, kBhMarks,
   kBhNodeEnd, kBhLevelCnt, kBhCounters, kBhWaves, kBhInter, kBhFlags,
   kBhRecCost, kBhRecBucket, kBhRecOrder, kBhRecHist, kBhBufCount
@@ -114,15 +112,14 @@ struct nb_bh_layout {
 constexpr nb_bh_layout nb_bh_layout_for(int64_t n) {
   nb_bh_layout L{};
   const int64_t sort_blocks = (n + kSortTile - 1) / kSortTile;
-  const int64_t hist = 256 * sort_blocks;
-  const int64_t scan_parts = ((hist > n ? hist : n) + kScanTile - 1) / kScanTile + 2;
+  const int64_t groups = (sort_blocks + kSortGroup - 1) / kSortGroup;
   const int64_t bound = nb_tree_bound(n);
   int64_t bytes[kBhBufCount] = {};
   bytes[kBhBbox] = 4 * 6 * kBboxBlocks;
   bytes[kBhGeom] = 4 * 32;
   bytes[kBhKey0] = bytes[kBhKey1] = bytes[kBhVal0] = bytes[kBhVal1] = bytes[kBhCodes] = 4 * n;
-  bytes[kBhHist] = 4 * 2 * hist;
-  bytes[kBhIscan] = 4 * scan_parts;
+  bytes[kBhHist] = 4 * 256 * sort_blocks;
+  bytes[kBhGroupHist] = 4 * 4 * 256 * groups;
   bytes[kBhPms] = 16 * (n + kSpare);
   bytes[kBhPrefix] = 32 * (n + 1);
   bytes[kBhScanPart] = 32 * ((n + kTreeTile - 1) / kTreeTile + 1);
@@ -165,7 +162,8 @@ struct nb_bh_state {
   uint32_t* keys[2] = {nullptr, nullptr};
   uint32_t* vals[2] = {nullptr, nullptr};
   uint32_t* codes = nullptr;    // unsorted codes (debug tap)
-  int* digit_hist = nullptr;       // radix: [256 * sort_blocks] counts, then offsets
+  int* digit_hist = nullptr;    // radix: [sort_blocks][256] digit counts of the current pass
+  int* group_hist = nullptr;    // radix: [4][groups][256] digit counts of each pass, kSortGroup tiles
   int sort_blocks = 0;
   int sorted_buf = 0;           // which of keys[]/vals[] holds the final order
   float4* pms = nullptr;        // bodies in sorted order (x, y, z, m)
@@ -179,7 +177,6 @@ struct nb_bh_state {
   unsigned char* marks = nullptr;  // per sorted body: levels at which a node starts there
   int* node_end = nullptr;      // end of each node's body range
   int* level_cnt = nullptr;     // [kLevels][tiles] node starts per tile, then their exclusive scan
-  int* iscan_part = nullptr;    // int scan block partials
   int* counters = nullptr;      // [0] wave ranges, [1] traversal ticket, [2 + l] nodes of level l
   int4* waves = nullptr;        // records of one or two sibling wave ranges (start, count, start, count)
   // traversal order: records by the device time their bodies took in the last pass

@@ -62,3 +62,21 @@ def test_workgroup_walk_equals_pair_walk(nb, n, leaf, eps2):
     assert np.percentile(rel_err(f[0], f[1]), 99) < 1e-5
     scale = np.linalg.norm(f[1][:, :3], axis=1).max()
     assert np.abs(f[0] - f[1]).max() <= 192 * 2.0 ** -24 * scale
+
+
+@pytest.mark.parametrize("n", [1, 63, 2047, 2049, 131071, 131073, 264193])
+def test_radix_sort_at_tile_and_group_edges(nb, ora, n):
+    """Tiles of 2048 keys in groups of 64: codes and the stable permutation."""
+    rng = np.random.default_rng(n)
+    pos = np.round(rng.normal(size=(n, 3)) * 8) if n % 4 == 1 else rng.normal(size=(n, 3))
+    m = np.ones(n, np.float32)
+    with nb.Simulation(n, EPS2, DT, solver=nb.SOLVER_BH) as sim:
+        sim.upload(pos, np.zeros_like(pos), m)
+        sim.forces()
+        codes, perm = sim.debug_morton()
+    p4 = np.zeros((n, 4), np.float32)
+    p4[:, :3], p4[:, 3] = pos, m
+    mn, mx = ora.bbox(p4)
+    ccodes = ora.morton(p4, mn, mx, cubic=True)
+    np.testing.assert_array_equal(codes, ccodes)
+    np.testing.assert_array_equal(perm, np.argsort(ccodes, kind="stable"))
