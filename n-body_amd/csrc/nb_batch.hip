@@ -85,7 +85,7 @@ __global__ __launch_bounds__(64 * K) void k_batch_force(
   const int nitems = counts[0];
   const int call_step = use_quota ? counts[4] : -1;
   __shared__ int s_item;
-  __shared__ float part[K][6][B][64];
+  __shared__ double part[K][3][B][64];
   for (;;) {
     if (threadIdx.x == 0) s_item = atomicAdd(&counts[2], 1);
     __syncthreads();
@@ -108,19 +108,11 @@ __global__ __launch_bounds__(64 * K) void k_batch_force(
       nbcore::accumulate<B, false>(pm, j0, j0 + jlen, eps2, t);
     else
       nbcore::accumulate<B, true>(pm, j0, j0 + jlen, eps2, t);
-    if constexpr (K > 1) nbcore::merge_waves<B, K>(part, wave, lane, t);
-    if (wave == 0) {
-      const double G = c_G[slot];
-#pragma unroll
-      for (int b = 0; b < B; ++b) {
-        const int i = ibase + 64 * b;
-        if (i - off < n) {
-          force[i] = G * ((double)t.sx[b] + (double)t.cx[b]);
-          force[cap + i] = G * ((double)t.sy[b] + (double)t.cy[b]);
-          force[2 * cap + i] = G * ((double)t.sz[b] + (double)t.cz[b]);
-        }
-      }
-    }
+    const double G = c_G[slot];
+    nbcore::merge_waves<B, K>(part, wave, lane, t, [&](int a, int b, double sum) {
+      const int i = ibase + 64 * b;
+      if (i - off < n) force[a * cap + i] = G * sum;
+    });
     if constexpr (K > 1) __syncthreads();  // LDS partials are reused by the next item
   }
 }

@@ -85,10 +85,10 @@ void to_caller_order(const nb_ctx* c, std::vector<T>& a, int comps) {
 
 }  // namespace
 
-// Built-in launch shapes, from a sweep on MI355X (Plummer spheres, force pass):
-// one body per lane; 16 waves per i-block up to 16384 bodies (4096 bodies:
-// 30 us against 83 us at 4 waves), 8 above (2^15: 0.41 ms against 0.61 ms;
-// 2^18: 19.8 ms against 20.2 ms).
+// Built-in launch shapes, from a sweep on MI355X (Plummer spheres, whole steps
+// with the best number of parts each): one body per lane; 16 waves per workgroup
+// up to 16384 bodies (4096 bodies: 16.6 us against 19.8 us at 8 waves), 8 above
+// (37,000 bodies: 379 us against 382 us at 16; 2^18: 17.38 ms against 17.37).
 void nb_default_shape(int64_t n, int* bpl, int* jsplit, int* leaf) {
   if (bpl && *bpl == 0) *bpl = 1;
   if (jsplit && *jsplit == 0) {
@@ -98,6 +98,36 @@ void nb_default_shape(int64_t n, int* bpl, int* jsplit, int* leaf) {
     *jsplit = k;
   }
   if (leaf && *leaf == 0) *leaf = 8;
+}
+
+// Workgroups per i-block of the direct sum. A compute unit works through
+// ceil(blocks * parts / 256) workgroups of n_pad / parts sources each, so one part
+// leaves most of the chip idle below 16,384 bodies (64 of 256 compute units at
+// 4096) and a nearly empty last round at many sizes above. The cost of a
+// workgroup beyond its pairs is that of about 256 sources (the wait for the first
+// ones, the merge). Among the part counts within 0.5% of the cheapest the largest
+// is taken: more, shorter workgroups end closer together. Slices are kept at 32
+// sources (at 2000 bodies four parts took 12.5 us, eight 14.6), and the partial
+// sums at 12 MB: from 2^19 bodies on the rounding costs less than 1.5%.
+// Steps in us, one part against this rule's number:
+//   1000 13.8 / 11.3, 4096 29.9 / 16.6, 8192 53.9 / 32.0, 12,345 74.5 / 58.3,
+//   16,384 100.9 / 85.9, 20,000 208 / 130, 37,000 525 / 379, 100,000 3060 / 2610, 2^18 17,635 / 17,428.
+int nb_direct_parts(int n_pad, int bpl, int jsplit) {
+  constexpr int kUnits = 256, kWorkgroupSources = 256, kMinSlice = 32, kMaxParts = 8;
+  constexpr int64_t kMaxPartBodies = 1 << 19;
+  const int64_t blocks = n_pad / (64 * bpl);
+  double cost[kMaxParts + 1], least = 0;
+  int most = 1;
+  for (int p = 1; p <= kMaxParts; ++p) {
+    if (p > 1 && (n_pad < p * jsplit * kMinSlice || (int64_t)p * n_pad > kMaxPartBodies)) break;
+    const int64_t rounds = (blocks * p + kUnits - 1) / kUnits;
+    const double slow = rounds * jsplit < 24 ? 1.2 : 1.0;
+    cost[p] = (double)rounds * (slow * n_pad / p + kWorkgroupSources);
+    least = p == 1 ? cost[p] : std::min(least, cost[p]);
+    most = p;
+  }
+  while (cost[most] > 1.005 * least) --most;
+  return most;
 }
 
 // Valid direct-sum launch shapes (see launch_b in nb_direct.hip).
@@ -287,6 +317,7 @@ int nb_create(nb_ctx** out, const nb_config* cfg) {
   // that (eps2)^{-3/2} overflows FP32. Below that, use the guarded kernel.
   c->guard = !(cfg->eps2 >= 1e-20f);
   default_direct_shape(c);
+  if (c->cfg.solver == NB_SOLVER_DIRECT) c->parts = nb_direct_parts(c->n_pad, c->bpl, c->jsplit);
 
   (void)hipGetDevice(&c->device);
   int rc = NB_OK;
@@ -298,9 +329,10 @@ int nb_create(nb_ctx** out, const nb_config* cfg) {
     return fail(NB_E_HIP, "nb_create: hipStreamCreate failed");
   const size_t n = c->n, np = c->n_pad;
   if (dalloc(&c->pos, 3 * n) || dalloc(&c->vel, 3 * n) || dalloc(&c->acc, 3 * n) ||
-      dalloc(&c->force, 3 * n) || dalloc(&c->mass, np) || dalloc(&c->pm, np) ||
+      dalloc(&c->force, 3 * n * (size_t)(c->parts > 1 ? 1 + c->parts : 1)) || dalloc(&c->mass, np) || dalloc(&c->pm, np) ||
       dalloc(&c->flags, 4))
     return fail(NB_E_OOM, "nb_create: device allocation failed (particle state)");
+  if (c->parts > 1) c->part = c->force + 3 * n;
   c->red_blocks = 256;
   if (dalloc(&c->red, 4 * (size_t)c->red_blocks + (np / 256) + 16))
     return fail(NB_E_OOM, "nb_create: device allocation failed (reductions)");
@@ -438,6 +470,7 @@ static int force_pass(nb_ctx* c) {
     c->tree_valid = true;
   } else {
     NB_HIP(nb_launch_direct(c));
+    NB_HIP(nb_launch_fold_parts(c));
   }
   NB_HIP(hipStreamSynchronize(c->stream));
   return check_flags(c);

@@ -23,43 +23,56 @@
 
 namespace {
 
+// Grid: (i-blocks, parts). The sources are cut into parts * K slices of whole
+// 16-source units; block (ib, p) takes the slices p * K .. p * K + K - 1. With one
+// part the block writes the forces; with more it writes its FP64 partial sums,
+// without G, to out[p][3][n], and whoever reads them adds the parts in order.
 template <int B, int K, bool kGuard>
 __global__ __launch_bounds__(64 * K) void k_direct(const float4* __restrict__ pm, int n,
                                                    int n_pad, float eps2, double G,
-                                                   double* __restrict__ force) {
+                                                   double* __restrict__ out) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ibase = blockIdx.x * (64 * B) + lane;
   nbcore::Targets<B> t;
   nbcore::load_targets<B>(pm, ibase, t);
-  const int jlen = n_pad / K;  // multiple of 64 (n_pad is a multiple of 256)
-  nbcore::accumulate<B, kGuard>(pm, wave * jlen, wave * jlen + jlen, eps2, t);
-  if constexpr (K > 1) {
-    __shared__ float part[K][6][B][64];
-    nbcore::merge_waves<B, K>(part, wave, lane, t);
-    if (wave != 0) return;
-  }
-#pragma unroll
-  for (int b = 0; b < B; ++b) {
+  const int64_t units = n_pad / 16, slices = (int64_t)gridDim.y * K;
+  const int64_t slice = (int64_t)blockIdx.y * K + wave;
+  nbcore::accumulate<B, kGuard>(pm, 16 * (int)(units * slice / slices),
+                                16 * (int)(units * (slice + 1) / slices), eps2, t);
+  __shared__ double part[K > 1 ? K : 1][3][B][64];
+  const double g = gridDim.y == 1 ? G : 1.0;
+  double* f = out + (int64_t)blockIdx.y * 3 * n;
+  nbcore::merge_waves<B, K>(part, wave, lane, t, [&](int a, int b, double sum) {
     const int i = ibase + 64 * b;
-    if (i < n) {
-      force[i] = G * ((double)t.sx[b] + (double)t.cx[b]);
-      force[n + i] = G * ((double)t.sy[b] + (double)t.cy[b]);
-      force[2 * n + i] = G * ((double)t.sz[b] + (double)t.cz[b]);
-    }
-  }
+    if (i < n) f[(int64_t)a * n + i] = g * sum;
+  });
 }
 
 template <int B, int K>
 hipError_t launch_bk(const nb_ctx* c) {
-  const int blocks = c->n_pad / (64 * B);
+  const dim3 grid(c->n_pad / (64 * B), c->parts);
+  double* out = c->parts > 1 ? c->part : c->force;
   if (c->guard)
-    hipLaunchKernelGGL((k_direct<B, K, true>), dim3(blocks), dim3(64 * K), 0, c->stream, c->pm,
-                       c->n, c->n_pad, c->cfg.eps2, c->G, c->force);
+    hipLaunchKernelGGL((k_direct<B, K, true>), grid, dim3(64 * K), 0, c->stream, c->pm, c->n,
+                       c->n_pad, c->cfg.eps2, c->G, out);
   else
-    hipLaunchKernelGGL((k_direct<B, K, false>), dim3(blocks), dim3(64 * K), 0, c->stream, c->pm,
-                       c->n, c->n_pad, c->cfg.eps2, c->G, c->force);
+    hipLaunchKernelGGL((k_direct<B, K, false>), grid, dim3(64 * K), 0, c->stream, c->pm, c->n,
+                       c->n_pad, c->cfg.eps2, c->G, out);
   return hipGetLastError();
+}
+
+// force = G * the sum of the parts, in order.
+__device__ __forceinline__ double fold_parts(const double* __restrict__ part, int parts,
+                                             int64_t stride, int64_t k, double G) {
+  double f = part[k];
+  for (int p = 1; p < parts; ++p) f += part[p * stride + k];
+  return G * f;
+}
+__global__ __launch_bounds__(256) void k_fold_parts(const double* __restrict__ part, int parts,
+                                                    int n, double G, double* __restrict__ force) {
+  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (k < 3 * (int64_t)n) force[k] = fold_parts(part, parts, 3 * (int64_t)n, k, G);
 }
 
 // Shapes: B in {1, 2, 4}; K in {1, 2, 4}, plus K = 8 for B <= 2 and K = 16 for
@@ -85,12 +98,13 @@ hipError_t launch_b(const nb_ctx* c) {
 //   v += a*dt/2; x += v*dt; a = F (evaluated at the pre-drift x); v += a*dt/2
 // and semi-implicit Euler (updateParticles.glsl:44-55): v += F*dt; x += v*dt.
 // Also refreshes the FP32 force view pm = (x, y, z, m) and flags non-finite state.
-template <bool kEuler>
+// kParts: `force` holds the direct sum's partial sums [parts][3][n].
+template <bool kEuler, bool kParts>
 __global__ __launch_bounds__(256) void k_integrate(int n, double dt, double* __restrict__ pos,
                                                    double* __restrict__ vel,
                                                    double* __restrict__ acc,
-                                                   const double* __restrict__ force,
-                                                   const float* __restrict__ mass,
+                                                   const double* __restrict__ force, int parts,
+                                                   double G, const float* __restrict__ mass,
                                                    float4* __restrict__ pm, int* __restrict__ flags) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
@@ -102,7 +116,7 @@ __global__ __launch_bounds__(256) void k_integrate(int n, double dt, double* __r
     const int k = a * n + i;
     double v = vel[k];
     double p = pos[k];
-    const double f = force[k];
+    const double f = kParts ? fold_parts(force, parts, 3 * (int64_t)n, k, G) : force[k];
     if (kEuler) {
       v = v + f * dt;
       p = p + v * dt;
@@ -255,16 +269,24 @@ hipError_t nb_launch_direct(nb_ctx* c) {
   }
 }
 
+hipError_t nb_launch_fold_parts(nb_ctx* c) {
+  if (c->parts == 1) return hipSuccess;
+  hipLaunchKernelGGL(k_fold_parts, dim3((unsigned)((3 * (int64_t)c->n + 255) / 256)), dim3(256), 0,
+                     c->stream, c->part, c->parts, c->n, c->G, c->force);
+  return hipGetLastError();
+}
+
 hipError_t nb_launch_integrate(nb_ctx* c) {
-  const int blocks = (c->n + 255) / 256;
+  const bool parts = c->parts > 1;
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((c->n + 255) / 256), dim3(256), 0, c->stream, c->n,
+                       (double)c->cfg.dt, c->pos, c->vel, c->acc, parts ? c->part : c->force,
+                       c->parts, c->G, c->mass, c->pm, c->flags);
+  };
   if (c->cfg.integrator == NB_INTEG_EULER)
-    hipLaunchKernelGGL((k_integrate<true>), dim3(blocks), dim3(256), 0, c->stream, c->n,
-                       (double)c->cfg.dt, c->pos, c->vel, c->acc, c->force, c->mass, c->pm,
-                       c->flags);
+    parts ? launch(k_integrate<true, true>) : launch(k_integrate<true, false>);
   else
-    hipLaunchKernelGGL((k_integrate<false>), dim3(blocks), dim3(256), 0, c->stream, c->n,
-                       (double)c->cfg.dt, c->pos, c->vel, c->acc, c->force, c->mass, c->pm,
-                       c->flags);
+    parts ? launch(k_integrate<false, true>) : launch(k_integrate<false, false>);
   return hipGetLastError();
 }
 

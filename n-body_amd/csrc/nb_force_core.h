@@ -104,41 +104,37 @@ __device__ __forceinline__ void load_targets(const float4* __restrict__ pm, int 
   }
 }
 
-// Merge the K wave partials of one i-block in wave order 0..K-1 through LDS.
-// All K waves must call it; afterwards wave 0 holds the merged sums.
-template <int B, int K>
-__device__ __forceinline__ void merge_waves(float (*part)[6][B][64], int wave, int lane,
-                                            Targets<B>& t) {
-#pragma unroll
-  for (int b = 0; b < B; ++b) {
-    part[wave][0][b][lane] = t.sx[b];
-    part[wave][1][b][lane] = t.sy[b];
-    part[wave][2][b][lane] = t.sz[b];
-    part[wave][3][b][lane] = t.cx[b];
-    part[wave][4][b][lane] = t.cy[b];
-    part[wave][5][b][lane] = t.cz[b];
-  }
-  __syncthreads();
-  if (wave == 0) {
+// Merge the K wave partials of one i-block, widened to FP64, in wave order 0..K-1
+// through LDS. All K waves must call it; put(component, b, sum) is called for
+// every component and target of the block, by the lane that holds the sum of its
+// lane's target: one wave per component where there are three.
+template <int B, int K, typename Put>
+__device__ __forceinline__ void merge_waves(double (*part)[3][B][64], int wave, int lane,
+                                            const Targets<B>& t, Put put) {
+  if constexpr (K == 1) {
 #pragma unroll
     for (int b = 0; b < B; ++b) {
-      t.sx[b] = part[0][0][b][lane];
-      t.sy[b] = part[0][1][b][lane];
-      t.sz[b] = part[0][2][b][lane];
-      t.cx[b] = part[0][3][b][lane];
-      t.cy[b] = part[0][4][b][lane];
-      t.cz[b] = part[0][5][b][lane];
-#pragma unroll
-      for (int w = 1; w < K; ++w) {
-        two_sum_fold(t.sx[b], t.cx[b], part[w][0][b][lane]);
-        two_sum_fold(t.sy[b], t.cy[b], part[w][1][b][lane]);
-        two_sum_fold(t.sz[b], t.cz[b], part[w][2][b][lane]);
-        t.cx[b] += part[w][3][b][lane];
-        t.cy[b] += part[w][4][b][lane];
-        t.cz[b] += part[w][5][b][lane];
-      }
+      put(0, b, (double)t.sx[b] + (double)t.cx[b]);
+      put(1, b, (double)t.sy[b] + (double)t.cy[b]);
+      put(2, b, (double)t.sz[b] + (double)t.cz[b]);
     }
+    return;
   }
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    part[wave][0][b][lane] = (double)t.sx[b] + (double)t.cx[b];
+    part[wave][1][b][lane] = (double)t.sy[b] + (double)t.cy[b];
+    part[wave][2][b][lane] = (double)t.sz[b] + (double)t.cz[b];
+  }
+  __syncthreads();
+  for (int a = wave; a < 3; a += K)
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      double f = part[0][a][b][lane];
+#pragma unroll
+      for (int w = 1; w < K; ++w) f += part[w][a][b][lane];
+      put(a, b, f);
+    }
 }
 
 }  // namespace nbcore

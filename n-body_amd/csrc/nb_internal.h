@@ -211,7 +211,9 @@ struct nb_ctx {
 
   // direct-sum launch shape
   int bpl = 2;     // i-bodies per lane
-  int jsplit = 2;  // waves per i-block
+  int jsplit = 2;  // waves per workgroup of an i-block
+  int parts = 1;   // workgroups per i-block, each with a part of the sources
+  double* part = nullptr;  // their partial sums [parts][3][n], behind force
   bool guard = false;
   int walk_stack = 0;  // BH traversal stack region cap (0: the full kStackCap); a test hook
 
@@ -247,8 +249,9 @@ inline void nb_drop_graph(hipStream_t s, hipGraphExec_t& exec, hipGraph_t& graph
 }
 
 // ---- launchers (return hipError_t of the launch) ---------------------------
-hipError_t nb_launch_direct(nb_ctx* c);  // pm -> force
-hipError_t nb_launch_integrate(nb_ctx* c);  // force + state -> state, pm
+hipError_t nb_launch_direct(nb_ctx* c);  // pm -> force, or part when parts > 1
+hipError_t nb_launch_fold_parts(nb_ctx* c);  // part -> force when parts > 1
+hipError_t nb_launch_integrate(nb_ctx* c);  // force or part + state -> state, pm
 hipError_t nb_launch_refresh_pm(nb_ctx* c);  // pos, mass -> pm
 hipError_t nb_launch_fill_i32(int* p, int v, int64_t count, hipStream_t s);
 hipError_t nb_launch_render_view(nb_ctx* c, float4* out);  // (x, y, z, |v|) per slot
@@ -277,6 +280,7 @@ hipError_t nb_bh_count_per_body(nb_ctx* c);
 // from the built-in defaults.
 bool nb_tuned_shape(int64_t n, int* bpl, int* jsplit, int* leaf);
 void nb_default_shape(int64_t n, int* bpl, int* jsplit, int* leaf);
+int nb_direct_parts(int n_pad, int bpl, int jsplit);  // workgroups per i-block
 bool nb_valid_shape(int bpl, int jsplit);  // a direct-sum kernel exists for it
 
 // step = forces + integration (no sync)

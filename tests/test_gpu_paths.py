@@ -80,3 +80,22 @@ def test_radix_sort_at_tile_and_group_edges(nb, ora, n):
     ccodes = ora.morton(p4, mn, mx, cubic=True)
     np.testing.assert_array_equal(codes, ccodes)
     np.testing.assert_array_equal(perm, np.argsort(ccodes, kind="stable"))
+
+
+@pytest.mark.parametrize("n, bpl, js", [(1, 0, 0), (511, 0, 0), (1025, 0, 0), (2049, 4, 4), (4097, 0, 0),
+                                        (6000, 2, 8), (8193, 1, 1), (16385, 0, 0), (37001, 0, 0)])
+def test_direct_sum_in_parts(nb, ora, n, bpl, js):
+    """Workgroups that each sum a part of the sources (1 to 8 parts at these sizes):
+    forces against FP64, and steps and force passes use the same sum."""
+    pos, vel, m = nb.ic_plummer(5 + n, n, 50.0, 1e4)
+    tgt = np.random.default_rng(n).choice(n, min(n, 500), replace=False)
+    ref = ora.direct_f64(pos.astype(np.float32).astype(np.float64), m.astype(np.float64), EPS2, targets=tgt)
+    with nb.Simulation(n, EPS2, DT, bodies_per_lane=bpl, j_split=js) as sim:
+        sim.upload(pos, vel, m)
+        f = sim.forces_f64()
+        sim.step(1)
+        _, _, acc = sim.download_f64()
+    np.testing.assert_array_equal(acc, f)  # the lagged step's forces are those at its start
+    scale = np.linalg.norm(ref, axis=1).max() + 1e-30
+    # 256-source FP32 sums, folded with compensation: 256 roundings of the largest force at worst
+    assert np.abs(f[tgt] - ref).max() <= 256 * 2.0 ** -24 * scale
