@@ -48,6 +48,8 @@ void free_ctx(nb_ctx* c) {
     if (e) (void)hipEventDestroy(e);
   nb_bh_free(c);
   if (c->tmp) (void)hipFree(c->tmp);
+  if (c->slot_of) (void)hipFree(c->slot_of);
+  nb_stage_free(c->stage);
   (void)hipFree(c->pos);
   (void)hipFree(c->vel);
   (void)hipFree(c->acc);
@@ -60,10 +62,7 @@ void free_ctx(nb_ctx* c) {
   delete c;
 }
 
-int check_flags(nb_ctx* c) {
-  int h = 0;
-  NB_HIP(hipMemcpyAsync(&h, c->flags, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  NB_HIP(hipStreamSynchronize(c->stream));
+int flags_status(int h) {
   if (h & 1) return nb_fail(NB_E_NONFINITE, "non-finite position or velocity in the particle state");
   if (h & 2) return nb_fail(NB_E_TREE_OVERFLOW, "octree node pool exhausted");
   if (h & 4) return nb_fail(NB_E_TREE_OVERFLOW, "octree traversal left the node range");
@@ -71,6 +70,20 @@ int check_flags(nb_ctx* c) {
   return NB_OK;
 }
 
+int check_flags(nb_ctx* c) {
+  int h = 0;
+  NB_HIP(hipMemcpyAsync(&h, c->flags, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  NB_HIP(hipStreamSynchronize(c->stream));
+  return flags_status(h);
+}
+
+// The context's arrays in the caller's order, for nb_fetch.
+nb_planes planes(const nb_ctx* c) {
+  nb_planes p;
+  p.n = p.stride = c->n;
+  p.slot_of = c->order.empty() ? nullptr : c->slot_of;
+  return p;
+}
 
 // Structure-of-arrays host copy [k][slot] -> [k][caller index] after nb_reorder.
 template <typename T>
@@ -380,6 +393,31 @@ static int upload_common(nb_ctx* c, const std::vector<double>& p, const std::vec
   return NB_OK;
 }
 
+static int upload_packed(nb_ctx* c, int layout, const void* pos, const void* vel, const void* acc,
+                         const float* mass) {
+  // Drop any captured step: it would be replayed against stale assumptions otherwise.
+  nb_drop_graph(c->stream, c->graph_exec, c->graph);
+  nb_put_args p{};
+  p.pos = pos;
+  p.vel = vel;
+  p.acc = acc;
+  p.mass = mass;
+  p.n = p.stride = c->n;
+  p.n_pad = c->n_pad;
+  p.dst[0] = c->pos;
+  p.dst[1] = c->vel;
+  p.dst[2] = c->acc;
+  p.mass_dst = c->mass;
+  p.pm = c->pm;
+  p.flags = c->flags;
+  const int rc = nb_put(c->stage, c->stream, c->force, layout, p);  // every force pass writes force anew
+  if (rc) return rc;
+  c->uploaded = true;
+  c->tree_valid = false;
+  c->order.clear();  // slots are in the caller's order again
+  return NB_OK;
+}
+
 int nb_upload(nb_ctx* c, const float* pos4, const float* vel4, const float* acc4,
               const float* mass, int64_t n) {
   NB_TRY
@@ -387,14 +425,7 @@ int nb_upload(nb_ctx* c, const float* pos4, const float* vel4, const float* acc4
   NB_API_SHARED;
   if (!c || !pos4 || !vel4 || !mass) return nb_fail(NB_E_ARG, "nb_upload: null argument");
   if (n != c->n) return nb_fail(NB_E_ARG, "nb_upload: n differs from the context's n");
-  std::vector<double> p(3 * n), v(3 * n), a(3 * n, 0.0);
-  for (int64_t i = 0; i < n; ++i)
-    for (int k = 0; k < 3; ++k) {
-      p[k * n + i] = pos4[4 * i + k];
-      v[k * n + i] = vel4[4 * i + k];
-      if (acc4) a[k * n + i] = acc4[4 * i + k];
-    }
-  return upload_common(c, p, v, a, mass);
+  return upload_packed(c, kPackF4, pos4, vel4, acc4, mass);
   NB_CATCH("nb_upload")
 }
 
@@ -405,14 +436,7 @@ int nb_upload_f64(nb_ctx* c, const double* pos3, const double* vel3, const doubl
   NB_API_SHARED;
   if (!c || !pos3 || !vel3 || !mass) return nb_fail(NB_E_ARG, "nb_upload_f64: null argument");
   if (n != c->n) return nb_fail(NB_E_ARG, "nb_upload_f64: n differs from the context's n");
-  std::vector<double> p(3 * n), v(3 * n), a(3 * n, 0.0);
-  for (int64_t i = 0; i < n; ++i)
-    for (int k = 0; k < 3; ++k) {
-      p[k * n + i] = pos3[3 * i + k];
-      v[k * n + i] = vel3[3 * i + k];
-      if (acc3) a[k * n + i] = acc3[3 * i + k];
-    }
-  return upload_common(c, p, v, a, mass);
+  return upload_packed(c, kPackD3, pos3, vel3, acc3, mass);
   NB_CATCH("nb_upload_f64")
 }
 
@@ -462,18 +486,25 @@ int nb_sync(nb_ctx* c) {
   NB_CATCH("nb_sync")
 }
 
-static int force_pass(nb_ctx* c) {
+static int force_pass(nb_ctx* c, int layout, void* out) {
   if (!c->uploaded) return nb_fail(NB_E_ARG, "no particle system uploaded");
+  nb_planes p = planes(c);
+  const double* src = c->force;
   if (c->cfg.solver == NB_SOLVER_BH) {
     NB_HIP(nb_bh_build(c));
     NB_HIP(nb_bh_traverse(c, false));
     c->tree_valid = true;
   } else {
     NB_HIP(nb_launch_direct(c));
-    NB_HIP(nb_launch_fold_parts(c));
+    if (c->parts > 1) {
+      src = c->part;
+      p.parts = c->parts;
+      p.G = c->G;
+    }
   }
-  NB_HIP(hipStreamSynchronize(c->stream));
-  return check_flags(c);
+  int flags = 0;
+  const int rc = nb_fetch(c->stage, c->stream, p, layout, 1, &src, &out, c->flags, &flags);
+  return rc ? rc : flags_status(flags);
 }
 
 int nb_forces(nb_ctx* c, float* force4) {
@@ -481,19 +512,7 @@ int nb_forces(nb_ctx* c, float* force4) {
   NB_RANGE("nb_forces");
   NB_API_SHARED;
   if (!c || !force4) return nb_fail(NB_E_ARG, "nb_forces: null argument");
-  int rc = force_pass(c);
-  if (rc) return rc;
-  const size_t n = c->n;
-  std::vector<double> f(3 * n);
-  NB_HIP(hipMemcpy(f.data(), c->force, 3 * n * sizeof(double), hipMemcpyDeviceToHost));
-  to_caller_order(c, f, 3);
-  for (size_t i = 0; i < n; ++i) {
-    force4[4 * i] = (float)f[i];
-    force4[4 * i + 1] = (float)f[n + i];
-    force4[4 * i + 2] = (float)f[2 * n + i];
-    force4[4 * i + 3] = 0.f;
-  }
-  return NB_OK;
+  return force_pass(c, kPackF4, force4);
   NB_CATCH("nb_forces")
 }
 
@@ -502,15 +521,7 @@ int nb_forces_f64(nb_ctx* c, double* force3) {
   NB_RANGE("nb_forces_f64");
   NB_API_SHARED;
   if (!c || !force3) return nb_fail(NB_E_ARG, "nb_forces_f64: null argument");
-  int rc = force_pass(c);
-  if (rc) return rc;
-  const size_t n = c->n;
-  std::vector<double> f(3 * n);
-  NB_HIP(hipMemcpy(f.data(), c->force, 3 * n * sizeof(double), hipMemcpyDeviceToHost));
-  to_caller_order(c, f, 3);
-  for (size_t i = 0; i < n; ++i)
-    for (int k = 0; k < 3; ++k) force3[3 * i + k] = f[k * n + i];
-  return NB_OK;
+  return force_pass(c, kPackD3, force3);
   NB_CATCH("nb_forces_f64")
 }
 
@@ -530,21 +541,29 @@ static int download_soa(nb_ctx* c, std::vector<double>& p, std::vector<double>& 
   return check_flags(c);
 }
 
+static int download_packed(nb_ctx* c, int layout, void* pos, void* vel, void* acc) {
+  const double* all[3] = {c->pos, c->vel, c->acc};
+  void* wanted[3] = {pos, vel, acc};
+  const double* src[3];
+  void* dst[3];
+  int arrays = 0;
+  for (int k = 0; k < 3; ++k)
+    if (wanted[k]) {
+      src[arrays] = all[k];
+      dst[arrays++] = wanted[k];
+    }
+  if (arrays == 0) return check_flags(c);
+  int flags = 0;
+  const int rc = nb_fetch(c->stage, c->stream, planes(c), layout, arrays, src, dst, c->flags, &flags);
+  return rc ? rc : flags_status(flags);
+}
+
 int nb_download(nb_ctx* c, float* pos4, float* vel4, float* acc4) {
   NB_TRY
   NB_RANGE("nb_download");
   NB_API_SHARED;
   if (!c) return nb_fail(NB_E_ARG, "nb_download: null context");
-  std::vector<double> p, v, a;
-  const int rc = download_soa(c, p, v, a);
-  const size_t n = c->n;
-  for (size_t i = 0; i < n; ++i)
-    for (int k = 0; k < 4; ++k) {
-      if (pos4) pos4[4 * i + k] = k < 3 ? (float)p[k * n + i] : 0.f;
-      if (vel4) vel4[4 * i + k] = k < 3 ? (float)v[k * n + i] : 0.f;
-      if (acc4) acc4[4 * i + k] = k < 3 ? (float)a[k * n + i] : 0.f;
-    }
-  return rc;
+  return download_packed(c, kPackF4, pos4, vel4, acc4);
   NB_CATCH("nb_download")
 }
 
@@ -553,16 +572,7 @@ int nb_download_f64(nb_ctx* c, double* pos3, double* vel3, double* acc3) {
   NB_RANGE("nb_download_f64");
   NB_API_SHARED;
   if (!c) return nb_fail(NB_E_ARG, "nb_download_f64: null context");
-  std::vector<double> p, v, a;
-  const int rc = download_soa(c, p, v, a);
-  const size_t n = c->n;
-  for (size_t i = 0; i < n; ++i)
-    for (int k = 0; k < 3; ++k) {
-      if (pos3) pos3[3 * i + k] = p[k * n + i];
-      if (vel3) vel3[3 * i + k] = v[k * n + i];
-      if (acc3) acc3[3 * i + k] = a[k * n + i];
-    }
-  return rc;
+  return download_packed(c, kPackD3, pos3, vel3, acc3);
   NB_CATCH("nb_download_f64")
 }
 
@@ -673,6 +683,10 @@ int nb_reorder(nb_ctx* c) {
   if (rc != NB_OK) return rc;
   rc = ensure_tmp(c);
   if (rc != NB_OK) return rc;
+  if (!c->slot_of && hipMalloc(&c->slot_of, sizeof(int) * (size_t)c->cap_n) != hipSuccess) {
+    c->slot_of = nullptr;
+    return nb_fail(NB_E_OOM, "device allocation failed (body order)");
+  }
   NB_HIP(nb_morton_sort(c));
   NB_HIP(nb_launch_permute_state(c));
   NB_HIP(nb_launch_refresh_pm(c));
@@ -684,6 +698,11 @@ int nb_reorder(nb_ctx* c) {
   std::vector<int32_t> order(n);
   for (size_t k = 0; k < n; ++k)
     order[k] = c->order.empty() ? (int32_t)perm[k] : c->order[perm[k]];
+  std::vector<int32_t> slot_of(n);
+  for (size_t k = 0; k < n; ++k) slot_of[order[k]] = (int32_t)k;
+  NB_HIP(hipMemcpyAsync(c->slot_of, slot_of.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice,
+                        c->stream));
+  NB_HIP(hipStreamSynchronize(c->stream));
   c->order.swap(order);
   c->tree_valid = false;
   return check_flags(c);
@@ -695,19 +714,11 @@ int nb_render_view(nb_ctx* c, float* xyzs) {
   NB_API_SHARED;
   if (!c || !xyzs) return nb_fail(NB_E_ARG, "nb_render_view: null argument");
   if (!c->uploaded) return nb_fail(NB_E_ARG, "nb_render_view: nothing uploaded");
-  int rc = ensure_tmp(c);
-  if (rc != NB_OK) return rc;
-  float4* view = reinterpret_cast<float4*>(c->tmp);  // 16 B of the 24 B per body staged
-  NB_HIP(nb_launch_render_view(c, view));
-  const size_t n = c->n;
-  std::vector<float> h(4 * n);
-  NB_HIP(hipMemcpyAsync(h.data(), view, sizeof(float4) * n, hipMemcpyDeviceToHost, c->stream));
-  NB_HIP(hipStreamSynchronize(c->stream));
-  for (size_t s = 0; s < n; ++s) {
-    const size_t i = c->order.empty() ? s : (size_t)c->order[s];
-    for (int k = 0; k < 4; ++k) xyzs[4 * i + k] = h[4 * s + k];
-  }
-  return check_flags(c);
+  const double* src[2] = {c->pos, c->vel};
+  void* dst = xyzs;
+  int flags = 0;
+  const int rc = nb_fetch(c->stage, c->stream, planes(c), kPackView, 2, src, &dst, c->flags, &flags);
+  return rc ? rc : flags_status(flags);
   NB_CATCH("nb_render_view")
 }
 

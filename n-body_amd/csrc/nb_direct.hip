@@ -69,12 +69,6 @@ __device__ __forceinline__ double fold_parts(const double* __restrict__ part, in
   for (int p = 1; p < parts; ++p) f += part[p * stride + k];
   return G * f;
 }
-__global__ __launch_bounds__(256) void k_fold_parts(const double* __restrict__ part, int parts,
-                                                    int n, double G, double* __restrict__ force) {
-  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (k < 3 * (int64_t)n) force[k] = fold_parts(part, parts, 3 * (int64_t)n, k, G);
-}
-
 // Shapes: B in {1, 2, 4}; K in {1, 2, 4}, plus K = 8 for B <= 2 and K = 16 for
 // B = 1 (small systems need the extra waves; the LDS merge holds K*6*B*64 floats).
 template <int B>
@@ -144,19 +138,6 @@ __global__ __launch_bounds__(256) void k_refresh_pm(int n, int n_pad, const doub
     pm[i] = make_float4((float)pos[i], (float)pos[n + i], (float)pos[2 * n + i], mass[i]);
   else
     pm[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-}
-
-// Render view: (x, y, z, |v|) per body, the inputs of the reference's point
-// shaders (vertexShader.glsl:3-9 reads positions and velocities;
-// fragmentShader.glsl colours by length(velocity)).
-__global__ __launch_bounds__(256) void k_render_view(int n, const double* __restrict__ pos,
-                                                     const double* __restrict__ vel,
-                                                     float4* __restrict__ out) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const double vx = vel[i], vy = vel[n + i], vz = vel[2 * n + i];
-  out[i] = make_float4((float)pos[i], (float)pos[n + i], (float)pos[2 * n + i],
-                       (float)sqrt(vx * vx + vy * vy + vz * vz));
 }
 
 __global__ __launch_bounds__(256) void k_fill_i32(int* __restrict__ p, int v, int64_t count) {
@@ -269,13 +250,6 @@ hipError_t nb_launch_direct(nb_ctx* c) {
   }
 }
 
-hipError_t nb_launch_fold_parts(nb_ctx* c) {
-  if (c->parts == 1) return hipSuccess;
-  hipLaunchKernelGGL(k_fold_parts, dim3((unsigned)((3 * (int64_t)c->n + 255) / 256)), dim3(256), 0,
-                     c->stream, c->part, c->parts, c->n, c->G, c->force);
-  return hipGetLastError();
-}
-
 hipError_t nb_launch_integrate(nb_ctx* c) {
   const bool parts = c->parts > 1;
   const auto launch = [&](auto kernel) {
@@ -293,12 +267,6 @@ hipError_t nb_launch_integrate(nb_ctx* c) {
 hipError_t nb_launch_refresh_pm(nb_ctx* c) {
   hipLaunchKernelGGL(k_refresh_pm, dim3(c->n_pad / 256), dim3(256), 0, c->stream, c->n, c->n_pad,
                      c->pos, c->mass, c->pm);
-  return hipGetLastError();
-}
-
-hipError_t nb_launch_render_view(nb_ctx* c, float4* out) {
-  hipLaunchKernelGGL(k_render_view, dim3((c->n + 255) / 256), dim3(256), 0, c->stream, c->n, c->pos,
-                     c->vel, out);
   return hipGetLastError();
 }
 

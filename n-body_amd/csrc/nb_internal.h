@@ -188,6 +188,16 @@ struct nb_bh_state {
   unsigned long long* inter = nullptr;  // interaction counter (diagnostic traversal)
 };
 
+// Pinned host buffer of one context or batch: what crosses the bus in small calls,
+// and large results in halves (nb_pack.hip). Used by one host thread at a time,
+// on the owner's stream only.
+constexpr int64_t kStageBytes = 2 << 20;
+struct nb_stage {
+  char* host = nullptr;
+  hipEvent_t done[2] = {};  // each half has been filled
+  bool busy = false;        // an enqueued kernel still reads it
+};
+
 struct nb_ctx {
   nb_config cfg{};
   int64_t cap_n = 0;  // bodies the device buffers were sized for (nb_ctx_rebind limit)
@@ -221,7 +231,9 @@ struct nb_ctx {
   // Morton reordering (nb_reorder): order[slot] = the caller's index of the
   // body held in that slot; empty while slots are in the caller's order.
   std::vector<int32_t> order;
+  int* slot_of = nullptr;    // its inverse on the device, allocated by the first nb_reorder
   double* tmp = nullptr;     // [3][n] permutation staging, allocated on first use
+  nb_stage stage;
   bool uploaded = false;
   bool tree_valid = false;
 
@@ -248,13 +260,41 @@ inline void nb_drop_graph(hipStream_t s, hipGraphExec_t& exec, hipGraph_t& graph
   graph = nullptr;
 }
 
+// ---- host copies (nb_pack.hip) ----------------------------------------------
+// Packed layouts: double[3] per body, float4 (x, y, z, 0), and the render view
+// (x, y, z, |v|), which reads positions and velocities into one array.
+enum nb_pack_layout { kPackD3, kPackF4, kPackView };
+struct nb_planes {
+  int64_t n = 0;       // bodies
+  int64_t stride = 0;  // from one component's plane to the next
+  const int* slot_of = nullptr;  // device: slot of each body, or null (body i in slot i)
+  int parts = 1;       // > 1: values are G times the sum of `parts` arrays of 3 * stride
+  double G = 1.0;
+};
+// Copies `arrays` device arrays to the host arrays dst, packed, and waits for
+// them; *flags_out receives the device word *flags (0 if null).
+int nb_fetch(nb_stage& st, hipStream_t s, const nb_planes& p, int layout, int arrays,
+             const double* const* src, void* const* dst, const int* flags, int* flags_out);
+struct nb_put_args {
+  const void *pos, *vel, *acc;  // host, packed (kPackD3 or kPackF4); acc may be null (zero)
+  const float* mass;            // host
+  int64_t n, n_pad;             // pm is zero from n to n_pad
+  int64_t stride;
+  double* dst[3];               // device: first planes of positions, velocities, accelerations
+  float* mass_dst;
+  float4* pm;
+  int* flags;                   // four words to clear, or null
+};
+// Copies a system to the device. The host arrays may be reused on return; the
+// copy is complete in stream order. dev_tmp: 24 n bytes of device scratch.
+int nb_put(nb_stage& st, hipStream_t s, void* dev_tmp, int layout, const nb_put_args& p);
+void nb_stage_free(nb_stage& st);
+
 // ---- launchers (return hipError_t of the launch) ---------------------------
 hipError_t nb_launch_direct(nb_ctx* c);  // pm -> force, or part when parts > 1
-hipError_t nb_launch_fold_parts(nb_ctx* c);  // part -> force when parts > 1
 hipError_t nb_launch_integrate(nb_ctx* c);  // force or part + state -> state, pm
 hipError_t nb_launch_refresh_pm(nb_ctx* c);  // pos, mass -> pm
 hipError_t nb_launch_fill_i32(int* p, int v, int64_t count, hipStream_t s);
-hipError_t nb_launch_render_view(nb_ctx* c, float4* out);  // (x, y, z, |v|) per slot
 hipError_t nb_launch_energy(nb_ctx* c, double* ekin_p, double* epot_p);
 // FP64 direct-sum accelerations of the bodies in slots[0..k) -> acc3[3k]
 hipError_t nb_launch_ref_f64(nb_ctx* c, const int* slots, int k, double* acc3);

@@ -99,3 +99,33 @@ def test_direct_sum_in_parts(nb, ora, n, bpl, js):
     scale = np.linalg.norm(ref, axis=1).max() + 1e-30
     # 256-source FP32 sums, folded with compensation: 256 roundings of the largest force at worst
     assert np.abs(f[tgt] - ref).max() <= 256 * 2.0 ** -24 * scale
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 29127, 29128, 43680, 43681, 65521, 131041])
+@pytest.mark.parametrize("layout", ["f64", "vec4"])
+def test_host_copies_at_stage_edges(nb, n, layout):
+    """State in and out through the pinned buffer (whole calls up to 2 MB, halves
+    above; uploads directly above), in the caller's order, also after a reorder."""
+    rng = np.random.default_rng(n)
+    pos, vel, acc = (rng.normal(size=(n, 3)) for _ in range(3))
+    m = rng.uniform(1, 2, n).astype(np.float32)
+    if layout == "vec4":
+        pos, vel, acc = (a.astype(np.float32).astype(np.float64) for a in (pos, vel, acc))
+    give = (lambda a: a) if layout == "f64" else nb.to_vec4
+    speed = np.sqrt(vel[:, 0] ** 2 + vel[:, 1] ** 2 + vel[:, 2] ** 2)
+    with nb.Simulation(n, EPS2, DT) as sim:
+        for again in range(2):  # the second upload reuses the buffer that a kernel still reads
+            sim.upload(give(np.roll(pos, again, 0)), give(vel), m, give(acc) if again else None)
+        pos = np.roll(pos, 1, 0)
+        for reordered in (False, True):
+            if reordered:
+                sim.reorder()
+            for got, want in zip(sim.download_f64(), (pos, vel, acc)):
+                np.testing.assert_array_equal(got, want)
+            for got, want in zip(sim.download(), (pos, vel, acc)):
+                np.testing.assert_array_equal(got[:, :3], want.astype(np.float32))
+                assert not got[:, 3].any()
+            view = sim.render_view()
+            np.testing.assert_array_equal(view[:, :3], pos.astype(np.float32))
+            np.testing.assert_allclose(view[:, 3], speed, rtol=2.0 ** -22)
+        np.testing.assert_array_equal(sim.forces(), sim.forces_f64().astype(np.float32) @ np.eye(3, 4, dtype=np.float32))
