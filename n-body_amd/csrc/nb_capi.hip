@@ -57,7 +57,6 @@ void free_ctx(nb_ctx* c) {
   (void)hipFree(c->mass);
   (void)hipFree(c->pm);
   (void)hipFree(c->flags);
-  (void)hipFree(c->red);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
@@ -346,9 +345,6 @@ int nb_create(nb_ctx** out, const nb_config* cfg) {
       dalloc(&c->flags, 4))
     return fail(NB_E_OOM, "nb_create: device allocation failed (particle state)");
   if (c->parts > 1) c->part = c->force + 3 * n;
-  c->red_blocks = 256;
-  if (dalloc(&c->red, 4 * (size_t)c->red_blocks + (np / 256) + 16))
-    return fail(NB_E_OOM, "nb_create: device allocation failed (reductions)");
   if (hipMemset(c->flags, 0, 4 * sizeof(int)) != hipSuccess ||
       hipMemset(c->mass, 0, np * sizeof(float)) != hipSuccess ||
       hipMemset(c->pm, 0, np * sizeof(float4)) != hipSuccess ||
@@ -582,14 +578,15 @@ int nb_energy(nb_ctx* c, double* ekin, double* epot, double p[3]) {
   NB_API_SHARED;
   if (!c) return nb_fail(NB_E_ARG, "nb_energy: null context");
   if (!c->uploaded) return nb_fail(NB_E_ARG, "nb_energy: no particle system uploaded");
-  const int kin_n = 4 * c->red_blocks;
-  const int pot_n = (c->n + 255) / 256;
-  NB_HIP(nb_launch_energy(c, c->red, c->red + kin_n));
-  std::vector<double> h(kin_n + pot_n);
-  NB_HIP(hipMemcpyAsync(h.data(), c->red, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  const int kin_n = 4 * kEnergyKinBlocks;
+  const int pot_n = nb_energy_pot_blocks(c->n);
+  const int rc = nb_stage_ready(c->stage, c->stream);
+  if (rc) return rc;
+  const double* h = reinterpret_cast<const double*>(c->stage.host);
+  NB_HIP(nb_launch_energy(c, reinterpret_cast<double*>(c->stage.host)));
   NB_HIP(hipStreamSynchronize(c->stream));
   double ek = 0, px = 0, py = 0, pz = 0, ep = 0;
-  for (int b = 0; b < c->red_blocks; ++b) {
+  for (int b = 0; b < kEnergyKinBlocks; ++b) {
     ek += h[4 * b];
     px += h[4 * b + 1];
     py += h[4 * b + 2];
@@ -597,9 +594,9 @@ int nb_energy(nb_ctx* c, double* ekin, double* epot, double p[3]) {
   }
   for (int b = 0; b < pot_n; ++b) ep += h[kin_n + b];
   if (ekin) *ekin = ek;
-  if (epot) *epot = -0.5 * c->G * ep;
+  if (epot) *epot = -c->G * ep;
   if (p) { p[0] = px; p[1] = py; p[2] = pz; }
-  return check_flags(c);
+  return flags_status(*reinterpret_cast<const int*>(h + kin_n + pot_n));
   NB_CATCH("nb_energy")
 }
 

@@ -216,8 +216,6 @@ struct nb_ctx {
   float* mass = nullptr;     // [n_pad], zero in the padding
   float4* pm = nullptr;      // FP32 force view (x, y, z, m), [n_pad]
   int* flags = nullptr;      // device status word (bit 0: non-finite state)
-  double* red = nullptr;     // reduction scratch for diagnostics
-  int red_blocks = 0;
 
   // direct-sum launch shape
   int bpl = 2;     // i-bodies per lane
@@ -271,6 +269,7 @@ struct nb_planes {
   int parts = 1;       // > 1: values are G times the sum of `parts` arrays of 3 * stride
   double G = 1.0;
 };
+int nb_stage_ready(nb_stage& st, hipStream_t s);  // allocated, and free for new content
 // Copies `arrays` device arrays to the host arrays dst, packed, and waits for
 // them; *flags_out receives the device word *flags (0 if null).
 int nb_fetch(nb_stage& st, hipStream_t s, const nb_planes& p, int layout, int arrays,
@@ -295,7 +294,11 @@ hipError_t nb_launch_direct(nb_ctx* c);  // pm -> force, or part when parts > 1
 hipError_t nb_launch_integrate(nb_ctx* c);  // force or part + state -> state, pm
 hipError_t nb_launch_refresh_pm(nb_ctx* c);  // pos, mass -> pm
 hipError_t nb_launch_fill_i32(int* p, int v, int64_t count, hipStream_t s);
-hipError_t nb_launch_energy(nb_ctx* c, double* ekin_p, double* epot_p);
+// state -> part: 4 * kEnergyKinBlocks kinetic, then nb_energy_pot_blocks(n) potential
+// partials, then the device status word (as an int)
+constexpr int kEnergyKinBlocks = 128;
+int nb_energy_pot_blocks(int n);
+hipError_t nb_launch_energy(nb_ctx* c, double* part);
 // FP64 direct-sum accelerations of the bodies in slots[0..k) -> acc3[3k]
 hipError_t nb_launch_ref_f64(nb_ctx* c, const int* slots, int k, double* acc3);
 

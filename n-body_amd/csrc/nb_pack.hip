@@ -150,8 +150,7 @@ int64_t body_bytes(int layout) { return layout == kPackD3 ? 24 : 16; }
 
 }  // namespace
 
-// The stage, allocated on first use and free for new content.
-static int stage_ready(nb_stage& st, hipStream_t s) {
+int nb_stage_ready(nb_stage& st, hipStream_t s) {
   if (!st.host) {
     if (hipHostMalloc(reinterpret_cast<void**>(&st.host), kStageBytes, hipHostMallocDefault) != hipSuccess) {
       st.host = nullptr;
@@ -174,7 +173,7 @@ void nb_stage_free(nb_stage& st) {
 
 int nb_fetch(nb_stage& st, hipStream_t s, const nb_planes& p, int layout, int arrays,
              const double* const* src, void* const* dst, const int* flags, int* flags_out) {
-  const int rc = stage_ready(st, s);
+  const int rc = nb_stage_ready(st, s);
   if (rc) return rc;
   int* stage_flags = reinterpret_cast<int*>(st.host + kStageBytes) - 1;
   PackArgs a{};
@@ -234,7 +233,7 @@ int nb_put(nb_stage& st, hipStream_t s, void* dev_tmp, int layout, const nb_put_
   const void* from[3] = {p.pos, p.vel, p.acc};
   if (3 * p.n * per + 4 * p.n <= kStageBytes) {
     // through the stage; nothing waits: the next use of the stage does
-    const int rc = stage_ready(st, s);
+    const int rc = nb_stage_ready(st, s);
     if (rc) return rc;
     char* at = st.host;
     for (int k = 0; k < 3; ++k) {

@@ -81,12 +81,11 @@ int64_t capacity(int64_t n) {
 }
 
 // Device bytes of a Barnes-Hut context sized for n bodies (nb_create +
-// nb_bh_alloc): FP64 state and forces, FP32 view and masses, reductions, and the
-// single octree block.
+// nb_bh_alloc): FP64 state and forces, FP32 view and masses, and the single octree
+// block.
 int64_t bh_bytes(int64_t n) {
   const int64_t np = (n + 255) / 256 * 256;
-  return 4 * 24 * n + np * (16 + 4) + 8 * (4 * 256 + np / 256 + 16) +
-         nb_bh_layout_for(n).off[kBhBufCount] + (1 << 20);
+  return 4 * 24 * n + np * (16 + 4) + nb_bh_layout_for(n).off[kBhBufCount] + (1 << 20);
 }
 
 int64_t padded(int64_t n) { return (n + kPadBodies - 1) / kPadBodies * kPadBodies; }
