@@ -56,6 +56,7 @@ void free_ctx(nb_ctx* c) {
   (void)hipFree(c->force);
   (void)hipFree(c->mass);
   (void)hipFree(c->pm);
+  if (c->pm_next) (void)hipFree(c->pm_next);
   (void)hipFree(c->flags);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -169,6 +170,7 @@ void default_direct_shape(nb_ctx* c) {
 hipError_t nb_enqueue_step(nb_ctx* c) {
   hipError_t e;
   const bool t = c->timing;
+  if (c->small && !t) return nb_launch_small_step(c);  // timed steps: the same sums in two launches
   if (t) (void)hipEventRecord(c->ev[0], c->stream);
   if (c->cfg.solver == NB_SOLVER_BH) {
     e = nb_bh_build(c);
@@ -208,7 +210,7 @@ static int accumulate_timing(nb_ctx* c) {
 // eight-step graph 0.0285 ms (N = 16384: 4% less; Barnes-Hut steps, bound by
 // their dependent build kernels, gained under 1%).
 constexpr int64_t kChunkMaxBodies = 32768;
-constexpr int kChunkSteps = 8;
+constexpr int kChunkSteps = 8;  // even: a small system's views are in place again after it
 
 int nb_prepare_step_graph(nb_ctx* c) {
   if (c->graph_exec || (c->cfg.flags & NB_F_NO_GRAPH)) return NB_OK;
@@ -217,11 +219,13 @@ int nb_prepare_step_graph(nb_ctx* c) {
       c->cfg.solver == NB_SOLVER_DIRECT && c->n <= kChunkMaxBodies ? kChunkSteps : 1;
   NB_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   hipError_t e = hipSuccess;
+  c->graph_pm = c->pm;
   for (int s = 0; s < steps && e == hipSuccess; ++s) e = nb_enqueue_step(c);
   hipGraph_t g = nullptr;
   hipError_t e2 = hipStreamEndCapture(c->stream, &g);
   if (e != hipSuccess || e2 != hipSuccess) {
     if (g) (void)hipGraphDestroy(g);
+    if (c->pm != c->graph_pm) std::swap(c->pm, c->pm_next);  // none of the steps ran
     return nb_fail(NB_E_HIP, std::string("nb_step: graph capture failed: ") +
                                  hipGetErrorString(e != hipSuccess ? e : e2));
   }
@@ -329,7 +333,11 @@ int nb_create(nb_ctx** out, const nb_config* cfg) {
   // that (eps2)^{-3/2} overflows FP32. Below that, use the guarded kernel.
   c->guard = !(cfg->eps2 >= 1e-20f);
   default_direct_shape(c);
-  if (c->cfg.solver == NB_SOLVER_DIRECT) c->parts = nb_direct_parts(c->n_pad, c->bpl, c->jsplit);
+  if (c->cfg.solver == NB_SOLVER_DIRECT) {
+    // an explicit launch shape is a choice of k_direct's
+    c->small = c->n_pad <= kSmallBodies && cfg->bodies_per_lane == 0 && cfg->j_split == 0;
+    c->parts = c->small ? 1 : nb_direct_parts(c->n_pad, c->bpl, c->jsplit);
+  }
 
   (void)hipGetDevice(&c->device);
   int rc = NB_OK;
@@ -342,12 +350,13 @@ int nb_create(nb_ctx** out, const nb_config* cfg) {
   const size_t n = c->n, np = c->n_pad;
   if (dalloc(&c->pos, 3 * n) || dalloc(&c->vel, 3 * n) || dalloc(&c->acc, 3 * n) ||
       dalloc(&c->force, 3 * n * (size_t)(c->parts > 1 ? 1 + c->parts : 1)) || dalloc(&c->mass, np) || dalloc(&c->pm, np) ||
-      dalloc(&c->flags, 4))
+      dalloc(&c->flags, 4) || (c->small && dalloc(&c->pm_next, np)))
     return fail(NB_E_OOM, "nb_create: device allocation failed (particle state)");
   if (c->parts > 1) c->part = c->force + 3 * n;
   if (hipMemset(c->flags, 0, 4 * sizeof(int)) != hipSuccess ||
       hipMemset(c->mass, 0, np * sizeof(float)) != hipSuccess ||
       hipMemset(c->pm, 0, np * sizeof(float4)) != hipSuccess ||
+      (c->small && hipMemset(c->pm_next, 0, np * sizeof(float4)) != hipSuccess) ||
       hipMemset(c->force, 0, 3 * n * sizeof(double)) != hipSuccess)
     return fail(NB_E_HIP, "nb_create: hipMemset failed");
   for (auto& e : c->ev)
@@ -464,7 +473,11 @@ int nb_step(nb_ctx* c, int32_t nsteps) {
     if (rc) return rc;
     // whole graphs, then the remainder as eager launches (identical results)
     int s = 0;
-    for (; s + c->graph_steps <= nsteps; s += c->graph_steps)
+    if (c->pm != c->graph_pm && nsteps > c->graph_steps) {  // a small system's other view is current
+      NB_HIP(nb_enqueue_step(c));
+      ++s;
+    }
+    for (; c->pm == c->graph_pm && s + c->graph_steps <= nsteps; s += c->graph_steps)
       NB_HIP(hipGraphLaunch(c->graph_exec, c->stream));
     for (; s < nsteps; ++s) NB_HIP(nb_enqueue_step(c));
   }

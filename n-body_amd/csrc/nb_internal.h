@@ -64,6 +64,9 @@ struct nb_trace_range {
 // multiples of 4 bodies, so every count is a multiple of 256.
 constexpr int kPadBodies = 256;
 
+// Largest direct sum that holds all its sources in one workgroup's LDS.
+constexpr int kSmallBodies = 8192;
+
 // Octree geometry: 30-bit Morton codes give at most 10 levels below the root.
 constexpr int kMaxLevel = 10;
 
@@ -220,6 +223,8 @@ struct nb_ctx {
   // direct-sum launch shape
   int bpl = 2;     // i-bodies per lane
   int jsplit = 2;  // waves per workgroup of an i-block
+  bool small = false;  // direct sum of a small system: one launch per step (k_direct_small)
+  float4* pm_next = nullptr;  // its second view: a step reads pm, writes pm_next and swaps them
   int parts = 1;   // workgroups per i-block, each with a part of the sources
   double* part = nullptr;  // their partial sums [parts][3][n], behind force
   bool guard = false;
@@ -240,6 +245,7 @@ struct nb_ctx {
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
   int graph_steps = 1;
+  const float4* graph_pm = nullptr;  // the view that the graph's first step reads
 
   // timing
   bool timing = false;
@@ -291,6 +297,7 @@ void nb_stage_free(nb_stage& st);
 
 // ---- launchers (return hipError_t of the launch) ---------------------------
 hipError_t nb_launch_direct(nb_ctx* c);  // pm -> force, or part when parts > 1
+hipError_t nb_launch_small_step(nb_ctx* c);  // force + integration of a `small` context
 hipError_t nb_launch_integrate(nb_ctx* c);  // force or part + state -> state, pm
 hipError_t nb_launch_refresh_pm(nb_ctx* c);  // pos, mass -> pm
 hipError_t nb_launch_fill_i32(int* p, int v, int64_t count, hipStream_t s);

@@ -129,3 +129,27 @@ def test_host_copies_at_stage_edges(nb, n, layout):
             np.testing.assert_array_equal(view[:, :3], pos.astype(np.float32))
             np.testing.assert_allclose(view[:, 3], speed, rtol=2.0 ** -22)
         np.testing.assert_array_equal(sim.forces(), sim.forces_f64().astype(np.float32) @ np.eye(3, 4, dtype=np.float32))
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1025, 2049, 4095, 4097, 8191, 8192, 8193])
+@pytest.mark.parametrize("integrator", [0, 1])
+def test_one_launch_steps(nb, n, integrator):
+    """Steps of small systems alternate two views of the bodies: any split of the
+    steps into calls, graphs or not, timed or not, gives the same bits."""
+    pos, vel, m = nb.ic_plummer(9 + n, n, 50.0, 1e4)
+    out = []
+    for flags, calls in ((0, [21]), (0, [1, 9, 2, 8, 1]), (nb.F_NO_GRAPH, [21]), (0, [3, -1, 18])):
+        with nb.Simulation(n, EPS2 if n % 2 else 0.0, DT, integrator=integrator, flags=flags) as sim:
+            sim.upload(pos, vel, m)
+            sim.step(1)  # an odd step first
+            sim.upload(pos, vel, m)
+            for k in calls:
+                if k < 0:
+                    sim.set_timing(True)
+                    f = sim.forces_f64()
+                else:
+                    sim.step(k)
+            sim.set_timing(False)
+            out.append(np.concatenate(sim.download_f64() + (sim.forces_f64(),)))
+    for o in out[1:]:
+        np.testing.assert_array_equal(o, out[0])
