@@ -8,11 +8,11 @@
 // device arrays indexed by slot.
 //
 // Work decomposition:
-//   force      work item = (slot, i-block of 64*B bodies); items are sorted by
-//              cluster size, largest first, and as many workgroups as can be
-//              resident at once pull them from an atomic ticket (persistent
-//              kernel; every workgroup exits once the ticket passes the item
-//              count). The K waves of a
+//   force      work item = (slot, i-block of 64*B bodies), with everything the
+//              kernel needs to know of its cluster; items are sorted by cluster
+//              size, largest first; as many workgroups as can be resident at
+//              once take one each, then more from an atomic ticket until none is
+//              left (persistent kernel). The K waves of a
 //              workgroup split the cluster's sources; partial sums merge in LDS
 //              in wave order, so a cluster's forces do not depend on scheduling
 //              or on the other clusters.
@@ -29,11 +29,18 @@
 #include "nb_force_core.h"
 #include "nb_internal.h"
 
+// One work item of the force pass.
+struct alignas(32) nb_batch_item {
+  int slot, ibase, off, npad, end;  // bodies [off, end), padded to npad; targets from ibase on
+  float eps2;
+  double G;
+};
+
 struct nb_batch {
   nb_batch_config cfg{};
   hipStream_t stream = nullptr;
   int64_t cap = 0;
-  int bpl = 1, jsplit = 4;
+  int bpl = 1, jsplit = 8;
   int cus = 256;  // compute units: the persistent grid fills every CU to its occupancy
   // device pool
   float4* pm = nullptr;
@@ -42,18 +49,19 @@ struct nb_batch {
   // device slot table
   int* c_off = nullptr;
   int* c_n = nullptr;
-  int* c_npad = nullptr;
-  float* c_eps2 = nullptr;
   double* c_dt = nullptr;
-  double* c_G = nullptr;
   int* c_quota = nullptr;  // steps the cluster takes per nb_batch_step call (INT32_MAX: all)
   // device work tables
-  int2* items = nullptr;   // (slot, i-block)
+  nb_batch_item* items = nullptr;
   int2* blocks = nullptr;  // (slot, first body) per 256-body block
-  int* counts = nullptr;   // [0] items, [1] blocks, [2] ticket, [3] flags, [4] step of the call
+  // [0] items, [1] blocks, [2] ticket, [4] step of the call, [5] the same for the integrator
+  int* counts = nullptr;
   double* red = nullptr;   // energy partials
   // host mirror
   std::vector<int> h_off, h_n, h_npad, h_quota;
+  std::vector<float> h_eps2;
+  std::vector<double> h_G;
+  nb_stage stage;
   std::vector<char> used;
   std::map<int64_t, int64_t> free_list;  // offset -> size
   int64_t used_bodies = 0;
@@ -73,47 +81,49 @@ constexpr int kUnlimited = NB_BATCH_UNLIMITED;
 
 // use_quota: skip the clusters whose quota is used up in this call (steps);
 // force-only passes (nb_batch_forces, nb_batch_tune) evaluate every cluster.
+// A workgroup's first item is its own index, so a small ensemble takes no tickets
+// (one per workgroup from one address: 100 clusters of 128 bodies took 45 us per
+// step with them, 17 without), and a next ticket is taken while the
+// current item is summed: an atomic's way across the chip, the item's record and
+// its targets are a chain of waits.
+// Nothing but this kernel and the integrator runs in a step: this one passes the
+// step on in counts[5], the integrator counts it in counts[4] and resets the ticket,
+// each where the other does not read.
 template <int B, int K>
 __global__ __launch_bounds__(64 * K) void k_batch_force(
-    const float4* __restrict__ pm, const int* __restrict__ c_off, const int* __restrict__ c_n,
-    const int* __restrict__ c_npad, const float* __restrict__ c_eps2,
-    const double* __restrict__ c_G, const int* __restrict__ c_quota, int use_quota,
-    const int2* __restrict__ items, int* __restrict__ counts, int64_t cap,
+    const float4* __restrict__ pm, const int* __restrict__ c_quota, int use_quota,
+    const nb_batch_item* __restrict__ items, int* __restrict__ counts, int64_t cap,
     double* __restrict__ force) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nitems = counts[0];
   const int call_step = use_quota ? counts[4] : -1;
-  __shared__ int s_item;
-  __shared__ double part[K][3][B][64];
-  for (;;) {
-    if (threadIdx.x == 0) s_item = atomicAdd(&counts[2], 1);
+  __shared__ int s_item[2];  // in turn, so that one barrier per item is enough
+  __shared__ double part[K > 1 ? K : 1][3][B][64];
+  if (use_quota && blockIdx.x == 0 && threadIdx.x == 0) counts[5] = call_step;
+  int next = blockIdx.x;
+  for (int turn = 0;; turn ^= 1) {
+    if (threadIdx.x == 0) s_item[turn] = next;
     __syncthreads();
-    const int item = __builtin_amdgcn_readfirstlane(s_item);
-    __syncthreads();  // every lane has read s_item before lane 0 overwrites it
+    const int item = __builtin_amdgcn_readfirstlane(s_item[turn]);
     if (item >= nitems) break;
-    const int2 it = items[item];
-    const int slot = __builtin_amdgcn_readfirstlane(it.x);
-    if (__builtin_amdgcn_readfirstlane(c_quota[slot]) <= call_step) continue;  // block-uniform
-    const int off = __builtin_amdgcn_readfirstlane(c_off[slot]);
-    const int npad = __builtin_amdgcn_readfirstlane(c_npad[slot]);
-    const int n = c_n[slot];
-    const float eps2 = c_eps2[slot];
-    const int ibase = off + it.y * (64 * B) + lane;
+    if (threadIdx.x == 0)
+      next = nitems > (int)gridDim.x ? (int)gridDim.x + atomicAdd(&counts[2], 1) : nitems;
+    const nb_batch_item it = items[item];  // wave-uniform
+    if (__builtin_amdgcn_readfirstlane(c_quota[it.slot]) <= call_step) continue;  // block-uniform
+    const int ibase = it.ibase + lane;
     nbcore::Targets<B> t;
     nbcore::load_targets<B>(pm, ibase, t);
-    const int jlen = npad / K;  // npad is a multiple of 256: a multiple of 16 for K <= 16
-    const int j0 = off + wave * jlen;
-    if (eps2 >= 1e-20f)
-      nbcore::accumulate<B, false>(pm, j0, j0 + jlen, eps2, t);
+    const int jlen = it.npad / K;  // npad is a multiple of 256: a multiple of 16 for K <= 16
+    const int j0 = it.off + wave * jlen;
+    if (it.eps2 >= 1e-20f)
+      nbcore::accumulate<B, false>(pm, j0, j0 + jlen, it.eps2, t);
     else
-      nbcore::accumulate<B, true>(pm, j0, j0 + jlen, eps2, t);
-    const double G = c_G[slot];
+      nbcore::accumulate<B, true>(pm, j0, j0 + jlen, it.eps2, t);
     nbcore::merge_waves<B, K>(part, wave, lane, t, [&](int a, int b, double sum) {
       const int i = ibase + 64 * b;
-      if (i - off < n) force[a * cap + i] = G * sum;
+      if (i < it.end) force[a * cap + i] = it.G * sum;
     });
-    if constexpr (K > 1) __syncthreads();  // LDS partials are reused by the next item
   }
 }
 
@@ -121,21 +131,20 @@ __global__ void k_batch_reset(int* __restrict__ counts) {
   if (threadIdx.x == 0 && blockIdx.x == 0) counts[2] = 0;
 }
 
-// End of one step: the next step of the same nb_batch_step call.
-__global__ void k_batch_advance(int* __restrict__ counts) {
-  if (threadIdx.x == 0 && blockIdx.x == 0 && counts[4] < 0x7fffffff) counts[4] += 1;
-}
-
 template <bool kEuler>
 __global__ __launch_bounds__(256) void k_batch_integrate(
-    const int2* __restrict__ blocks, const int* __restrict__ counts, const int* __restrict__ c_off,
+    const int2* __restrict__ blocks, int* __restrict__ counts, const int* __restrict__ c_off,
     const int* __restrict__ c_n, const double* __restrict__ c_dt, const int* __restrict__ c_quota,
     int64_t cap, double* __restrict__ pos, double* __restrict__ vel, double* __restrict__ acc,
     const double* __restrict__ force, const float* __restrict__ mass, float4* __restrict__ pm) {
   // grid-stride over the pool blocks in use: the launch is sized for the
   // device, not for the pool's capacity, so an almost empty pool costs little
   const int nblocks = counts[1];
-  const int step = counts[4];
+  const int step = counts[5];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // the next step's force pass
+    counts[2] = 0;
+    if (step < 0x7fffffff) counts[4] = step + 1;
+  }
   for (int blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
     const int2 bl = blocks[blk];
     if (c_quota[bl.x] <= step) continue;  // quota used up in this call
@@ -167,15 +176,14 @@ __global__ __launch_bounds__(256) void k_batch_integrate(
   }
 }
 
-__global__ __launch_bounds__(256) void k_batch_refresh(int off, int n, int npad, int64_t cap,
-                                                       const double* __restrict__ pos,
-                                                       const float* __restrict__ mass,
-                                                       float4* __restrict__ pm) {
-  const int k = blockIdx.x * 256 + threadIdx.x;
-  if (k >= npad) return;
-  const int i = off + k;
-  pm[i] = k < n ? make_float4((float)pos[i], (float)pos[cap + i], (float)pos[2 * cap + i], mass[i])
-                : make_float4(0.f, 0.f, 0.f, 0.f);
+__global__ void k_batch_admit(int slot, int off, int n, double dt, int* __restrict__ c_off,
+                              int* __restrict__ c_n, double* __restrict__ c_dt,
+                              int* __restrict__ c_quota) {
+  if (threadIdx.x != 0) return;
+  c_off[slot] = off;
+  c_n[slot] = n;
+  c_dt[slot] = dt;
+  c_quota[slot] = kUnlimited;
 }
 
 // FP64 energy of one cluster: block partials of (ekin, sum_i m_i phi_i).
@@ -215,9 +223,7 @@ template <int B, int K>
 hipError_t launch_force(nb_batch* b, int use_quota) {
   // Persistent: as many blocks as can be resident at once, which depends on the
   // shape's registers and LDS (one body per lane fits 8 waves per SIMD, two
-  // bodies 4). A fixed 16 waves per CU left the one-body shapes at half
-  // occupancy: 1x4 took 16.08 ms on the 512-cluster ensemble, 14.37 ms at full
-  // occupancy.
+  // bodies 4).
   // (Queried per launch, for the current device: a host-side query, and steps
   // replay a captured graph, so it runs once per capture.)
   int per_cu = 0;
@@ -227,8 +233,7 @@ hipError_t launch_force(nb_batch* b, int use_quota) {
     per_cu = std::max(1, 16 / K);
   const int grid = b->cus * per_cu;
   hipLaunchKernelGGL((k_batch_force<B, K>), dim3(grid), dim3(64 * K), 0, b->stream, b->pm,
-                     b->c_off, b->c_n, b->c_npad, b->c_eps2, b->c_G, b->c_quota, use_quota,
-                     b->items, b->counts, b->cap, b->force);
+                     b->c_quota, use_quota, b->items, b->counts, b->cap, b->force);
   return hipGetLastError();
 }
 
@@ -248,14 +253,19 @@ hipError_t launch_force_b(nb_batch* b, int use_quota) {
   }
 }
 
+// Every pass finds the ticket at zero: a step's integrator leaves it so, and a
+// force pass without one is followed by a reset.
 hipError_t enqueue_force(nb_batch* b, int use_quota = 0) {
-  hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, b->stream, b->counts);
+  hipError_t e = hipErrorInvalidValue;
   switch (b->bpl) {
-    case 1: return launch_force_b<1>(b, use_quota);
-    case 2: return launch_force_b<2>(b, use_quota);
-    case 4: return launch_force_b<4>(b, use_quota);
-    default: return hipErrorInvalidValue;
+    case 1: e = launch_force_b<1>(b, use_quota); break;
+    case 2: e = launch_force_b<2>(b, use_quota); break;
+    case 4: e = launch_force_b<4>(b, use_quota); break;
+    default: break;
   }
+  if (e != hipSuccess || use_quota) return e;
+  hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, b->stream, b->counts);
+  return hipGetLastError();
 }
 
 hipError_t enqueue_step(nb_batch* b) {
@@ -271,7 +281,6 @@ hipError_t enqueue_step(nb_batch* b) {
     hipLaunchKernelGGL((k_batch_integrate<false>), dim3(nblk), dim3(256), 0, b->stream, b->blocks,
                        b->counts, b->c_off, b->c_n, b->c_dt, b->c_quota, b->cap, b->pos, b->vel,
                        b->acc, b->force, b->mass, b->pm);
-  hipLaunchKernelGGL(k_batch_advance, dim3(1), dim3(64), 0, b->stream, b->counts);
   return hipGetLastError();
 }
 
@@ -283,11 +292,14 @@ int rebuild_tables(nb_batch* b) {
     if (b->used[s]) slots.push_back(s);
   std::stable_sort(slots.begin(), slots.end(),
                    [&](int a, int c) { return b->h_npad[a] > b->h_npad[c]; });
-  std::vector<int2> items, blocks;
+  std::vector<nb_batch_item> items;
+  std::vector<int2> blocks;
   int64_t inter = 0;
   const int iblock = 64 * b->bpl;
   for (int s : slots) {
-    for (int q = 0; q < b->h_npad[s] / iblock; ++q) items.push_back(make_int2(s, q));
+    for (int q = 0; q < b->h_npad[s] / iblock; ++q)
+      items.push_back({s, b->h_off[s] + q * iblock, b->h_off[s], b->h_npad[s], b->h_off[s] + b->h_n[s],
+                       b->h_eps2[s], b->h_G[s]});
     inter += (int64_t)b->h_n[s] * (b->h_n[s] - 1);
   }
   std::vector<int> by_off(slots);
@@ -296,8 +308,8 @@ int rebuild_tables(nb_batch* b) {
     for (int q = 0; q < b->h_npad[s]; q += 256) blocks.push_back(make_int2(s, b->h_off[s] + q));
   const int counts[2] = {(int)items.size(), (int)blocks.size()};
   if (!items.empty())
-    NB_HIP(hipMemcpyAsync(b->items, items.data(), items.size() * sizeof(int2), hipMemcpyHostToDevice,
-                          b->stream));
+    NB_HIP(hipMemcpyAsync(b->items, items.data(), items.size() * sizeof(nb_batch_item),
+                          hipMemcpyHostToDevice, b->stream));
   if (!blocks.empty())
     NB_HIP(hipMemcpyAsync(b->blocks, blocks.data(), blocks.size() * sizeof(int2),
                           hipMemcpyHostToDevice, b->stream));
@@ -311,11 +323,11 @@ int rebuild_tables(nb_batch* b) {
 void free_batch(nb_batch* b) {
   if (!b) return;
   nb_drop_graph(b->stream, b->graph_exec, b->graph);
+  nb_stage_free(b->stage);
   for (auto& e : b->ev)
     if (e) (void)hipEventDestroy(e);
   void* ps[] = {b->pm,     b->pos,    b->vel,   b->acc,   b->force, b->mass,  b->c_off,
-                b->c_n,    b->c_npad, b->c_eps2, b->c_dt, b->c_G,   b->items, b->blocks,
-                b->counts, b->red,    b->c_quota};
+                b->c_n,    b->c_dt,   b->items, b->blocks, b->counts, b->red,  b->c_quota};
   for (void* p : ps)
     if (p) (void)hipFree(p);
   if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -360,13 +372,13 @@ int nb_batch_create(nb_batch** out, const nb_batch_config* cfg) {
   if (!b) return nb_fail(NB_E_OOM, "nb_batch_create: host allocation failed");
   b->cfg = *cfg;
   b->cap = (cfg->max_bodies + 255) / 256 * 256;
-  // Built-in shape, measured on MI355X on the 512-cluster ensemble
-  // (N_c log-uniform in [256, 32768]) with occupancy-sized launches: one body
-  // per lane and four waves per work item, 14.4 ms per force pass against
-  // 14.7 ms for 1x8 and 15.4 ms for 2x4. nb_batch_tune times every shape on the
-  // batch's own clusters.
+  // Built-in shape, measured on MI355X over whole steps: one body per lane and eight
+  // waves per work item. In us, four / eight / sixteen waves: 512 clusters of 256 to
+  // 32,768 bodies 13,750 / 13,369 / 13,670; 256 of 256 to 8192 781 / 735 / 711; 24 of
+  // 256 to 16,384 267 / 217 / 221; 500 of 64 to 1024 94 / 78 / 76. nb_batch_tune times
+  // every shape on the batch's own clusters.
   b->bpl = cfg->bodies_per_lane > 0 ? cfg->bodies_per_lane : 1;
-  b->jsplit = cfg->j_split > 0 ? cfg->j_split : 4;
+  b->jsplit = cfg->j_split > 0 ? cfg->j_split : 8;
   int dev = 0, cus = 256;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -383,10 +395,9 @@ int nb_batch_create(nb_batch** out, const nb_batch_config* cfg) {
       A((void**)&b->vel, 3 * cap * sizeof(double)) || A((void**)&b->acc, 3 * cap * sizeof(double)) ||
       A((void**)&b->force, 3 * cap * sizeof(double)) || A((void**)&b->mass, cap * sizeof(float)) ||
       A((void**)&b->c_off, mc * sizeof(int)) || A((void**)&b->c_n, mc * sizeof(int)) ||
-      A((void**)&b->c_npad, mc * sizeof(int)) || A((void**)&b->c_eps2, mc * sizeof(float)) ||
-      A((void**)&b->c_dt, mc * sizeof(double)) || A((void**)&b->c_G, mc * sizeof(double)) ||
+      A((void**)&b->c_dt, mc * sizeof(double)) ||
       A((void**)&b->c_quota, mc * sizeof(int)) ||
-      A((void**)&b->items, (cap / 64) * sizeof(int2)) ||
+      A((void**)&b->items, (cap / 64) * sizeof(nb_batch_item)) ||
       A((void**)&b->blocks, (cap / 256) * sizeof(int2)) || A((void**)&b->counts, 16 * sizeof(int)) ||
       A((void**)&b->red, (2 * (cap / 256) + 16) * sizeof(double)))
     return fail(NB_E_OOM, "nb_batch_create: device allocation failed");
@@ -400,6 +411,8 @@ int nb_batch_create(nb_batch** out, const nb_batch_config* cfg) {
   b->h_off.assign(mc, 0);
   b->h_n.assign(mc, 0);
   b->h_npad.assign(mc, 0);
+  b->h_eps2.assign(mc, 0.f);
+  b->h_G.assign(mc, 1.0);
   b->used.assign(mc, 0);
   b->h_quota.assign(mc, kUnlimited);
   b->free_list[0] = b->cap;
@@ -435,55 +448,39 @@ int nb_batch_add(nb_batch* b, const double* pos3, const double* vel3, const doub
   const int64_t off = it->first, len = it->second;
   b->free_list.erase(it);
   if (len > npad) b->free_list[off + npad] = len - npad;
-  // stage the FP64 state as structure-of-arrays slices of the pool
-  const size_t cap = b->cap;
-  std::vector<double> p(3 * n), v(3 * n), a(3 * n, 0.0);
-  for (int64_t i = 0; i < n; ++i)
-    for (int k = 0; k < 3; ++k) {
-      p[k * n + i] = pos3[3 * i + k];
-      v[k * n + i] = vel3[3 * i + k];
-      if (acc3) a[k * n + i] = acc3[3 * i + k];
-    }
-  std::vector<float> m(npad, 0.f);
-  std::copy(mass, mass + n, m.begin());
   const int io = (int)off, in = (int)n, inp = (int)npad;
-  const double ddt = dt, dG = G == 0.f ? 1.0 : (double)G;
-  auto upload = [&]() -> hipError_t {
-    hipError_t e = hipSuccess;
-    auto put = [&](void* dst, const void* src, size_t bytes) {
-      if (e == hipSuccess) e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, b->stream);
-    };
-    for (int k = 0; k < 3; ++k) {
-      put(b->pos + k * cap + off, p.data() + k * n, n * sizeof(double));
-      put(b->vel + k * cap + off, v.data() + k * n, n * sizeof(double));
-      put(b->acc + k * cap + off, a.data() + k * n, n * sizeof(double));
-    }
-    put(b->mass + off, m.data(), npad * sizeof(float));
-    put(b->c_off + slot, &io, sizeof(int));
-    put(b->c_n + slot, &in, sizeof(int));
-    put(b->c_npad + slot, &inp, sizeof(int));
-    put(b->c_eps2 + slot, &eps2, sizeof(float));
-    put(b->c_dt + slot, &ddt, sizeof(double));
-    put(b->c_G + slot, &dG, sizeof(double));
-    put(b->c_quota + slot, &kUnlimited, sizeof(int));
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_batch_refresh, dim3((unsigned)(npad / 256)), dim3(256), 0, b->stream, io,
-                       in, inp, b->cap, b->pos, b->mass, b->pm);
-    e = hipGetLastError();
-    const hipError_t es = hipStreamSynchronize(b->stream);  // host staging buffers die here
-    return e != hipSuccess ? e : es;
-  };
-  const hipError_t ue = upload();
-  if (ue != hipSuccess) {
+  nb_put_args p{};
+  p.pos = pos3;
+  p.vel = vel3;
+  p.acc = acc3;
+  p.mass = mass;
+  p.n = n;
+  p.n_pad = npad;
+  p.stride = b->cap;
+  p.dst[0] = b->pos + off;
+  p.dst[1] = b->vel + off;
+  p.dst[2] = b->acc + off;
+  p.mass_dst = b->mass + off;
+  p.pm = b->pm + off;
+  int rc = nb_put(b->stage, b->stream, b->force, kPackD3, p);  // every force pass writes force anew
+  if (rc == NB_OK) {
+    hipLaunchKernelGGL(k_batch_admit, dim3(1), dim3(64), 0, b->stream, slot, io, in, (double)dt,
+                       b->c_off, b->c_n, b->c_dt, b->c_quota);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) rc = nb_fail(NB_E_HIP, std::string("nb_batch_add: ") + hipGetErrorString(e));
+  }
+  if (rc != NB_OK) {
     // give the segment back (coalescing happens on the next remove)
     if (len > npad) b->free_list.erase(off + npad);
     b->free_list[off] = len;
-    return nb_fail(NB_E_HIP, std::string("nb_batch_add: upload failed: ") + hipGetErrorString(ue));
+    return rc;
   }
   b->used[slot] = 1;
   b->h_off[slot] = io;
   b->h_n[slot] = in;
   b->h_npad[slot] = inp;
+  b->h_eps2[slot] = eps2;
+  b->h_G[slot] = G == 0.f ? 1.0 : (double)G;
   b->h_quota[slot] = kUnlimited;
   b->used_bodies += npad;
   b->dirty = true;
@@ -497,11 +494,10 @@ int nb_batch_remove(nb_batch* b, int32_t id) {
   NB_API_SHARED;
   int rc = check_slot(b, id);
   if (rc) return rc;
-  NB_HIP(hipStreamSynchronize(b->stream));
   int64_t off = b->h_off[id], len = b->h_npad[id];
-  // zero the FP32 view so a stale body can never be read as a source
-  NB_HIP(hipMemsetAsync(b->pm + off, 0, len * sizeof(float4), b->stream));
-  NB_HIP(hipStreamSynchronize(b->stream));
+  // zero the FP32 view so a stale body can never be read as a source (in stream
+  // order: after the steps that still use it, before a later cluster's upload)
+  NB_HIP(nb_launch_fill_i32(reinterpret_cast<int*>(b->pm + off), 0, 4 * len, b->stream));
   b->used[id] = 0;
   b->used_bodies -= len;
   // return the segment to the free list, coalescing neighbours
@@ -611,14 +607,23 @@ int nb_batch_sync(nb_batch* b) {
   NB_CATCH("nb_batch_sync")
 }
 
-static int copy_slices(nb_batch* b, int32_t id, const double* src, double* dst) {
-  const int64_t n = b->h_n[id], off = b->h_off[id];
-  std::vector<double> buf(n);
-  for (int k = 0; k < 3; ++k) {
-    NB_HIP(hipMemcpy(buf.data(), src + k * b->cap + off, n * sizeof(double), hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < n; ++i) dst[3 * i + k] = buf[i];
+static int fetch(nb_batch* b, int32_t id, const double* const* src, double* const* dst, int arrays) {
+  nb_planes p;
+  p.n = b->h_n[id];
+  p.stride = b->cap;
+  const double* from[3];
+  void* to[3];
+  int count = 0;
+  for (int k = 0; k < arrays; ++k)
+    if (dst[k]) {
+      from[count] = src[k] + b->h_off[id];
+      to[count++] = dst[k];
+    }
+  if (count == 0) {
+    NB_HIP(hipStreamSynchronize(b->stream));
+    return NB_OK;
   }
-  return NB_OK;
+  return nb_fetch(b->stage, b->stream, p, kPackD3, count, from, to, nullptr, nullptr);
 }
 
 int nb_batch_forces(nb_batch* b, int32_t id, double* force3) {
@@ -631,8 +636,8 @@ int nb_batch_forces(nb_batch* b, int32_t id, double* force3) {
   rc = rebuild_tables(b);
   if (rc) return rc;
   NB_HIP(enqueue_force(b));
-  NB_HIP(hipStreamSynchronize(b->stream));
-  return copy_slices(b, id, b->force, force3);
+  const double* src = b->force;
+  return fetch(b, id, &src, &force3, 1);
   NB_CATCH("nb_batch_forces")
 }
 
@@ -641,11 +646,9 @@ int nb_batch_download(nb_batch* b, int32_t id, double* pos3, double* vel3, doubl
   NB_API_SHARED;
   int rc = check_slot(b, id);
   if (rc) return rc;
-  NB_HIP(hipStreamSynchronize(b->stream));
-  if (pos3 && (rc = copy_slices(b, id, b->pos, pos3))) return rc;
-  if (vel3 && (rc = copy_slices(b, id, b->vel, vel3))) return rc;
-  if (acc3 && (rc = copy_slices(b, id, b->acc, acc3))) return rc;
-  return NB_OK;
+  const double* src[3] = {b->pos, b->vel, b->acc};
+  double* dst[3] = {pos3, vel3, acc3};
+  return fetch(b, id, src, dst, 3);
   NB_CATCH("nb_batch_download")
 }
 
@@ -656,11 +659,8 @@ int nb_batch_energy(nb_batch* b, int32_t id, double* ekin, double* epot) {
   if (rc) return rc;
   const int n = b->h_n[id], off = b->h_off[id];
   const int blocks = (n + 255) / 256;
-  float eps2 = 0.f;
-  double G = 1.0;
-  NB_HIP(hipMemcpyAsync(&eps2, b->c_eps2 + id, sizeof(float), hipMemcpyDeviceToHost, b->stream));
-  NB_HIP(hipMemcpyAsync(&G, b->c_G + id, sizeof(double), hipMemcpyDeviceToHost, b->stream));
-  NB_HIP(hipStreamSynchronize(b->stream));
+  const float eps2 = b->h_eps2[id];
+  const double G = b->h_G[id];
   hipLaunchKernelGGL(k_batch_energy, dim3(blocks), dim3(256), 0, b->stream, off, n, b->cap,
                      (double)eps2, b->pos, b->vel, b->mass, b->red);
   NB_HIP(hipGetLastError());
