@@ -31,8 +31,9 @@
 
 // One work item of the force pass.
 struct alignas(32) nb_batch_item {
-  int slot, ibase, off, npad, end;  // bodies [off, end), padded to npad; targets from ibase on
-  float eps2;
+  int slot_equal;  // 2 * slot, + 1 for equal masses
+  int ibase, off, npad, end;  // bodies [off, end), padded to npad; targets from ibase on
+  float eps2;                 // of the scaled view (nb_equal_mass)
   double G;
 };
 
@@ -50,6 +51,7 @@ struct nb_batch {
   int* c_off = nullptr;
   int* c_n = nullptr;
   double* c_dt = nullptr;
+  float* c_scale = nullptr;  // of the cluster's FP32 view
   int* c_quota = nullptr;  // steps the cluster takes per nb_batch_step call (INT32_MAX: all)
   // device work tables
   nb_batch_item* items = nullptr;
@@ -61,6 +63,7 @@ struct nb_batch {
   std::vector<int> h_off, h_n, h_npad, h_quota;
   std::vector<float> h_eps2;
   std::vector<double> h_G;
+  std::vector<nb_equal_mass> h_equal;
   nb_stage stage;
   std::vector<char> used;
   std::map<int64_t, int64_t> free_list;  // offset -> size
@@ -89,8 +92,11 @@ constexpr int kUnlimited = NB_BATCH_UNLIMITED;
 // Nothing but this kernel and the integrator runs in a step: this one passes the
 // step on in counts[5], the integrator counts it in counts[4] and resets the ticket,
 // each where the other does not read.
+// At most 80 scalar registers: with 96 the hardware holds seven waves per SIMD, not
+// eight, and a CU one workgroup of sixteen waves instead of two (256 clusters of 256
+// to 8192 bodies: 711 and 876 us at eight and sixteen waves, 675 and 666 with 80).
 template <int B, int K>
-__global__ __launch_bounds__(64 * K) void k_batch_force(
+__global__ __launch_bounds__(64 * K) __attribute__((amdgpu_num_sgpr(80))) void k_batch_force(
     const float4* __restrict__ pm, const int* __restrict__ c_quota, int use_quota,
     const nb_batch_item* __restrict__ items, int* __restrict__ counts, int64_t cap,
     double* __restrict__ force) {
@@ -110,16 +116,18 @@ __global__ __launch_bounds__(64 * K) void k_batch_force(
     if (threadIdx.x == 0)
       next = nitems > (int)gridDim.x ? (int)gridDim.x + atomicAdd(&counts[2], 1) : nitems;
     const nb_batch_item it = items[item];  // wave-uniform
-    if (__builtin_amdgcn_readfirstlane(c_quota[it.slot]) <= call_step) continue;  // block-uniform
+    if (__builtin_amdgcn_readfirstlane(c_quota[it.slot_equal >> 1]) <= call_step) continue;  // block-uniform
     const int ibase = it.ibase + lane;
     nbcore::Targets<B> t;
     nbcore::load_targets<B>(pm, ibase, t);
     const int jlen = it.npad / K;  // npad is a multiple of 256: a multiple of 16 for K <= 16
     const int j0 = it.off + wave * jlen;
-    if (it.eps2 >= 1e-20f)
-      nbcore::accumulate<B, false>(pm, j0, j0 + jlen, it.eps2, t);
+    if (it.slot_equal & 1)
+      nbcore::accumulate<B, false, true>(pm, j0, j0 + jlen, it.eps2, t);
+    else if (it.eps2 >= 1e-20f)
+      nbcore::accumulate<B, false, false>(pm, j0, j0 + jlen, it.eps2, t);
     else
-      nbcore::accumulate<B, true>(pm, j0, j0 + jlen, it.eps2, t);
+      nbcore::accumulate<B, true, false>(pm, j0, j0 + jlen, it.eps2, t);
     nbcore::merge_waves<B, K>(part, wave, lane, t, [&](int a, int b, double sum) {
       const int i = ibase + 64 * b;
       if (i < it.end) force[a * cap + i] = it.G * sum;
@@ -134,8 +142,8 @@ __global__ void k_batch_reset(int* __restrict__ counts) {
 template <bool kEuler>
 __global__ __launch_bounds__(256) void k_batch_integrate(
     const int2* __restrict__ blocks, int* __restrict__ counts, const int* __restrict__ c_off,
-    const int* __restrict__ c_n, const double* __restrict__ c_dt, const int* __restrict__ c_quota,
-    int64_t cap, double* __restrict__ pos, double* __restrict__ vel, double* __restrict__ acc,
+    const int* __restrict__ c_n, const double* __restrict__ c_dt, const float* __restrict__ c_scale,
+    const int* __restrict__ c_quota, int64_t cap, double* __restrict__ pos, double* __restrict__ vel, double* __restrict__ acc,
     const double* __restrict__ force, const float* __restrict__ mass, float4* __restrict__ pm) {
   // grid-stride over the pool blocks in use: the launch is sized for the
   // device, not for the pool's capacity, so an almost empty pool costs little
@@ -152,6 +160,7 @@ __global__ __launch_bounds__(256) void k_batch_integrate(
     if (i - c_off[bl.x] >= c_n[bl.x]) continue;  // padding keeps zero mass
     const double dt = c_dt[bl.x];
     const double h = dt * 0.5;
+    const float scale = c_scale[bl.x];
     double x[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -172,17 +181,19 @@ __global__ __launch_bounds__(256) void k_batch_integrate(
       pos[k] = p;
       x[a] = p;
     }
-    pm[i] = make_float4((float)x[0], (float)x[1], (float)x[2], mass[i]);
+    pm[i] = make_float4((float)x[0] * scale, (float)x[1] * scale, (float)x[2] * scale, mass[i]);
   }
 }
 
-__global__ void k_batch_admit(int slot, int off, int n, double dt, int* __restrict__ c_off,
-                              int* __restrict__ c_n, double* __restrict__ c_dt,
+__global__ void k_batch_admit(int slot, int off, int n, double dt, float scale,
+                              int* __restrict__ c_off, int* __restrict__ c_n,
+                              double* __restrict__ c_dt, float* __restrict__ c_scale,
                               int* __restrict__ c_quota) {
   if (threadIdx.x != 0) return;
   c_off[slot] = off;
   c_n[slot] = n;
   c_dt[slot] = dt;
+  c_scale[slot] = scale;
   c_quota[slot] = kUnlimited;
 }
 
@@ -275,11 +286,11 @@ hipError_t enqueue_step(nb_batch* b) {
   const unsigned nblk = (unsigned)std::min<int64_t>(b->cap / 256, (int64_t)b->cus * 64);
   if (b->cfg.integrator == NB_INTEG_EULER)
     hipLaunchKernelGGL((k_batch_integrate<true>), dim3(nblk), dim3(256), 0, b->stream, b->blocks,
-                       b->counts, b->c_off, b->c_n, b->c_dt, b->c_quota, b->cap, b->pos, b->vel,
+                       b->counts, b->c_off, b->c_n, b->c_dt, b->c_scale, b->c_quota, b->cap, b->pos, b->vel,
                        b->acc, b->force, b->mass, b->pm);
   else
     hipLaunchKernelGGL((k_batch_integrate<false>), dim3(nblk), dim3(256), 0, b->stream, b->blocks,
-                       b->counts, b->c_off, b->c_n, b->c_dt, b->c_quota, b->cap, b->pos, b->vel,
+                       b->counts, b->c_off, b->c_n, b->c_dt, b->c_scale, b->c_quota, b->cap, b->pos, b->vel,
                        b->acc, b->force, b->mass, b->pm);
   return hipGetLastError();
 }
@@ -298,8 +309,9 @@ int rebuild_tables(nb_batch* b) {
   const int iblock = 64 * b->bpl;
   for (int s : slots) {
     for (int q = 0; q < b->h_npad[s] / iblock; ++q)
-      items.push_back({s, b->h_off[s] + q * iblock, b->h_off[s], b->h_npad[s], b->h_off[s] + b->h_n[s],
-                       b->h_eps2[s], b->h_G[s]});
+      items.push_back({2 * s + (b->h_equal[s].on ? 1 : 0), b->h_off[s] + q * iblock, b->h_off[s],
+                       b->h_npad[s], b->h_off[s] + b->h_n[s], b->h_equal[s].eps2,
+                       b->h_equal[s].factor});
     inter += (int64_t)b->h_n[s] * (b->h_n[s] - 1);
   }
   std::vector<int> by_off(slots);
@@ -327,7 +339,8 @@ void free_batch(nb_batch* b) {
   for (auto& e : b->ev)
     if (e) (void)hipEventDestroy(e);
   void* ps[] = {b->pm,     b->pos,    b->vel,   b->acc,   b->force, b->mass,  b->c_off,
-                b->c_n,    b->c_dt,   b->items, b->blocks, b->counts, b->red,  b->c_quota};
+                b->c_n,    b->c_dt,   b->items, b->blocks, b->counts, b->red,  b->c_quota,
+                b->c_scale};
   for (void* p : ps)
     if (p) (void)hipFree(p);
   if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -374,8 +387,8 @@ int nb_batch_create(nb_batch** out, const nb_batch_config* cfg) {
   b->cap = (cfg->max_bodies + 255) / 256 * 256;
   // Built-in shape, measured on MI355X over whole steps: one body per lane and eight
   // waves per work item. In us, four / eight / sixteen waves: 512 clusters of 256 to
-  // 32,768 bodies 13,750 / 13,369 / 13,670; 256 of 256 to 8192 781 / 735 / 711; 24 of
-  // 256 to 16,384 267 / 217 / 221; 500 of 64 to 1024 94 / 78 / 76. nb_batch_tune times
+  // 32,768 bodies 12,495 / 12,193 / 12,733; 256 of 256 to 8192 733 / 675 / 666; 24 of
+  // 256 to 16,384 274 / 205 / 207; 500 of 64 to 1024 91 / 76 / 74. nb_batch_tune times
   // every shape on the batch's own clusters.
   b->bpl = cfg->bodies_per_lane > 0 ? cfg->bodies_per_lane : 1;
   b->jsplit = cfg->j_split > 0 ? cfg->j_split : 8;
@@ -395,7 +408,7 @@ int nb_batch_create(nb_batch** out, const nb_batch_config* cfg) {
       A((void**)&b->vel, 3 * cap * sizeof(double)) || A((void**)&b->acc, 3 * cap * sizeof(double)) ||
       A((void**)&b->force, 3 * cap * sizeof(double)) || A((void**)&b->mass, cap * sizeof(float)) ||
       A((void**)&b->c_off, mc * sizeof(int)) || A((void**)&b->c_n, mc * sizeof(int)) ||
-      A((void**)&b->c_dt, mc * sizeof(double)) ||
+      A((void**)&b->c_dt, mc * sizeof(double)) || A((void**)&b->c_scale, mc * sizeof(float)) ||
       A((void**)&b->c_quota, mc * sizeof(int)) ||
       A((void**)&b->items, (cap / 64) * sizeof(nb_batch_item)) ||
       A((void**)&b->blocks, (cap / 256) * sizeof(int2)) || A((void**)&b->counts, 16 * sizeof(int)) ||
@@ -413,6 +426,7 @@ int nb_batch_create(nb_batch** out, const nb_batch_config* cfg) {
   b->h_npad.assign(mc, 0);
   b->h_eps2.assign(mc, 0.f);
   b->h_G.assign(mc, 1.0);
+  b->h_equal.assign(mc, nb_equal_mass{});
   b->used.assign(mc, 0);
   b->h_quota.assign(mc, kUnlimited);
   b->free_list[0] = b->cap;
@@ -462,10 +476,12 @@ int nb_batch_add(nb_batch* b, const double* pos3, const double* vel3, const doub
   p.dst[2] = b->acc + off;
   p.mass_dst = b->mass + off;
   p.pm = b->pm + off;
+  const nb_equal_mass equal = nb_find_equal_mass(mass, n, eps2, G == 0.f ? 1.0 : (double)G);
+  p.scale = equal.scale;
   int rc = nb_put(b->stage, b->stream, b->force, kPackD3, p);  // every force pass writes force anew
   if (rc == NB_OK) {
     hipLaunchKernelGGL(k_batch_admit, dim3(1), dim3(64), 0, b->stream, slot, io, in, (double)dt,
-                       b->c_off, b->c_n, b->c_dt, b->c_quota);
+                       p.scale, b->c_off, b->c_n, b->c_dt, b->c_scale, b->c_quota);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) rc = nb_fail(NB_E_HIP, std::string("nb_batch_add: ") + hipGetErrorString(e));
   }
@@ -481,6 +497,7 @@ int nb_batch_add(nb_batch* b, const double* pos3, const double* vel3, const doub
   b->h_npad[slot] = inp;
   b->h_eps2[slot] = eps2;
   b->h_G[slot] = G == 0.f ? 1.0 : (double)G;
+  b->h_equal[slot] = equal;
   b->h_quota[slot] = kUnlimited;
   b->used_bodies += npad;
   b->dirty = true;

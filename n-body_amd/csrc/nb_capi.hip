@@ -143,6 +143,28 @@ int nb_direct_parts(int n_pad, int bpl, int jsplit) {
   return most;
 }
 
+nb_equal_mass nb_find_equal_mass(const float* mass, int64_t n, float eps2, double G) {
+  nb_equal_mass e;
+  e.factor = G;
+  e.eps2 = eps2;
+  const float m = mass[0];
+  if (!(m > 0.f) || !std::isfinite(m)) return e;
+  for (int64_t i = 0; i < n; i += 4096) {  // whole blocks compare without a branch per body
+    const int64_t end = std::min(n, i + 4096);
+    bool same = true;
+    for (int64_t k = i; k < end; ++k) same = same && mass[k] == m;
+    if (!same) return e;
+  }
+  const int shift = std::max(0, (std::ilogb(m) + 3) / 3);  // 2^(3 shift) > m
+  const float scale = std::ldexp(1.f, -shift);
+  if (!(eps2 * scale * scale >= 1e-20f)) return e;
+  e.on = true;
+  e.scale = scale;
+  e.eps2 = eps2 * scale * scale;
+  e.factor = G * (double)m * ((double)scale * (double)scale);
+  return e;
+}
+
 // Valid direct-sum launch shapes (see launch_b in nb_direct.hip).
 bool nb_valid_shape(int bpl, int jsplit) {
   switch (bpl) {
@@ -380,6 +402,15 @@ void nb_destroy(nb_ctx* ctx) {
   free_ctx(ctx);
 }
 
+// What the inner loop may leave out for these masses. k_direct_small and Barnes-Hut
+// have no such form.
+static void choose_form(nb_ctx* c, const float* mass) {
+  c->equal = nb_equal_mass{};
+  c->equal.factor = c->G;
+  if (c->cfg.solver == NB_SOLVER_DIRECT && !c->small)
+    c->equal = nb_find_equal_mass(mass, c->n, c->cfg.eps2, c->G);
+}
+
 static int upload_common(nb_ctx* c, const std::vector<double>& p, const std::vector<double>& v,
                          const std::vector<double>& a, const float* mass) {
   const size_t n = c->n;
@@ -390,7 +421,8 @@ static int upload_common(nb_ctx* c, const std::vector<double>& p, const std::vec
   NB_HIP(hipMemcpyAsync(c->acc, a.data(), 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   NB_HIP(hipMemcpyAsync(c->mass, mass, n * sizeof(float), hipMemcpyHostToDevice, c->stream));
   NB_HIP(nb_launch_fill_i32(c->flags, 0, 4, c->stream));
-  NB_HIP(nb_launch_refresh_pm(c));
+  choose_form(c, mass);
+  NB_HIP(nb_launch_refresh_pm(c, c->equal.scale));
   NB_HIP(hipStreamSynchronize(c->stream));
   c->uploaded = true;
   c->tree_valid = false;
@@ -414,6 +446,8 @@ static int upload_packed(nb_ctx* c, int layout, const void* pos, const void* vel
   p.dst[2] = c->acc;
   p.mass_dst = c->mass;
   p.pm = c->pm;
+  choose_form(c, mass);
+  p.scale = c->equal.scale;
   p.flags = c->flags;
   const int rc = nb_put(c->stage, c->stream, c->force, layout, p);  // every force pass writes force anew
   if (rc) return rc;
@@ -508,7 +542,7 @@ static int force_pass(nb_ctx* c, int layout, void* out) {
     if (c->parts > 1) {
       src = c->part;
       p.parts = c->parts;
-      p.G = c->G;
+      p.G = c->equal.factor;
     }
   }
   int flags = 0;
@@ -697,9 +731,10 @@ int nb_reorder(nb_ctx* c) {
     c->slot_of = nullptr;
     return nb_fail(NB_E_OOM, "device allocation failed (body order)");
   }
+  if (c->equal.scale != 1.f) NB_HIP(nb_launch_refresh_pm(c, 1.f));  // codes of the bodies themselves
   NB_HIP(nb_morton_sort(c));
   NB_HIP(nb_launch_permute_state(c));
-  NB_HIP(nb_launch_refresh_pm(c));
+  NB_HIP(nb_launch_refresh_pm(c, c->equal.scale));
   const size_t n = c->n;
   std::vector<uint32_t> perm(n);
   NB_HIP(hipMemcpyAsync(perm.data(), c->bh.vals[0], sizeof(uint32_t) * n, hipMemcpyDeviceToHost,

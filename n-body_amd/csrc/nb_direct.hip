@@ -30,7 +30,7 @@ namespace {
 // 16-source units; block (ib, p) takes the slices p * K .. p * K + K - 1. With one
 // part the block writes the forces; with more it writes its FP64 partial sums,
 // without G, to out[p][3][n], and whoever reads them adds the parts in order.
-template <int B, int K, bool kGuard>
+template <int B, int K, bool kGuard, bool kUniform>
 __global__ __launch_bounds__(64 * K) void k_direct(const float4* __restrict__ pm, int n,
                                                    int n_pad, float eps2, double G,
                                                    double* __restrict__ out) {
@@ -41,7 +41,7 @@ __global__ __launch_bounds__(64 * K) void k_direct(const float4* __restrict__ pm
   nbcore::load_targets<B>(pm, ibase, t);
   const int64_t units = n_pad / 16, slices = (int64_t)gridDim.y * K;
   const int64_t slice = (int64_t)blockIdx.y * K + wave;
-  nbcore::accumulate<B, kGuard>(pm, 16 * (int)(units * slice / slices),
+  nbcore::accumulate<B, kGuard, kUniform>(pm, 16 * (int)(units * slice / slices),
                                 16 * (int)(units * (slice + 1) / slices), eps2, t);
   __shared__ double part[K > 1 ? K : 1][3][B][64];
   const double g = gridDim.y == 1 ? G : 1.0;
@@ -56,12 +56,13 @@ template <int B, int K>
 hipError_t launch_bk(const nb_ctx* c) {
   const dim3 grid(c->n_pad / (64 * B), c->parts);
   double* out = c->parts > 1 ? c->part : c->force;
-  if (c->guard)
-    hipLaunchKernelGGL((k_direct<B, K, true>), grid, dim3(64 * K), 0, c->stream, c->pm, c->n,
-                       c->n_pad, c->cfg.eps2, c->G, out);
-  else
-    hipLaunchKernelGGL((k_direct<B, K, false>), grid, dim3(64 * K), 0, c->stream, c->pm, c->n,
-                       c->n_pad, c->cfg.eps2, c->G, out);
+  const auto launch = [&](auto kernel, float eps2) {
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * K), 0, c->stream, c->pm, c->n, c->n_pad, eps2,
+                       c->equal.factor, out);
+  };
+  if (c->equal.on) launch(k_direct<B, K, false, true>, c->equal.eps2);
+  else if (c->guard) launch(k_direct<B, K, true, false>, c->cfg.eps2);
+  else launch(k_direct<B, K, false, false>, c->cfg.eps2);
   return hipGetLastError();
 }
 
@@ -102,7 +103,8 @@ __global__ __launch_bounds__(256) void k_integrate(int n, double dt, double* __r
                                                    double* __restrict__ acc,
                                                    const double* __restrict__ force, int parts,
                                                    double G, const float* __restrict__ mass,
-                                                   float4* __restrict__ pm, int* __restrict__ flags) {
+                                                   float scale, float4* __restrict__ pm,
+                                                   int* __restrict__ flags) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   const double h = dt * 0.5;
@@ -128,7 +130,7 @@ __global__ __launch_bounds__(256) void k_integrate(int n, double dt, double* __r
     x[a] = p;
     finite = finite && isfinite(p) && isfinite(v);
   }
-  pm[i] = make_float4((float)x[0], (float)x[1], (float)x[2], mass[i]);
+  pm[i] = make_float4((float)x[0] * scale, (float)x[1] * scale, (float)x[2] * scale, mass[i]);
   if (!finite) atomicOr(flags, 1);
 }
 
@@ -250,14 +252,15 @@ hipError_t launch_small(const nb_ctx* c, float4* pm_next) {
 }
 
 __global__ __launch_bounds__(256) void k_refresh_pm(int n, int n_pad, const double* __restrict__ pos,
-                                                    const float* __restrict__ mass,
+                                                    const float* __restrict__ mass, float scale,
                                                     float4* __restrict__ pm) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n_pad) return;
   if (i < n)
-    pm[i] = make_float4((float)pos[i], (float)pos[n + i], (float)pos[2 * n + i], mass[i]);
+    pm[i] = make_float4((float)pos[i] * scale, (float)pos[n + i] * scale,
+                        (float)pos[2 * n + i] * scale, mass[i]);
   else
-    pm[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    pm[i] = nbcore::far_pad();
 }
 
 __global__ __launch_bounds__(256) void k_fill_i32(int* __restrict__ p, int v, int64_t count) {
@@ -362,15 +365,16 @@ __global__ __launch_bounds__(kEnergyThreads) void k_energy(int n, const double* 
 // fixed tree, so the result does not depend on scheduling.
 __global__ __launch_bounds__(256) void k_ref_f64(const float4* __restrict__ pm, int n,
                                                  const int* __restrict__ slots, double eps2,
-                                                 double G, double* __restrict__ acc3) {
+                                                 double G, double unscale,
+                                                 double* __restrict__ acc3) {
   __shared__ double red[3][256];
   const int i = slots[blockIdx.x];
   const float4 me = pm[i];
-  const double xi = me.x, yi = me.y, zi = me.z;
+  const double xi = me.x * unscale, yi = me.y * unscale, zi = me.z * unscale;  // exact
   double ax = 0.0, ay = 0.0, az = 0.0;
   for (int j = threadIdx.x; j < n; j += 256) {
     const float4 q = pm[j];
-    const double dx = (double)q.x - xi, dy = (double)q.y - yi, dz = (double)q.z - zi;
+    const double dx = q.x * unscale - xi, dy = q.y * unscale - yi, dz = q.z * unscale - zi;
     const double r2 = dx * dx + dy * dy + dz * dz + eps2;
     const double s = j == i ? 0.0 : (double)q.w / (r2 * sqrt(r2));
     ax += s * dx;
@@ -394,7 +398,7 @@ __global__ __launch_bounds__(256) void k_ref_f64(const float4* __restrict__ pm, 
 hipError_t nb_launch_ref_f64(nb_ctx* c, const int* slots, int k, double* acc3) {
   if (k <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_ref_f64, dim3(k), dim3(256), 0, c->stream, c->pm, c->n, slots,
-                     (double)c->cfg.eps2, c->G, acc3);
+                     (double)c->cfg.eps2, c->G, 1.0 / c->equal.scale, acc3);
   return hipGetLastError();
 }
 
@@ -421,7 +425,7 @@ hipError_t nb_launch_integrate(nb_ctx* c) {
   const auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((c->n + 255) / 256), dim3(256), 0, c->stream, c->n,
                        (double)c->cfg.dt, c->pos, c->vel, c->acc, parts ? c->part : c->force,
-                       c->parts, c->G, c->mass, c->pm, c->flags);
+                       c->parts, c->equal.factor, c->mass, c->equal.scale, c->pm, c->flags);
   };
   if (c->cfg.integrator == NB_INTEG_EULER)
     parts ? launch(k_integrate<true, true>) : launch(k_integrate<true, false>);
@@ -430,9 +434,9 @@ hipError_t nb_launch_integrate(nb_ctx* c) {
   return hipGetLastError();
 }
 
-hipError_t nb_launch_refresh_pm(nb_ctx* c) {
+hipError_t nb_launch_refresh_pm(nb_ctx* c, float scale) {
   hipLaunchKernelGGL(k_refresh_pm, dim3(c->n_pad / 256), dim3(256), 0, c->stream, c->n, c->n_pad,
-                     c->pos, c->mass, c->pm);
+                     c->pos, c->mass, scale, c->pm);
   return hipGetLastError();
 }
 

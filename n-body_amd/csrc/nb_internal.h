@@ -201,6 +201,19 @@ struct nb_stage {
   bool busy = false;        // an enqueued kernel still reads it
 };
 
+// Equal masses m > 0 leave the direct sum's inner loop. The coordinates of its FP32
+// view are then multiplied by `scale`, a power of two (exact), at or below m^{-1/3}
+// and at most 1, and the sum by m * scale^2: its terms r^-3 are then no smaller than the
+// m r^-3 they stand for, so nothing underflows that did not before, and with the
+// scaled eps2 at 1e-20 or more nothing overflows. Not used where eps2 is smaller
+// (the guarded kernels).
+struct nb_equal_mass {
+  bool on = false;
+  float scale = 1.f, eps2 = 0.f;  // of the view
+  double factor = 1.0;            // G times the sum's factor
+};
+nb_equal_mass nb_find_equal_mass(const float* mass, int64_t n, float eps2, double G);
+
 struct nb_ctx {
   nb_config cfg{};
   int64_t cap_n = 0;  // bodies the device buffers were sized for (nb_ctx_rebind limit)
@@ -217,7 +230,7 @@ struct nb_ctx {
   double* acc = nullptr;
   double* force = nullptr;   // last force pass, [3][n]
   float* mass = nullptr;     // [n_pad], zero in the padding
-  float4* pm = nullptr;      // FP32 force view (x, y, z, m), [n_pad]
+  float4* pm = nullptr;      // FP32 force view (x, y, z, m), [n_pad], far-away padding
   int* flags = nullptr;      // device status word (bit 0: non-finite state)
 
   // direct-sum launch shape
@@ -228,6 +241,7 @@ struct nb_ctx {
   int parts = 1;   // workgroups per i-block, each with a part of the sources
   double* part = nullptr;  // their partial sums [parts][3][n], behind force
   bool guard = false;
+  nb_equal_mass equal;  // k_direct's form for equal masses
   int walk_stack = 0;  // BH traversal stack region cap (0: the full kStackCap); a test hook
 
   nb_bh_state bh;
@@ -288,6 +302,7 @@ struct nb_put_args {
   double* dst[3];               // device: first planes of positions, velocities, accelerations
   float* mass_dst;
   float4* pm;
+  float scale;                  // of the coordinates in pm
   int* flags;                   // four words to clear, or null
 };
 // Copies a system to the device. The host arrays may be reused on return; the
@@ -299,7 +314,7 @@ void nb_stage_free(nb_stage& st);
 hipError_t nb_launch_direct(nb_ctx* c);  // pm -> force, or part when parts > 1
 hipError_t nb_launch_small_step(nb_ctx* c);  // force + integration of a `small` context
 hipError_t nb_launch_integrate(nb_ctx* c);  // force or part + state -> state, pm
-hipError_t nb_launch_refresh_pm(nb_ctx* c);  // pos, mass -> pm
+hipError_t nb_launch_refresh_pm(nb_ctx* c, float scale);  // pos * scale, mass -> pm
 hipError_t nb_launch_fill_i32(int* p, int v, int64_t count, hipStream_t s);
 // state -> part: 4 * kEnergyKinBlocks kinetic, then nb_energy_pot_blocks(n) potential
 // partials, then the device status word (as an int)

@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "nb_force_core.h"
 #include "nb_internal.h"
 
 namespace {
@@ -108,9 +109,10 @@ struct UnpackArgs {
   const float* mass;   // n masses
   double* dst[3];      // first plane of each array (null: the array is not part of this call)
   int64_t stride;
-  int n, n_pad;        // bodies, and the entries of pm to fill (zero mass past n)
+  int n, n_pad;        // bodies, and the entries of pm to fill (padding past n)
   float* mass_dst;     // null: the masses are in place
   float4* pm;          // written with the positions
+  float scale;         // of the coordinates in pm
   int* flags;          // four words set to zero, or null
 };
 
@@ -134,8 +136,9 @@ __global__ __launch_bounds__(256) void k_unpack(UnpackArgs a) {
 #pragma unroll
       for (int c = 0; c < 3; ++c) a.dst[k][c * a.stride + i] = v[c];
     if (k == 0 && a.pm && i < a.n_pad)
-      a.pm[i] = body ? make_float4((float)v[0], (float)v[1], (float)v[2], m)
-                     : make_float4(0.f, 0.f, 0.f, 0.f);
+      a.pm[i] = body ? make_float4((float)v[0] * a.scale, (float)v[1] * a.scale,
+                                   (float)v[2] * a.scale, m)
+                     : nbcore::far_pad();
   }
 }
 
@@ -229,6 +232,7 @@ int nb_put(nb_stage& st, hipStream_t s, void* dev_tmp, int layout, const nb_put_
   a.stride = p.stride;
   a.n = (int)p.n;
   a.n_pad = (int)p.n_pad;
+  a.scale = p.scale;
   const int64_t per = body_bytes(layout);
   const void* from[3] = {p.pos, p.vel, p.acc};
   if (3 * p.n * per + 4 * p.n <= kStageBytes) {

@@ -153,3 +153,36 @@ def test_one_launch_steps(nb, n, integrator):
             out.append(np.concatenate(sim.download_f64() + (sim.forces_f64(),)))
     for o in out[1:]:
         np.testing.assert_array_equal(o, out[0])
+
+
+@pytest.mark.parametrize("m, radius, eps2, G", [(1.0, 100.0, 40.0, 1.0), (2.4, 50.0, 0.5, 1.0), (1e-9, 1e-3, 1e-9, 1.0),
+                                                (2e30, 1e13, 1e20, 6.674e-11), (3e38, 1e15, 1e26, 1e-11),
+                                                (7.0, 1e14, 1e20, 1.0), (5.0, 10.0, 1e-19, 1.0)])
+@pytest.mark.parametrize("n", [1, 257, 9001])
+def test_equal_masses_over_the_range_of_scales(nb, ora, m, radius, eps2, G, n):
+    """Equal masses leave the inner loop and the view is scaled by a power of two:
+    forces against FP64 at masses and lengths where r^-3 alone would leave FP32's
+    range, for a single system and a cluster, before and after a step and a reorder;
+    one different mass takes the general form."""
+    pos, vel, _ = nb.ic_ball(3 + n, n, radius, 1.0)
+    tgt = np.arange(0, n, max(1, n // 200))
+    for mass in (np.full(n, m, np.float32), np.concatenate([np.full(n - 1, m), [m / 2]]).astype(np.float32)):
+        ref = G * ora.direct_f64(pos.astype(np.float32).astype(np.float64), mass.astype(np.float64), np.float32(eps2),
+                                 targets=tgt)
+        scale = np.linalg.norm(ref, axis=1).max() + 1e-300
+        with nb.Simulation(n, eps2, 0.0, G=G) as sim:  # dt = 0: a step moves nothing
+            sim.upload(pos, np.zeros_like(pos), mass)
+            got = [sim.forces_f64(), sim.direct_f64(tgt)]
+            sim.step(1)
+            got.append(sim.download_f64()[2])
+            sim.reorder()
+            got += [sim.forces_f64(), sim.direct_f64(tgt)]
+        with nb.Batch(n + 255, 1) as b:
+            c = b.add(pos, np.zeros_like(pos), mass, eps2, 0.0, G)
+            got.append(b.forces(c))
+            b.step(2)
+            got.append(b.download(c)[2])
+        for f in got:
+            f = f if len(f) == len(tgt) else f[tgt]
+            # 256-source FP32 sums, folded: 256 roundings of the largest force at worst
+            assert np.abs(f - ref).max() <= 256 * 2.0 ** -24 * scale
