@@ -627,7 +627,7 @@ int nb_energy(nb_ctx* c, double* ekin, double* epot, double p[3]) {
   if (!c->uploaded) return nb_fail(NB_E_ARG, "nb_energy: no particle system uploaded");
   const int kin_n = 4 * kEnergyKinBlocks;
   const int pot_n = nb_energy_pot_blocks(c->n);
-  const int rc = nb_stage_ready(c->stage, c->stream);
+  const int rc = nb_stage_ready(c->stage, c->stream, kStageBytes);
   if (rc) return rc;
   const double* h = reinterpret_cast<const double*>(c->stage.host);
   NB_HIP(nb_launch_energy(c, reinterpret_cast<double*>(c->stage.host)));

@@ -195,8 +195,10 @@ struct nb_bh_state {
 // and large results in halves (nb_pack.hip). Used by one host thread at a time,
 // on the owner's stream only.
 constexpr int64_t kStageBytes = 2 << 20;
+constexpr int64_t kLargeStageBytes = 16 << 20;  // from twice as many bytes in one call on
 struct nb_stage {
   char* host = nullptr;
+  int64_t bytes = 0;
   hipEvent_t done[2] = {};  // each half has been filled
   bool busy = false;        // an enqueued kernel still reads it
 };
@@ -289,7 +291,7 @@ struct nb_planes {
   int parts = 1;       // > 1: values are G times the sum of `parts` arrays of 3 * stride
   double G = 1.0;
 };
-int nb_stage_ready(nb_stage& st, hipStream_t s);  // allocated, and free for new content
+int nb_stage_ready(nb_stage& st, hipStream_t s, int64_t bytes);  // at least that large, and free
 // Copies `arrays` device arrays to the host arrays dst, packed, and waits for
 // them; *flags_out receives the device word *flags (0 if null).
 int nb_fetch(nb_stage& st, hipStream_t s, const nb_planes& p, int layout, int arrays,

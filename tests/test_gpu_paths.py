@@ -186,3 +186,20 @@ def test_equal_masses_over_the_range_of_scales(nb, ora, m, radius, eps2, G, n):
             f = f if len(f) == len(tgt) else f[tgt]
             # 256-source FP32 sums, folded: 256 roundings of the largest force at worst
             assert np.abs(f - ref).max() <= 256 * 2.0 ** -24 * scale
+
+
+@pytest.mark.parametrize("n", [89000, 250001, 700001])
+def test_large_host_copies(nb, n):
+    """Downloads above 4 MB, where several threads copy, and above 32 MB, through the
+    larger stage (which replaces the smaller one on the way)."""
+    rng = np.random.default_rng(n)
+    pos, vel, acc = (rng.normal(size=(n, 3)) for _ in range(3))
+    with nb.Simulation(n, EPS2, DT, solver=nb.SOLVER_BH) as sim:
+        sim.upload(pos, vel, np.ones(n, np.float32), acc)
+        np.testing.assert_array_equal(sim.render_view()[:, :3], pos.astype(np.float32))
+        for _ in range(2):
+            for got, want in zip(sim.download_f64(), (pos, vel, acc)):
+                np.testing.assert_array_equal(got, want)
+            for got, want in zip(sim.download(), (pos, vel, acc)):
+                np.testing.assert_array_equal(got[:, :3], want.astype(np.float32))
+        sim.energy() if n < 100000 else sim.sync()
