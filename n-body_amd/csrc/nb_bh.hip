@@ -458,8 +458,8 @@ __global__ __launch_bounds__(256) void k_permute_f32(const float* __restrict__ s
 }
 
 // ---- 6. octree ------------------------------------------------------------------------
-__device__ __forceinline__ int link_count(int w) { return w >> 4; }
-__device__ __forceinline__ int link_level(int w) { return w & 15; }
+__device__ __forceinline__ int span_count(int w) { return w >> 4; }
+__device__ __forceinline__ int span_level(int w) { return w & 15; }
 
 // Octal digits that two 30-bit codes share from the top (0..10).
 __device__ __forceinline__ int common_level(uint32_t a, uint32_t b) {
@@ -645,8 +645,8 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_emit(
     const float4* __restrict__ pms, int n, const double4* __restrict__ part,
     const unsigned char* __restrict__ marks, const int* __restrict__ level_cnt,
     const int* __restrict__ counters, int64_t max_nodes, double4* __restrict__ prefix,
-    int4* __restrict__ link, int* __restrict__ node_end, int* __restrict__ level_off,
-    int* __restrict__ flags) {
+    nb_node* __restrict__ nodes, int* __restrict__ next, int* __restrict__ node_end,
+    int* __restrict__ level_off, int* __restrict__ flags) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint64_t lt = (uint64_t(1) << lane) - 1;
   const int e = blockIdx.x * kTreeTile + threadIdx.x;
@@ -687,7 +687,6 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_emit(
   const double4 below = shfl_up4(x, 1);  // inclusive value of the lane below
   const double4 start = s_mom[wave];
   if (e < n) prefix[e] = lane > 0 ? add4(start, below) : start;
-  int* words = reinterpret_cast<int*>(link);
   // idx[l]: index of a node of level l that starts at e
   int idx[kLevels + 1], rope = -1;
 #pragma unroll
@@ -704,12 +703,13 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_emit(
     if (__ballot(starts || ends) == 0) continue;
     const int64_t at = idx[l];
     if (starts && at < max_nodes) {
-      words[4 * at] = l < D ? idx[l + 1] : -1;
-      *reinterpret_cast<int2*>(words + 4 * at + 2) = make_int2(e, l);
+      nodes[at].first = l < D ? idx[l + 1] : -1;
+      nodes[at].start = e;
+      nodes[at].span = l;
     }
     const int64_t in = at - (starts ? 0 : 1);  // the node of level l around e
     if (ends && in >= 0 && in < max_nodes) {
-      words[4 * in + 1] = rope;
+      next[in] = rope;
       node_end[in] = e + 1;
     }
     over = over || (starts && at >= max_nodes);
@@ -839,10 +839,10 @@ __device__ __forceinline__ float open_radius2(float4 cm, uint32_t code, int l,
 }
 
 // One thread per node: its centre of mass from the prefix, its opening radius,
-// its link's last word (count << 4 | level), and the wave ranges of the children
+// its span (count << 4 | level), and the wave ranges of the children
 // of nodes holding more than kWaveBodies bodies, in records of one or two: one
 // atomic per wave reserves the records of all its lanes.
-__global__ __launch_bounds__(256) void k_tree_com(int4* __restrict__ link,
+__global__ __launch_bounds__(256) void k_tree_com(nb_node* __restrict__ nodes,
                                                   const int* __restrict__ node_end, int n,
                                                   int64_t max_nodes,
                                                   const int* __restrict__ level_off,
@@ -852,46 +852,45 @@ __global__ __launch_bounds__(256) void k_tree_com(int4* __restrict__ link,
                                                   const float* __restrict__ geom, int cubic,
                                                   float theta, int leaf, int pairs,
                                                   int4* __restrict__ waves,
-                                                  int* __restrict__ wctl,
-                                                  float4* __restrict__ com,
-                                                  float* __restrict__ r2) {
+                                                  int* __restrict__ wctl) {
   const int total = (int)min((int64_t)level_off[kMaxLevel + 1], max_nodes);
   const int lane = threadIdx.x & 63;
-  int* words = reinterpret_cast<int*>(link);
   // Rounds are uniform across the block, so every lane of a wave reaches the
   // wave-wide record reservation.
   for (int k0 = blockIdx.x * 256; k0 < total; k0 += gridDim.x * 256) {
     const int k = k0 + threadIdx.x;
     int starts[8], ends[8], nc = 0, nrec = 0, l = 0;
     if (k < total) {
-      const int4 nd = link[k];
-      const int first = nd.x, start = nd.z;
-      l = nd.w & 15;
+      const int first = nodes[k].first, start = nodes[k].start;
+      l = nodes[k].span & 15;
       const int end = node_end[k], cnt = end - start;
-      words[4 * (int64_t)k + 3] = cnt << 4 | l;
-      float4 cm;
+      nb_node nd{make_float4(0.f, 0.f, 0.f, 0.f), -1.f, first, start, cnt << 4 | l};
       if (start < 0 || cnt < 1 || end > n) {
-        com[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-        r2[k] = -1.f;
+        nodes[k].com = nd.com;
+        nodes[k].r2 = nd.r2;
+        nodes[k].span = nd.span;
       } else {
         if (cnt == 1) {
-          cm = pms[start];
+          nd.com = pms[start];
         } else {
           const double4 a = prefix[start], b = prefix[end];
           const double m = b.x - a.x;
           const double inv = m > 0.0 ? 1.0 / m : 0.0;
-          cm = make_float4((float)((b.y - a.y) * inv), (float)((b.z - a.z) * inv),
-                           (float)((b.w - a.w) * inv), (float)m);
+          nd.com = make_float4((float)((b.y - a.y) * inv), (float)((b.z - a.z) * inv),
+                               (float)((b.w - a.w) * inv), (float)m);
         }
-        com[k] = cm;
-        r2[k] = open_radius2(cm, codes[start], l, geom, cubic, theta);
+        nd.r2 = open_radius2(nd.com, codes[start], l, geom, cubic, theta);
+        // the other threads read `first` and `start` only, which stay as they are
+        nodes[k].com = nd.com;
+        nodes[k].r2 = nd.r2;
+        nodes[k].span = nd.span;
         if (cnt > kWaveBodies && first >= 0 && l < kMaxLevel) {
           // the children are consecutive nodes of the next level and tile the range
           const int last = min(level_off[l + 2], total);
           int s[8];  // eight independent loads; past the last child: >= end
 #pragma unroll
           for (int q = 0; q < 8; ++q)
-            s[q] = first + q < last ? words[4 * (int64_t)(first + q) + 2] : end;
+            s[q] = first + q < last ? nodes[first + q].start : end;
 #pragma unroll
           for (int q = 0; q < 8; ++q)
             if (s[q] < end) {
@@ -913,21 +912,20 @@ __global__ __launch_bounds__(256) void k_tree_com(int4* __restrict__ link,
 }
 
 // ---- 8. traversal ---------------------------------------------------------------------------
-// kModified: open with the default traversal's radius (r2[i] < d^2) instead of
+// kModified: open with the default traversal's radius (r2 < d^2) instead of
 // the reference's test; used only to count what that test needs per body.
 template <bool kCount, bool kModified = false>
 __global__ __launch_bounds__(256) void k_traverse(const float4* __restrict__ pms,
                                                   const uint32_t* __restrict__ perm, int n,
-                                                  const float4* __restrict__ com,
-                                                  const int4* __restrict__ link,
+                                                  const nb_node* __restrict__ nodes,
+                                                  const int* __restrict__ next,
                                                   const int* __restrict__ level_off,
                                                   int64_t max_nodes,
                                                   const float* __restrict__ geom, float theta2,
                                                   float eps2, double G,
                                                   double* __restrict__ force,
                                                   unsigned long long* __restrict__ inter,
-                                                  int* __restrict__ flags,
-                                                  const float* __restrict__ r2 = nullptr) {
+                                                  int* __restrict__ flags) {
   __shared__ float side2[kMaxLevel + 1];
   if (threadIdx.x <= kMaxLevel) side2[threadIdx.x] = geom[6 + threadIdx.x];
   __syncthreads();
@@ -945,11 +943,11 @@ __global__ __launch_bounds__(256) void k_traverse(const float4* __restrict__ pms
         atomicOr(flags, 4);
         break;
       }
-      const float4 c = com[i];
-      const int4 nd = link[i];
+      const nb_node nd = nodes[i];
+      const float4 c = nd.com;
       const float dx = c.x - me.x, dy = c.y - me.y, dz = c.z - me.z;
       const float d2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-      if (kModified ? r2[i] < d2 : side2[link_level(nd.w)] < theta2 * d2) {
+      if (kModified ? nd.r2 < d2 : side2[span_level(nd.span)] < theta2 * d2) {
         if (c.w > 0.f && d2 > 0.f) {
           const float inv = __builtin_amdgcn_rsqf(d2 + eps2);
           const float s = (c.w * inv) * (inv * inv);
@@ -958,10 +956,10 @@ __global__ __launch_bounds__(256) void k_traverse(const float4* __restrict__ pms
           az = fmaf(dz, s, az);
           if (kCount) ++cnt;
         }
-        i = nd.y;
-      } else if (nd.x < 0) {
-        const int e = min(nd.z + link_count(nd.w), n);
-        for (int b = max(nd.z, 0); b < e; ++b) {
+        i = next[i];
+      } else if (nd.first < 0) {
+        const int e = min(nd.start + span_count(nd.span), n);
+        for (int b = max(nd.start, 0); b < e; ++b) {
           const float4 q = pms[b];
           const float bx = q.x - me.x, by = q.y - me.y, bz = q.z - me.z;
           const float b2 = fmaf(bz, bz, fmaf(by, by, bx * bx));
@@ -974,9 +972,9 @@ __global__ __launch_bounds__(256) void k_traverse(const float4* __restrict__ pms
             if (kCount) ++cnt;
           }
         }
-        i = nd.y;
+        i = next[i];
       } else {
-        i = nd.x;
+        i = nd.first;
       }
     }
     const uint32_t o = perm[t];
@@ -1051,7 +1049,7 @@ constexpr uint32_t kCellBit = 0x80000000u;    // list entry refers to a cell, no
 template <bool kCount, bool kGuard>
 __device__ __forceinline__ void list_flush(const uint32_t* list, int lc, float4* stage, int lane,
                                            int slice, int log2S, const float4* __restrict__ pms,
-                                           const float4* __restrict__ com, float4 me, float eps2_s,
+                                           const nb_node* __restrict__ nodes, float4 me, float eps2_s,
                                            float& sx, float& sy, float& sz, float& cx, float& cy,
                                            float& cz, unsigned long long& cnt) {
   float ax = 0.f, ay = 0.f, az = 0.f;
@@ -1066,7 +1064,7 @@ __device__ __forceinline__ void list_flush(const uint32_t* list, int lc, float4*
     float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
     if (e + lane < lc) {
       const uint32_t id = list[e + lane];
-      g = (id & kCellBit) ? com[id & ~kCellBit] : pms[id];
+      g = (id & kCellBit) ? nodes[id & ~kCellBit].com : pms[id];
     }
     return g;
   };
@@ -1101,6 +1099,47 @@ __device__ __forceinline__ void list_flush(const uint32_t* list, int lc, float4*
   nbcore::two_sum_fold(sx, cx, ax);
   nbcore::two_sum_fold(sy, cy, ay);
   nbcore::two_sum_fold(sz, cz, az);
+}
+
+// Bits of m below this lane.
+__device__ __forceinline__ int bits_below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+}
+
+// Append the bodies of the leaves that the lanes hold (in lane order) to a list of
+// kCap entries. A prefix sum places each lane's bodies, which it writes itself: at
+// most leaf_size rounds for all of them. One round per leaf, the lanes together, was a
+// chain of scalar waits that near ranges paid for a dozen leaves per iteration (20,011
+// bodies: traversal 120 us, now 73; 65,536 199, now 162). Leaves that do not fit
+// together go one by one, 64 bodies at a time.
+template <int kCap, typename Flush>
+__device__ __forceinline__ void list_leaves(uint32_t* list, int& lc, int lane, bool leaf, int start,
+                                            int count, int n, Flush flush) {
+  uint64_t bl = __ballot(leaf);
+  if (bl == 0) return;
+  const int mine = leaf ? count : 0;
+  const int incl = wave_incl_scan(mine);
+  const int total = __builtin_amdgcn_readlane(incl, 63);
+  if (total <= kCap) {
+    if (lc + total > kCap) flush();
+    uint32_t* at = list + lc + incl - mine;
+    for (int k = 0; __ballot(k < mine); ++k)
+      if (k < mine) at[k] = (uint32_t)min(start + k, n - 1);
+    lc += total;
+    return;
+  }
+  while (bl) {
+    const int src = __ffsll((unsigned long long)bl) - 1;
+    bl &= bl - 1;
+    const int ls = __builtin_amdgcn_readlane(start, src);
+    const int lcount = __builtin_amdgcn_readlane(count, src);
+    for (int off = 0; off < lcount; off += 64) {
+      const int m = min(64, lcount - off);
+      if (lc + 64 > kCap) flush();
+      if (lane < m) list[lc + lane] = (uint32_t)min(ls + off + lane, n - 1);
+      lc += m;
+    }
+  }
 }
 
 // Shared LDS of one traversing wave. The stack region holds the walk's stack
@@ -1141,17 +1180,15 @@ __device__ __forceinline__ float box_dist2(const Box& b, const float4& c) {
 // and a deferred cell is decided by each range's own test.
 template <bool kCount, bool kGuard, bool kShared>
 __device__ void walk(const WaveLds& L, int lane, int slice, int log2S, float4 me, int n,
-                     const float4* __restrict__ pms, const float4* __restrict__ com,
-                     const int4* __restrict__ link, const float* __restrict__ r2, float eps2,
+                     const float4* __restrict__ pms, const nb_node* __restrict__ nodes, float eps2,
                      int* __restrict__ flags, const Box& U, const Box& A, const Box& B, int& nd,
                      float& ax, float& ay, float& az, float& cx, float& cy, float& cz,
                      unsigned long long& cnt) {
-  const uint64_t lt = (uint64_t(1) << lane) - 1;
   int2* stack = L.stack;
   uint32_t* list = L.list;
 #define NB_FLUSH()                                                                              \
   do {                                                                                          \
-    list_flush<kCount, kGuard>(list, lc, L.stage, lane, slice, log2S, pms, com, me, eps2, ax, ay, \
+    list_flush<kCount, kGuard>(list, lc, L.stage, lane, slice, log2S, pms, nodes, me, eps2, ax, ay, \
                                az, cx, cy, cz, cnt);                                           \
     lc = 0;                                                                                     \
   } while (0)
@@ -1172,9 +1209,7 @@ __device__ void walk(const WaveLds& L, int lane, int slice, int log2S, float4 me
     // nothing of the iteration is live
     if (lc + 64 > kListCap) NB_FLUSH();
     int child = -1, efirst = 0;
-    int4 cl = make_int4(-1, -1, 0, 0);
-    float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
-    float rr = 0.f;
+    nb_node cl{make_float4(0.f, 0.f, 0.f, 0.f), 0.f, -1, 0, 0};
     if (!kShared && sp < 8 && dpos < nd) {
       // deferred entries: up to 32 of them, at most 64 cells, listed in the
       // staging area (free while walking) so that lane j takes the j-th cell
@@ -1194,9 +1229,7 @@ __device__ void walk(const WaveLds& L, int lane, int slice, int log2S, float4 me
       const int T = __builtin_amdgcn_readlane(incl, kd - 1);
       if (lane < T) {
         child = cells[lane];
-        cl = link[child];
-        c = com[child];
-        rr = r2[child];
+        cl = nodes[child];
       }
       __builtin_amdgcn_wave_barrier();
       dpos += kd;
@@ -1215,10 +1248,8 @@ __device__ void walk(const WaveLds& L, int lane, int slice, int log2S, float4 me
         const int pend = (int)(w & ((1u << 27) - 1));
         if (ci < slots) {
           const int cand = e.x + ci;
-          cl = link[cand];
-          c = com[cand];
-          rr = r2[cand];
-          if (cl.z < pend) child = cand;
+          cl = nodes[cand];
+          if (cl.start < pend) child = cand;
         }
       }
       __builtin_amdgcn_wave_barrier();
@@ -1227,19 +1258,19 @@ __device__ void walk(const WaveLds& L, int lane, int slice, int log2S, float4 me
     if (child >= 0) {
       // the group's modified test (see open_radius2); a pair shares what both accept
       if (kShared) {
-        const bool a = rr < box_dist2(A, c), b = rr < box_dist2(B, c);
+        const bool a = cl.r2 < box_dist2(A, cl.com), b = cl.r2 < box_dist2(B, cl.com);
         accept = a && b;
         defer = a != b;
       } else {
-        accept = rr < box_dist2(U, c);
+        accept = cl.r2 < box_dist2(U, cl.com);
       }
-      leaf = !accept && !defer && cl.x < 0;
-      open = !accept && !defer && cl.x >= 0;
+      leaf = !accept && !defer && cl.first < 0;
+      open = !accept && !defer && cl.first >= 0;
     }
     // accepted cells with mass -> list
-    const bool acc = accept && c.w > 0.f;
+    const bool acc = accept && cl.com.w > 0.f;
     const uint64_t ba = __ballot(acc);
-    if (acc) list[lc + __popcll(ba & lt)] = (uint32_t)child | kCellBit;
+    if (acc) list[lc + bits_below(ba)] = (uint32_t)child | kCellBit;
     lc += __popcll(ba);
     // deferred cells -> one entry per stack entry that has any
     int nd_add = 0;
@@ -1262,28 +1293,17 @@ __device__ void walk(const WaveLds& L, int lane, int slice, int log2S, float4 me
       if (lane == 0) atomicOr(flags, 8);
       break;
     }
-    if (kShared && head) stack[L.cap - 1 - (nd + __popcll(bg & lt))] = make_int2(efirst, (int)dmask);
+    if (kShared && head) stack[L.cap - 1 - (nd + bits_below(bg))] = make_int2(efirst, (int)dmask);
     nd += nd_add;
     if (open) {
-      const uint32_t pend = (uint32_t)(cl.z + link_count(cl.w));
-      const int slots = max(0, min(8, L.lvl[link_level(cl.w) + 2] - cl.x));
-      stack[sp + __popcll(bo & lt)] = make_int2(cl.x, (int)(((uint32_t)slots << 27) | pend));
+      const uint32_t pend = (uint32_t)(cl.start + span_count(cl.span));
+      const int slots = max(0, min(8, L.lvl[span_level(cl.span) + 2] - cl.first));
+      stack[sp + bits_below(bo)] = make_int2(cl.first, (int)(((uint32_t)slots << 27) | pend));
     }
     sp += __popcll(bo);
     // leaves that are not accepted -> the indices of their bodies
-    uint64_t bl = __ballot(leaf);
-    while (bl) {
-      const int src = __ffsll((unsigned long long)bl) - 1;
-      bl &= bl - 1;
-      const int ls = __builtin_amdgcn_readlane(cl.z, src);
-      const int lcount = __builtin_amdgcn_readlane(link_count(cl.w), src);
-      for (int off = 0; off < lcount; off += 64) {
-        const int m = min(64, lcount - off);
-        if (lc + 64 > kListCap) NB_FLUSH();
-        if (lane < m) list[lc + lane] = (uint32_t)min(ls + off + lane, n - 1);
-        lc += m;
-      }
-    }
+    list_leaves<kListCap>(list, lc, lane, leaf, cl.start, span_count(cl.span), n,
+                          [&] { NB_FLUSH(); });
     __builtin_amdgcn_wave_barrier();
   }
   NB_FLUSH();
@@ -1338,8 +1358,7 @@ __device__ __forceinline__ void lane_boxes(float4 me, int keep, int from0, int f
 template <bool kCount, bool kGuard>
 __global__ __launch_bounds__(64 * kListWaves, kCount ? 5 : kListBlocksPerCU) void k_traverse_list(
     const float4* __restrict__ pms, const uint32_t* __restrict__ perm, int n,
-    const float4* __restrict__ com, const int4* __restrict__ link,
-    const int* __restrict__ level_off, int64_t max_nodes, const float* __restrict__ r2,
+    const nb_node* __restrict__ nodes, const int* __restrict__ level_off, int64_t max_nodes,
     float eps2, double G, double* __restrict__ force,
     unsigned long long* __restrict__ inter, int* __restrict__ flags,
     const int4* __restrict__ waves, int* __restrict__ wctl, const int* __restrict__ order,
@@ -1382,10 +1401,10 @@ __global__ __launch_bounds__(64 * kListWaves, kCount ? 5 : kListBlocksPerCU) voi
     unsigned long long c = 0;
     int nd = 0;
     if (pair)
-      walk<kCount, kGuard, true>(L, lane, slice, log2S, me, n, pms, com, link, r2, eps2, flags, A,
+      walk<kCount, kGuard, true>(L, lane, slice, log2S, me, n, pms, nodes, eps2, flags, A,
                                  A, B, nd, ax, ay, az, cx, cy, cz, c);
     else
-      walk<kCount, kGuard, false>(L, lane, slice, log2S, me, n, pms, com, link, r2, eps2, flags,
+      walk<kCount, kGuard, false>(L, lane, slice, log2S, me, n, pms, nodes, eps2, flags,
                                   A, A, B, nd, ax, ay, az, cx, cy, cz, c);
     // each slice's compensated sum in FP64, then the slices added (butterfly
     // over the slice bits, fixed order)
@@ -1417,8 +1436,8 @@ __global__ __launch_bounds__(64 * kListWaves, kCount ? 5 : kListBlocksPerCU) voi
       const float4 me2 = pms[t2];
       ax = ay = az = cx = cy = cz = 0.f;
       c = 0;
-      walk<kCount, kGuard, false>(L, lane, lane / P, 6 - (31 - __clz(P)), me2, n, pms, com, link,
-                                  r2, eps2, flags, h ? B : A, A, B, nd, ax, ay, az, cx, cy, cz, c);
+      walk<kCount, kGuard, false>(L, lane, lane / P, 6 - (31 - __clz(P)), me2, n, pms, nodes,
+                                  eps2, flags, h ? B : A, A, B, nd, ax, ay, az, cx, cy, cz, c);
       double gx = (double)ax + (double)cx, gy = (double)ay + (double)cy,
              gz = (double)az + (double)cz;
       for (int off = P; off < 64; off <<= 1) {
@@ -1478,23 +1497,24 @@ constexpr int block_stack(int waves) { return (9 * 56 + 64) * waves; }
 constexpr int kBlockListCap = 256;  // source indices per wave
 // Waves per range by the system's size. Measured Barnes-Hut steps in us (Plummer
 // sphere / uniform ball, leaf size 8), one, two, four and eight waves per range:
-//     4,000 bodies  333/269  243/204  198/164  169/140
-//    20,000         448/294  337/234  253/196  212/180
-//    65,536         404/342  339/279  330/267  333/272
-//   131,072         494/399  440/354  456/371  483/395
-//   262,144         662/522  661/534  742/596  812/647
-// Sixteen were 3% faster than eight at 4,000 bodies and 27% slower at 20,000; four
-// would be the best in a narrow band, by 3%. From 262,144 bodies on there are
-// enough ranges for every wave and the barriers only cost.
-constexpr int kBlock8Bodies = 5 << 14;    // below: eight waves per range
-constexpr int kBlockMaxBodies = 1 << 18;  // below: two; from here on k_traverse_list
+//     4,000 bodies  224/197  153/137  121/107  105/ 90
+//    20,000         305/225  208/159  152/126  131/115
+//    40,000         283/248  215/185  175/147  174/142
+//    65,536         309/252  256/201  224/177  230/187
+//   131,072         421/331  347/275  332/262  355/287
+//   262,144         586/453  542/410  535/402  611/481
+//   400,000         777/582  757/561  769/575  897/719
+//   524,288         961/680  946/672  971/710 1157/902
+// Two would be the best in a narrow band, by 2%. Above it there are enough ranges
+// for every wave and the barriers only cost.
+constexpr int kBlock8Bodies = 5 << 13;    // below: eight waves per range
+constexpr int kBlockMaxBodies = 7 << 16;  // below: four; from here on k_traverse_list
 constexpr int kBlockWavesPerCU = 24;      // by LDS and 80 VGPRs, as k_traverse_list
 
 template <bool kGuard, int kWaves>
 __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_block(
     const float4* __restrict__ pms, const uint32_t* __restrict__ perm, int n,
-    const float4* __restrict__ com, const int4* __restrict__ link,
-    const int* __restrict__ level_off, int64_t max_nodes, const float* __restrict__ r2,
+    const nb_node* __restrict__ nodes, const int* __restrict__ level_off, int64_t max_nodes,
     float eps2, double G, double* __restrict__ force, int* __restrict__ flags,
     const int4* __restrict__ waves, int* __restrict__ wctl, const int* __restrict__ order,
     float* __restrict__ cost, int stack_cap) {
@@ -1509,7 +1529,6 @@ __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_
     s_lvl[threadIdx.x] = (int)min((int64_t)level_off[threadIdx.x], max_nodes);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint64_t lt = (uint64_t(1) << lane) - 1;
   uint32_t* list = s_list[wave];
   float4* stage = s_stage[wave];
   const int cap = stack_cap > 0 && stack_cap < block_stack(kWaves) ? stack_cap : block_stack(kWaves);
@@ -1533,7 +1552,7 @@ __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_
     float ax = 0.f, ay = 0.f, az = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
     int lc = 0, sp = 1;
     auto flush = [&]() {
-      list_flush<false, kGuard>(list, lc, stage, lane, slice, log2S, pms, com, me, eps2, ax, ay, az,
+      list_flush<false, kGuard>(list, lc, stage, lane, slice, log2S, pms, nodes, me, eps2, ax, ay, az,
                                 cx, cy, cz, unused);
       lc = 0;
     };
@@ -1549,43 +1568,27 @@ __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_
       sp -= k;
       const int q = 8 * wave + (lane >> 3), ci = lane & 7;
       int child = -1;
-      int4 cl = make_int4(-1, -1, 0, 0);
-      float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
-      float rr = 0.f;
+      nb_node cl{make_float4(0.f, 0.f, 0.f, 0.f), 0.f, -1, 0, 0};
       if (q < k) {  // entries and their candidates as in walk()
         const int2 e = stack[sp + q];
         const uint32_t ew = (uint32_t)e.y;
         if (ci < (int)(ew >> 27)) {
           const int cand = e.x + ci;
-          cl = link[cand];
-          c = com[cand];
-          rr = r2[cand];
-          if (cl.z < (int)(ew & ((1u << 27) - 1))) child = cand;
+          cl = nodes[cand];
+          if (cl.start < (int)(ew & ((1u << 27) - 1))) child = cand;
         }
       }
       bool accept = false, leaf = false, open = false;
       if (child >= 0) {
-        accept = rr < box_dist2(A, c);
-        leaf = !accept && cl.x < 0;
-        open = !accept && cl.x >= 0;
+        accept = cl.r2 < box_dist2(A, cl.com);
+        leaf = !accept && cl.first < 0;
+        open = !accept && cl.first >= 0;
       }
-      const bool acc = accept && c.w > 0.f;
+      const bool acc = accept && cl.com.w > 0.f;
       const uint64_t ba = __ballot(acc);
-      if (acc) list[lc + __popcll(ba & lt)] = (uint32_t)child | kCellBit;
+      if (acc) list[lc + bits_below(ba)] = (uint32_t)child | kCellBit;
       lc += __popcll(ba);
-      uint64_t bl = __ballot(leaf);
-      while (bl) {  // the bodies of leaves that are not accepted
-        const int src = __ffsll((unsigned long long)bl) - 1;
-        bl &= bl - 1;
-        const int ls = __builtin_amdgcn_readlane(cl.z, src);
-        const int lcount = __builtin_amdgcn_readlane(link_count(cl.w), src);
-        for (int off = 0; off < lcount; off += 64) {
-          const int m = min(64, lcount - off);
-          if (lc + 64 > kBlockListCap) flush();
-          if (lane < m) list[lc + lane] = (uint32_t)min(ls + off + lane, n - 1);
-          lc += m;
-        }
-      }
+      list_leaves<kBlockListCap>(list, lc, lane, leaf, cl.start, span_count(cl.span), n, flush);
       const uint64_t bo = __ballot(open);
       if (lane == 0) s_cnt[wave] = make_int2(__popcll(bo), lc);
       __syncthreads();  // counts are in, and every wave has read its entries
@@ -1603,9 +1606,9 @@ __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_
         break;
       }
       if (open) {
-        const uint32_t pend = (uint32_t)(cl.z + link_count(cl.w));
-        const int slots = max(0, min(8, s_lvl[link_level(cl.w) + 2] - cl.x));
-        stack[sp + before + __popcll(bo & lt)] = make_int2(cl.x, (int)(((uint32_t)slots << 27) | pend));
+        const uint32_t pend = (uint32_t)(cl.start + span_count(cl.span));
+        const int slots = max(0, min(8, s_lvl[span_level(cl.span) + 2] - cl.first));
+        stack[sp + before + bits_below(bo)] = make_int2(cl.first, (int)(((uint32_t)slots << 27) | pend));
       }
       sp += opened;
       // room for the next iteration's accepted cells (at most 64 per wave)
@@ -1747,9 +1750,8 @@ void nb_bh_carve(nb_ctx* c, char* base, int upto) {
   b.pms = (float4*)at(kBhPms);
   b.prefix = (double4*)at(kBhPrefix);
   b.scan_part = (double4*)at(kBhScanPart);
-  b.node_com = (float4*)at(kBhCom);
-  b.node_r2 = (float*)at(kBhR2);
-  b.node_link = (int4*)at(kBhLink);
+  b.nodes = (nb_node*)at(kBhNode);
+  b.node_next = (int*)at(kBhNext);
   b.level_off = (int*)at(kBhLevel);
   b.marks = (unsigned char*)at(kBhMarks);
   b.node_end = (int*)at(kBhNodeEnd);
@@ -1873,14 +1875,14 @@ hipError_t nb_bh_build(nb_ctx* c) {
   hipLaunchKernelGGL(k_tree_scan, dim3(1 + kLevels), dim3(kScanThreads), 0, s, b.scan_part,
                      b.level_cnt, tiles, n, leaf, pairs, b.counters, b.waves, b.rec_hist);
   hipLaunchKernelGGL(k_tree_emit, dim3(tiles), dim3(kTreeTile), 0, s, b.pms, n, b.scan_part,
-                     b.marks, b.level_cnt, b.counters, b.max_nodes, b.prefix, b.node_link,
+                     b.marks, b.level_cnt, b.counters, b.max_nodes, b.prefix, b.nodes, b.node_next,
                      b.node_end, b.level_off, c->flags);
   // 7. centre of mass, wave ranges
   const int cgrid = (int)std::max<int64_t>(1, std::min<int64_t>((b.max_nodes + 255) / 256, 8192));
   const int cubic = (c->cfg.flags & NB_F_BH_AXIS_BOX) ? 0 : 1;
-  hipLaunchKernelGGL(k_tree_com, dim3(cgrid), dim3(256), 0, s, b.node_link, b.node_end, n,
+  hipLaunchKernelGGL(k_tree_com, dim3(cgrid), dim3(256), 0, s, b.nodes, b.node_end, n,
                      b.max_nodes, b.level_off, b.prefix, b.pms, codes_sorted, b.geom, cubic,
-                     c->cfg.theta, leaf, pairs, b.waves, b.counters, b.node_com, b.node_r2);
+                     c->cfg.theta, leaf, pairs, b.waves, b.counters);
   return hipGetLastError();
 }
 
@@ -1892,7 +1894,7 @@ hipError_t nb_bh_traverse(nb_ctx* c, bool count_interactions) {
   if (count_interactions)
     hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, b.inter);
 #define NB_TRAVERSE_ARGS                                                                       \
-  b.pms, b.vals[0], n, b.node_com, b.node_link, b.level_off, b.max_nodes, b.geom, c->theta2, \
+  b.pms, b.vals[0], n, b.nodes, b.node_next, b.level_off, b.max_nodes, b.geom, c->theta2, \
       c->cfg.eps2, c->G, c->force, b.inter, c->flags
   const bool guard = c->guard;
   const int gl = b.persist_blocks;  // persistent blocks pulling wave ranges
@@ -1908,8 +1910,8 @@ hipError_t nb_bh_traverse(nb_ctx* c, bool count_interactions) {
                        b.rec_bucket, b.rec_hist, b.rec_order);
   }
 #define NB_LIST_ARGS                                                                     \
-  b.pms, b.vals[0], n, b.node_com, b.node_link, b.level_off, b.max_nodes, b.node_r2,     \
-      c->cfg.eps2, c->G, c->force, b.inter, c->flags, b.waves, b.counters,                \
+  b.pms, b.vals[0], n, b.nodes, b.level_off, b.max_nodes, c->cfg.eps2,     \
+      c->G, c->force, b.inter, c->flags, b.waves, b.counters,                \
       ordered ? b.rec_order : nullptr, ordered ? b.rec_cost : nullptr, c->walk_stack
   if (group && count_interactions && guard)
     hipLaunchKernelGGL((k_traverse_list<true, true>), dim3(gl), dim3(64 * kListWaves), 0, c->stream,
@@ -1921,7 +1923,7 @@ hipError_t nb_bh_traverse(nb_ctx* c, bool count_interactions) {
     const auto launch = [&](auto kernel, int waves) {
       const int blocks = b.persist_blocks / kListBlocksPerCU * (kBlockWavesPerCU / waves);
       hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * waves), 0, c->stream, b.pms, b.vals[0], n,
-                         b.node_com, b.node_link, b.level_off, b.max_nodes, b.node_r2, c->cfg.eps2,
+                         b.nodes, b.level_off, b.max_nodes, c->cfg.eps2,
                          c->G, c->force, c->flags, b.waves, b.counters,
                          ordered ? b.rec_order : nullptr, ordered ? b.rec_cost : nullptr,
                          c->walk_stack);
@@ -1929,7 +1931,7 @@ hipError_t nb_bh_traverse(nb_ctx* c, bool count_interactions) {
     if (n < kBlock8Bodies)
       guard ? launch(k_traverse_block<true, 8>, 8) : launch(k_traverse_block<false, 8>, 8);
     else
-      guard ? launch(k_traverse_block<true, 2>, 2) : launch(k_traverse_block<false, 2>, 2);
+      guard ? launch(k_traverse_block<true, 4>, 4) : launch(k_traverse_block<false, 4>, 4);
   } else if (group && guard)
     hipLaunchKernelGGL((k_traverse_list<false, true>), dim3(gl), dim3(64 * kListWaves), 0, c->stream,
                        NB_LIST_ARGS);
@@ -1950,8 +1952,8 @@ hipError_t nb_bh_count_per_body(nb_ctx* c) {
   const int n = c->n;
   hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, b.inter);
   hipLaunchKernelGGL((k_traverse<true, true>), dim3((n + 255) / 256), dim3(256), 0, c->stream, b.pms,
-                     b.vals[0], n, b.node_com, b.node_link, b.level_off, b.max_nodes, b.geom,
-                     c->theta2, c->cfg.eps2, c->G, c->force, b.inter, c->flags, b.node_r2);
+                     b.vals[0], n, b.nodes, b.node_next, b.level_off, b.max_nodes, b.geom,
+                     c->theta2, c->cfg.eps2, c->G, c->force, b.inter, c->flags);
   return hipGetLastError();
 }
 
@@ -1994,24 +1996,22 @@ extern "C" int nb_debug_tree(nb_ctx* c, nb_node_view* nodes, int64_t cap, int64_
   if (bbox) NB_HIP(hipMemcpy(bbox, c->bh.geom, sizeof(float) * 6, hipMemcpyDeviceToHost));
   const int64_t m = std::min<int64_t>(cap, total);
   if (nodes && m > 0) {
-    std::vector<int4> link(m);
-    std::vector<float4> com(m);
-    std::vector<float> r2(m);
-    NB_HIP(hipMemcpy(link.data(), c->bh.node_link, sizeof(int4) * m, hipMemcpyDeviceToHost));
-    NB_HIP(hipMemcpy(com.data(), c->bh.node_com, sizeof(float4) * m, hipMemcpyDeviceToHost));
-    NB_HIP(hipMemcpy(r2.data(), c->bh.node_r2, sizeof(float) * m, hipMemcpyDeviceToHost));
+    std::vector<nb_node> nd(m);
+    std::vector<int> next(m);
+    NB_HIP(hipMemcpy(nd.data(), c->bh.nodes, sizeof(nb_node) * m, hipMemcpyDeviceToHost));
+    NB_HIP(hipMemcpy(next.data(), c->bh.node_next, sizeof(int) * m, hipMemcpyDeviceToHost));
     for (int64_t k = 0; k < m; ++k) {
       nb_node_view& v = nodes[k];
-      v.com[0] = com[k].x;
-      v.com[1] = com[k].y;
-      v.com[2] = com[k].z;
-      v.mass = com[k].w;
-      v.first_child = link[k].x;
-      v.next = link[k].y;
-      v.body_start = link[k].z;
-      v.body_count = link[k].w >> 4;
-      v.level = link[k].w & 15;
-      v.open_r2 = r2[k];
+      v.com[0] = nd[k].com.x;
+      v.com[1] = nd[k].com.y;
+      v.com[2] = nd[k].com.z;
+      v.mass = nd[k].com.w;
+      v.first_child = nd[k].first;
+      v.next = next[k];
+      v.body_start = nd[k].start;
+      v.body_count = nd[k].span >> 4;
+      v.level = nd[k].span & 15;
+      v.open_r2 = nd[k].r2;
     }
   }
   return NB_OK;

@@ -92,7 +92,7 @@ inline bool nb_bh_pairs(int64_t n, int flags) {
 
 enum nb_bh_buf {
   kBhBbox, kBhGeom, kBhKey0, kBhKey1, kBhVal0, kBhVal1, kBhCodes, kBhHist, kBhGroupHist,
-  kBhPms, kBhPrefix, kBhScanPart, kBhCom, kBhR2, kBhLink, kBhLevel, kBhMarks,
+  kBhPms, kBhPrefix, kBhScanPart, kBhNode, kBhNext, kBhLevel, kBhMarks,
   kBhNodeEnd, kBhLevelCnt, kBhCounters, kBhWaves, kBhInter, kBhFlags,
   kBhRecCost, kBhRecBucket, kBhRecOrder, kBhRecHist, kBhBufCount
 };
@@ -126,9 +126,8 @@ constexpr nb_bh_layout nb_bh_layout_for(int64_t n) {
   bytes[kBhPms] = 16 * (n + kSpare);
   bytes[kBhPrefix] = 32 * (n + 1);
   bytes[kBhScanPart] = 32 * ((n + kTreeTile - 1) / kTreeTile + 1);
-  bytes[kBhCom] = 16 * bound;
-  bytes[kBhR2] = 4 * bound;
-  bytes[kBhLink] = 16 * bound;
+  bytes[kBhNode] = 32 * bound;
+  bytes[kBhNext] = 4 * bound;
   bytes[kBhLevel] = 4 * (kMaxLevel + 2);
   bytes[kBhMarks] = n;
   bytes[kBhNodeEnd] = 4 * bound;
@@ -149,6 +148,16 @@ constexpr nb_bh_layout nb_bh_layout_for(int64_t n) {
   L.max_nodes = bound;
   return L;
 }
+
+// An octree node, 32 bytes: all that a walk reads of it. The eight children of a
+// node are two cache lines.
+struct alignas(32) nb_node {
+  float4 com;  // (cx, cy, cz, m)
+  float r2;    // squared opening radius (s / theta + |COM - cell centre|)^2
+  int first;   // first child, -1 for a leaf
+  int start;   // first sorted body
+  int span;    // count << 4 | level
+};
 
 // Largest system nb_bh_forces_noalloc accepts (its static scratch is sized for it).
 constexpr int64_t kNoAllocMaxBodies = NB_NOALLOC_MAX_BODIES;
@@ -173,9 +182,8 @@ struct nb_bh_state {
   double4* prefix = nullptr;    // exclusive FP64 prefix of (m, m x, m y, m z), n+1 entries
   double4* scan_part = nullptr; // scan block partials
   // octree, breadth-first
-  float4* node_com = nullptr;   // (cx, cy, cz, m)
-  float* node_r2 = nullptr;     // squared opening radius (s / theta + |COM - cell centre|)^2
-  int4* node_link = nullptr;    // (first_child, next, start, count << 4 | level)
+  nb_node* nodes = nullptr;
+  int* node_next = nullptr;     // rope: next node in pre-order after the subtree, -1 at the end
   int* level_off = nullptr;     // [kMaxLevel + 2] node index where each level begins
   unsigned char* marks = nullptr;  // per sorted body: levels at which a node starts there
   int* node_end = nullptr;      // end of each node's body range
