@@ -277,6 +277,9 @@ __device__ __forceinline__ double4 shfl_up4(double4 v, int off) {
   return make_double4(__shfl_up(v.x, off), __shfl_up(v.y, off), __shfl_up(v.z, off),
                       __shfl_up(v.w, off));
 }
+__device__ __forceinline__ double4 shfl4(double4 v, int lane) {
+  return make_double4(__shfl(v.x, lane), __shfl(v.y, lane), __shfl(v.z, lane), __shfl(v.w, lane));
+}
 __device__ __forceinline__ double4 wave_incl_scan4(double4 v) {
   return make_double4(wave_incl_scan(v.x), wave_incl_scan(v.y), wave_incl_scan(v.z),
                       wave_incl_scan(v.w));
@@ -559,165 +562,6 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_mark(
   }
 }
 
-// Block 0: exclusive scan of the tiles' moments in a fixed order: each thread
-// folds a contiguous run of tiles, the 256 run totals are scanned (wave DPP
-// prefixes, then the 4 wave totals in wave order), then each thread rewrites its
-// run; part[tiles] receives the total. Block 1 + l: the same for the tiles' node
-// counts of level l, whose total goes to counters[2 + l]. Block 1 also resets the
-// traversal's work items and ticket, and lists the ranges of a system that no
-// node packs.
-__global__ __launch_bounds__(kScanThreads) void k_tree_scan(double4* __restrict__ part,
-                                                            int* __restrict__ level_cnt,
-                                                            int tiles, int n, int leaf, int pairs,
-                                                            int* __restrict__ counters,
-                                                            int4* __restrict__ waves,
-                                                            int* __restrict__ rec_hist) {
-  const int per = (tiles + kScanThreads - 1) / kScanThreads;
-  const int b0 = min((int)threadIdx.x * per, tiles);
-  const int b1 = min(b0 + per, tiles);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (blockIdx.x == 0) {
-    double4 tot = make_double4(0, 0, 0, 0);
-    for (int b = b0; b < b1; ++b) tot = add4(tot, part[b]);
-    const double4 incl = wave_incl_scan4(tot);
-    __shared__ double4 wtot[kScanWaves];
-    if (lane == 63) wtot[wave] = incl;
-    __syncthreads();
-    double4 run = make_double4(0, 0, 0, 0), grand = make_double4(0, 0, 0, 0);
-    for (int w = 0; w < kScanWaves; ++w) {
-      if (w < wave) run = add4(run, wtot[w]);
-      grand = add4(grand, wtot[w]);
-    }
-    const double4 below = shfl_up4(incl, 1);  // inclusive value of the lane below
-    if (lane > 0) run = add4(run, below);
-    for (int b = b0; b < b1; ++b) {
-      const double4 v = part[b];
-      part[b] = run;
-      run = add4(run, v);
-    }
-    if (threadIdx.x == 0) part[tiles] = grand;
-    return;
-  }
-  int* cnt = level_cnt + (blockIdx.x - 1) * tiles;
-  __shared__ int wsum[kScanWaves];
-  int sum = 0, total = 0;
-  for (int b = b0; b < b1; ++b) sum += cnt[b];
-  int run = block_excl_scan(sum, wsum, total);
-  for (int b = b0; b < b1; ++b) {
-    const int v = cnt[b];
-    cnt[b] = run;
-    run += v;
-  }
-  if (threadIdx.x == 0) counters[1 + blockIdx.x] = total;
-  if (blockIdx.x != 1) return;
-  if (threadIdx.x < kCostBuckets) rec_hist[threadIdx.x] = 0;  // this pass's traversal order starts empty
-  if (threadIdx.x == 0) {
-    int r = 0;
-    if (n <= kWaveBodies) {
-      waves[r++] = make_int4(0, n, 0, 0);
-    } else if (n <= leaf) {
-      // the root is itself a leaf, so no node packs ranges below it: chunk it,
-      // two full chunks per record, a shorter last chunk on its own
-      for (int o = 0; o < n; o += kWaveBodies) {
-        const int k = min(kWaveBodies, n - o), o2 = o + kWaveBodies;
-        if (pairs && k == kWaveBodies && n - o2 >= kWaveBodies) {
-          waves[r++] = make_int4(o, k, o2, kWaveBodies);
-          o = o2;
-        } else {
-          waves[r++] = make_int4(o, k, 0, 0);
-        }
-      }
-    }
-    counters[0] = r;
-    counters[1] = 0;  // traversal ticket
-  }
-}
-
-// Per tile: the exclusive FP64 prefix of the moments (wave DPP prefixes, then a
-// DPP prefix of the 16 wave totals: a fixed association, no atomics) and the
-// nodes that start or end in it. The body i that starts a node writes its first
-// child (which starts at i too), its start and its level; the last body i of a
-// node writes its end and its rope: the node of the lowest level that starts at
-// i + 1, which is a sibling of it or of the closest ancestor that has one. Few
-// levels are active in 64 neighbouring bodies, so the others are branched over
-// (at 2^22 bodies 141 us without that, 94 us with it).
-__global__ __launch_bounds__(kTreeTile) void k_tree_emit(
-    const float4* __restrict__ pms, int n, const double4* __restrict__ part,
-    const unsigned char* __restrict__ marks, const int* __restrict__ level_cnt,
-    const int* __restrict__ counters, int64_t max_nodes, double4* __restrict__ prefix,
-    nb_node* __restrict__ nodes, int* __restrict__ next, int* __restrict__ node_end,
-    int* __restrict__ level_off, int* __restrict__ flags) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint64_t lt = (uint64_t(1) << lane) - 1;
-  const int e = blockIdx.x * kTreeTile + threadIdx.x;
-  __shared__ double4 s_mom[kTreeWaves];
-  __shared__ int s_off[kLevels][kTreeWaves];  // node starts per wave, then their first index
-  const double4 x0 = e < n ? body_moments(pms[e]) : make_double4(0, 0, 0, 0);
-  const int mark = e < n ? marks[e] : kLevels << 4;
-  const int dn = e + 1 < n ? marks[e + 1] >> 4 : 0;  // after the last body every node ends
-  const int d = mark >> 4, D = e < n ? mark & 15 : -1;
-  const double4 x = wave_incl_scan4(x0);
-  int cnt = 0;
-#pragma unroll
-  for (int l = 0; l < kLevels; ++l) {
-    const int c = __popcll(__ballot(d <= l && l <= D));
-    cnt = lane == l ? c : cnt;
-  }
-  if (lane == 63) s_mom[wave] = x;
-  if (lane < kLevels) s_off[lane][wave] = cnt;
-  __syncthreads();
-  if (wave < kLevels) {  // wave l: level l's node index at the start of every wave
-    const int l = wave;
-    int lo = 0;
-    for (int k = 0; k < l; ++k) lo += counters[2 + k];
-    const int v = lane < kTreeWaves ? s_off[l][lane] : 0;
-    const int at = wave_incl_scan(v) - v;
-    if (lane < kTreeWaves) s_off[l][lane] = lo + level_cnt[l * gridDim.x + blockIdx.x] + at;
-    if (blockIdx.x == 0 && lane == 0) {
-      level_off[l] = lo;
-      if (l == kMaxLevel) level_off[l + 1] = lo + counters[2 + l];
-    }
-  } else if (wave == kLevels) {
-    const double4 v = lane < kTreeWaves ? s_mom[lane] : make_double4(0, 0, 0, 0);
-    const double4 below = shfl_up4(wave_incl_scan4(v), 1);
-    const double4 run = part[blockIdx.x];  // exclusive start of this tile
-    if (lane < kTreeWaves) s_mom[lane] = lane > 0 ? add4(run, below) : run;
-  }
-  __syncthreads();
-  const double4 below = shfl_up4(x, 1);  // inclusive value of the lane below
-  const double4 start = s_mom[wave];
-  if (e < n) prefix[e] = lane > 0 ? add4(start, below) : start;
-  // idx[l]: index of a node of level l that starts at e
-  int idx[kLevels + 1], rope = -1;
-#pragma unroll
-  for (int l = 0; l < kLevels; ++l) {
-    const bool starts = d <= l && l <= D;
-    idx[l] = s_off[l][wave] + __popcll(__ballot(starts) & lt);
-    if (l == dn && e + 1 < n) rope = idx[l] + (starts ? 1 : 0);
-  }
-  idx[kLevels] = -1;
-  bool over = false;
-#pragma unroll
-  for (int l = 0; l < kLevels; ++l) {
-    const bool starts = d <= l && l <= D, ends = dn <= l && l <= D;
-    if (__ballot(starts || ends) == 0) continue;
-    const int64_t at = idx[l];
-    if (starts && at < max_nodes) {
-      nodes[at].first = l < D ? idx[l + 1] : -1;
-      nodes[at].start = e;
-      nodes[at].span = l;
-    }
-    const int64_t in = at - (starts ? 0 : 1);  // the node of level l around e
-    if (ends && in >= 0 && in < max_nodes) {
-      next[in] = rope;
-      node_end[in] = e + 1;
-    }
-    over = over || (starts && at >= max_nodes);
-  }
-  if (over) atomicOr(flags, 2);
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) prefix[n] = part[gridDim.x];
-}
-
 // Wave ranges of one node's children (see kWaveBodies): calls out(start, count)
 // for each range in order; returns how many there are.
 template <typename Out>
@@ -800,6 +644,211 @@ __device__ __forceinline__ void emit_records(int4* __restrict__ waves, int first
 #pragma unroll
   for (int j = 0; j < 4; ++j)
     if (wait[j].y > 0) put(make_int4(wait[j].x, wait[j].y, 0, 0));
+}
+
+// Where the traversal's work items go.
+struct Records {
+  int4* waves;
+  int* ctl;   // [0] records, [1] traversal ticket
+  int* hist;  // [kCostBuckets] records per cost bucket, then [kCostBuckets] cursors
+};
+
+// Before a build's first record: no records, a fresh ticket, empty buckets, and the
+// ranges of a system that no node packs. One workgroup.
+__device__ __forceinline__ void start_records(const Records& R, int n, int leaf, int pairs) {
+  for (int k = threadIdx.x; k < 2 * kCostBuckets; k += blockDim.x) R.hist[k] = 0;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  int r = 0;
+  if (n <= kWaveBodies) {
+    R.waves[r++] = make_int4(0, n, 0, 0);
+  } else if (n <= leaf) {
+    // the root is itself a leaf, so no node packs ranges below it: chunk it,
+    // two full chunks per record, a shorter last chunk on its own
+    for (int o = 0; o < n; o += kWaveBodies) {
+      const int k = min(kWaveBodies, n - o), o2 = o + kWaveBodies;
+      if (pairs && k == kWaveBodies && n - o2 >= kWaveBodies) {
+        R.waves[r++] = make_int4(o, k, o2, kWaveBodies);
+        o = o2;
+      } else {
+        R.waves[r++] = make_int4(o, k, 0, 0);
+      }
+    }
+  }
+  R.ctl[0] = r;
+  R.ctl[1] = 0;  // traversal ticket
+}
+
+// ---- 6b. scan and emission -------------------------------------------------------------
+// Block 0: exclusive scan of the tiles' moments in a fixed order: each thread
+// folds a contiguous run of tiles, the 256 run totals are scanned (wave DPP
+// prefixes, then the 4 wave totals in wave order), then each thread rewrites its
+// run; part[tiles] receives the total. Block 1 + l: the same for the tiles' node
+// counts of level l, whose total goes to counters[2 + l]. The last block starts the
+// records. A system of at most 64 tiles needs no launch for this (k_tree_emit).
+__global__ __launch_bounds__(kScanThreads) void k_tree_scan(double4* __restrict__ part,
+                                                            int* __restrict__ level_cnt,
+                                                            int tiles, int n, int leaf, int pairs,
+                                                            int* __restrict__ counters,
+                                                            Records records) {
+  if (blockIdx.x == 1 + kLevels) {
+    start_records(records, n, leaf, pairs);
+    return;
+  }
+  const int per = (tiles + kScanThreads - 1) / kScanThreads;
+  const int b0 = min((int)threadIdx.x * per, tiles);
+  const int b1 = min(b0 + per, tiles);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (blockIdx.x == 0) {
+    double4 tot = make_double4(0, 0, 0, 0);
+    for (int b = b0; b < b1; ++b) tot = add4(tot, part[b]);
+    const double4 incl = wave_incl_scan4(tot);
+    __shared__ double4 wtot[kScanWaves];
+    if (lane == 63) wtot[wave] = incl;
+    __syncthreads();
+    double4 run = make_double4(0, 0, 0, 0), grand = make_double4(0, 0, 0, 0);
+    for (int w = 0; w < kScanWaves; ++w) {
+      if (w < wave) run = add4(run, wtot[w]);
+      grand = add4(grand, wtot[w]);
+    }
+    const double4 below = shfl_up4(incl, 1);  // inclusive value of the lane below
+    if (lane > 0) run = add4(run, below);
+    for (int b = b0; b < b1; ++b) {
+      const double4 v = part[b];
+      part[b] = run;
+      run = add4(run, v);
+    }
+    if (threadIdx.x == 0) part[tiles] = grand;
+    return;
+  }
+  int* cnt = level_cnt + (blockIdx.x - 1) * tiles;
+  __shared__ int wsum[kScanWaves];
+  int sum = 0, total = 0;
+  for (int b = b0; b < b1; ++b) sum += cnt[b];
+  int run = block_excl_scan(sum, wsum, total);
+  for (int b = b0; b < b1; ++b) {
+    const int v = cnt[b];
+    cnt[b] = run;
+    run += v;
+  }
+  if (threadIdx.x == 0) counters[1 + blockIdx.x] = total;
+}
+
+// Per tile: the exclusive FP64 prefix of the moments (wave DPP prefixes, then a
+// DPP prefix of the 16 wave totals: a fixed association, no atomics) and the
+// nodes that start or end in it. The body i that starts a node writes its first
+// child (which starts at i too), its start and its level; the last body i of a
+// node writes its end and its rope: the node of the lowest level that starts at
+// i + 1, which is a sibling of it or of the closest ancestor that has one. Few
+// levels are active in 64 neighbouring bodies, so the others are branched over
+// (at 2^22 bodies 141 us without that, 94 us with it).
+// kSelf: at most 64 tiles, whose counts and moments every block scans itself, one
+// lane per tile (a launch less: 4.6 us of 65,536 bodies' step); the first block
+// starts the records.
+template <bool kSelf>
+__global__ __launch_bounds__(kTreeTile) void k_tree_emit(
+    const float4* __restrict__ pms, int n, int leaf, int pairs, const double4* __restrict__ part,
+    const unsigned char* __restrict__ marks, const int* __restrict__ level_cnt,
+    const int* __restrict__ counters, Records records, int64_t max_nodes, double4* __restrict__ prefix,
+    nb_node* __restrict__ nodes, int* __restrict__ next, int* __restrict__ node_end,
+    int* __restrict__ level_off, int* __restrict__ flags) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t lt = (uint64_t(1) << lane) - 1;
+  const int e = blockIdx.x * kTreeTile + threadIdx.x;
+  __shared__ double4 s_mom[kTreeWaves];
+  __shared__ int s_off[kLevels][kTreeWaves];  // node starts per wave, then their first index
+  __shared__ int s_tot[kLevels];              // nodes of each level
+  const int tile = blockIdx.x, tiles = gridDim.x;
+  if (kSelf && tile == 0) start_records(records, n, leaf, pairs);
+  const double4 x0 = e < n ? body_moments(pms[e]) : make_double4(0, 0, 0, 0);
+  const int mark = e < n ? marks[e] : kLevels << 4;
+  const int dn = e + 1 < n ? marks[e + 1] >> 4 : 0;  // after the last body every node ends
+  const int d = mark >> 4, D = e < n ? mark & 15 : -1;
+  const double4 x = wave_incl_scan4(x0);
+  int cnt = 0;
+#pragma unroll
+  for (int l = 0; l < kLevels; ++l) {
+    const int c = __popcll(__ballot(d <= l && l <= D));
+    cnt = lane == l ? c : cnt;
+  }
+  if (lane == 63) s_mom[wave] = x;
+  if (lane < kLevels) s_off[lane][wave] = cnt;
+  // level `wave`: its nodes in earlier tiles, and in all
+  int earlier = 0;
+  if (wave < kLevels) {
+    int total;
+    if (kSelf) {
+      const int v = lane < tiles ? level_cnt[wave * tiles + lane] : 0;
+      const int incl = wave_incl_scan(v);
+      earlier = __shfl(incl - v, tile);
+      total = __shfl(incl, 63);
+    } else {
+      earlier = level_cnt[wave * tiles + tile];
+      total = counters[2 + wave];
+    }
+    if (lane == 0) s_tot[wave] = total;
+  }
+  __syncthreads();
+  if (wave < kLevels) {  // level l's node index at the start of every wave
+    const int l = wave;
+    int lo = 0;
+    for (int k = 0; k < l; ++k) lo += s_tot[k];
+    const int v = lane < kTreeWaves ? s_off[l][lane] : 0;
+    const int at = wave_incl_scan(v) - v;
+    if (lane < kTreeWaves) s_off[l][lane] = lo + earlier + at;
+    if (tile == 0 && lane == 0) {
+      level_off[l] = lo;
+      if (l == kMaxLevel) level_off[l + 1] = lo + s_tot[l];
+    }
+  } else if (wave == kLevels) {
+    const double4 v = lane < kTreeWaves ? s_mom[lane] : make_double4(0, 0, 0, 0);
+    const double4 below = shfl_up4(wave_incl_scan4(v), 1);
+    double4 run, all;  // exclusive start of this tile, and the total
+    if (kSelf) {
+      const double4 t = lane < tiles ? part[lane] : make_double4(0, 0, 0, 0);
+      const double4 incl = wave_incl_scan4(t);
+      const double4 before = shfl4(incl, max(tile - 1, 0));
+      run = tile > 0 ? before : make_double4(0, 0, 0, 0);
+      all = shfl4(incl, 63);
+    } else {
+      run = part[tile];
+      all = part[tiles];
+    }
+    if (lane < kTreeWaves) s_mom[lane] = lane > 0 ? add4(run, below) : run;
+    if (tile == tiles - 1 && lane == 0) prefix[n] = all;
+  }
+  __syncthreads();
+  const double4 below = shfl_up4(x, 1);  // inclusive value of the lane below
+  const double4 start = s_mom[wave];
+  if (e < n) prefix[e] = lane > 0 ? add4(start, below) : start;
+  // idx[l]: index of a node of level l that starts at e
+  int idx[kLevels + 1], rope = -1;
+#pragma unroll
+  for (int l = 0; l < kLevels; ++l) {
+    const bool starts = d <= l && l <= D;
+    idx[l] = s_off[l][wave] + __popcll(__ballot(starts) & lt);
+    if (l == dn && e + 1 < n) rope = idx[l] + (starts ? 1 : 0);
+  }
+  idx[kLevels] = -1;
+  bool over = false;
+#pragma unroll
+  for (int l = 0; l < kLevels; ++l) {
+    const bool starts = d <= l && l <= D, ends = dn <= l && l <= D;
+    if (__ballot(starts || ends) == 0) continue;
+    const int64_t at = idx[l];
+    if (starts && at < max_nodes) {
+      nodes[at].first = l < D ? idx[l + 1] : -1;
+      nodes[at].start = e;
+      nodes[at].span = l;
+    }
+    const int64_t in = at - (starts ? 0 : 1);  // the node of level l around e
+    if (ends && in >= 0 && in < max_nodes) {
+      next[in] = rope;
+      node_end[in] = e + 1;
+    }
+    over = over || (starts && at >= max_nodes);
+  }
+  if (over) atomicOr(flags, 2);
 }
 
 // ---- 7. centre of mass and opening radius -------------------------------------------
@@ -1640,7 +1689,7 @@ __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_
   }
 }
 
-// ---- 8. traversal order ---------------------------------------------------------------
+// ---- 8c. traversal order ---------------------------------------------------------------
 // A persistent launch ends when its last wave finishes its last record, so the
 // records are taken costliest first: each record's estimate is the device time
 // its bodies' records took in the previous pass (stored per body, by original
@@ -1658,12 +1707,14 @@ __device__ __forceinline__ int cost_bucket(float est) {
 
 // Records are handled in chunks of kOrderChunk by a grid of at most kOrderBlocks
 // blocks; each block counts in LDS and makes one global atomic per bucket per
-// chunk, so the few busy buckets see few atomics.
+// chunk, so the few busy buckets see few atomics. (Bucketing a record where it is
+// made, in k_tree_com, spares a launch of 4.7 us but its gathers made that kernel 7
+// us longer at 65,536 bodies and 35 at 2^22.)
 constexpr int kOrderChunk = 1024;
 constexpr int kOrderBlocks = 256;
-// Below this the three ordering launches cost more than the tail they save
-// (Plummer steps with single ranges, ordered against not: 0.577 against 0.583
-// ms at 65,536 bodies, 0.858 against 0.881 at 262,144, 1.267 against 1.296 at
+// Below this the ordering costs more than the tail it saves (Plummer steps with
+// single ranges, ordered against not, when it took three launches: 0.577 against
+// 0.583 ms at 65,536 bodies, 0.858 against 0.881 at 262,144, 1.267 against 1.296 at
 // 524,288).
 constexpr int kOrderMinBodies = 1 << 16;
 
@@ -1689,22 +1740,20 @@ __global__ __launch_bounds__(256) void k_rec_bucket(const int4* __restrict__ wav
   if (threadIdx.x < kCostBuckets && h[threadIdx.x] > 0) atomicAdd(&hist[threadIdx.x], h[threadIdx.x]);
 }
 
-// One wave: cursor[b] = records in buckets above b (costliest first); the
-// counts are cleared for the next pass's k_rec_bucket.
-__global__ __launch_bounds__(64) void k_rec_offsets(int* __restrict__ hist) {
-  const int lane = threadIdx.x;
-  const int v = hist[kCostBuckets - 1 - lane];
-  hist[kCostBuckets + kCostBuckets - 1 - lane] = wave_incl_scan(v) - v;
-  hist[kCostBuckets - 1 - lane] = 0;
-}
-
+// Tickets -> records: the first place of each bucket (the records in the buckets
+// above, one wave's scan in every block) plus a place within it.
 __global__ __launch_bounds__(256) void k_rec_scatter(const int* __restrict__ wctl, int n,
                                                      const int* __restrict__ bucket,
                                                      int* __restrict__ hist,
                                                      int* __restrict__ order) {
-  __shared__ int h[kCostBuckets], base[kCostBuckets];
+  __shared__ int h[kCostBuckets], base[kCostBuckets], first[kCostBuckets];
   constexpr int kPer = kOrderChunk / 256;
+  static_assert(kCostBuckets == 64, "one wave scans the buckets");
   const int nrec = min(wctl[0], n);
+  if (threadIdx.x < 64) {  // records in the buckets above
+    const int b = kCostBuckets - 1 - threadIdx.x, v = hist[b];
+    first[b] = wave_incl_scan(v) - v;
+  }
   for (int c0 = blockIdx.x * kOrderChunk; c0 < nrec; c0 += gridDim.x * kOrderChunk) {
     if (threadIdx.x < kCostBuckets) h[threadIdx.x] = 0;
     __syncthreads();
@@ -1717,7 +1766,8 @@ __global__ __launch_bounds__(256) void k_rec_scatter(const int* __restrict__ wct
     }
     __syncthreads();
     if (threadIdx.x < kCostBuckets && h[threadIdx.x] > 0)
-      base[threadIdx.x] = atomicAdd(&hist[kCostBuckets + threadIdx.x], h[threadIdx.x]);
+      base[threadIdx.x] =
+          first[threadIdx.x] + atomicAdd(&hist[kCostBuckets + threadIdx.x], h[threadIdx.x]);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
@@ -1872,11 +1922,19 @@ hipError_t nb_bh_build(nb_ctx* c) {
   // 4-6. bodies in sorted order, FP64 moment prefix, octree
   hipLaunchKernelGGL(k_tree_mark, dim3(tiles), dim3(kTreeTile), 0, s, codes_sorted, perm, c->pm,
                      n, leaf, b.pms, b.scan_part, b.marks, b.level_cnt);
-  hipLaunchKernelGGL(k_tree_scan, dim3(1 + kLevels), dim3(kScanThreads), 0, s, b.scan_part,
-                     b.level_cnt, tiles, n, leaf, pairs, b.counters, b.waves, b.rec_hist);
-  hipLaunchKernelGGL(k_tree_emit, dim3(tiles), dim3(kTreeTile), 0, s, b.pms, n, b.scan_part,
-                     b.marks, b.level_cnt, b.counters, b.max_nodes, b.prefix, b.nodes, b.node_next,
-                     b.node_end, b.level_off, c->flags);
+  const Records records{b.waves, b.counters, b.rec_hist};
+  const auto emit = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(kTreeTile), 0, s, b.pms, n, leaf, pairs,
+                       b.scan_part, b.marks, b.level_cnt, b.counters, records, b.max_nodes,
+                       b.prefix, b.nodes, b.node_next, b.node_end, b.level_off, c->flags);
+  };
+  if (tiles <= 64) {
+    emit(k_tree_emit<true>);
+  } else {
+    hipLaunchKernelGGL(k_tree_scan, dim3(2 + kLevels), dim3(kScanThreads), 0, s, b.scan_part,
+                       b.level_cnt, tiles, n, leaf, pairs, b.counters, records);
+    emit(k_tree_emit<false>);
+  }
   // 7. centre of mass, wave ranges
   const int cgrid = (int)std::max<int64_t>(1, std::min<int64_t>((b.max_nodes + 255) / 256, 8192));
   const int cubic = (c->cfg.flags & NB_F_BH_AXIS_BOX) ? 0 : 1;
@@ -1905,7 +1963,6 @@ hipError_t nb_bh_traverse(nb_ctx* c, bool count_interactions) {
     const int og = std::max(1, std::min((n + kOrderChunk - 1) / kOrderChunk, kOrderBlocks));
     hipLaunchKernelGGL(k_rec_bucket, dim3(og), dim3(256), 0, c->stream, b.waves, b.counters, n,
                        b.rec_cost, b.vals[0], b.rec_bucket, b.rec_hist);
-    hipLaunchKernelGGL(k_rec_offsets, dim3(1), dim3(64), 0, c->stream, b.rec_hist);
     hipLaunchKernelGGL(k_rec_scatter, dim3(og), dim3(256), 0, c->stream, b.counters, n,
                        b.rec_bucket, b.rec_hist, b.rec_order);
   }
