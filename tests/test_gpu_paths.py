@@ -203,3 +203,24 @@ def test_large_host_copies(nb, n):
             for got, want in zip(sim.download(), (pos, vel, acc)):
                 np.testing.assert_array_equal(got[:, :3], want.astype(np.float32))
         sim.energy() if n < 100000 else sim.sync()
+
+
+@pytest.mark.parametrize("sizes", [(1, 4096, 4097), (8192, 300, 8193), (16384, 16385), (20481, 33000)])
+def test_batch_clusters_in_parts(nb, ora, sizes):
+    """Large clusters are summed in 1 to 4 parts: forces against FP64, the same bits
+    alone and together, and steps use the forces of the force pass."""
+    sys_ = [nb.ic_plummer(50 + n, n, 50.0, 1e4) for n in sizes]
+    with nb.Batch(sum(n + 256 for n in sizes), len(sizes)) as b:
+        ids = [b.add(p, v, m, EPS2, DT) for p, v, m in sys_]
+        f = [b.forces(c) for c in ids]
+        b.step(1)
+        acc = [b.download(c)[2] for c in ids]
+    for (pos, vel, m), n, mine, a in zip(sys_, sizes, f, acc):
+        np.testing.assert_array_equal(mine, a)
+        with nb.Batch(n + 256, 1) as b:
+            c = b.add(pos, vel, m, EPS2, DT)
+            np.testing.assert_array_equal(b.forces(c), mine)
+        tgt = np.arange(0, n, max(1, n // 300))
+        ref = ora.direct_f64(pos.astype(np.float32).astype(np.float64), m.astype(np.float64), EPS2, targets=tgt)
+        # 256-source FP32 sums, folded: 256 roundings of the largest force at worst
+        assert np.abs(mine[tgt] - ref).max() <= 256 * 2.0 ** -24 * (np.linalg.norm(ref, axis=1).max() + 1e-30)
