@@ -144,11 +144,39 @@ __global__ __launch_bounds__(256) void k_integrate(int n, double dt, double* __r
 // sources. Bound by latencies (staging, merge) and the LDS reads; fewer lanes with
 // more bodies each halve the reads but lengthen the merge (2048 bodies: 8 x 1 5.9 us,
 // 4 x 2 7.3, 2 x 4 10.6; 4096: 16 x 1 10.6, 8 x 2 11.7). Steps in us, k_direct and
-// k_integrate against this: 256 bodies 6.9 / 4.7, 1000 9.7 / 5.1, 2048 11.0 / 5.9,
+// k_integrate against this: 256 bodies 6.9 / 4.2, 1000 9.7 / 4.7, 2048 11.0 / 5.8,
 // 4096 14.5 / 10.4, 6000 22.3 / 21.2, 8192 29.7 / 26.9, where the LDS ends it.
 // A slice is at most 128 terms in FP32; slices are added in FP64.
 // kMode 0: forces only, to `force`; 1: KDK step; 2: Euler step (as k_integrate).
 constexpr int kSmallThreads = 1024;
+
+// The sum over the lanes l, l + kLanes, l + 2 kLanes, ... of a wave, in every one of
+// them: lane swaps and rotations in registers, without the LDS round trips of a
+// shuffle (steps: 256 bodies 4.8 -> 4.2 us, 1000 5.1 -> 4.7, 2048 6.0 -> 5.8).
+template <int kLanes>
+__device__ __forceinline__ double sum_slices(double v) {
+  static_assert(kLanes == 4 || kLanes == 8 || kLanes == 16, "rows of 16 lanes");
+  const auto halves = [](double x, auto exchange) {  // both halves of x moved alike, added
+    const uint64_t b = (uint64_t)__double_as_longlong(x);
+    const auto lo = exchange((uint32_t)b), hi = exchange((uint32_t)(b >> 32));
+    return __longlong_as_double((long long)((uint64_t)hi[0] << 32 | lo[0])) +
+           __longlong_as_double((long long)((uint64_t)hi[1] << 32 | lo[1]));
+  };
+  // swapping a register's odd rows (or upper half) with the even ones of its copy
+  // leaves the two lanes' values side by side
+  v = halves(v, [](uint32_t w) { return __builtin_amdgcn_permlane32_swap(w, w, false, false); });
+  v = halves(v, [](uint32_t w) { return __builtin_amdgcn_permlane16_swap(w, w, false, false); });
+  const auto rotate = [](double x, auto ctrl) {
+    const uint64_t b = (uint64_t)__double_as_longlong(x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, decltype(ctrl)::value, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), decltype(ctrl)::value, 0xf, 0xf, false);
+    return x + __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+  };
+  if constexpr (kLanes <= 8) v = rotate(v, std::integral_constant<int, 0x128>{});  // row_ror:8
+  if constexpr (kLanes <= 4) v = rotate(v, std::integral_constant<int, 0x124>{});  // row_ror:4
+  return v;
+}
+
 template <int kLanes, int kPer, int kMaxPad, bool kGuard, int kMode>
 __global__ __launch_bounds__(kSmallThreads) void k_direct_small(
     const float4* __restrict__ pm, int n, int n_pad, float eps2, double G, double dt,
@@ -201,8 +229,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_direct_small(
     double f[3] = {fx[r], fy[r], fz[r]};
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-#pragma unroll
-      for (int off = kLanes; off < 64; off <<= 1) f[c] += __shfl_xor(f[c], off);
+      f[c] = sum_slices<kLanes>(f[c]);
       if (lane < kLanes) sums[wave][c][lane + kLanes * r] = f[c];
     }
   }
