@@ -1150,9 +1150,32 @@ __device__ __forceinline__ void list_flush(const uint32_t* list, int lc, float4*
   nbcore::two_sum_fold(sz, cz, az);
 }
 
+// The lanes whose b is true; __ballot takes an int and would make one of b first.
+__device__ __forceinline__ uint64_t lanes_where(bool b) { return __builtin_amdgcn_ballot_w64(b); }
+
 // Bits of m below this lane.
 __device__ __forceinline__ int bits_below(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+}
+
+// A stack entry: the children of an opened node.
+__device__ __forceinline__ int2 stack_entry(int first, int level, int body_end) {
+  return make_int2(first, (int)(((uint32_t)level << 27) | (uint32_t)body_end));
+}
+
+// Child slot ci (0..7) of entry e: true where the slot holds a child, whose index and
+// record are then in child and cl. The nodes from the entry's first on are its children
+// as long as they are of the children's level (the last parent of a level is followed by
+// the next level) and start before the parent's end. A lane without a candidate reads
+// the root's record: no lane is masked off, and the record needs no initial value.
+__device__ __forceinline__ bool child_at(int2 e, int ci, bool have, int total,
+                                         const nb_node* __restrict__ nodes, int& child, nb_node& cl) {
+  const int cand = e.x + ci;
+  const bool ok = have && (uint32_t)cand < (uint32_t)total;
+  child = ok ? cand : 0;
+  cl = nodes[child];
+  const uint32_t w = (uint32_t)e.y;
+  return ok && cl.start < (int)(w & ((1u << 27) - 1)) && span_level(cl.span) == (int)(w >> 27);
 }
 
 // Append the bodies of the leaves that the lanes hold (in lane order) to a list of
@@ -1164,7 +1187,7 @@ __device__ __forceinline__ int bits_below(uint64_t m) {
 template <int kCap, typename Flush>
 __device__ __forceinline__ void list_leaves(uint32_t* list, int& lc, int lane, bool leaf, int start,
                                             int count, int n, Flush flush) {
-  uint64_t bl = __ballot(leaf);
+  uint64_t bl = lanes_where(leaf);
   if (bl == 0) return;
   const int mine = leaf ? count : 0;
   const int incl = wave_incl_scan(mine);
@@ -1172,7 +1195,7 @@ __device__ __forceinline__ void list_leaves(uint32_t* list, int& lc, int lane, b
   if (total <= kCap) {
     if (lc + total > kCap) flush();
     uint32_t* at = list + lc + incl - mine;
-    for (int k = 0; __ballot(k < mine); ++k)
+    for (int k = 0; lanes_where(k < mine); ++k)
       if (k < mine) at[k] = (uint32_t)min(start + k, n - 1);
     lc += total;
     return;
@@ -1197,7 +1220,6 @@ struct WaveLds {
   int2* stack;
   uint32_t* list;
   float4* stage;
-  const int* lvl;      // first node of each level (kMaxLevel + 2 entries)
   int cap;             // entries of the stack region in use (<= kStackCap)
 };
 
@@ -1229,8 +1251,8 @@ __device__ __forceinline__ float box_dist2(const Box& b, const float4& c) {
 // and a deferred cell is decided by each range's own test.
 template <bool kCount, bool kGuard, bool kShared>
 __device__ void walk(const WaveLds& L, int lane, int slice, int log2S, float4 me, int n,
-                     const float4* __restrict__ pms, const nb_node* __restrict__ nodes, float eps2,
-                     int* __restrict__ flags, const Box& U, const Box& A, const Box& B, int& nd,
+                     const float4* __restrict__ pms, const nb_node* __restrict__ nodes, int total,
+                     float eps2, int* __restrict__ flags, const Box& U, const Box& A, const Box& B, int& nd,
                      float& ax, float& ay, float& az, float& cx, float& cy, float& cz,
                      unsigned long long& cnt) {
   int2* stack = L.stack;
@@ -1244,21 +1266,22 @@ __device__ void walk(const WaveLds& L, int lane, int slice, int log2S, float4 me
   int sp = 0, lc = 0, dpos = 0;
   if (kShared || nd == 0) {
     // a virtual parent whose only child is the root
-    if (lane == 0) stack[0] = make_int2(0, (int)((1u << 27) | (uint32_t)n));
+    if (lane == 0) stack[0] = stack_entry(0, 0, n);
     sp = 1;
     __builtin_amdgcn_wave_barrier();
   }
-  const int q = lane >> 3, ci = lane & 7;
-  for (int iter = 0; sp > 0 || (!kShared && dpos < nd); ++iter) {
-    if (iter > L.lvl[kMaxLevel + 1]) {  // every node is examined at most once
-      if (lane == 0) atomicOr(flags, 4);
-      break;
-    }
+  int left = total;  // iterations: every node is examined at most once
+  for (; left >= 0 && (sp > 0 || (!kShared && dpos < nd)); --left) {
     // room for this iteration's accepted cells (at most 64), flushed while
     // nothing of the iteration is live
     if (lc + 64 > kListCap) NB_FLUSH();
-    int child = -1, efirst = 0;
-    nb_node cl{make_float4(0.f, 0.f, 0.f, 0.f), 0.f, -1, 0, 0};
+    // opaque per iteration: what follows from the lane is computed where it is used
+    // instead of being held, and then spilled, over the whole walk
+    asm volatile("" : "+v"(lane));
+    const int q = lane >> 3, ci = lane & 7;
+    int child, efirst = 0;
+    nb_node cl;
+    bool valid;
     if (!kShared && sp < 8 && dpos < nd) {
       // deferred entries: up to 32 of them, at most 64 cells, listed in the
       // staging area (free while walking) so that lane j takes the j-th cell
@@ -1267,58 +1290,41 @@ __device__ void walk(const WaveLds& L, int lane, int slice, int log2S, float4 me
       if (have) d = stack[L.cap - 1 - (dpos + lane)];
       const int pc = __popc((uint32_t)d.y);
       const int incl = wave_incl_scan(pc);
-      const uint64_t fit = __ballot(have && incl <= 64);
-      const int kd = __popcll(fit);  // >= 1: one entry has at most 8 cells
+      const bool fits = have && incl <= 64;
+      const int kd = __popcll(lanes_where(fits));  // >= 1: one entry has at most 8 cells
       int* cells = reinterpret_cast<int*>(L.stage);
-      if ((fit >> lane) & 1) {
+      if (fits) {
         int o = incl - pc;
         for (uint32_t mm = (uint32_t)d.y; mm; mm &= mm - 1) cells[o++] = d.x + __ffs(mm) - 1;
       }
       __builtin_amdgcn_wave_barrier();
-      const int T = __builtin_amdgcn_readlane(incl, kd - 1);
-      if (lane < T) {
-        child = cells[lane];
-        cl = nodes[child];
-      }
+      valid = lane < __builtin_amdgcn_readlane(incl, kd - 1);
+      child = valid ? cells[lane] : 0;
+      cl = nodes[child];
       __builtin_amdgcn_wave_barrier();
       dpos += kd;
     } else {
       const int k = min(sp, 8);
       sp -= k;
-      if (q < k) {
-        // entry: first child, and (slots << 27 | parent's body end); the slots
-        // stop at the end of the children's level, so every load below is in
-        // bounds and the three are issued together (a child is one whose bodies
-        // start before the parent's end)
-        const int2 e = stack[sp + q];
-        efirst = e.x;
-        const uint32_t w = (uint32_t)e.y;
-        const int slots = (int)(w >> 27);
-        const int pend = (int)(w & ((1u << 27) - 1));
-        if (ci < slots) {
-          const int cand = e.x + ci;
-          cl = nodes[cand];
-          if (cl.start < pend) child = cand;
-        }
-      }
+      const int2 e = stack[sp + min(q, k - 1)];
+      efirst = e.x;
+      valid = child_at(e, ci, q < k, total, nodes, child, cl);
       __builtin_amdgcn_wave_barrier();
     }
-    bool accept = false, defer = false, leaf = false, open = false;
-    if (child >= 0) {
-      // the group's modified test (see open_radius2); a pair shares what both accept
-      if (kShared) {
-        const bool a = cl.r2 < box_dist2(A, cl.com), b = cl.r2 < box_dist2(B, cl.com);
-        accept = a && b;
-        defer = a != b;
-      } else {
-        accept = cl.r2 < box_dist2(U, cl.com);
-      }
-      leaf = !accept && !defer && cl.first < 0;
-      open = !accept && !defer && cl.first >= 0;
+    // the group's modified test (see open_radius2); a pair shares what both accept
+    bool accept, defer = false;
+    if (kShared) {
+      const bool a = cl.r2 < box_dist2(A, cl.com), b = cl.r2 < box_dist2(B, cl.com);
+      accept = valid && a && b;
+      defer = valid && a != b;
+    } else {
+      accept = valid && cl.r2 < box_dist2(U, cl.com);
     }
+    const bool rest = valid && !accept && !defer;
+    const bool leaf = rest && cl.first < 0, open = rest && cl.first >= 0;
     // accepted cells with mass -> list
     const bool acc = accept && cl.com.w > 0.f;
-    const uint64_t ba = __ballot(acc);
+    const uint64_t ba = lanes_where(acc);
     if (acc) list[lc + bits_below(ba)] = (uint32_t)child | kCellBit;
     lc += __popcll(ba);
     // deferred cells -> one entry per stack entry that has any
@@ -1327,34 +1333,36 @@ __device__ void walk(const WaveLds& L, int lane, int slice, int log2S, float4 me
     uint32_t dmask = 0;
     uint64_t bg = 0;
     if (kShared) {
-      const uint64_t bd = __ballot(defer);
+      const uint64_t bd = lanes_where(defer);
       if (bd) {
         const uint32_t half = q < 4 ? (uint32_t)bd : (uint32_t)(bd >> 32);
         dmask = (half >> (lane & 24)) & 0xffu;  // bits 8q .. 8q + 7
         head = ci == 0 && dmask != 0;
-        bg = __ballot(head);
+        bg = lanes_where(head);
         nd_add = __popcll(bg);
       }
     }
     // opened cells -> stack
-    const uint64_t bo = __ballot(open);
-    if (sp + __popcll(bo) + nd + nd_add > L.cap) {
+    const uint64_t bo = lanes_where(open);
+    const int opened = __popcll(bo);
+    if (sp + opened + nd + nd_add > L.cap) {  // reported; nothing more is walked
       if (lane == 0) atomicOr(flags, 8);
-      break;
+      sp = 0;
+      dpos = nd;
+    } else {
+      if (kShared && head) stack[L.cap - 1 - (nd + bits_below(bg))] = make_int2(efirst, (int)dmask);
+      nd += nd_add;
+      if (open)
+        stack[sp + bits_below(bo)] =
+            stack_entry(cl.first, span_level(cl.span) + 1, cl.start + span_count(cl.span));
+      sp += opened;
     }
-    if (kShared && head) stack[L.cap - 1 - (nd + bits_below(bg))] = make_int2(efirst, (int)dmask);
-    nd += nd_add;
-    if (open) {
-      const uint32_t pend = (uint32_t)(cl.start + span_count(cl.span));
-      const int slots = max(0, min(8, L.lvl[span_level(cl.span) + 2] - cl.first));
-      stack[sp + bits_below(bo)] = make_int2(cl.first, (int)(((uint32_t)slots << 27) | pend));
-    }
-    sp += __popcll(bo);
     // leaves that are not accepted -> the indices of their bodies
     list_leaves<kListCap>(list, lc, lane, leaf, cl.start, span_count(cl.span), n,
                           [&] { NB_FLUSH(); });
     __builtin_amdgcn_wave_barrier();
   }
+  if (left < 0 && lane == 0) atomicOr(flags, 4);
   NB_FLUSH();
 #undef NB_FLUSH
 }
@@ -1415,13 +1423,10 @@ __global__ __launch_bounds__(64 * kListWaves, kCount ? 5 : kListBlocksPerCU) voi
   __shared__ int2 s_stack[kListWaves][kStackCap];
   __shared__ uint32_t s_list[kListWaves][kListCap];
   __shared__ float4 s_stage[kListWaves][64];
-  __shared__ int s_lvl[kMaxLevel + 2];
-  if (threadIdx.x < kMaxLevel + 2)
-    s_lvl[threadIdx.x] = (int)min((int64_t)level_off[threadIdx.x], max_nodes);
-  __syncthreads();
+  const int total = (int)min((int64_t)level_off[kMaxLevel + 1], max_nodes);
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const WaveLds L{s_stack[wave], s_list[wave], s_stage[wave], s_lvl,
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const WaveLds L{s_stack[wave], s_list[wave], s_stage[wave],
                   stack_cap > 0 && stack_cap < kStackCap ? stack_cap : kStackCap};
   const int nrec = min(wctl[0], n);
   unsigned long long cnt = 0;
@@ -1450,10 +1455,10 @@ __global__ __launch_bounds__(64 * kListWaves, kCount ? 5 : kListBlocksPerCU) voi
     unsigned long long c = 0;
     int nd = 0;
     if (pair)
-      walk<kCount, kGuard, true>(L, lane, slice, log2S, me, n, pms, nodes, eps2, flags, A,
-                                 A, B, nd, ax, ay, az, cx, cy, cz, c);
+      walk<kCount, kGuard, true>(L, lane, slice, log2S, me, n, pms, nodes, total, eps2, flags,
+                                 A, A, B, nd, ax, ay, az, cx, cy, cz, c);
     else
-      walk<kCount, kGuard, false>(L, lane, slice, log2S, me, n, pms, nodes, eps2, flags,
+      walk<kCount, kGuard, false>(L, lane, slice, log2S, me, n, pms, nodes, total, eps2, flags,
                                   A, A, B, nd, ax, ay, az, cx, cy, cz, c);
     // each slice's compensated sum in FP64, then the slices added (butterfly
     // over the slice bits, fixed order)
@@ -1486,7 +1491,7 @@ __global__ __launch_bounds__(64 * kListWaves, kCount ? 5 : kListBlocksPerCU) voi
       ax = ay = az = cx = cy = cz = 0.f;
       c = 0;
       walk<kCount, kGuard, false>(L, lane, lane / P, 6 - (31 - __clz(P)), me2, n, pms, nodes,
-                                  eps2, flags, h ? B : A, A, B, nd, ax, ay, az, cx, cy, cz, c);
+                                  total, eps2, flags, h ? B : A, A, B, nd, ax, ay, az, cx, cy, cz, c);
       double gx = (double)ax + (double)cx, gy = (double)ay + (double)cy,
              gz = (double)az + (double)cz;
       for (int off = P; off < 64; off <<= 1) {
@@ -1571,11 +1576,9 @@ __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_
   __shared__ uint32_t s_list[kWaves][kBlockListCap];
   __shared__ float4 s_stage[kWaves][64];
   __shared__ int2 s_cnt[kWaves];  // (opened children, list length) of each wave
-  __shared__ int s_lvl[kMaxLevel + 2];
   __shared__ int s_rec;
   static_assert(sizeof(s_stage[0]) >= 3 * kWaveBodies * sizeof(double), "a wave's sums fit its stage");
-  if (threadIdx.x < kMaxLevel + 2)
-    s_lvl[threadIdx.x] = (int)min((int64_t)level_off[threadIdx.x], max_nodes);
+  const int total = (int)min((int64_t)level_off[kMaxLevel + 1], max_nodes);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint32_t* list = s_list[wave];
@@ -1606,39 +1609,28 @@ __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_
       lc = 0;
     };
     // a virtual parent whose only child is the root
-    if (threadIdx.x == 0) stack[0] = make_int2(0, (int)((1u << 27) | (uint32_t)n));
+    if (threadIdx.x == 0) stack[0] = stack_entry(0, 0, n);
     __syncthreads();
     for (int iter = 0; sp > 0; ++iter) {  // sp is the same in every wave
-      if (iter > s_lvl[kMaxLevel + 1]) {  // every node is examined at most once
+      if (iter > total) {  // every node is examined at most once
         if (threadIdx.x == 0) atomicOr(flags, 4);
         break;
       }
       const int k = min(sp, 8 * kWaves);
       sp -= k;
       const int q = 8 * wave + (lane >> 3), ci = lane & 7;
-      int child = -1;
-      nb_node cl{make_float4(0.f, 0.f, 0.f, 0.f), 0.f, -1, 0, 0};
-      if (q < k) {  // entries and their candidates as in walk()
-        const int2 e = stack[sp + q];
-        const uint32_t ew = (uint32_t)e.y;
-        if (ci < (int)(ew >> 27)) {
-          const int cand = e.x + ci;
-          cl = nodes[cand];
-          if (cl.start < (int)(ew & ((1u << 27) - 1))) child = cand;
-        }
-      }
-      bool accept = false, leaf = false, open = false;
-      if (child >= 0) {
-        accept = cl.r2 < box_dist2(A, cl.com);
-        leaf = !accept && cl.first < 0;
-        open = !accept && cl.first >= 0;
-      }
+      int child;
+      nb_node cl;
+      const bool valid = child_at(stack[sp + min(q, k - 1)], ci, q < k, total, nodes, child, cl);
+      const bool accept = valid && cl.r2 < box_dist2(A, cl.com);
+      const bool rest = valid && !accept;
+      const bool leaf = rest && cl.first < 0, open = rest && cl.first >= 0;
       const bool acc = accept && cl.com.w > 0.f;
-      const uint64_t ba = __ballot(acc);
+      const uint64_t ba = lanes_where(acc);
       if (acc) list[lc + bits_below(ba)] = (uint32_t)child | kCellBit;
       lc += __popcll(ba);
       list_leaves<kBlockListCap>(list, lc, lane, leaf, cl.start, span_count(cl.span), n, flush);
-      const uint64_t bo = __ballot(open);
+      const uint64_t bo = lanes_where(open);
       if (lane == 0) s_cnt[wave] = make_int2(__popcll(bo), lc);
       __syncthreads();  // counts are in, and every wave has read its entries
       int before = 0, opened = 0, longest = 0;
@@ -1654,11 +1646,9 @@ __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_
         if (threadIdx.x == 0) atomicOr(flags, 8);
         break;
       }
-      if (open) {
-        const uint32_t pend = (uint32_t)(cl.start + span_count(cl.span));
-        const int slots = max(0, min(8, s_lvl[span_level(cl.span) + 2] - cl.first));
-        stack[sp + before + bits_below(bo)] = make_int2(cl.first, (int)(((uint32_t)slots << 27) | pend));
-      }
+      if (open)
+        stack[sp + before + bits_below(bo)] =
+            stack_entry(cl.first, span_level(cl.span) + 1, cl.start + span_count(cl.span));
       sp += opened;
       // room for the next iteration's accepted cells (at most 64 per wave)
       if (__builtin_amdgcn_readfirstlane(longest) + 64 > kBlockListCap) flush();
