@@ -1168,6 +1168,9 @@ __device__ __forceinline__ int2 stack_entry(int first, int level, int body_end) 
 // as long as they are of the children's level (the last parent of a level is followed by
 // the next level) and start before the parent's end. A lane without a candidate reads
 // the root's record: no lane is masked off, and the record needs no initial value.
+// With the entry read in one piece, nothing looked up per level and nothing held in
+// scratch memory a walk's iteration is about a quarter shorter (traversal of 2^22
+// bodies 4,672 us, now 4,385).
 __device__ __forceinline__ bool child_at(int2 e, int ci, bool have, int total,
                                          const nb_node* __restrict__ nodes, int& child, nb_node& cl) {
   const int cand = e.x + ci;
@@ -1404,14 +1407,17 @@ __device__ __forceinline__ void lane_boxes(float4 me, int keep, int from0, int f
 }
 
 // Persistent: every wave takes records from a ticket until none is left, so the
-// cost of uneven ranges balances dynamically. A record is one wave range or a
+// cost of uneven ranges balances dynamically. Its first record it has from its
+// own number: that many tickets at once are that many atomics on one address, about
+// 10 ns each, so the last of 6,144 waves began 60 us after the first (traversal of
+// 2^22 bodies 4,385 us, now 4,229; with workgroups as below 65,536 bodies 147, now
+// 132, 20,011 68, now 61). A record is one wave range or a
 // pair of sibling ranges (x, y) and (z, w), w > 0. A pair first walks once for
 // both (its lanes: [slice][range][slot], P1 lanes per copy of a range), then,
 // if cells were deferred, each range walks them with its own lanes ([slice][slot]);
 // each body's force is the sum of the two parts in FP64, in that order. The
 // counting variant (diagnostics only) needs more registers and is allowed five
-// blocks per CU; its surplus blocks start when others retire and take what
-// tickets are left.
+// blocks per CU; its surplus blocks start when others retire.
 template <bool kCount, bool kGuard>
 __global__ __launch_bounds__(64 * kListWaves, kCount ? 5 : kListBlocksPerCU) void k_traverse_list(
     const float4* __restrict__ pms, const uint32_t* __restrict__ perm, int n,
@@ -1430,11 +1436,8 @@ __global__ __launch_bounds__(64 * kListWaves, kCount ? 5 : kListBlocksPerCU) voi
                   stack_cap > 0 && stack_cap < kStackCap ? stack_cap : kStackCap};
   const int nrec = min(wctl[0], n);
   unsigned long long cnt = 0;
-  for (;;) {
-    int w = 0;
-    if (lane == 0) w = atomicAdd(&wctl[1], 1);
-    w = __builtin_amdgcn_readfirstlane(w);
-    if (w >= nrec) break;
+  const int static_recs = gridDim.x * kListWaves;
+  for (int w = wave * gridDim.x + blockIdx.x; w < nrec;) {
     const uint64_t t_start = wall_clock64();
     const int ri = order ? order[w] : w;
     const int4 rec = waves[(unsigned)ri < (unsigned)nrec ? ri : w];  // wave-uniform: scalar registers
@@ -1518,6 +1521,9 @@ __global__ __launch_bounds__(64 * kListWaves, kCount ? 5 : kListBlocksPerCU) voi
       const uint32_t o = perm[t];
       if (o < (uint32_t)n) cost[o] = share;
     }
+    if (nrec <= static_recs) break;
+    if (lane == 0) w = static_recs + atomicAdd(&wctl[1], 1);
+    w = __builtin_amdgcn_readfirstlane(w);
   }
   if (kCount) {
     __shared__ unsigned long long red[64 * kListWaves];
@@ -1550,19 +1556,20 @@ __global__ __launch_bounds__(64 * kListWaves, kCount ? 5 : kListBlocksPerCU) voi
 constexpr int block_stack(int waves) { return (9 * 56 + 64) * waves; }
 constexpr int kBlockListCap = 256;  // source indices per wave
 // Waves per range by the system's size. Measured Barnes-Hut steps in us (Plummer
-// sphere / uniform ball, leaf size 8), one, two, four and eight waves per range:
-//     4,000 bodies  224/197  153/137  121/107  105/ 90
-//    20,000         305/225  208/159  152/126  131/115
-//    40,000         283/248  215/185  175/147  174/142
-//    65,536         309/252  256/201  224/177  230/187
-//   131,072         421/331  347/275  332/262  355/287
-//   262,144         586/453  542/410  535/402  611/481
-//   400,000         777/582  757/561  769/575  897/719
-//   524,288         961/680  946/672  971/710 1157/902
-// Two would be the best in a narrow band, by 2%. Above it there are enough ranges
-// for every wave and the barriers only cost.
-constexpr int kBlock8Bodies = 5 << 13;    // below: eight waves per range
-constexpr int kBlockMaxBodies = 7 << 16;  // below: four; from here on k_traverse_list
+// sphere / uniform ball, leaf size 8), one (k_traverse_list), four and eight waves:
+//     4,000 bodies  148/121  103/ 88   96/ 81
+//    20,011         223/145  133/107  122/106
+//    30,011         267/158  154/120  146/119
+//    40,000         209/174  159/129  165/132
+//    65,536         255/180  205/158  220/174
+//   131,072         339/260  312/244  340/277
+//   200,000         415/319  412/312  470/370
+//   300,007         547/423  575/434  672/544
+//   524,288         823/580  931/677
+// Two gained 2% over four and one in a narrow band below the upper line. Above it
+// there are enough ranges for every wave and the barriers only cost.
+constexpr int kBlock8Bodies = 1 << 15;    // below: eight waves per range
+constexpr int kBlockMaxBodies = 1 << 18;  // below: four; from here on k_traverse_list
 constexpr int kBlockWavesPerCU = 24;      // by LDS and 80 VGPRs, as k_traverse_list
 
 template <bool kGuard, int kWaves>
@@ -1586,11 +1593,7 @@ __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_
   const int cap = stack_cap > 0 && stack_cap < block_stack(kWaves) ? stack_cap : block_stack(kWaves);
   const int nrec = min(wctl[0], n);
   unsigned long long unused = 0;
-  for (;;) {
-    if (threadIdx.x == 0) s_rec = atomicAdd(&wctl[1], 1);
-    __syncthreads();
-    const int w = __builtin_amdgcn_readfirstlane(s_rec);
-    if (w >= nrec) break;
+  for (int w = blockIdx.x; w < nrec;) {
     const uint64_t t_start = wall_clock64();
     const int ri = order ? order[w] : w;
     const int4 rec = waves[(unsigned)ri < (unsigned)nrec ? ri : w];
@@ -1676,6 +1679,10 @@ __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_
       // the range's device time, shared out over its bodies for the next pass's order
       if (cost) cost[o] = (float)(wall_clock64() - t_start) / (float)rec.y;
     }
+    if (nrec <= (int)gridDim.x) break;
+    if (threadIdx.x == 0) s_rec = gridDim.x + atomicAdd(&wctl[1], 1);
+    __syncthreads();  // the waves' sums have been read, too
+    w = __builtin_amdgcn_readfirstlane(s_rec);
   }
 }
 

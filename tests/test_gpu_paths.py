@@ -44,7 +44,8 @@ def test_tree_build_at_tile_edges(nb, ora, n, leaf):
 
 
 @pytest.mark.parametrize("n, leaf, eps2", [(3, 8, EPS2), (300, 64, EPS2), (5001, 1, 0.0), (20011, 64, EPS2),
-                                           (40959, 8, EPS2), (40960, 16, 0.0), (458751, 8, EPS2)])
+                                           (32767, 8, EPS2), (32768, 16, 0.0), (262143, 8, EPS2),
+                                           (262144, 8, EPS2)])
 def test_workgroup_walk_equals_pair_walk(nb, n, leaf, eps2):
     """Eight, then four waves per range, against the walk that one wave does for a
     pair of ranges: the same interactions, summed in another order. A level-10
