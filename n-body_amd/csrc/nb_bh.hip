@@ -144,6 +144,18 @@ __device__ __forceinline__ void block_bounds(float (&mn)[3], float (&mx)[3], flo
     }
 }
 
+// One thread's share of the bounds: bodies from, from + step, ...
+__device__ __forceinline__ void fold_bounds(const float4* __restrict__ pm, int from, int step, int n,
+                                            float (&mn)[3], float (&mx)[3]) {
+#pragma unroll 4
+  for (int i = from; i < n; i += step) {
+    const float4 p = pm[i];
+    mn[0] = fminf(mn[0], p.x); mx[0] = fmaxf(mx[0], p.x);
+    mn[1] = fminf(mn[1], p.y); mx[1] = fmaxf(mx[1], p.y);
+    mn[2] = fminf(mn[2], p.z); mx[2] = fmaxf(mx[2], p.z);
+  }
+}
+
 // Partial bounds per block, folded by every block of k_morton. Also clears the
 // radix passes' group counts.
 __global__ __launch_bounds__(1024) void k_bbox_partial(const float4* __restrict__ pm, int n,
@@ -154,13 +166,7 @@ __global__ __launch_bounds__(1024) void k_bbox_partial(const float4* __restrict_
   float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX};
   float mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
   for (int i = blockIdx.x * 1024 + threadIdx.x; i < counts; i += step) group_hist[i] = 0;
-#pragma unroll 4
-  for (int i = blockIdx.x * 1024 + threadIdx.x; i < n; i += step) {
-    const float4 p = pm[i];
-    mn[0] = fminf(mn[0], p.x); mx[0] = fmaxf(mx[0], p.x);
-    mn[1] = fminf(mn[1], p.y); mx[1] = fmaxf(mx[1], p.y);
-    mn[2] = fminf(mn[2], p.z); mx[2] = fmaxf(mx[2], p.z);
-  }
+  fold_bounds(pm, blockIdx.x * 1024 + threadIdx.x, step, n, mn, mx);
   block_bounds<16>(mn, mx, red);
   if (threadIdx.x == 0)
     for (int a = 0; a < 3; ++a) {
@@ -208,11 +214,13 @@ __device__ __forceinline__ void publish_counts(const int* h, int* __restrict__ h
   }
 }
 
-// Codes, and the digit counts of the first radix pass. Every block folds the
-// partial bounds itself (6 KB of L2 reads), which spares a launch of one block.
+// Codes, and the digit counts of the first radix pass. Every block folds
+// the partial bounds itself (6 KB of L2 reads), which spares a launch of one block;
+// kSelf: it takes the bounds of all bodies itself, which spares that launch, too.
 // cubic = 1: one extent E = max_a max(max_a - min_a, 1e-6) on every axis (a cubic
 // root cell, so every cell is a cube of side E / 2^level); cubic = 0: each axis
 // over its own extent max(max_a - min_a, 1e-6), exactly morton.glsl's inputs.
+template <bool kSelf>
 __global__ __launch_bounds__(1024) void k_morton(const float4* __restrict__ pm, int n, int cubic,
                                                  const float* __restrict__ part, int nparts,
                                                  float* __restrict__ geom,
@@ -224,11 +232,14 @@ __global__ __launch_bounds__(1024) void k_morton(const float4* __restrict__ pm, 
   if (threadIdx.x < 256) h[threadIdx.x] = 0;
   float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX};
   float mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-  if ((int)threadIdx.x < nparts)  // nparts <= kBboxBlocks
+  if (kSelf) {
+    fold_bounds(pm, threadIdx.x, 1024, n, mn, mx);
+  } else if ((int)threadIdx.x < nparts) {  // nparts <= kBboxBlocks
     for (int a = 0; a < 3; ++a) {
       mn[a] = part[6 * threadIdx.x + a];
       mx[a] = part[6 * threadIdx.x + 3 + a];
     }
+  }
   block_bounds<16>(mn, mx, red);  // ends behind a barrier: h is clear
   float ext[3], E = 0.f;
 #pragma unroll
@@ -257,9 +268,10 @@ __global__ __launch_bounds__(1024) void k_morton(const float4* __restrict__ pm, 
       const uint32_t qz = quantize(p.z, mn[2], cubic ? E : ext[2]);
       const uint32_t code = expand_bits(qx) * 4u + expand_bits(qy) * 2u + expand_bits(qz);
       codes[i] = code;
-      atomicAdd(&h[code & 255u], 1);
+      if (!kSelf) atomicAdd(&h[code & 255u], 1);
     }
   }
+  if (kSelf) return;  // as its digits are counted where they are sorted
   __syncthreads();
   publish_counts(h, hist, group_hist);
 }
@@ -301,19 +313,20 @@ __global__ __launch_bounds__(1024) void k_radix_hist(const uint32_t* __restrict_
   publish_counts(h, hist, group_hist);
 }
 
-// Mask of the active lanes whose 8-bit digit equals this lane's digit.
+// Mask of the active lanes whose digit of kBits bits equals this lane's digit.
+template <int kBits>
 __device__ __forceinline__ uint64_t match_digit(uint32_t d, uint64_t active) {
   uint64_t m = active;
 #pragma unroll
-  for (int b = 0; b < 8; ++b) {
+  for (int b = 0; b < kBits; ++b) {
     const bool bit = (d >> b) & 1u;
-    const uint64_t bb = __ballot(bit);
+    const uint64_t bb = __builtin_amdgcn_ballot_w64(bit);
     m &= bit ? bb : ~bb;
   }
   return m;
 }
 
-// Stable scatter of one 8-bit digit pass. A tile's first output index of a digit
+// Stable scatter of one digit's pass. A tile's first output index of a digit
 // is the number of smaller digits anywhere plus the number of its own digit in
 // earlier tiles: each block adds these up itself from the groups' counts and the
 // counts of the tiles before it in its group (four threads per digit; at 2^22
@@ -324,18 +337,25 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, uint64_t active) {
 // addresses instead of 64 scattered lines per wave store. Two keys per thread: a
 // pass over a small system is a chain of latencies (65,536 keys, counts and scatter:
 // 27 us in four launches with eight keys per thread, 11 us now; 2^22 keys 56 and 53).
+// Eight bits per pass: four passes. kSelf: the blocks count the digits of all keys
+// themselves, before and after their tile, which spares the counting launches, and
+// as no table of counts goes through memory the digits have ten bits: three passes,
+// three launches of 8.3 us at 20,011 keys in place of seven (30 us in all).
 // kFirst: the values are the indices themselves.
-template <bool kFirst>
+constexpr int kCopies = 2;  // of a count, for even and odd lanes: fewer atomics on one word
+template <bool kFirst, bool kSelf>
 __global__ __launch_bounds__(1024) void k_radix_scatter(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, int n, int shift,
     const int* __restrict__ hist, const int* __restrict__ group_hist, int groups,
     uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out) {
   constexpr int kRounds = kSortTile / 1024;
-  __shared__ int whist[16][256];  // per wave: digit counts, then first tile slots
-  __shared__ int s_part[2][4][256];
-  __shared__ int s_to_global[256];  // a digit's first output index minus its first tile slot
+  constexpr int kBits = kSelf ? 10 : 8, kDigits = 1 << kBits, kShare = kSelf ? kCopies : 1024 / kDigits;
+  __shared__ int whist[16][kDigits];  // per wave: digit counts, then those of the waves before
+  __shared__ int s_part[2][kShare][kDigits + (kSelf ? 64 / kCopies : 0)];
+  __shared__ int s_local[kDigits];      // a digit's first tile slot
+  __shared__ int s_to_global[kDigits];  // a digit's first output index minus its first tile slot
   __shared__ uint32_t sk[kSortTile], sv[kSortTile];
-  __shared__ int wsum[2][4];
+  __shared__ int wsum[2][kDigits / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint64_t lt = (uint64_t(1) << lane) - 1;
   const int tile0 = blockIdx.x * kSortTile;
@@ -348,28 +368,49 @@ __global__ __launch_bounds__(1024) void k_radix_scatter(
     key[r] = e < n ? keys_in[e] : 0u;
     val[r] = kFirst ? (uint32_t)e : e < n ? vals_in[e] : 0u;
   }
-  {
-    const int d = threadIdx.x & 255, q = threadIdx.x >> 8;
+  if (kSelf) {
+    // s_part[0]: digits of the tiles after this one, s_part[1]: of those before
+    int* const parts = &s_part[0][0][0];
+    for (int i = threadIdx.x; i < (int)(sizeof(s_part) / 4); i += 1024) parts[i] = 0;
+    __syncthreads();
+    const auto count = [&](int from, int to, int* h) {  // from: a multiple of four
+      for (int e = from + 4 * threadIdx.x; e < to; e += 4096) {
+        uint32_t k[4];
+        if (e + 3 < to) {
+          const uint4 v = *reinterpret_cast<const uint4*>(keys_in + e);
+          k[0] = v.x, k[1] = v.y, k[2] = v.z, k[3] = v.w;
+        } else {
+          for (int u = 0; u < 4; ++u) k[u] = e + u < to ? keys_in[e + u] : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (e + u < to) atomicAdd(&h[(k[u] >> shift) & (kDigits - 1)], 1);
+      }
+    };
+    count(0, tile0, s_part[1][lane & (kCopies - 1)]);
+    count(tile0 + kSortTile, n, s_part[0][lane & (kCopies - 1)]);
+  } else {
+    const int d = threadIdx.x & (kDigits - 1), q = threadIdx.x >> kBits;
     const int mine = blockIdx.x / kSortGroup;
     int total = 0, before = 0;
-    for (int g = q; g < groups; g += 4) {
-      const int c = group_hist[g * 256 + d];
+    for (int g = q; g < groups; g += kShare) {
+      const int c = group_hist[g * kDigits + d];
       total += c;
       before += g < mine ? c : 0;
     }
-    for (int t = mine * kSortGroup + q; t < (int)blockIdx.x; t += 4) before += hist[t * 256 + d];
+    for (int t = mine * kSortGroup + q; t < (int)blockIdx.x; t += kShare) before += hist[t * kDigits + d];
     s_part[0][q][d] = total;
     s_part[1][q][d] = before;
   }
 #pragma unroll
-  for (int k = 0; k < 4; ++k) whist[wave][64 * k + lane] = 0;  // the wave's own row
+  for (int k = 0; k < kDigits / 64; ++k) whist[wave][64 * k + lane] = 0;  // the wave's own row
   __builtin_amdgcn_wave_barrier();
   int rank[kRounds];
 #pragma unroll
   for (int r = 0; r < kRounds; ++r) {
     const bool in = base + 64 * r < n;
-    const uint32_t d = (key[r] >> shift) & 255u;
-    const uint64_t m = match_digit(d, __ballot(in));
+    const uint32_t d = (key[r] >> shift) & (kDigits - 1);
+    const uint64_t m = match_digit<kBits>(d, __builtin_amdgcn_ballot_w64(in));
     rank[r] = whist[wave][d] + __popcll(m & lt);
     __builtin_amdgcn_wave_barrier();
     if (in && (m & lt) == 0) whist[wave][d] += __popcll(m);
@@ -377,7 +418,7 @@ __global__ __launch_bounds__(1024) void k_radix_scatter(
   }
   __syncthreads();
   int cnt = 0, total = 0, before = 0, incl_c = 0, incl_t = 0;
-  if (threadIdx.x < 256) {
+  if (threadIdx.x < kDigits) {
     const int d = threadIdx.x;
 #pragma unroll
     for (int w = 0; w < 16; ++w) {
@@ -386,10 +427,11 @@ __global__ __launch_bounds__(1024) void k_radix_scatter(
       cnt += c;
     }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < kShare; ++q) {
       total += s_part[0][q][d];
       before += s_part[1][q][d];
     }
+    if (kSelf) total += before + cnt;
     incl_c = wave_incl_scan(cnt);
     incl_t = wave_incl_scan(total);
     if (lane == 63) {
@@ -398,21 +440,21 @@ __global__ __launch_bounds__(1024) void k_radix_scatter(
     }
   }
   __syncthreads();
-  if (threadIdx.x < 256) {
+  if (threadIdx.x < kDigits) {
     const int d = threadIdx.x;
     int local = incl_c - cnt, global = incl_t - total + before;
     for (int w = 0; w < wave; ++w) {
       local += wsum[0][w];
       global += wsum[1][w];
     }
-#pragma unroll
-    for (int w = 0; w < 16; ++w) whist[w][d] += local;
+    s_local[d] = local;
     s_to_global[d] = global - local;
   }
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < kRounds; ++r) {
-    const int slot = whist[wave][(key[r] >> shift) & 255u] + rank[r];
+    const uint32_t d = (key[r] >> shift) & (kDigits - 1);
+    const int slot = s_local[d] + whist[wave][d] + rank[r];
     if (base + 64 * r < n && slot >= 0 && slot < kSortTile) {  // always, for consistent counts
       sk[slot] = key[r];
       sv[slot] = val[r];
@@ -425,7 +467,7 @@ __global__ __launch_bounds__(1024) void k_radix_scatter(
     const int i = r * 1024 + threadIdx.x;
     if (i < count) {
       const uint32_t k = sk[i];
-      const int dst = i + s_to_global[(k >> shift) & 255u];
+      const int dst = i + s_to_global[(k >> shift) & (kDigits - 1)];
       if (dst >= 0 && dst < n) {
         keys_out[dst] = k;
         vals_out[dst] = sv[i];
@@ -1859,30 +1901,54 @@ void nb_bh_free(nb_ctx* c) {
   b = nb_bh_state{};
 }
 
+// Up to here each block takes bounds and counts from all bodies instead of from other
+// launches' partial ones. Measured Barnes-Hut steps in us (Plummer sphere / uniform
+// ball), partial and own:
+//     4,000 bodies   96.4/ 80.8   84.9/ 69.9
+//    10,000         113.9/ 96.2  106.9/ 87.9
+//    20,011         121.0/105.4  118.9/100.5
+//    30,011         145.9/118.3  145.0/116.4
+//    40,000         157.1/130.1  162.5/131.3
+//    65,536         204.9/158.0  217.3/161.9
+constexpr int kSelfBodies = 3 << 13;
+
 hipError_t nb_morton_sort(nb_ctx* c) {
   nb_bh_state& b = c->bh;
   const int n = c->n;
   hipStream_t s = c->stream;
   const int tiles = b.sort_blocks, groups = (tiles + kSortGroup - 1) / kSortGroup;
-  // 1. bbox
-  const int parts = std::min(b.bbox_blocks, (n + 1023) / 1024);
-  hipLaunchKernelGGL(k_bbox_partial, dim3(parts), dim3(1024), 0, s, c->pm, n, b.bbox_part,
-                     b.group_hist, 4 * 256 * groups);
-  // 2. encode
   const int cubic = (c->cfg.flags & NB_F_BH_AXIS_BOX) ? 0 : 1;
-  hipLaunchKernelGGL(k_morton, dim3(tiles), dim3(1024), 0, s, c->pm, n, cubic, b.bbox_part, parts,
-                     b.geom, b.codes, b.digit_hist, b.group_hist);
-  // 3. sort: 4 passes of 8 bits, codes -> 1 -> 0 -> 1 -> 0
-  hipLaunchKernelGGL((k_radix_scatter<true>), dim3(tiles), dim3(1024), 0, s, b.codes, nullptr, n, 0,
-                     b.digit_hist, b.group_hist, groups, b.keys[1], b.vals[1]);
-  for (int pass = 1; pass < 4; ++pass) {
-    const int in = pass & 1, out = in ^ 1;
-    int* gh = b.group_hist + pass * groups * 256;
-    hipLaunchKernelGGL(k_radix_hist, dim3(tiles), dim3(1024), 0, s, b.keys[in], n, 8 * pass,
-                       b.digit_hist, gh);
-    hipLaunchKernelGGL((k_radix_scatter<false>), dim3(tiles), dim3(1024), 0, s, b.keys[in],
-                       b.vals[in], n, 8 * pass, b.digit_hist, gh, groups, b.keys[out],
-                       b.vals[out]);
+  const bool self = n <= kSelfBodies;
+  // 1-2. bounding box and codes
+  if (self) {
+    hipLaunchKernelGGL(k_morton<true>, dim3(tiles), dim3(1024), 0, s, c->pm, n, cubic, nullptr, 0,
+                       b.geom, b.codes, nullptr, nullptr);
+  } else {
+    const int parts = std::min(b.bbox_blocks, (n + 1023) / 1024);
+    hipLaunchKernelGGL(k_bbox_partial, dim3(parts), dim3(1024), 0, s, c->pm, n, b.bbox_part,
+                       b.group_hist, 4 * 256 * groups);
+    hipLaunchKernelGGL(k_morton<false>, dim3(tiles), dim3(1024), 0, s, c->pm, n, cubic, b.bbox_part,
+                       parts, b.geom, b.codes, b.digit_hist, b.group_hist);
+  }
+  // 3. sort: the last pass writes keys[0] and vals[0]
+  const auto scatter = [&](auto kernel, const uint32_t* keys, const uint32_t* vals, int shift,
+                           const int* gh, int out) {
+    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(1024), 0, s, keys, vals, n, shift, b.digit_hist, gh,
+                       groups, b.keys[out], b.vals[out]);
+  };
+  if (self) {
+    scatter(k_radix_scatter<true, true>, b.codes, nullptr, 0, nullptr, 0);
+    scatter(k_radix_scatter<false, true>, b.keys[0], b.vals[0], 10, nullptr, 1);
+    scatter(k_radix_scatter<false, true>, b.keys[1], b.vals[1], 20, nullptr, 0);
+  } else {
+    scatter(k_radix_scatter<true, false>, b.codes, nullptr, 0, b.group_hist, 1);
+    for (int pass = 1; pass < 4; ++pass) {
+      const int in = pass & 1;
+      int* gh = b.group_hist + pass * groups * 256;
+      hipLaunchKernelGGL(k_radix_hist, dim3(tiles), dim3(1024), 0, s, b.keys[in], n, 8 * pass,
+                         b.digit_hist, gh);
+      scatter(k_radix_scatter<false, false>, b.keys[in], b.vals[in], 8 * pass, gh, in ^ 1);
+    }
   }
   b.sorted_buf = 0;
   return hipGetLastError();

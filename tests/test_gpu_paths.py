@@ -65,9 +65,9 @@ def test_workgroup_walk_equals_pair_walk(nb, n, leaf, eps2):
     assert np.abs(f[0] - f[1]).max() <= 192 * 2.0 ** -24 * scale
 
 
-@pytest.mark.parametrize("n", [1, 63, 2047, 2049, 131071, 131073, 264193])
+@pytest.mark.parametrize("n", [1, 63, 2047, 2049, 24576, 24577, 131071, 131073, 264193])
 def test_radix_sort_at_tile_and_group_edges(nb, ora, n):
-    """Tiles of 2048 keys in groups of 64: codes and the stable permutation."""
+    """Tiles of 2048 keys, in groups of 64 above 24,576: codes and the stable permutation."""
     rng = np.random.default_rng(n)
     pos = np.round(rng.normal(size=(n, 3)) * 8) if n % 4 == 1 else rng.normal(size=(n, 3))
     m = np.ones(n, np.float32)
