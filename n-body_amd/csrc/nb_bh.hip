@@ -1171,18 +1171,24 @@ __device__ __forceinline__ void list_flush(const uint32_t* list, int lc, float4*
     // slice's block; entries at or past m are zero-mass pads.
     const int T = __builtin_amdgcn_readfirstlane((((m + S - 1) >> log2S) + 3) & ~3);
     for (int t = 0; t < T; t += 4) {
+      float dx[4], dy[4], dz[4], r2[4], inv[4], w[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const float4 src = mine[t + u];  // few distinct addresses: LDS broadcast
-        const float dx = src.x - me.x, dy = src.y - me.y, dz = src.z - me.z;
-        const float r2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, eps2)));
-        const float inv = __builtin_amdgcn_rsqf(r2);
-        float s = (src.w * inv) * (inv * inv);
-        if (kGuard) s = r2 > 0.f ? s : 0.f;
-        ax = fmaf(dx, s, ax);
-        ay = fmaf(dy, s, ay);
-        az = fmaf(dz, s, az);
-        if (kCount) cnt += (src.w > 0.f && fmaf(dz, dz, fmaf(dy, dy, dx * dx)) > 0.f) ? 1 : 0;
+        w[u] = src.w;
+        dx[u] = src.x - me.x, dy[u] = src.y - me.y, dz[u] = src.z - me.z;
+        r2[u] = fmaf(dz[u], dz[u], fmaf(dy[u], dy[u], fmaf(dx[u], dx[u], eps2)));
+      }
+      nbcore::rsq_group(r2, inv);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        float s = (w[u] * inv[u]) * (inv[u] * inv[u]);
+        if (kGuard) s = r2[u] > 0.f ? s : 0.f;
+        ax = fmaf(dx[u], s, ax);
+        ay = fmaf(dy[u], s, ay);
+        az = fmaf(dz[u], s, az);
+        if (kCount)
+          cnt += (w[u] > 0.f && fmaf(dz[u], dz[u], fmaf(dy[u], dy[u], dx[u] * dx[u])) > 0.f) ? 1 : 0;
       }
     }
     __builtin_amdgcn_wave_barrier();
@@ -1648,11 +1654,15 @@ __global__ __launch_bounds__(64 * kWaves, kBlockWavesPerCU / 4) void k_traverse_
     lane_boxes(me, 0, 0, 0, A, B);
     float ax = 0.f, ay = 0.f, az = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
     int lc = 0, sp = 1;
+    // the walk, a chain of loads, goes before other waves' arithmetic
     auto flush = [&]() {
+      __builtin_amdgcn_s_setprio(0);
       list_flush<false, kGuard>(list, lc, stage, lane, slice, log2S, pms, nodes, me, eps2, ax, ay, az,
                                 cx, cy, cz, unused);
+      __builtin_amdgcn_s_setprio(1);
       lc = 0;
     };
+    __builtin_amdgcn_s_setprio(1);
     // a virtual parent whose only child is the root
     if (threadIdx.x == 0) stack[0] = stack_entry(0, 0, n);
     __syncthreads();

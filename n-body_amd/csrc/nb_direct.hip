@@ -145,7 +145,7 @@ __global__ __launch_bounds__(256) void k_integrate(int n, double dt, double* __r
 // more bodies each halve the reads but lengthen the merge (2048 bodies: 8 x 1 5.9 us,
 // 4 x 2 7.3, 2 x 4 10.6; 4096: 16 x 1 10.6, 8 x 2 11.7). Steps in us, k_direct and
 // k_integrate against this: 256 bodies 6.9 / 4.2, 1000 9.7 / 4.7, 2048 11.0 / 5.8,
-// 4096 14.5 / 10.4, 6000 22.3 / 21.2, 8192 29.7 / 26.9, where the LDS ends it.
+// 4096 14.5 / 10.4, 6000 22.3 / 19.7, 8192 29.7 / 24.9, where the LDS ends it.
 // A slice is at most 128 terms in FP32; slices are added in FP64.
 // kMode 0: forces only, to `force`; 1: KDK step; 2: Euler step (as k_integrate).
 constexpr int kSmallThreads = 1024;
@@ -209,21 +209,37 @@ __global__ __launch_bounds__(kSmallThreads) void k_direct_small(
     z[r] = q.z;
     fx[r] = fy[r] = fz[r] = 0.f;
   }
-#pragma unroll 4
-  for (int k = tid / kLanes; k < n_pad; k += kSlices) {
-    const float4 q = src[k];
+  const auto pairs = [&](auto count, int k) {  // with sources k, k + kSlices, ...
+    constexpr int kCount = decltype(count)::value;
+    float dx[kCount * kPer], dy[kCount * kPer], dz[kCount * kPer], r2[kCount * kPer],
+        inv[kCount * kPer], w[kCount];
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const float dx = q.x - x[r], dy = q.y - y[r], dz = q.z - z[r];
-      const float r2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, eps2)));
-      const float inv = __builtin_amdgcn_rsqf(r2);
-      float s = (q.w * inv) * (inv * inv);
-      if (kGuard) s = r2 > 0.f ? s : 0.f;
-      fx[r] = fmaf(dx, s, fx[r]);
-      fy[r] = fmaf(dy, s, fy[r]);
-      fz[r] = fmaf(dz, s, fz[r]);
+    for (int u = 0; u < kCount; ++u) {
+      const float4 q = src[k + u * kSlices];
+      w[u] = q.w;
+#pragma unroll
+      for (int r = 0; r < kPer; ++r) {
+        const int e = u * kPer + r;
+        dx[e] = q.x - x[r], dy[e] = q.y - y[r], dz[e] = q.z - z[r];
+        r2[e] = fmaf(dz[e], dz[e], fmaf(dy[e], dy[e], fmaf(dx[e], dx[e], eps2)));
+      }
     }
-  }
+    nbcore::rsq_group(r2, inv);
+#pragma unroll
+    for (int u = 0; u < kCount; ++u)
+#pragma unroll
+      for (int r = 0; r < kPer; ++r) {
+        const int e = u * kPer + r;
+        float s = (w[u] * inv[e]) * (inv[e] * inv[e]);
+        if (kGuard) s = r2[e] > 0.f ? s : 0.f;
+        fx[r] = fmaf(dx[e], s, fx[r]);
+        fy[r] = fmaf(dy[e], s, fy[r]);
+        fz[r] = fmaf(dz[e], s, fz[r]);
+      }
+  };
+  int k = tid / kLanes;
+  for (; k + 3 * kSlices < n_pad; k += 4 * kSlices) pairs(std::integral_constant<int, 4>{}, k);
+  for (; k < n_pad; k += kSlices) pairs(std::integral_constant<int, 1>{}, k);
 #pragma unroll
   for (int r = 0; r < kPer; ++r) {
     double f[3] = {fx[r], fy[r], fz[r]};

@@ -4,7 +4,8 @@
 // A lane owns B target bodies held in VGPRs; the sources [j0, j1) are read at
 // wave-uniform addresses, so they come through the scalar cache into SGPRs and
 // feed the VALU as scalar operands. One interaction is
-//   3 v_sub + 3 v_fma (r^2) + v_rsq + 3 v_mul (2 for equal masses) + 3 v_fma.
+//   3 v_sub + 3 v_fma (r^2) + v_rsq + 3 v_mul (2 for equal masses) + 3 v_fma,
+// the reciprocal square roots four by four (rsq_group).
 // Sums are plain FP32 within a chunk of kChunk sources and folded into a
 // (sum, error) pair with Knuth's TwoSum once per chunk.
 #pragma once
@@ -24,6 +25,28 @@ __device__ __forceinline__ void two_sum_fold(float& s, float& c, float x) {
   const float e = (s - (t - bp)) + (x - bp);
   s = t;
   c += e;
+}
+
+// inv = 1 / sqrt(r2), N of them one after the other, at raised wave priority.
+// A SIMD takes full-rate vector instructions of two waves at a time, one per 2.0 to 2.4
+// cycles (4.1 from one wave alone), and a reciprocal square root in 8.1. Mixed, with
+// all waves alike, they do not add up: an interaction of eleven and one took 40 to 52
+// cycles at eight waves per SIMD, by the order of its instructions, as waves waiting for
+// the slow unit hold up the pairing of the others. With the four of a group raised it
+// takes 33 in any order, which is the sum of the parts; groups of two, six or eight,
+// or a raise some instructions earlier or later, are within 3%. Direct sum of 2^18
+// bodies 15.8 -> 14.6 ms, 65,536 1.044 -> 0.962; ensembles of 256 clusters 659 -> 609 us,
+// of 512 12.3 -> 11.3 ms; Barnes-Hut traversal of 300,007 bodies 488 -> 450 us, 2^22
+// 4.31 -> 4.13 ms. The barriers keep the scheduler from moving the group apart.
+template <int N>
+__device__ __forceinline__ void rsq_group(const float (&r2)[N], float (&inv)[N]) {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_setprio(3);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int k = 0; k < N; ++k) inv[k] = __builtin_amdgcn_rsqf(r2[k]);
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_setprio(0);
 }
 
 template <int B>
@@ -49,44 +72,49 @@ __device__ __forceinline__ void accumulate(const float4* __restrict__ pm, int j0
     float px[B], py[B], pz[B];
 #pragma unroll
     for (int b = 0; b < B; ++b) px[b] = py[b] = pz[b] = 0.f;
-    auto step = [&](const float4* qq) {
+    // One register set of four sources: once their differences are taken, the scalar
+    // loads of the next four are issued, so the load latency overlaps the rest of the
+    // arithmetic. Two sets gained 10% over loads right before their use at N = 2^18;
+    // with the sums in the order below one does as well. The memory clobbers keep the
+    // compiler from sinking the loads next to their first use.
+    // je - jc is a multiple of 4 (ranges are multiples of 16 sources).
+    float4 q[4];
+    auto load = [&](int j) {
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int u = 0; u < 4; ++u) q[u] = pm[j + u];  // wave-uniform: scalar loads
+      asm volatile("" ::: "memory");
+    };
+    load(jc);
+    for (int j = jc; j < je; j += 4) {
+      float dx[4 * B], dy[4 * B], dz[4 * B], r2[4 * B], inv[4 * B], w[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const float4 q = qq[u];
+        w[u] = q[u].w;
 #pragma unroll
         for (int b = 0; b < B; ++b) {
-          const float dx = q.x - t.x[b];
-          const float dy = q.y - t.y[b];
-          const float dz = q.z - t.z[b];
-          const float r2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, eps2)));
-          const float inv = __builtin_amdgcn_rsqf(r2);
-          float s = (kUniform ? inv : q.w * inv) * (inv * inv);
-          if (kGuard) s = r2 > 0.f ? s : 0.f;
-          px[b] = fmaf(dx, s, px[b]);
-          py[b] = fmaf(dy, s, py[b]);
-          pz[b] = fmaf(dz, s, pz[b]);
+          const int k = u * B + b;
+          dx[k] = q[u].x - t.x[b];
+          dy[k] = q[u].y - t.y[b];
+          dz[k] = q[u].z - t.z[b];
+          r2[k] = fmaf(dz[k], dz[k], fmaf(dy[k], dy[k], fmaf(dx[k], dx[k], eps2)));
         }
       }
-    };
-    // Two register sets of four sources: the scalar loads of one set are
-    // issued before the other set's arithmetic, so the load latency overlaps
-    // the math instead of stalling every four sources (measured 10% faster at
-    // N = 2^18 than loading each set right before its use). The memory clobber
-    // keeps the compiler from sinking the loads next to their first use.
-    // je - jc is a multiple of 8 (ranges are multiples of 16 sources).
-    float4 qa[4], qb[4];
+      __builtin_amdgcn_sched_barrier(0);
+      load(j + 4 < je ? j + 4 : j);  // the last step reloads its own (in range)
+      rsq_group(r2, inv);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) qa[u] = pm[jc + u];
-    for (int j = jc; j < je; j += 8) {
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) qb[u] = pm[j + 4 + u];  // wave-uniform: scalar loads
-      asm volatile("" ::: "memory");
-      step(qa);
-      const int jn = j + 8 < je ? j + 8 : j;  // the last step reloads its own (in range)
-#pragma unroll
-      for (int u = 0; u < 4; ++u) qa[u] = pm[jn + u];
-      asm volatile("" ::: "memory");
-      step(qb);
+        for (int b = 0; b < B; ++b) {
+          const int k = u * B + b;
+          float s = (kUniform ? inv[k] : w[u] * inv[k]) * (inv[k] * inv[k]);
+          if (kGuard) s = r2[k] > 0.f ? s : 0.f;
+          px[b] = fmaf(dx[k], s, px[b]);
+          py[b] = fmaf(dy[k], s, py[b]);
+          pz[b] = fmaf(dz[k], s, pz[b]);
+        }
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int b = 0; b < B; ++b) {
