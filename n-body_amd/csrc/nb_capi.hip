@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstring>
 #include <new>
+#include <numeric>
 #include <vector>
 
 #include "nb_internal.h"
@@ -113,34 +114,38 @@ void nb_default_shape(int64_t n, int* bpl, int* jsplit, int* leaf) {
   if (leaf && *leaf == 0) *leaf = 8;
 }
 
-// Workgroups per i-block of the direct sum. A compute unit works through
-// ceil(blocks * parts / 256) workgroups of n_pad / parts sources each, so one part
-// leaves most of the chip idle below 16,384 bodies (64 of 256 compute units at
-// 4096) and a nearly empty last round at many sizes above. The cost of a
-// workgroup beyond its pairs is that of about 256 sources (the wait for the first
-// ones, the merge). Among the part counts within 0.5% of the cheapest the largest
-// is taken: more, shorter workgroups end closer together. Slices are kept at 32
-// sources (at 2000 bodies four parts took 12.5 us, eight 14.6), and the partial
-// sums at 12 MB: from 2^19 bodies on the rounding costs less than 1.5%.
-// Steps in us, one part against this rule's number:
-//   1000 13.8 / 11.3, 4096 29.9 / 16.6, 8192 53.9 / 32.0, 12,345 74.5 / 58.3,
-//   16,384 100.9 / 85.9, 20,000 208 / 130, 37,000 525 / 379, 100,000 3060 / 2610, 2^18 17,635 / 17,428.
-int nb_direct_parts(int n_pad, int bpl, int jsplit) {
-  constexpr int kUnits = 256, kWorkgroupSources = 256, kMinSlice = 32, kMaxParts = 8;
-  constexpr int64_t kMaxPartBodies = 1 << 19;
-  const int64_t blocks = n_pad / (64 * bpl);
-  double cost[kMaxParts + 1], least = 0;
-  int most = 1;
-  for (int p = 1; p <= kMaxParts; ++p) {
-    if (p > 1 && (n_pad < p * jsplit * kMinSlice || (int64_t)p * n_pad > kMaxPartBodies)) break;
-    const int64_t rounds = (blocks * p + kUnits - 1) / kUnits;
-    const double slow = rounds * jsplit < 24 ? 1.2 : 1.0;
-    cost[p] = (double)rounds * (slow * n_pad / p + kWorkgroupSources);
-    least = p == 1 ? cost[p] : std::min(least, cost[p]);
-    most = p;
-  }
-  while (cost[most] > 1.005 * least) --most;
-  return most;
+// The direct sum's work (units of an i-block and 16 sources, see k_direct) in equal
+// shares, `rounds` of them for each workgroup that the chip holds at a time. Whole
+// i-blocks leave most of it idle below 16,384 bodies (64 of 256 compute units at 4096)
+// and a nearly empty last round at many sizes above; shares fit any size. Their ends
+// spread by about a tenth of their length, as a SIMD does not serve its waves evenly,
+// and each costs what a few hundred sources do (the first loads, the merge), so their
+// number grows with the square root of the work. It is a multiple of the compute units,
+// unless that would make a wave's slice shorter than 32 sources or an i-block's shares
+// more than eight. From 2^19 bodies on whole i-blocks lose less than 1.5%.
+// Steps in us, whole i-blocks or i-blocks in equal parts (the better one) against
+// this, both with equal masses:
+//   8193 34.0 / 31.0, 10,000 40.5 / 37.0, 12,345 52.0 / 49.6, 16,384 80.0 / 72.1,
+//   20,000 118 / 105, 32,768 263 / 249, 37,000 330 / 321, 65,536 965 / 940,
+//   80,000 1448 / 1400, 200,000 8840 / 8590, 300,000 20,400 / 20,050.
+// Shares per resident workgroup 1, 2, 4, 8: 12,345 49.6, 52.3, 58.0, 66.7; 20,000 109,
+// 105, 108, 120; 37,000 341, 325, 321, 327; 65,536 1004, 970, 946, 936.
+nb_shares nb_direct_shares(int n_pad, int bpl, int jsplit, int cus) {
+  constexpr int kWavesPerUnit = 32, kMaxRounds = 8, kMinSlice = 2;
+  constexpr double kRoundSources = 1300;
+  constexpr int kMaxShareBodies = 1 << 19;
+  const int64_t units = n_pad / 16, blocks = n_pad / (64 * bpl), work = blocks * units;
+  const int resident = std::max(1, kWavesPerUnit / jsplit);  // workgroups per compute unit
+  const int rounds = std::clamp((int)std::sqrt(16.0 * work / cus / resident / kRoundSources), 1, kMaxRounds);
+  const int64_t least = std::max<int64_t>(units / 8, kMinSlice * jsplit);
+  const int64_t per_cu = std::clamp<int64_t>(work / cus / least, 1, resident * rounds);
+  const int64_t share = std::max((work + cus * per_cu - 1) / (cus * per_cu), least);
+  if (n_pad > kMaxShareBodies) return {(int)units, 1};
+  const int64_t most = (share - std::gcd(share, units) + units - 1) / share + 1;  // reached by enough blocks
+  int64_t parts = 1;
+  for (int64_t b = 0; b < blocks && parts < most; ++b)
+    parts = std::max(parts, ((b + 1) * units - 1) / share - b * units / share + 1);
+  return parts > 1 ? nb_shares{(int)share, (int)parts} : nb_shares{(int)units, 1};
 }
 
 nb_equal_mass nb_find_equal_mass(const float* mass, int64_t n, float eps2, double G) {
@@ -358,10 +363,16 @@ int nb_create(nb_ctx** out, const nb_config* cfg) {
   if (c->cfg.solver == NB_SOLVER_DIRECT) {
     // an explicit launch shape is a choice of k_direct's
     c->small = c->n_pad <= kSmallBodies && cfg->bodies_per_lane == 0 && cfg->j_split == 0;
-    c->parts = c->small ? 1 : nb_direct_parts(c->n_pad, c->bpl, c->jsplit);
   }
 
   (void)hipGetDevice(&c->device);
+  if (c->cfg.solver == NB_SOLVER_DIRECT && !c->small) {
+    int cus = 256;
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
+    const nb_shares d = nb_direct_shares(c->n_pad, c->bpl, c->jsplit, cus);
+    c->share = d.units;
+    c->parts = d.parts;
+  }
   int rc = NB_OK;
   auto fail = [&](int code, const std::string& m) {
     free_ctx(c);

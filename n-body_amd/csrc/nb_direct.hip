@@ -26,43 +26,74 @@
 
 namespace {
 
-// Grid: (i-blocks, parts). The sources are cut into parts * K slices of whole
-// 16-source units; block (ib, p) takes the slices p * K .. p * K + K - 1. With one
-// part the block writes the forces; with more it writes its FP64 partial sums,
-// without G, to out[p][3][n], and whoever reads them adds the parts in order.
-template <int B, int K, bool kGuard, bool kUniform>
+// The work is the pairs of i-blocks and units of 16 sources, block by block; a
+// workgroup takes `share` of them, whatever blocks they belong to, and its waves cut
+// each block's stretch into K slices. share = a whole block's units: the workgroup
+// writes the block's forces. Otherwise it writes FP64 partial sums, without G, to
+// out[p][3][n], p counting the workgroups of that block, and whoever reads them adds
+// the parts in order; the block's last workgroup sets the unused ones to zero.
+template <int B, int K, bool kGuard, bool kUniform, bool kShares>
 __global__ __launch_bounds__(64 * K) void k_direct(const float4* __restrict__ pm, int n,
-                                                   int n_pad, float eps2, double G,
-                                                   double* __restrict__ out) {
+                                                   int n_pad, float eps2, double G, int share,
+                                                   int parts, double* __restrict__ out) {
+  __shared__ double part[K > 1 ? K : 1][3][B][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ibase = blockIdx.x * (64 * B) + lane;
-  nbcore::Targets<B> t;
-  nbcore::load_targets<B>(pm, ibase, t);
-  const int64_t units = n_pad / 16, slices = (int64_t)gridDim.y * K;
-  const int64_t slice = (int64_t)blockIdx.y * K + wave;
-  nbcore::accumulate<B, kGuard, kUniform>(pm, 16 * (int)(units * slice / slices),
-                                16 * (int)(units * (slice + 1) / slices), eps2, t);
-  __shared__ double part[K > 1 ? K : 1][3][B][64];
-  const double g = gridDim.y == 1 ? G : 1.0;
-  double* f = out + (int64_t)blockIdx.y * 3 * n;
-  nbcore::merge_waves<B, K>(part, wave, lane, t, [&](int a, int b, double sum) {
-    const int i = ibase + 64 * b;
-    if (i < n) f[(int64_t)a * n + i] = g * sum;
-  });
+  const uint32_t units = n_pad / 16, blocks = n_pad / (64 * B);
+  // the pairs of this workgroup's waves in block, len units from the given one on
+  const auto sum = [&](uint32_t block, uint32_t from, uint32_t len, auto put) {
+    const int ibase = block * (64 * B) + lane;
+    nbcore::Targets<B> t;
+    nbcore::load_targets<B>(pm, ibase, t);
+    const uint32_t begin = 16 * (from + len * wave / K), end = 16 * (from + len * (wave + 1) / K);
+    nbcore::accumulate<B, kGuard, kUniform>(pm, (int)begin, (int)end, eps2, t,
+                                            kShares ? nbcore::even_chunk(end - begin) : nbcore::kChunk);
+    nbcore::merge_waves<B, K>(part, wave, lane, t, [&](int a, int b, double f) {
+      const int i = ibase + 64 * b;
+      if (i < n) put((int64_t)a * n + i, f);
+    });
+  };
+  if (!kShares) {
+    sum(blockIdx.x, 0, units, [&](int64_t at, double f) { out[at] = G * f; });
+    return;
+  }
+  const uint32_t x = blockIdx.x * (uint32_t)share;  // blocks * units fits 32 bits
+  uint32_t block = x / units, from = x - block * units, left = share;
+  for (;;) {
+    const uint32_t len = min(left, units - from);
+    const uint32_t p = blockIdx.x - block * units / (uint32_t)share;
+    const bool last = from + len == units;
+    sum(block, from, len, [&](int64_t at, double f) {
+      out[3 * (int64_t)n * p + at] = f;
+      if (last)
+        for (int r = p + 1; r < parts; ++r) out[3 * (int64_t)n * r + at] = 0.0;
+    });
+    left -= len;
+    if (left == 0 || ++block == blocks) return;
+    from = 0;
+    __syncthreads();  // the sums are read before the next block's replace them
+  }
 }
 
 template <int B, int K>
 hipError_t launch_bk(const nb_ctx* c) {
-  const dim3 grid(c->n_pad / (64 * B), c->parts);
+  const int64_t work = (int64_t)(c->n_pad / (64 * B)) * (c->n_pad / 16);
+  const dim3 grid((unsigned)((work + c->share - 1) / c->share));
   double* out = c->parts > 1 ? c->part : c->force;
   const auto launch = [&](auto kernel, float eps2) {
     hipLaunchKernelGGL(kernel, grid, dim3(64 * K), 0, c->stream, c->pm, c->n, c->n_pad, eps2,
-                       c->equal.factor, out);
+                       c->equal.factor, c->share, c->parts, out);
   };
-  if (c->equal.on) launch(k_direct<B, K, false, true>, c->equal.eps2);
-  else if (c->guard) launch(k_direct<B, K, true, false>, c->cfg.eps2);
-  else launch(k_direct<B, K, false, false>, c->cfg.eps2);
+  const bool shares = c->parts > 1;
+  if (c->equal.on)
+    shares ? launch(k_direct<B, K, false, true, true>, c->equal.eps2)
+           : launch(k_direct<B, K, false, true, false>, c->equal.eps2);
+  else if (c->guard)
+    shares ? launch(k_direct<B, K, true, false, true>, c->cfg.eps2)
+           : launch(k_direct<B, K, true, false, false>, c->cfg.eps2);
+  else
+    shares ? launch(k_direct<B, K, false, false, true>, c->cfg.eps2)
+           : launch(k_direct<B, K, false, false, false>, c->cfg.eps2);
   return hipGetLastError();
 }
 

@@ -224,6 +224,12 @@ struct nb_equal_mass {
 };
 nb_equal_mass nb_find_equal_mass(const float* mass, int64_t n, float eps2, double G);
 
+// Division of the direct sum: units of (i-block, 16 sources) per workgroup, and the
+// most workgroups that any i-block is divided among.
+struct nb_shares {
+  int units, parts;
+};
+
 struct nb_ctx {
   nb_config cfg{};
   int64_t cap_n = 0;  // bodies the device buffers were sized for (nb_ctx_rebind limit)
@@ -248,7 +254,8 @@ struct nb_ctx {
   int jsplit = 2;  // waves per workgroup of an i-block
   bool small = false;  // direct sum of a small system: one launch per step (k_direct_small)
   float4* pm_next = nullptr;  // its second view: a step reads pm, writes pm_next and swaps them
-  int parts = 1;   // workgroups per i-block, each with a part of the sources
+  int share = 0;   // units of work per workgroup of the direct sum (nb_shares)
+  int parts = 1;   // most workgroups that share an i-block
   double* part = nullptr;  // their partial sums [parts][3][n], behind force
   bool guard = false;
   nb_equal_mass equal;  // k_direct's form for equal masses
@@ -355,7 +362,7 @@ hipError_t nb_bh_count_per_body(nb_ctx* c);
 // from the built-in defaults.
 bool nb_tuned_shape(int64_t n, int* bpl, int* jsplit, int* leaf);
 void nb_default_shape(int64_t n, int* bpl, int* jsplit, int* leaf);
-int nb_direct_parts(int n_pad, int bpl, int jsplit);  // workgroups per i-block
+nb_shares nb_direct_shares(int n_pad, int bpl, int jsplit, int cus);
 bool nb_valid_shape(int bpl, int jsplit);  // a direct-sum kernel exists for it
 
 // step = forces + integration (no sync)
