@@ -232,18 +232,20 @@ static int accumulate_timing(nb_ctx* c) {
   return NB_OK;
 }
 
-// Direct-sum systems up to this size capture kChunkSteps steps per graph: at
-// N = 4096 a step replayed from a one-step graph took 0.0333 ms and from an
-// eight-step graph 0.0285 ms (N = 16384: 4% less; Barnes-Hut steps, bound by
-// their dependent build kernels, gained under 1%).
-constexpr int64_t kChunkMaxBodies = 32768;
+// Steps per captured graph. Shorter calls, and what is left of others, are launched one
+// by one: a graph of one step costs 4 to 5 us more than its dozen Barnes-Hut launches
+// (one step and its wait, 20,011 bodies 148 us, launched 143). Eight steps per graph cost
+// as little as launches, on less of the host's time (20,011 bodies 115 us per step, 4096
+// 83 against 88), but their capture takes about 200 us at a context's first such call, so
+// Barnes-Hut calls of up to 31 steps are launched, too. Direct sum, N = 4096: 33.3 us from
+// one-step graphs, 28.5 from eight-step graphs, when a step was two launches.
 constexpr int kChunkSteps = 8;  // even: a small system's views are in place again after it
+constexpr int kGraphStepsBh = 4 * kChunkSteps;
 
 int nb_prepare_step_graph(nb_ctx* c) {
   if (c->graph_exec || (c->cfg.flags & NB_F_NO_GRAPH)) return NB_OK;
   NB_API_CAPTURE;
-  const int steps =
-      c->cfg.solver == NB_SOLVER_DIRECT && c->n <= kChunkMaxBodies ? kChunkSteps : 1;
+  const int steps = kChunkSteps;
   NB_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   hipError_t e = hipSuccess;
   c->graph_pm = c->pm;
@@ -508,10 +510,11 @@ int nb_step(nb_ctx* c, int32_t nsteps) {
     c->tree_valid = c->cfg.solver == NB_SOLVER_BH;
     return NB_OK;
   }
-  // The step is captured once per context and replayed (cheap launches for the
-  // ~47-kernel Barnes-Hut step); graph and eager launches give identical results.
+  // Steps are captured once per context and replayed; graph and eager launches give
+  // identical results.
   const bool use_graph = !(c->cfg.flags & NB_F_NO_GRAPH);
-  if (!use_graph) {
+  const int worth = c->cfg.solver == NB_SOLVER_BH ? kGraphStepsBh : kChunkSteps;
+  if (!use_graph || nsteps < worth) {
     for (int s = 0; s < nsteps; ++s) NB_HIP(nb_enqueue_step(c));
   } else {
     const int rc = nb_prepare_step_graph(c);

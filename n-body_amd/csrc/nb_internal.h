@@ -271,8 +271,7 @@ struct nb_ctx {
   bool uploaded = false;
   bool tree_valid = false;
 
-  // captured step graph: graph_steps consecutive steps (more than one for small
-  // direct-sum systems, whose steps are short enough for the graph launch to show)
+  // captured step graph: graph_steps consecutive steps
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
   int graph_steps = 1;

@@ -225,3 +225,20 @@ def test_batch_clusters_in_parts(nb, ora, sizes):
         ref = ora.direct_f64(pos.astype(np.float32).astype(np.float64), m.astype(np.float64), EPS2, targets=tgt)
         # 256-source FP32 sums, folded: 256 roundings of the largest force at worst
         assert np.abs(mine[tgt] - ref).max() <= 256 * 2.0 ** -24 * (np.linalg.norm(ref, axis=1).max() + 1e-30)
+
+
+@pytest.mark.parametrize("solver, n, calls", [("direct", 300, (7, 8, 9, 17)), ("direct", 9000, (8, 3)),
+                                              ("bh", 700, (31, 32)), ("bh", 5001, (1, 35, 2))])
+def test_calls_of_any_length_take_the_same_steps(nb, solver, n, calls):
+    """Launched steps, whole graphs and what is left of them, against launched steps only."""
+    pos, vel, m = nb.ic_plummer(n, n, 50.0, 1e4)
+    out = []
+    for flags in (0, nb.F_NO_GRAPH):
+        with nb.Simulation(n, EPS2, DT, solver=nb.SOLVER_BH if solver == "bh" else nb.SOLVER_DIRECT,
+                           flags=flags) as sim:
+            sim.upload(pos, vel, m)
+            for k in calls:
+                sim.step(k)
+            out.append(sim.download_f64())
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
