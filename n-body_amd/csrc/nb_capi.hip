@@ -99,10 +99,10 @@ void to_caller_order(const nb_ctx* c, std::vector<T>& a, int comps) {
 
 }  // namespace
 
-// Built-in launch shapes, from a sweep on MI355X (Plummer spheres, whole steps
-// with the best number of parts each): one body per lane; 16 waves per workgroup
-// up to 16384 bodies (4096 bodies: 16.6 us against 19.8 us at 8 waves), 8 above
-// (37,000 bodies: 379 us against 382 us at 16; 2^18: 17.38 ms against 17.37).
+// Built-in launch shapes, from a sweep on MI355X (Plummer spheres, whole steps): one body
+// per lane; 16 waves per workgroup up to 16384 bodies (12,345 bodies: 47.7 us against
+// 50.4 us at 8 waves), 8 above (37,000 bodies: 322.6 us against 320.6 us at 16; 100,000:
+// 2184 against 2186).
 void nb_default_shape(int64_t n, int* bpl, int* jsplit, int* leaf) {
   if (bpl && *bpl == 0) *bpl = 1;
   if (jsplit && *jsplit == 0) {
