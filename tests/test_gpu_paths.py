@@ -242,3 +242,21 @@ def test_calls_of_any_length_take_the_same_steps(nb, solver, n, calls):
             out.append(sim.download_f64())
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("clusters", [1023, 1025, 1040, 3100])
+def test_batch_items_beyond_the_first(nb, clusters):
+    """More work items than workgroups: every cluster is stepped once per step, and all
+    alike ones come out as a cluster does alone."""
+    pos, vel, m = nb.ic_plummer(clusters, 64, 50.0, 1e4)
+    with nb.Batch(256, 1) as one, nb.Batch(256 * clusters, clusters) as many:
+        alone = one.add(pos, vel, m, EPS2, DT)
+        ids = [many.add(pos, vel, m, EPS2, DT) for _ in range(clusters)]
+        for b in (one, many):
+            b.step(3)
+        ref = one.download(alone)
+        for k in range(0, clusters, 31):
+            for a, b in zip(ref, many.download(ids[k])):
+                np.testing.assert_array_equal(a, b)
+        for a, b in zip(ref, many.download(ids[-1])):
+            np.testing.assert_array_equal(a, b)
