@@ -260,3 +260,21 @@ def test_batch_items_beyond_the_first(nb, clusters):
                 np.testing.assert_array_equal(a, b)
         for a, b in zip(ref, many.download(ids[-1])):
             np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("n, bpl, js, eps2", [(8193, 0, 0, 0.0), (12289, 2, 4, 0.0), (16385, 4, 1, EPS2),
+                                              (20001, 1, 16, EPS2), (24833, 4, 4, 0.0), (33001, 2, 8, EPS2)])
+def test_direct_sum_shares_of_unequal_masses(nb, ora, n, bpl, js, eps2):
+    """Shares that end inside a block of targets, with masses of their own and without
+    softening: forces against FP64 at the first, last and random targets."""
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(-100, 100, (n, 3))
+    m = rng.uniform(0.5, 2, n).astype(np.float32)
+    tgt = np.unique(np.concatenate([[0, 63, 64, n - 1], rng.choice(n, 300, replace=False)]))
+    ref = ora.direct_f64(pos.astype(np.float32).astype(np.float64), m.astype(np.float64), eps2, targets=tgt)
+    with nb.Simulation(n, eps2, DT, bodies_per_lane=bpl, j_split=js) as sim:
+        sim.upload(pos, np.zeros_like(pos), m)
+        f = sim.forces_f64()
+    scale = np.linalg.norm(ref, axis=1).max()
+    # 256-source FP32 sums, folded with compensation: 256 roundings of the largest force at worst
+    assert np.abs(f[tgt] - ref).max() <= 256 * 2.0 ** -24 * scale
