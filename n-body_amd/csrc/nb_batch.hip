@@ -31,10 +31,10 @@
 
 // One work item of the force pass.
 struct alignas(32) nb_batch_item {
-  int slot_equal;  // 2 * slot, + 1 for equal masses
+  int head;             // slot << 6 | parts - 1 << 4 | its part << 2 | all parts << 1 | equal masses
   int ibase, off, end;  // bodies [off, end); targets from ibase on
-  int units_part;       // 16-source units << 4 | parts - 1 << 2 | part of the sources (see batch_parts)
-  float eps2;                 // of the scaled view (nb_equal_mass)
+  int shift;            // from a body's index to where its sums go
+  float eps2;           // of the scaled view (nb_equal_mass)
   double G;
 };
 
@@ -47,9 +47,8 @@ struct nb_batch {
   // device pool
   float4* pm = nullptr;
   double *pos = nullptr, *vel = nullptr, *acc = nullptr;
-  double* force = nullptr;  // [3][cap]; [kMaxParts][3][cap] once a cluster has parts
-  bool wide = false;
-  int max_parts = 4;        // 1 if there was no memory for the partial sums
+  double* force = nullptr;  // [3][force_cap]; past the bodies and in free segments: partial sums
+  int64_t force_cap = 0;
   float* mass = nullptr;
   // device slot table
   int* c_off = nullptr;
@@ -59,7 +58,8 @@ struct nb_batch {
   int* c_quota = nullptr;  // steps the cluster takes per nb_batch_step call (INT32_MAX: all)
   // device work tables
   nb_batch_item* items = nullptr;
-  int2* blocks = nullptr;  // (slot, first body) per 256-body block
+  int4* blocks = nullptr;  // per 256-body block: slot, first body, n_pad << 2 | stored parts - 1,
+                           // from a body's index to its sum of part 1
   // [0] items, [1] blocks, [4] step of the call, [5] the same for the integrator, then
   // the tickets
   int* counts = nullptr;
@@ -69,6 +69,7 @@ struct nb_batch {
   std::vector<float> h_eps2;
   std::vector<double> h_G;
   std::vector<nb_equal_mass> h_equal;
+  std::vector<int> h_stored, h_shift;  // a cluster's parts stored apart, as in blocks
   nb_stage stage;
   std::vector<char> used;
   std::map<int64_t, int64_t> free_list;  // offset -> size
@@ -95,9 +96,15 @@ constexpr int kUnlimited = NB_BATCH_UNLIMITED;
 // on the others. Steps in us without / with parts: 16 clusters of 1000 to 16,000
 // bodies 111 / 101, four of 8000 109 / 101, 24 of 256 to 16,384 203 / 197, 256 of 256
 // to 8192 671 / 655, 512 of 256 to 32,768 12,152 / 12,330; 24 served jobs 9.16 / 7.34 ms.
+// The sums of the parts past the first lie where the force array has no bodies: in the
+// pool's free segments and, in a batch of its own, in kSpareBodies entries behind the
+// pool. Parts help while the clusters do not fill the chip, so that is room enough; a
+// cluster that finds none has an item sum its parts one after the other, with the same
+// bits. The parts thus cost a server's pool no memory.
 constexpr int kMaxParts = 4;
-int batch_parts(const nb_batch* b, int npad) {
-  return std::max(1, std::min({b->max_parts, (npad + 4095) / 4096, 1024 / (npad / 64)}));
+constexpr int64_t kSpareBodies = 3 << 17;
+int batch_parts(int npad) {
+  return std::max(1, std::min({kMaxParts, (npad + 4095) / 4096, 1024 / (npad / 64)}));
 }
 
 // Ticket k of the force pass. Its workgroups are dealt to kTickets classes, which take every
@@ -124,7 +131,7 @@ __device__ __forceinline__ int* ticket(int* counts, int k) { return counts + 64 
 template <int B, int K>
 __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_num_sgpr(80))) void k_batch_force(
     const float4* __restrict__ pm, const int* __restrict__ c_quota, int use_quota,
-    const nb_batch_item* __restrict__ items, int* __restrict__ counts, int64_t cap,
+    const nb_batch_item* __restrict__ items, int* __restrict__ counts, int64_t force_cap,
     double* __restrict__ force) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -144,26 +151,34 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_num_sgpr(80))) void k
       next = nitems > (int)gridDim.x
                  ? (int)gridDim.x + mine + tickets * atomicAdd(ticket(counts, mine), 1)
                  : nitems;
-    const nb_batch_item it = items[item];  // wave-uniform
-    if (__builtin_amdgcn_readfirstlane(c_quota[it.slot_equal >> 1]) <= call_step) continue;  // block-uniform
+    const nb_batch_item& it = items[item];  // wave-uniform
+    if (__builtin_amdgcn_readfirstlane(c_quota[it.head >> 6]) <= call_step) continue;  // block-uniform
     const int ibase = it.ibase + lane;
-    nbcore::Targets<B> t;
-    nbcore::load_targets<B>(pm, ibase, t);
-    const int units = it.units_part >> 4, part_no = it.units_part & 3;
-    const int slices = K * (((it.units_part >> 2) & 3) + 1), slice = K * part_no + wave;
-    const int j0 = it.off + 16 * (int)((int64_t)units * slice / slices);
-    const int j1 = it.off + 16 * (int)((int64_t)units * (slice + 1) / slices);
-    if (it.slot_equal & 1)
-      nbcore::accumulate<B, false, true>(pm, j0, j1, it.eps2, t);
-    else if (it.eps2 >= 1e-20f)
-      nbcore::accumulate<B, false, false>(pm, j0, j1, it.eps2, t);
-    else
-      nbcore::accumulate<B, true, false>(pm, j0, j1, it.eps2, t);
-    double* out = force + part_no * 3 * cap;
-    nbcore::merge_waves<B, K>(part, wave, lane, t, [&](int a, int b, double sum) {
-      const int i = ibase + 64 * b;
-      if (i < it.end) out[a * cap + i] = it.G * sum;
-    });
+    const int parts = (it.head >> 4 & 3) + 1, first = it.head >> 2 & 3;
+    const int last = it.head & 2 ? parts - 1 : first;
+    const int units = (it.end - it.off + 255) / 256 * 16;  // of 16 sources
+    for (int q = first; q <= last; ++q) {
+      nbcore::Targets<B> t;
+      nbcore::load_targets<B>(pm, ibase, t);
+      const int slices = K * parts, slice = K * q + wave;
+      const int j0 = it.off + 16 * (int)((int64_t)units * slice / slices);
+      const int j1 = it.off + 16 * (int)((int64_t)units * (slice + 1) / slices);
+      if (it.head & 1)
+        nbcore::accumulate<B, false, true>(pm, j0, j1, it.eps2, t);
+      else if (it.eps2 >= 1e-20f)
+        nbcore::accumulate<B, false, false>(pm, j0, j1, it.eps2, t);
+      else
+        nbcore::accumulate<B, true, false>(pm, j0, j1, it.eps2, t);
+      if (q > first) __syncthreads();  // the last part's sums are read before these replace them
+      nbcore::merge_waves<B, K>(part, wave, lane, t, [&](int a, int b, double sum) {
+#pragma clang fp contract(off)  // parts are added rounded, as the integrator adds stored ones
+        const int i = ibase + 64 * b;
+        if (i >= it.end) return;
+        double* at = force + a * force_cap + i + it.shift;
+        const double f = it.G * sum;
+        *at = q > first ? *at + f : f;
+      });
+    }
   }
 }
 
@@ -173,10 +188,10 @@ __global__ void k_batch_reset(int* __restrict__ counts) {
 
 template <bool kEuler>
 __global__ __launch_bounds__(256) void k_batch_integrate(
-    const int2* __restrict__ blocks, int* __restrict__ counts, const int* __restrict__ c_off,
+    const int4* __restrict__ blocks, int* __restrict__ counts, const int* __restrict__ c_off,
     const int* __restrict__ c_n, const double* __restrict__ c_dt, const float* __restrict__ c_scale,
     const int* __restrict__ c_quota, int64_t cap, double* __restrict__ pos, double* __restrict__ vel, double* __restrict__ acc,
-    const double* __restrict__ force, const float* __restrict__ mass, float4* __restrict__ pm) {
+    const double* __restrict__ force, int64_t force_cap, const float* __restrict__ mass, float4* __restrict__ pm) {
   // grid-stride over the pool blocks in use: the launch is sized for the
   // device, not for the pool's capacity, so an almost empty pool costs little
   const int nblocks = counts[1];
@@ -186,9 +201,8 @@ __global__ __launch_bounds__(256) void k_batch_integrate(
     if (threadIdx.x == 0 && step < 0x7fffffff) counts[4] = step + 1;
   }
   for (int blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
-    int2 bl = blocks[blk];
-    const int parts = (bl.y & 3) + 1;  // block starts are multiples of 256
-    bl.y &= ~3;
+    const int4 bl = blocks[blk];
+    const int stored = (bl.z & 3) + 1, npad = bl.z >> 2;
     if (c_quota[bl.x] <= step) continue;  // quota used up in this call
     const int i = bl.y + threadIdx.x;
     if (i - c_off[bl.x] >= c_n[bl.x]) continue;  // padding keeps zero mass
@@ -201,8 +215,9 @@ __global__ __launch_bounds__(256) void k_batch_integrate(
       const int64_t k = a * cap + i;
       double v = vel[k];
       double p = pos[k];
-      double f = force[k];
-      for (int q = 1; q < parts; ++q) f += force[3 * cap * q + k];
+      const double* mine = force + a * force_cap + i;
+      double f = *mine;
+      for (int q = 1; q < stored; ++q) f += mine[bl.w + (q - 1) * npad];
       if (kEuler) {
         v = v + f * dt;
         p = p + v * dt;
@@ -279,7 +294,7 @@ hipError_t launch_force(nb_batch* b, int use_quota) {
     per_cu = std::max(1, 16 / K);
   const int grid = b->cus * per_cu;
   hipLaunchKernelGGL((k_batch_force<B, K>), dim3(grid), dim3(64 * K), 0, b->stream, b->pm,
-                     b->c_quota, use_quota, b->items, b->counts, b->cap, b->force);
+                     b->c_quota, use_quota, b->items, b->counts, b->force_cap, b->force);
   return hipGetLastError();
 }
 
@@ -322,11 +337,11 @@ hipError_t enqueue_step(nb_batch* b) {
   if (b->cfg.integrator == NB_INTEG_EULER)
     hipLaunchKernelGGL((k_batch_integrate<true>), dim3(nblk), dim3(256), 0, b->stream, b->blocks,
                        b->counts, b->c_off, b->c_n, b->c_dt, b->c_scale, b->c_quota, b->cap, b->pos, b->vel,
-                       b->acc, b->force, b->mass, b->pm);
+                       b->acc, b->force, b->force_cap, b->mass, b->pm);
   else
     hipLaunchKernelGGL((k_batch_integrate<false>), dim3(nblk), dim3(256), 0, b->stream, b->blocks,
                        b->counts, b->c_off, b->c_n, b->c_dt, b->c_scale, b->c_quota, b->cap, b->pos, b->vel,
-                       b->acc, b->force, b->mass, b->pm);
+                       b->acc, b->force, b->force_cap, b->mass, b->pm);
   return hipGetLastError();
 }
 
@@ -337,34 +352,52 @@ int rebuild_tables(nb_batch* b) {
   for (int s = 0; s < (int)b->used.size(); ++s)
     if (b->used[s]) slots.push_back(s);
   std::stable_sort(slots.begin(), slots.end(),
+                   [&](int a, int c) { return b->h_npad[a] > b->h_npad[c]; });
+  // partial sums, largest clusters first, in free segments of the force array
+  std::vector<std::pair<int64_t, int64_t>> room(b->free_list.begin(), b->free_list.end());
+  room.push_back({b->cap, b->force_cap - b->cap});
+  for (int s : slots) {
+    const int npad = b->h_npad[s], parts = batch_parts(npad);
+    const int64_t need = (int64_t)(parts - 1) * npad;
+    b->h_stored[s] = 1;
+    b->h_shift[s] = 0;
+    if (parts == 1) continue;
+    const auto seg = std::find_if(room.begin(), room.end(), [&](const auto& r) { return r.second >= need; });
+    if (seg == room.end()) continue;
+    b->h_stored[s] = parts;
+    b->h_shift[s] = (int)(seg->first - b->h_off[s]);
+    seg->first += need;
+    seg->second -= need;
+  }
+  std::stable_sort(slots.begin(), slots.end(),
                    [&](int a, int c) {  // sources per item
-                     return b->h_npad[a] / batch_parts(b, b->h_npad[a]) > b->h_npad[c] / batch_parts(b, b->h_npad[c]);
+                     return b->h_npad[a] / b->h_stored[a] > b->h_npad[c] / b->h_stored[c];
                    });
   std::vector<nb_batch_item> items;
-  std::vector<int2> blocks;
+  std::vector<int4> blocks;
   int64_t inter = 0;
   const int iblock = 64 * b->bpl;
   for (int s : slots) {
-    const int parts = batch_parts(b, b->h_npad[s]);
-    for (int q = 0; q < b->h_npad[s] / iblock; ++q)
-      for (int part = 0; part < parts; ++part)
-        items.push_back({2 * s + (b->h_equal[s].on ? 1 : 0), b->h_off[s] + q * iblock, b->h_off[s],
-                         b->h_off[s] + b->h_n[s],
-                         (b->h_npad[s] / 16) << 4 | (parts - 1) << 2 | part, b->h_equal[s].eps2,
-                         b->h_equal[s].factor});
+    const int npad = b->h_npad[s], off = b->h_off[s], stored = b->h_stored[s], parts = batch_parts(npad);
+    for (int q = 0; q < npad / iblock; ++q)
+      for (int p = 0; p < stored; ++p)
+        items.push_back({s << 6 | (parts - 1) << 4 | p << 2 | (stored < parts) << 1 | (b->h_equal[s].on ? 1 : 0),
+                         off + q * iblock, off, off + b->h_n[s], p > 0 ? b->h_shift[s] + (p - 1) * npad : 0,
+                         b->h_equal[s].eps2, b->h_equal[s].factor});
     inter += (int64_t)b->h_n[s] * (b->h_n[s] - 1);
   }
   std::vector<int> by_off(slots);
   std::sort(by_off.begin(), by_off.end(), [&](int a, int c) { return b->h_off[a] < b->h_off[c]; });
   for (int s : by_off)
     for (int q = 0; q < b->h_npad[s]; q += 256)
-      blocks.push_back(make_int2(s, b->h_off[s] + q + batch_parts(b, b->h_npad[s]) - 1));
+      blocks.push_back(make_int4(s, b->h_off[s] + q, b->h_stored[s] > 1 ? b->h_npad[s] << 2 | (b->h_stored[s] - 1) : 0,
+                                 b->h_shift[s]));
   const int counts[2] = {(int)items.size(), (int)blocks.size()};
   if (!items.empty())
     NB_HIP(hipMemcpyAsync(b->items, items.data(), items.size() * sizeof(nb_batch_item),
                           hipMemcpyHostToDevice, b->stream));
   if (!blocks.empty())
-    NB_HIP(hipMemcpyAsync(b->blocks, blocks.data(), blocks.size() * sizeof(int2),
+    NB_HIP(hipMemcpyAsync(b->blocks, blocks.data(), blocks.size() * sizeof(int4),
                           hipMemcpyHostToDevice, b->stream));
   NB_HIP(hipMemcpyAsync(b->counts, counts, sizeof(counts), hipMemcpyHostToDevice, b->stream));
   NB_HIP(hipStreamSynchronize(b->stream));  // the host vectors die here
@@ -397,9 +430,7 @@ int check_slot(nb_batch* b, int32_t id) {
 
 }  // namespace
 
-extern "C" {
-
-int nb_batch_create(nb_batch** out, const nb_batch_config* cfg) {
+int nb_batch_create_with(nb_batch** out, const nb_batch_config* cfg, bool spare) {
   NB_TRY
   NB_API_SHARED;
   if (!out || !cfg) return nb_fail(NB_E_ARG, "nb_batch_create: null argument");
@@ -445,19 +476,26 @@ int nb_batch_create(nb_batch** out, const nb_batch_config* cfg) {
     return fail(NB_E_HIP, "nb_batch_create: hipStreamCreate failed");
   const size_t cap = b->cap, mc = cfg->max_clusters;
   auto A = [](void** p, size_t bytes) { return hipMalloc(p, bytes < 256 ? 256 : bytes); };
+  b->force_cap = b->cap + (spare && b->cap > 4096 ? std::min(3 * b->cap, kSpareBodies) : 0);
+  if (A((void**)&b->force, 3 * b->force_cap * sizeof(double))) {  // the spare entries may go
+    (void)hipGetLastError();
+    b->force_cap = b->cap;
+    if (A((void**)&b->force, 3 * cap * sizeof(double)))
+      return fail(NB_E_OOM, "nb_batch_create: device allocation failed");
+  }
+  const size_t fcap = b->force_cap;
   if (A((void**)&b->pm, cap * sizeof(float4)) || A((void**)&b->pos, 3 * cap * sizeof(double)) ||
       A((void**)&b->vel, 3 * cap * sizeof(double)) || A((void**)&b->acc, 3 * cap * sizeof(double)) ||
-      A((void**)&b->force, 3 * cap * sizeof(double)) || A((void**)&b->mass, cap * sizeof(float)) ||
-      A((void**)&b->c_off, mc * sizeof(int)) || A((void**)&b->c_n, mc * sizeof(int)) ||
+      A((void**)&b->mass, cap * sizeof(float)) || A((void**)&b->c_off, mc * sizeof(int)) || A((void**)&b->c_n, mc * sizeof(int)) ||
       A((void**)&b->c_dt, mc * sizeof(double)) || A((void**)&b->c_scale, mc * sizeof(float)) ||
       A((void**)&b->c_quota, mc * sizeof(int)) ||
-      A((void**)&b->items, (cap / 64) * kMaxParts * sizeof(nb_batch_item)) ||
-      A((void**)&b->blocks, (cap / 256) * sizeof(int2)) || A((void**)&b->counts, kCounts * sizeof(int)) ||
+      A((void**)&b->items, fcap / 64 * sizeof(nb_batch_item)) ||
+      A((void**)&b->blocks, (cap / 256) * sizeof(int4)) || A((void**)&b->counts, kCounts * sizeof(int)) ||
       A((void**)&b->red, (2 * (cap / 256) + 16) * sizeof(double)))
     return fail(NB_E_OOM, "nb_batch_create: device allocation failed");
   if (hipMemset(b->pm, 0, cap * sizeof(float4)) != hipSuccess ||
       hipMemset(b->mass, 0, cap * sizeof(float)) != hipSuccess ||
-      hipMemset(b->force, 0, 3 * cap * sizeof(double)) != hipSuccess ||
+      hipMemset(b->force, 0, 3 * fcap * sizeof(double)) != hipSuccess ||
       hipMemset(b->counts, 0, kCounts * sizeof(int)) != hipSuccess)
     return fail(NB_E_HIP, "nb_batch_create: hipMemset failed");
   for (auto& e : b->ev)
@@ -468,12 +506,20 @@ int nb_batch_create(nb_batch** out, const nb_batch_config* cfg) {
   b->h_eps2.assign(mc, 0.f);
   b->h_G.assign(mc, 1.0);
   b->h_equal.assign(mc, nb_equal_mass{});
+  b->h_stored.assign(mc, 1);
+  b->h_shift.assign(mc, 0);
   b->used.assign(mc, 0);
   b->h_quota.assign(mc, kUnlimited);
   b->free_list[0] = b->cap;
   *out = b;
   return NB_OK;
   NB_CATCH("nb_batch_create")
+}
+
+extern "C" {
+
+int nb_batch_create(nb_batch** out, const nb_batch_config* cfg) {
+  return nb_batch_create_with(out, cfg, true);
 }
 
 void nb_batch_destroy(nb_batch* b) {
@@ -492,20 +538,6 @@ int nb_batch_add(nb_batch* b, const double* pos3, const double* vel3, const doub
   if (!(eps2 >= 0.f) || !std::isfinite(eps2) || !std::isfinite(dt))
     return nb_fail(NB_E_ARG, "nb_batch_add: bad eps2 or dt");
   const int64_t npad = (n + 255) / 256 * 256;
-  if (!b->wide && npad <= b->cap && batch_parts(b, (int)npad) > 1) {  // room for partial sums
-    double* wide = nullptr;
-    if (hipMalloc(reinterpret_cast<void**>(&wide), (size_t)kMaxParts * 3 * b->cap * sizeof(double)) ==
-        hipSuccess) {
-      nb_drop_graph(b->stream, b->graph_exec, b->graph);  // holds the old address
-      NB_HIP(hipStreamSynchronize(b->stream));
-      (void)hipFree(b->force);
-      b->force = wide;
-      b->wide = true;
-    } else {
-      (void)hipGetLastError();
-      b->max_parts = 1;
-    }
-  }
   int slot = -1;
   for (int s = 0; s < (int)b->used.size(); ++s)
     if (!b->used[s]) { slot = s; break; }
@@ -679,12 +711,8 @@ int nb_batch_sync(nb_batch* b) {
   NB_CATCH("nb_batch_sync")
 }
 
-static int fetch(nb_batch* b, int32_t id, const double* const* src, double* const* dst, int arrays,
-                 int parts = 1) {
-  nb_planes p;
-  p.n = b->h_n[id];
-  p.stride = b->cap;
-  p.parts = parts;
+static int fetch(nb_batch* b, const nb_planes& p, int32_t id, const double* const* src, double* const* dst,
+                 int arrays) {
   const double* from[3];
   void* to[3];
   int count = 0;
@@ -710,8 +738,14 @@ int nb_batch_forces(nb_batch* b, int32_t id, double* force3) {
   rc = rebuild_tables(b);
   if (rc) return rc;
   NB_HIP(enqueue_force(b));
+  nb_planes p;
+  p.n = b->h_n[id];
+  p.stride = b->force_cap;
+  p.parts = b->h_stored[id];
+  p.part_first = b->h_shift[id];
+  p.part_stride = b->h_npad[id];
   const double* src = b->force;
-  return fetch(b, id, &src, &force3, 1, batch_parts(b, b->h_npad[id]));
+  return fetch(b, p, id, &src, &force3, 1);
   NB_CATCH("nb_batch_forces")
 }
 
@@ -720,9 +754,12 @@ int nb_batch_download(nb_batch* b, int32_t id, double* pos3, double* vel3, doubl
   NB_API_SHARED;
   int rc = check_slot(b, id);
   if (rc) return rc;
+  nb_planes p;
+  p.n = b->h_n[id];
+  p.stride = b->cap;
   const double* src[3] = {b->pos, b->vel, b->acc};
   double* dst[3] = {pos3, vel3, acc3};
-  return fetch(b, id, src, dst, 3);
+  return fetch(b, p, id, src, dst, 3);
   NB_CATCH("nb_batch_download")
 }
 

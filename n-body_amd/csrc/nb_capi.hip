@@ -556,6 +556,7 @@ static int force_pass(nb_ctx* c, int layout, void* out) {
     if (c->parts > 1) {
       src = c->part;
       p.parts = c->parts;
+      p.part_first = p.part_stride = 3 * p.stride;
       p.G = c->equal.factor;
     }
   }

@@ -302,7 +302,8 @@ struct nb_planes {
   int64_t n = 0;       // bodies
   int64_t stride = 0;  // from one component's plane to the next
   const int* slot_of = nullptr;  // device: slot of each body, or null (body i in slot i)
-  int parts = 1;       // > 1: values are G times the sum of `parts` arrays of 3 * stride
+  int parts = 1;       // > 1: values are G times the sum of part 0, in place, and the others:
+  int64_t part_first = 0, part_stride = 0;  // from it to part 1, from one to the next
   double G = 1.0;
 };
 int nb_stage_ready(nb_stage& st, hipStream_t s, int64_t bytes);  // at least that large, and free
@@ -356,6 +357,9 @@ hipError_t nb_bh_traverse(nb_ctx* c, bool count_interactions);  // -> force
 // Per-body traversal with the default (modified) opening test, counting only:
 // the interactions the group traversal's test needs body by body -> bh.inter
 hipError_t nb_bh_count_per_body(nb_ctx* c);
+
+// nb_batch_create; spare: with room for partial sums beyond the pool (see batch_parts)
+int nb_batch_create_with(nb_batch** out, const nb_batch_config* cfg, bool spare);
 
 // Launch-shape defaults: fill the zero fields from the autotuner's table, then
 // from the built-in defaults.

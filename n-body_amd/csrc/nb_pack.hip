@@ -22,7 +22,7 @@ namespace {
 struct PackArgs {
   const double* src[3];  // first plane of each array
   int64_t stride;        // from one plane to the next
-  int64_t part_stride;   // parts > 1: each value is G times the sum of `parts` values this far apart
+  int64_t part_first, part_stride;  // parts > 1: each value is G times a sum (nb_planes)
   double G;
   int parts;
   int n;               // bodies to pack
@@ -36,7 +36,7 @@ struct PackArgs {
 __device__ __forceinline__ double pack_value(const PackArgs& a, const double* src, int64_t k) {
   double f = src[k];
   if (a.parts > 1) {
-    for (int p = 1; p < a.parts; ++p) f += src[p * a.part_stride + k];
+    for (int p = 1; p < a.parts; ++p) f += src[a.part_first + (p - 1) * a.part_stride + k];
     f *= a.G;
   }
   return f;
@@ -259,7 +259,8 @@ int nb_fetch(nb_stage& st, hipStream_t s, const nb_planes& p, int layout, int ar
   int* stage_flags = reinterpret_cast<int*>(st.host + st.bytes) - 1;
   PackArgs a{};
   a.stride = p.stride;
-  a.part_stride = 3 * p.stride;
+  a.part_first = p.part_first;
+  a.part_stride = p.part_stride;
   a.parts = p.parts;
   a.G = p.G;
   a.slot_of = p.slot_of;

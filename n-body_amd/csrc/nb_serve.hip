@@ -378,7 +378,9 @@ int nb_server_create(nb_server** out, const nb_server_config* cfg) {
     return nb_fail(NB_E_HIP, "nb_server_create: hipMemGetInfo failed");
   }
   int64_t budget = s->cfg.hbm_budget > 0 ? s->cfg.hbm_budget : (int64_t)(0.6 * (double)free_b);
-  const int64_t pool_bytes = s->cfg.direct_pool * 116;  // pm, mass, state, force per body
+  // pm, mass, state, force per body; partial sums go to free segments, and no later call
+  // allocates
+  const int64_t pool_bytes = s->cfg.direct_pool * 116;
   if (pool_bytes >= budget) {
     delete s;
     return nb_fail(NB_E_BUDGET, "nb_server_create: the direct-sum pool exceeds the HBM budget");
@@ -386,7 +388,7 @@ int nb_server_create(nb_server** out, const nb_server_config* cfg) {
   nb_batch_config bc{};
   bc.max_bodies = s->cfg.direct_pool;
   bc.max_clusters = s->cfg.max_jobs;
-  int rc = nb_batch_create(&s->batch, &bc);
+  int rc = nb_batch_create_with(&s->batch, &bc, false);
   if (rc != NB_OK) {
     delete s;
     return rc;

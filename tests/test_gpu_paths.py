@@ -278,3 +278,28 @@ def test_direct_sum_shares_of_unequal_masses(nb, ora, n, bpl, js, eps2):
     scale = np.linalg.norm(ref, axis=1).max()
     # 256-source FP32 sums, folded with compensation: 256 roundings of the largest force at worst
     assert np.abs(f[tgt] - ref).max() <= 256 * 2.0 ** -24 * scale
+
+
+def test_batch_parts_with_and_without_room(nb):
+    """More clusters in parts than there is room for partial sums: those without it, and a
+    batch whose removed clusters make room, give the same forces and steps."""
+    n, clusters = 16000, 12  # four parts each
+    pos, vel, m = nb.ic_plummer(9, n, 50.0, 1e4)
+    with nb.Batch(clusters * 16128, clusters) as b:
+        ids = [b.add(pos, vel, m, EPS2, DT) for _ in range(clusters)]
+        f = [b.forces(c) for c in ids]
+        b.step(2)
+        for c in ids[: clusters // 2]:
+            b.remove(c)
+        b.step(1)
+        end = [b.download(c) for c in ids[clusters // 2:]]
+    with nb.Batch(16128, 1) as b:
+        c = b.add(pos, vel, m, EPS2, DT)
+        ref = b.forces(c)
+        b.step(3)
+        last = b.download(c)
+    for mine in f:
+        np.testing.assert_array_equal(mine, ref)
+    for mine in end:
+        for x, y in zip(mine, last):
+            np.testing.assert_array_equal(x, y)

@@ -1,6 +1,7 @@
 """GPU checks of the serving loop (nb_server_*): results are identical alone and
 in a mix, direct-sum jobs match the FP64 oracle, Barnes-Hut jobs match a
 standalone context bit for bit, and admission respects the HBM budget."""
+import ctypes
 import time
 
 import numpy as np
@@ -254,3 +255,38 @@ def test_c5_stream_at_full_shape(nb, ora):
         alone, _ = run_server(nb, [(n, st, ic, seed)], max_jobs=1, bh_threshold=65536, direct_pool=1 << 17)
         for a, b in zip(alone[0], results[i]):
             assert np.array_equal(a, b), n
+
+
+def free_device_bytes(nb):
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert nb.load().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_large_clusters_take_no_memory_from_the_budget(nb):
+    # the pool's bytes are reserved when the server is created: a cluster that is summed
+    # in parts (above 4096 bodies) finds room for its partial sums in them
+    with nb.Server(direct_pool=1 << 20) as s:
+        def serve(n):
+            i = s.submit(n, 2, 0, 1)
+            t0 = time.monotonic()
+            while s.status(i)["state"] != nb.JOB_DONE and time.monotonic() - t0 < 60:
+                s.tick()
+            assert s.status(i)["state"] == nb.JOB_DONE
+            s.result(i)
+
+        serve(300)
+        before = free_device_bytes(nb)
+        serve(6000)
+        serve(30000)
+        assert before - free_device_bytes(nb) < 8 << 20  # far below 24 bytes for each of 2^20 bodies
+
+
+@pytest.mark.parametrize("n", [4097, 8192, 12289, 21504, 30000])
+def test_full_pool_gives_the_same_bits(nb, n):
+    # no free segment for partial sums: the parts are added one after the other
+    padded = (n + 255) // 256 * 256
+    (full,), _ = run_server(nb, [(n, 3, 0, 7)], bh_threshold=65536, direct_pool=padded)
+    (roomy,), _ = run_server(nb, [(n, 3, 0, 7)], bh_threshold=65536, direct_pool=8 * padded)
+    for a, b in zip(full, roomy):
+        np.testing.assert_array_equal(a, b)
