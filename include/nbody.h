@@ -230,6 +230,10 @@ int nb_debug_tree(nb_ctx* ctx, nb_node_view* nodes, int64_t cap, int64_t* node_c
  * the pass returns NB_E_TREE_OVERFLOW. No counterpart in the reference. */
 int nb_debug_set_walk_stack(nb_ctx* ctx, int32_t entries);
 
+/* Step graphs captured by this process's contexts (nb_step) so far. For tests of
+ * what captures them. No counterpart in the reference. */
+int64_t nb_debug_graph_captures(void);
+
 /* ---- timing ------------------------------------------------------------ */
 typedef struct nb_timing {
   double force_ms;      /* summed device time of force kernels (direct or traversal) */

@@ -6,6 +6,7 @@
 // sequences of ParticleSolverGPU.cpp:31-41 and ParticleSolverBHutGPU.cpp:25-61,
 // and buffer read-back (OpenGLBuffer.cpp:135-165).
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -242,9 +243,13 @@ static int accumulate_timing(nb_ctx* c) {
 constexpr int kChunkSteps = 8;  // even: a small system's views are in place again after it
 constexpr int kGraphStepsBh = 4 * kChunkSteps;
 
-int nb_prepare_step_graph(nb_ctx* c) {
-  if (c->graph_exec || (c->cfg.flags & NB_F_NO_GRAPH)) return NB_OK;
+static std::atomic<int64_t> g_captures{0};
+
+// Captures and instantiates the graph of kChunkSteps steps if there is none (launches nothing).
+static int prepare_step_graph(nb_ctx* c) {
+  if (c->graph_exec) return NB_OK;
   NB_API_CAPTURE;
+  g_captures.fetch_add(1, std::memory_order_relaxed);
   const int steps = kChunkSteps;
   NB_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   hipError_t e = hipSuccess;
@@ -517,7 +522,7 @@ int nb_step(nb_ctx* c, int32_t nsteps) {
   if (!use_graph || nsteps < worth) {
     for (int s = 0; s < nsteps; ++s) NB_HIP(nb_enqueue_step(c));
   } else {
-    const int rc = nb_prepare_step_graph(c);
+    const int rc = prepare_step_graph(c);
     if (rc) return rc;
     // whole graphs, then the remainder as eager launches (identical results)
     int s = 0;
@@ -533,6 +538,8 @@ int nb_step(nb_ctx* c, int32_t nsteps) {
   return NB_OK;
   NB_CATCH("nb_step")
 }
+
+int64_t nb_debug_graph_captures(void) { return g_captures.load(std::memory_order_relaxed); }
 
 int nb_sync(nb_ctx* c) {
   NB_TRY

@@ -370,8 +370,6 @@ bool nb_valid_shape(int bpl, int jsplit);  // a direct-sum kernel exists for it
 
 // step = forces + integration (no sync)
 hipError_t nb_enqueue_step(nb_ctx* c);
-// Capture and instantiate the one-step graph if there is none (launches nothing).
-int nb_prepare_step_graph(nb_ctx* c);
 // Reuse a Barnes-Hut context for another system of the same solver:
 // cfg->n <= c->cap_n; the buffers are re-laid out for cfg->n, the captured step
 // graph is dropped and the state must be uploaded again. Allocates nothing.

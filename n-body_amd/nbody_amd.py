@@ -212,6 +212,7 @@ _SIGS = {
     "nb_debug_morton": (C.c_int, [_P, _P, _P]),
     "nb_debug_tree": (C.c_int, [_P, _P, C.c_int64, C.POINTER(C.c_int64), _P]),
     "nb_debug_set_walk_stack": (C.c_int, [_P, C.c_int32]),
+    "nb_debug_graph_captures": (C.c_int64, []),
     "nb_bh_forces_noalloc": (C.c_int, [_P, C.c_int64, C.c_float, C.c_float, C.c_float, C.c_int32,
                                        C.c_int32, _P, _P, _P]),
     "nb_reorder": (C.c_int, [_P]),

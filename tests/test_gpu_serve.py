@@ -290,3 +290,11 @@ def test_full_pool_gives_the_same_bits(nb, n):
     (roomy,), _ = run_server(nb, [(n, 3, 0, 7)], bh_threshold=65536, direct_pool=8 * padded)
     for a, b in zip(full, roomy):
         np.testing.assert_array_equal(a, b)
+
+
+def test_short_jobs_capture_no_graph(nb):
+    # Barnes-Hut calls of up to 31 steps are launched, so nothing may pay for a graph
+    before = nb.load().nb_debug_graph_captures()
+    out, st = run_server(nb, [(9000, 3, 0, k) for k in range(5)])
+    assert all(x["state"] == nb.JOB_DONE and x["solver"] == nb.SOLVER_BH for x in st)
+    assert nb.load().nb_debug_graph_captures() == before
