@@ -11,7 +11,10 @@
 // for the state of 1000 bodies and 92 ms at 4,194,304; now 12 us and 5.4 ms.
 #include <algorithm>
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
 #include <cstring>
+#include <mutex>
 #include <thread>
 
 #include "nb_force_core.h"
@@ -154,7 +157,8 @@ hipError_t launch_unpack(int layout, const UnpackArgs& a, hipStream_t s) {
 // Copies between the stage and the caller's memory by a few threads that live as
 // long as one call: one core moves 10 to 14 GB/s, fresh pages included, and the bus
 // 50. The helpers only copy; every HIP call stays on the caller's thread. If none can
-// be started the caller copies alone.
+// be started the caller copies alone. Until the first chunk is there, behind all steps
+// that are still queued, and in longer pauses they sleep.
 class CopyTeam {
  public:
   explicit CopyTeam(int64_t bytes) {
@@ -166,7 +170,11 @@ class CopyTeam {
     }
   }
   ~CopyTeam() {
-    stop_.store(true, std::memory_order_release);
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      stop_.store(true, std::memory_order_release);
+    }
+    cv_.notify_all();
     for (int k = 0; k < count_; ++k) helpers_[k].join();
   }
   CopyTeam(const CopyTeam&) = delete;
@@ -181,7 +189,11 @@ class CopyTeam {
     src_ = static_cast<const char*>(src);
     bytes_ = bytes;
     busy_.store(count_, std::memory_order_relaxed);
-    job_.fetch_add(1, std::memory_order_release);
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      job_.fetch_add(1, std::memory_order_release);
+    }
+    cv_.notify_all();
     slice(count_);
     while (busy_.load(std::memory_order_acquire) > 0) std::this_thread::yield();
   }
@@ -190,6 +202,7 @@ class CopyTeam {
   static constexpr int64_t kMinBytes = 4 << 20;  // below: starting helpers costs what they save
   static constexpr int kHelpers = 5;  // 201 MB into fresh memory: none 14 GB/s, one 20, three 28,
                                       // five 38, seven 40; 12.6 MB: one 24, seven 23
+  static constexpr std::chrono::microseconds kSpin{200};  // a chunk of 8 MB is 160 us on the bus
 
   void slice(int k) {  // of count_ + 1, whole pages each
     const size_t per = (bytes_ / (count_ + 1) + 4095) & ~size_t(4095);
@@ -197,13 +210,18 @@ class CopyTeam {
     std::memcpy(dst_ + at, src_ + at, end - at);
   }
   void help(int k) {
-    for (int64_t seen = 0;;) {
-      int64_t job;
-      while ((job = job_.load(std::memory_order_acquire)) == seen) {
-        if (stop_.load(std::memory_order_acquire)) return;
-        std::this_thread::yield();
+    using clock = std::chrono::steady_clock;
+    for (int64_t seen = 0;; ++seen) {  // jobs follow each other only when all have done the last
+      const auto idle = [&] {
+        return job_.load(std::memory_order_acquire) == seen && !stop_.load(std::memory_order_acquire);
+      };
+      if (seen > 0)  // the next chunk is on its way
+        for (const auto until = clock::now() + kSpin; idle() && clock::now() < until;) std::this_thread::yield();
+      if (idle()) {
+        std::unique_lock<std::mutex> lk(mu_);
+        cv_.wait(lk, [&] { return !idle(); });
       }
-      seen = job;
+      if (job_.load(std::memory_order_acquire) == seen) return;  // stopped
       slice(k);
       busy_.fetch_sub(1, std::memory_order_acq_rel);
     }
@@ -215,6 +233,8 @@ class CopyTeam {
   std::atomic<int64_t> job_{0};
   std::atomic<int> busy_{0};
   std::atomic<bool> stop_{false};
+  std::mutex mu_;
+  std::condition_variable cv_;
   int count_ = 0;  // helpers that started; they read it only after a job is posted
   std::thread helpers_[kHelpers];
 };

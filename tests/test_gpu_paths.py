@@ -1,5 +1,7 @@
 """Kernel variants and dispatch rules at the sizes where they can go wrong: tile
 edges, remainders, the smallest and largest of a range."""
+import time
+
 import numpy as np
 import pytest
 
@@ -303,3 +305,19 @@ def test_batch_parts_with_and_without_room(nb):
     for mine in end:
         for x, y in zip(mine, last):
             np.testing.assert_array_equal(x, y)
+
+
+def test_download_waits_without_spinning(nb):
+    """A large download behind queued steps occupies the calling thread at most: the
+    threads that will copy sleep until there is something to copy."""
+    n = 1 << 18
+    pos, vel, m = nb.ic_ball(1, n, 100.0, 1.0)
+    with nb.Simulation(n, EPS2, DT) as sim:
+        sim.upload(pos, vel, m)
+        sim.step(1)
+        sim.download_f64()
+        sim.step(30)  # some 400 ms
+        wall, cpu = time.monotonic(), time.process_time()
+        sim.download_f64()
+        wall, cpu = time.monotonic() - wall, time.process_time() - cpu
+    assert cpu < 2.0 * wall
