@@ -410,9 +410,10 @@ int nb_server_get_stats(nb_server* s, nb_server_stats* out);
  * nb_create / nb_batch_create calls for systems in the same power-of-two size
  * class (explicit non-zero config fields still win). Candidates: direct sum
  * bodies_per_lane x j_split in {1,2,4} x {1,2,4,8,16} (the shapes a kernel
- * exists for: 8 needs bodies_per_lane <= 2, 16 needs 1); Barnes-Hut leaf_size in
- * {1,2,4,8,16,32}. The reference hard-codes its work-group sizes (64, 320,
- * 1024) in the shaders. */
+ * exists for: 8 needs bodies_per_lane <= 2, 16 needs 1), and up to 8192 bodies the
+ * kernel that takes a step in one launch, which has no shape (0, 0) and is the
+ * built-in default there; Barnes-Hut leaf_size in {1,2,4,8,16,32}. The reference
+ * hard-codes its work-group sizes (64, 320, 1024) in the shaders. */
 typedef struct nb_tuning {
   int64_t n;
   int32_t bodies_per_lane;
@@ -420,7 +421,8 @@ typedef struct nb_tuning {
   int32_t leaf_size;
   int32_t bh_single_ranges;  /* nb_tune_leaf: 1 if single ranges timed faster than pairs
                                 (NB_F_BH_SINGLE_RANGES set), 0 if pairs (NB_F_BH_PAIRS set) */
-  double direct_ms;  /* force pass at the chosen shape (0 if not tuned) */
+  double direct_ms;  /* force pass at the chosen shape (0 if not tuned); up to 8192
+                        bodies the shape is chosen by whole steps */
   double bh_ms;      /* Barnes-Hut build + traversal at the chosen leaf size */
 } nb_tuning;
 #define NB_TUNE_DIRECT 0x1
@@ -439,7 +441,9 @@ int nb_batch_tune(nb_batch* b, int32_t reps, nb_tuning* out);
  * candidate serves the context's later steps; out->leaf_size,
  * out->bh_single_ranges and out->bh_ms (its fastest pass) receive the choice. */
 int nb_tune_leaf(nb_ctx* ctx, int32_t reps, nb_tuning* out);
-/* The defaults nb_create would use for n bodies (tuned or built in). */
+/* The defaults nb_create would use for n bodies (tuned or built in). Up to 8192
+ * bodies, unless a shape was tuned, steps take one launch without one, and the
+ * shape is that of a context with only one of its fields given. */
 int nb_get_tuning(int64_t n, nb_tuning* out);
 
 /* Library / device description for logs: writes a NUL-terminated string. */

@@ -183,9 +183,11 @@ bool nb_valid_shape(int bpl, int jsplit) {
 
 namespace {
 
-void default_direct_shape(nb_ctx* c) {
+void default_direct_shape(nb_ctx* c, bool tuned) {
   int bpl = c->cfg.bodies_per_lane, js = c->cfg.j_split, leaf = c->cfg.leaf_size;
-  nb_tuned_shape(c->cfg.n, &bpl, &js, &leaf);
+  if (tuned) nb_tuned_shape(c->cfg.n, &bpl, &js, &leaf);
+  // a launch shape, the caller's or the tuner's, is a choice of k_direct's
+  c->small = c->cfg.solver == NB_SOLVER_DIRECT && c->n_pad <= kSmallBodies && bpl == 0 && js == 0;
   nb_default_shape(c->cfg.n, &bpl, &js, &leaf);
   if (!nb_valid_shape(bpl, js)) js = std::min(js, bpl == 1 ? 16 : bpl == 2 ? 8 : 4);
   c->bpl = bpl;
@@ -311,9 +313,7 @@ int nb_ctx_rebind(nb_ctx* c, const nb_config* cfg) {
   NB_CATCH("nb_ctx_rebind")
 }
 
-extern "C" {
-
-int nb_create(nb_ctx** out, const nb_config* cfg) {
+int nb_create_with(nb_ctx** out, const nb_config* cfg, bool tuned) {
   NB_TRY
   NB_RANGE("nb_create");
   NB_API_SHARED;
@@ -366,11 +366,7 @@ int nb_create(nb_ctx** out, const nb_config* cfg) {
   // The self pair gives dx = 0; its term is exactly 0 unless eps2 is so small
   // that (eps2)^{-3/2} overflows FP32. Below that, use the guarded kernel.
   c->guard = !(cfg->eps2 >= 1e-20f);
-  default_direct_shape(c);
-  if (c->cfg.solver == NB_SOLVER_DIRECT) {
-    // an explicit launch shape is a choice of k_direct's
-    c->small = c->n_pad <= kSmallBodies && cfg->bodies_per_lane == 0 && cfg->j_split == 0;
-  }
+  default_direct_shape(c, tuned);
 
   (void)hipGetDevice(&c->device);
   if (c->cfg.solver == NB_SOLVER_DIRECT && !c->small) {
@@ -412,6 +408,10 @@ int nb_create(nb_ctx** out, const nb_config* cfg) {
   return NB_OK;
   NB_CATCH("nb_create")
 }
+
+extern "C" {
+
+int nb_create(nb_ctx** out, const nb_config* cfg) { return nb_create_with(out, cfg, true); }
 
 void nb_destroy(nb_ctx* ctx) {
   NB_API_SHARED;

@@ -361,6 +361,9 @@ hipError_t nb_bh_count_per_body(nb_ctx* c);
 // nb_batch_create; spare: with room for partial sums beyond the pool (see batch_parts)
 int nb_batch_create_with(nb_batch** out, const nb_batch_config* cfg, bool spare);
 
+// nb_create; tuned: zero shape fields take the autotuner's values, if there are any
+int nb_create_with(nb_ctx** out, const nb_config* cfg, bool tuned);
+
 // Launch-shape defaults: fill the zero fields from the autotuner's table, then
 // from the built-in defaults.
 bool nb_tuned_shape(int64_t n, int* bpl, int* jsplit, int* leaf);

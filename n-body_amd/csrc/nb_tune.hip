@@ -36,10 +36,10 @@ Input plummer(int64_t n) {
   return in;
 }
 
-// Mean device time of `reps` force passes (after one warm-up pass).
-int time_forces(const nb_config& cfg, const Input& in, int reps, double* ms) {
+// Mean device time of `reps` force passes, or steps (after one warm-up pass).
+int time_passes(const nb_config& cfg, const Input& in, int reps, bool steps, double* ms) {
   nb_ctx* c = nullptr;
-  int rc = nb_create(&c, &cfg);
+  int rc = nb_create_with(&c, &cfg, false);
   if (rc) return rc;
   rc = nb_upload_f64(c, in.pos.data(), in.vel.data(), nullptr, in.mass.data(), cfg.n);
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -48,7 +48,9 @@ int time_forces(const nb_config& cfg, const Input& in, int reps, double* ms) {
   for (int r = -1; !rc && r < reps; ++r) {
     if (r == 0) (void)hipEventRecord(e0, c->stream);
     hipError_t e;
-    if (cfg.solver == NB_SOLVER_BH) {
+    if (steps) {
+      e = nb_enqueue_step(c);
+    } else if (cfg.solver == NB_SOLVER_BH) {
       e = nb_bh_build(c);
       if (e == hipSuccess) e = nb_bh_traverse(c, false);
     } else {
@@ -99,27 +101,37 @@ extern "C" int nb_autotune(int64_t n, int32_t what, int32_t reps, nb_tuning* out
     best.j_split = t.j_split;
   }
   if (what & NB_TUNE_DIRECT) {
+    // up to kSmallBodies one launch per step (shape 0, 0) stands against two, so whole
+    // steps are timed there, enough of them for launches of a few us
+    const bool small = (n + kPadBodies - 1) / kPadBodies * kPadBodies <= kSmallBodies;
     double best_ms = DBL_MAX;
+    nb_config cfg{};
+    cfg.n = n;
+    cfg.eps2 = 40.f;
+    cfg.dt = 0.0035f;
+    cfg.solver = NB_SOLVER_DIRECT;
+    const auto time_shape = [&](int b, int k) -> int {
+      cfg.bodies_per_lane = b;
+      cfg.j_split = k;
+      double ms = 0;
+      const int rc = time_passes(cfg, in, small ? 16 * reps : reps, small, &ms);
+      if (rc || ms >= best_ms) return rc;
+      best_ms = ms;
+      best.bodies_per_lane = b;
+      best.j_split = k;
+      best.direct_ms = ms;
+      return NB_OK;
+    };
+    int rc = small ? time_shape(0, 0) : NB_OK;
     for (int b : {1, 2, 4})
-      for (int k : {1, 2, 4, 8, 16}) {
-        if (!nb_valid_shape(b, k)) continue;
-        nb_config cfg{};
-        cfg.n = n;
-        cfg.eps2 = 40.f;
-        cfg.dt = 0.0035f;
-        cfg.solver = NB_SOLVER_DIRECT;
-        cfg.bodies_per_lane = b;
-        cfg.j_split = k;
-        double ms = 0;
-        const int rc = time_forces(cfg, in, reps, &ms);
-        if (rc) return rc;
-        if (ms < best_ms) {
-          best_ms = ms;
-          best.bodies_per_lane = b;
-          best.j_split = k;
-          best.direct_ms = ms;
-        }
-      }
+      for (int k : {1, 2, 4, 8, 16})
+        if (!rc && nb_valid_shape(b, k)) rc = time_shape(b, k);
+    if (!rc && small) {
+      cfg.bodies_per_lane = best.bodies_per_lane;
+      cfg.j_split = best.j_split;
+      rc = time_passes(cfg, in, 16 * reps, false, &best.direct_ms);
+    }
+    if (rc) return rc;
   }
   if (what & NB_TUNE_BH) {
     double best_ms = DBL_MAX;
@@ -131,7 +143,7 @@ extern "C" int nb_autotune(int64_t n, int32_t what, int32_t reps, nb_tuning* out
       cfg.solver = NB_SOLVER_BH;
       cfg.leaf_size = leaf;
       double ms = 0;
-      const int rc = time_forces(cfg, in, reps, &ms);
+      const int rc = time_passes(cfg, in, reps, false, &ms);
       if (rc) return rc;
       if (ms < best_ms) {
         best_ms = ms;

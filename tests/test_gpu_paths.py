@@ -321,3 +321,23 @@ def test_download_waits_without_spinning(nb):
         sim.download_f64()
         wall, cpu = time.monotonic() - wall, time.process_time() - cpu
     assert cpu < 2.0 * wall
+
+
+@pytest.mark.parametrize("n", [300, 3000, 8000])
+def test_small_sizes_use_what_the_tuner_reports(nb, n):
+    """Shape 0, 0 is the kernel that takes a step in one launch."""
+    t = nb.autotune(n, nb.TUNE_DIRECT, 3)
+    assert t["direct_ms"] > 0 and (t["bodies_per_lane"] == 0) == (t["j_split"] == 0)
+    pos, vel, m = nb.ic_plummer(n, n, 50.0, 1e4)
+    m[::3] *= 1.5  # no equal masses: the kernels add in different orders
+    out = []
+    for shape in ((0, 0), (t["bodies_per_lane"], t["j_split"])):
+        with nb.Simulation(n, EPS2, DT, bodies_per_lane=shape[0], j_split=shape[1]) as sim:
+            sim.upload(pos, vel, m)
+            sim.step(2)
+            out.append(sim.download_f64())
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+    if t["bodies_per_lane"]:
+        got = nb.get_tuning(n)
+        assert (got["bodies_per_lane"], got["j_split"]) == (t["bodies_per_lane"], t["j_split"])
