@@ -236,7 +236,8 @@ int64_t nb_debug_graph_captures(void);
 
 /* ---- timing ------------------------------------------------------------ */
 typedef struct nb_timing {
-  double force_ms;      /* summed device time of force kernels (direct or traversal) */
+  double force_ms;      /* summed device time of force kernels (direct or traversal);
+                           of the whole step where one launch takes it (nb_autotune) */
   int64_t force_calls;
   double step_ms;       /* summed device time of whole steps (first to last kernel) */
   int64_t step_calls;

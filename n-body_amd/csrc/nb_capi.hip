@@ -200,8 +200,12 @@ void default_direct_shape(nb_ctx* c, bool tuned) {
 hipError_t nb_enqueue_step(nb_ctx* c) {
   hipError_t e;
   const bool t = c->timing;
-  if (c->small && !t) return nb_launch_small_step(c);  // timed steps: the same sums in two launches
   if (t) (void)hipEventRecord(c->ev[0], c->stream);
+  if (c->small) {
+    e = nb_launch_small_step(c);
+    if (t) (void)hipEventRecord(c->ev[3], c->stream);
+    return e;
+  }
   if (c->cfg.solver == NB_SOLVER_BH) {
     e = nb_bh_build(c);
     if (e != hipSuccess) return e;
@@ -221,9 +225,13 @@ hipError_t nb_enqueue_step(nb_ctx* c) {
 static int accumulate_timing(nb_ctx* c) {
   NB_HIP(hipEventSynchronize(c->ev[3]));
   float build = 0.f, force = 0.f, step = 0.f;
-  NB_HIP(hipEventElapsedTime(&build, c->ev[0], c->ev[1]));
-  NB_HIP(hipEventElapsedTime(&force, c->ev[1], c->ev[2]));
   NB_HIP(hipEventElapsedTime(&step, c->ev[0], c->ev[3]));
+  if (c->small) {
+    force = step;  // one launch
+  } else {
+    NB_HIP(hipEventElapsedTime(&build, c->ev[0], c->ev[1]));
+    NB_HIP(hipEventElapsedTime(&force, c->ev[1], c->ev[2]));
+  }
   c->tim.force_ms += force;
   c->tim.force_calls += 1;
   c->tim.step_ms += step;

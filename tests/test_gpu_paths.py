@@ -341,3 +341,31 @@ def test_small_sizes_use_what_the_tuner_reports(nb, n):
     if t["bodies_per_lane"]:
         got = nb.get_tuning(n)
         assert (got["bodies_per_lane"], got["j_split"]) == (t["bodies_per_lane"], t["j_split"])
+
+
+@pytest.mark.parametrize("n", [1, 1024, 4095, 4097])
+def test_timed_small_steps_are_the_steps_that_run(nb, n):
+    """One launch per step has one time, with and without timing the same result, and its
+    forces are those of the force pass."""
+    pos, vel, m = nb.ic_plummer(n + 1, n, 50.0, 1e4)
+    with nb.Simulation(n, EPS2, DT) as sim:
+        sim.upload(pos, vel, m)
+        f = sim.forces_f64()
+        sim.set_timing(True)
+        sim.step(5)
+        t = sim.timing()
+        sim.set_timing(False)
+        timed = sim.download_f64()
+        sim.upload(pos, vel, m)
+        sim.step(1)
+        p, v, a = sim.download_f64()
+        sim.step(4)
+        plain = sim.download_f64()
+    assert t["step_calls"] == t["force_calls"] == 5 and 0 < t["force_ms"] == t["step_ms"]
+    for x, y in zip(timed, plain):
+        np.testing.assert_array_equal(x, y)
+    np.testing.assert_array_equal(a, f)
+    # a first lagged step, from no acceleration; three FP64 roundings of each term
+    h = 0.5 * float(np.float32(DT))
+    np.testing.assert_allclose(v, vel + f * h, rtol=0, atol=4 * 2.0 ** -53 * (np.abs(vel).max() + np.abs(f).max()))
+    np.testing.assert_allclose(p, pos + vel * 2 * h, rtol=0, atol=4 * 2.0 ** -53 * (np.abs(pos).max() + np.abs(vel).max()))
