@@ -323,26 +323,6 @@ def test_download_waits_without_spinning(nb):
     assert cpu < 2.0 * wall
 
 
-@pytest.mark.parametrize("n", [300, 3000, 8000])
-def test_small_sizes_use_what_the_tuner_reports(nb, n):
-    """Shape 0, 0 is the kernel that takes a step in one launch."""
-    t = nb.autotune(n, nb.TUNE_DIRECT, 3)
-    assert t["direct_ms"] > 0 and (t["bodies_per_lane"] == 0) == (t["j_split"] == 0)
-    pos, vel, m = nb.ic_plummer(n, n, 50.0, 1e4)
-    m[::3] *= 1.5  # no equal masses: the kernels add in different orders
-    out = []
-    for shape in ((0, 0), (t["bodies_per_lane"], t["j_split"])):
-        with nb.Simulation(n, EPS2, DT, bodies_per_lane=shape[0], j_split=shape[1]) as sim:
-            sim.upload(pos, vel, m)
-            sim.step(2)
-            out.append(sim.download_f64())
-    for a, b in zip(*out):
-        np.testing.assert_array_equal(a, b)
-    if t["bodies_per_lane"]:
-        got = nb.get_tuning(n)
-        assert (got["bodies_per_lane"], got["j_split"]) == (t["bodies_per_lane"], t["j_split"])
-
-
 @pytest.mark.parametrize("n", [1, 1024, 4095, 4097])
 def test_timed_small_steps_are_the_steps_that_run(nb, n):
     """One launch per step has one time, with and without timing the same result, and its
@@ -369,3 +349,24 @@ def test_timed_small_steps_are_the_steps_that_run(nb, n):
     h = 0.5 * float(np.float32(DT))
     np.testing.assert_allclose(v, vel + f * h, rtol=0, atol=4 * 2.0 ** -53 * (np.abs(vel).max() + np.abs(f).max()))
     np.testing.assert_allclose(p, pos + vel * 2 * h, rtol=0, atol=4 * 2.0 ** -53 * (np.abs(pos).max() + np.abs(vel).max()))
+
+
+@pytest.mark.parametrize("n", [300, 3000, 8000])
+def test_small_sizes_use_what_the_tuner_reports(nb, n):
+    """Shape 0, 0 is the kernel that takes a step in one launch. Last in the file: a shape
+    that wins stays the default of its size class in this process."""
+    t = nb.autotune(n, nb.TUNE_DIRECT, 3)
+    assert t["direct_ms"] > 0 and (t["bodies_per_lane"] == 0) == (t["j_split"] == 0)
+    pos, vel, m = nb.ic_plummer(n, n, 50.0, 1e4)
+    m[::3] *= 1.5  # no equal masses: the kernels add in different orders
+    out = []
+    for shape in ((0, 0), (t["bodies_per_lane"], t["j_split"])):
+        with nb.Simulation(n, EPS2, DT, bodies_per_lane=shape[0], j_split=shape[1]) as sim:
+            sim.upload(pos, vel, m)
+            sim.step(2)
+            out.append(sim.download_f64())
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+    if t["bodies_per_lane"]:
+        got = nb.get_tuning(n)
+        assert (got["bodies_per_lane"], got["j_split"]) == (t["bodies_per_lane"], t["j_split"])
