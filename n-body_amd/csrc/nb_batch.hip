@@ -2,7 +2,7 @@
 // in one persistent force launch (see the nb_batch_* block of nbody.h).
 //
 // Layout in HBM: one body pool of `cap` bodies. A cluster occupies a contiguous
-// segment [off, off + n_pad) (n_pad = n rounded up to 256, zero-mass padding),
+// segment [off, off + n_pad) (n_pad = n rounded up to 256, far-away padding),
 // so its FP32 view pm[off..], FP64 state pos/vel/acc[k * cap + off..] and forces
 // are plain slices. Per-slot parameters (offset, n, n_pad, eps2, dt, G) live in
 // device arrays indexed by slot.
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(256) void k_batch_integrate(
     const int stored = (bl.z & 3) + 1, npad = bl.z >> 2;
     if (c_quota[bl.x] <= step) continue;  // quota used up in this call
     const int i = bl.y + threadIdx.x;
-    if (i - c_off[bl.x] >= c_n[bl.x]) continue;  // padding keeps zero mass
+    if (i - c_off[bl.x] >= c_n[bl.x]) continue;  // padding stays far away
     const double dt = c_dt[bl.x];
     const double h = dt * 0.5;
     const float scale = c_scale[bl.x];

@@ -14,6 +14,7 @@
 #include <numeric>
 #include <vector>
 
+#include "nb_force_core.h"
 #include "nb_internal.h"
 
 static thread_local std::string g_last_error;
@@ -400,9 +401,13 @@ int nb_create_with(nb_ctx** out, const nb_config* cfg, bool tuned) {
   if (hipMemset(c->flags, 0, 4 * sizeof(int)) != hipSuccess ||
       hipMemset(c->mass, 0, np * sizeof(float)) != hipSuccess ||
       hipMemset(c->pm, 0, np * sizeof(float4)) != hipSuccess ||
-      (c->small && hipMemset(c->pm_next, 0, np * sizeof(float4)) != hipSuccess) ||
       hipMemset(c->force, 0, 3 * n * sizeof(double)) != hipSuccess)
     return fail(NB_E_HIP, "nb_create: hipMemset failed");
+  if (c->small) {  // an upload pads pm; steps write the bodies only
+    const std::vector<float4> pad(np, nbcore::far_pad());
+    if (hipMemcpy(c->pm_next, pad.data(), np * sizeof(float4), hipMemcpyHostToDevice) != hipSuccess)
+      return fail(NB_E_HIP, "nb_create: hipMemcpy failed");
+  }
   for (auto& e : c->ev)
     if (hipEventCreate(&e) != hipSuccess) return fail(NB_E_HIP, "nb_create: hipEventCreate failed");
   if (c->cfg.solver == NB_SOLVER_BH) {

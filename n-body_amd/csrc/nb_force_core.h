@@ -26,8 +26,9 @@ __device__ __forceinline__ int even_chunk(uint32_t len) {
 }
 
 // Coordinates of the padding of an FP32 view, and its mass: r^2 is infinite and
-// 1/r zero against any body, so it adds nothing with or without its mass.
-__device__ __forceinline__ float4 far_pad() { return make_float4(1e30f, 1e30f, 1e30f, 0.f); }
+// 1/r zero against any body, so it adds nothing with or without its mass. (Zero mass
+// alone is not enough: at a distance whose r^-2 overflows, its term is not a number.)
+__host__ __device__ __forceinline__ float4 far_pad() { return make_float4(1e30f, 1e30f, 1e30f, 0.f); }
 
 __device__ __forceinline__ void two_sum_fold(float& s, float& c, float x) {
   const float t = s + x;

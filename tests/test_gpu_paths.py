@@ -351,6 +351,22 @@ def test_timed_small_steps_are_the_steps_that_run(nb, n):
     np.testing.assert_allclose(p, pos + vel * 2 * h, rtol=0, atol=4 * 2.0 ** -53 * (np.abs(pos).max() + np.abs(vel).max()))
 
 
+@pytest.mark.parametrize("n", [1, 3, 1000, 4097])
+def test_padding_of_both_views_adds_nothing(nb, n):
+    """Without softening, a body closer to the origin than FP32 has inverse squares for:
+    the padding of either view (steps alternate them) must not be there."""
+    pos, _, m = nb.ic_ball(5, n, 100.0, 1.0)
+    pos[0] = (1e-20, 0, 0)
+    zero = np.zeros_like(pos)
+    with nb.Simulation(n, 0.0, 0.0) as sim:  # dt = 0: the forces stay
+        sim.upload(pos, zero, m)
+        f = sim.forces_f64()
+        assert np.isfinite(f).all()
+        for _ in range(3):
+            sim.step(1)
+            np.testing.assert_array_equal(sim.download_f64()[2], f)
+
+
 @pytest.mark.parametrize("n", [300, 3000, 8000])
 def test_small_sizes_use_what_the_tuner_reports(nb, n):
     """Shape 0, 0 is the kernel that takes a step in one launch. Last in the file: a shape
