@@ -1151,9 +1151,9 @@ __device__ __forceinline__ void list_flush(const uint32_t* list, int lc, float4*
   const int per = 64 >> log2S;  // entries per slice
   const int put = (lane & (S - 1)) * per + (lane >> log2S);  // slice-major slot of entry `lane`
   const float4* mine = stage + slice * per;
-  // lane's source of the chunk starting at e (a zero-mass pad past the list)
+  // lane's source of the chunk starting at e (a far-away pad past the list)
   auto gather = [&](int e) {
-    float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 g = nbcore::far_pad();
     if (e + lane < lc) {
       const uint32_t id = list[e + lane];
       g = (id & kCellBit) ? nodes[id & ~kCellBit].com : pms[id];
@@ -1169,7 +1169,7 @@ __device__ __forceinline__ void list_flush(const uint32_t* list, int lc, float4*
     if (e + 64 < lc) q = gather(e + 64);
     // T = ceil(m / S) rounded up to 4 entries per slice; S <= 16 divides 64, so
     // 64 / S is a multiple of 4 and T <= 64 / S: every read stays inside this
-    // slice's block; entries at or past m are zero-mass pads.
+    // slice's block; entries at or past m are far-away pads.
     const int T = __builtin_amdgcn_readfirstlane((((m + S - 1) >> log2S) + 3) & ~3);
     for (int t = 0; t < T; t += 4) {
       float dx[4], dy[4], dz[4], r2[4], inv[4], w[4];

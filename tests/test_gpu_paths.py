@@ -367,6 +367,22 @@ def test_padding_of_both_views_adds_nothing(nb, n):
             np.testing.assert_array_equal(sim.download_f64()[2], f)
 
 
+@pytest.mark.parametrize("n", [3, 40, 5001])
+@pytest.mark.parametrize("pairs", [False, True])
+def test_padding_of_walk_lists_adds_nothing(nb, ora, n, pairs):
+    """As above for the lists of both Barnes-Hut walks; leaves of single bodies, theta so
+    small that every body is listed."""
+    pos, vel, m = nb.ic_ball(6, n, 100.0, 1.0)
+    pos[0] = (1e-20, 0, 0)
+    with nb.Simulation(n, 0.0, DT, solver=nb.SOLVER_BH, theta=1e-6, leaf_size=1,
+                       flags=nb.F_BH_PAIRS if pairs else 0) as sim:
+        sim.upload(pos, vel, m)
+        f = sim.forces_f64()
+    ref = ora.direct_f64(pos.astype(np.float32).astype(np.float64), m.astype(np.float64), 0.0)
+    # FP32 sums of at most 384 terms, folded: as many roundings of the largest force at worst
+    assert np.abs(f - ref).max() <= 384 * 2.0 ** -24 * np.linalg.norm(ref, axis=1).max()
+
+
 @pytest.mark.parametrize("n", [300, 3000, 8000])
 def test_small_sizes_use_what_the_tuner_reports(nb, n):
     """Shape 0, 0 is the kernel that takes a step in one launch. Last in the file: a shape
