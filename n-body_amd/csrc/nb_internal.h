@@ -177,7 +177,6 @@ struct nb_bh_state {
   int* digit_hist = nullptr;    // radix: [sort_blocks][256] digit counts of the current pass
   int* group_hist = nullptr;    // radix: [4][groups][256] digit counts of each pass, kSortGroup tiles
   int sort_blocks = 0;
-  int sorted_buf = 0;           // which of keys[]/vals[] holds the final order
   float4* pms = nullptr;        // bodies in sorted order (x, y, z, m)
   double4* prefix = nullptr;    // exclusive FP64 prefix of (m, m x, m y, m z), n+1 entries
   double4* scan_part = nullptr; // scan block partials

@@ -383,6 +383,34 @@ def test_padding_of_walk_lists_adds_nothing(nb, ora, n, pairs):
     assert np.abs(f - ref).max() <= 384 * 2.0 ** -24 * np.linalg.norm(ref, axis=1).max()
 
 
+@pytest.mark.parametrize("n", [31 * 131072, 31 * 131072 + 1, 64 * 131072 + 1, 9000001])
+def test_radix_sort_of_many_groups(nb, n):
+    """Below and above the line at which the groups' counts are added up in a launch of
+    their own: the permutation is the stable sort of the codes."""
+    rng = np.random.default_rng(n)
+    pos = rng.random((n, 3)) ** 3
+    with nb.Simulation(n, EPS2, DT, solver=nb.SOLVER_BH, theta=2.0) as sim:
+        sim.upload(pos, np.zeros_like(pos), np.ones(n, np.float32))
+        sim.step(1)
+        codes, perm = sim.debug_morton()
+    np.testing.assert_array_equal(perm, np.argsort(codes, kind="stable"))
+
+
+def test_build_time_stays_linear(nb):
+    """A body of 2^26 costs what one of 2^23 does: no pass of the build adds up a table
+    that grows with the system in each of its blocks."""
+    cost = []
+    for n in (1 << 23, 1 << 26):
+        pos = np.random.default_rng(1).random((n, 3))
+        with nb.Simulation(n, 1e-4, 0.0, solver=nb.SOLVER_BH, theta=1.0) as sim:
+            sim.upload(pos, np.zeros_like(pos), np.ones(n, np.float32))
+            sim.step(1)
+            sim.set_timing(True)
+            sim.step(3)
+            cost.append(sim.timing()["build_ms"] / n)
+    assert cost[1] < 1.25 * cost[0]
+
+
 @pytest.mark.parametrize("n", [300, 3000, 8000])
 def test_small_sizes_use_what_the_tuner_reports(nb, n):
     """Shape 0, 0 is the kernel that takes a step in one launch. Last in the file: a shape
