@@ -90,14 +90,16 @@ int64_t bh_bytes(int64_t n) {
 
 int64_t padded(int64_t n) { return (n + kPadBodies - 1) / kPadBodies * kPadBodies; }
 
-// Estimated device time of one step, from rates measured on MI355X: the
-// compensated direct sum runs about 3.2e12 pair interactions/s once the device
-// is full, and a Barnes-Hut step (theta = 0.5, build + traversal) costs about
-// 1.7 ns per body plus some 0.35 ms of latency-bound launches (7.3 ms at
-// 4,194,304 bodies, about 0.5 ms at 65,536).
+// Estimated device time of one step, from times measured on MI355X. A cluster's share
+// of a direct-sum step: 4e12 pair interactions/s (ms alone / one of four: 16,384 bodies
+// 0.078 / 0.062, 20,000 0.115 / 0.097, 30,000 0.240 / 0.207, 45,000 0.534 / 0.452,
+// 65,535 1.00 / 0.93; estimated 0.069, 0.102, 0.227, 0.508, 1.08). A Barnes-Hut step
+// (theta = 0.5, Plummer spheres): 65,536 bodies 0.195 ms, 131,072 0.311, 262,144 0.503,
+// 524,288 0.869, 2^20 1.61, 2^22 6.04; estimated 0.203, 0.296, 0.482, 0.854, 1.60, 6.07
+// (uniform balls a quarter less).
 double step_cost_ms(int64_t n, int32_t solver) {
-  if (solver == NB_SOLVER_DIRECT) return 2e-3 + (double)n * (double)n / 3.2e9;
-  return 0.35 + (double)n * 1.7e-6;
+  if (solver == NB_SOLVER_DIRECT) return 2e-3 + (double)n * (double)n / 4e9;
+  return 0.11 + (double)n * 1.42e-6;
 }
 
 // Most steps a job takes in one tick (bounds the batch's replays per tick).

@@ -298,3 +298,17 @@ def test_short_jobs_capture_no_graph(nb):
     out, st = run_server(nb, [(9000, 3, 0, k) for k in range(5)])
     assert all(x["state"] == nb.JOB_DONE and x["solver"] == nb.SOLVER_BH for x in st)
     assert nb.load().nb_debug_graph_captures() == before
+
+
+@pytest.mark.parametrize("n, budget", [(65536, 5.0), (200000, 8.0), (45000, 6.0)])
+def test_ticks_fill_their_budget(nb, n, budget):
+    # a tick of a job's steps takes about as long as the budget that they were chosen for
+    with nb.Server(direct_pool=1 << 17, tick_budget_ms=budget) as s:
+        i = s.submit(n, 1000, 0, 1)
+        while s.status(i)["steps_done"] == 0:
+            s.tick()
+        t0 = time.monotonic()
+        for _ in range(8):
+            s.tick()
+        took = (time.monotonic() - t0) / 8 * 1e3
+    assert 0.6 * budget < took < 1.4 * budget
