@@ -1941,9 +1941,7 @@ int nb_bh_alloc(nb_ctx* c) {
     return nb_fail(NB_E_OOM, "nb_create: device allocation failed (octree)");
   }
   nb_bh_carve(c, (char*)b.block, kBhBufCount);
-  // the batched leaf loop may read up to kSpare bodies past the end: zero mass
-  if (hipMemset(b.pms + c->n, 0, sizeof(float4) * kSpare) != hipSuccess ||
-      hipMemset(b.geom, 0, sizeof(float) * 32) != hipSuccess ||
+  if (hipMemset(b.geom, 0, sizeof(float) * 32) != hipSuccess ||
       hipMemset(b.rec_cost, 0, sizeof(float) * c->n) != hipSuccess)
     return nb_fail(NB_E_HIP, "nb_create: hipMemset failed (octree)");
   return NB_OK;

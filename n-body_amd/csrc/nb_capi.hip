@@ -311,7 +311,6 @@ int nb_ctx_rebind(nb_ctx* c, const nb_config* cfg) {
   c->bh = nb_bh_state{};
   c->bh.block = block;
   nb_bh_carve(c, static_cast<char*>(block), kBhBufCount);
-  NB_HIP(nb_launch_fill_i32(reinterpret_cast<int*>(c->bh.pms + c->n), 0, 4 * kSpare, c->stream));
   NB_HIP(nb_launch_fill_i32(c->flags, 0, 4, c->stream));
   NB_HIP(hipStreamSynchronize(c->stream));
   c->uploaded = false;

@@ -80,7 +80,6 @@ constexpr int kBboxBlocks = 256;                      // bbox partial blocks
 constexpr int kSortTile = 2048;                       // keys per block in the radix passes
 constexpr int kSortGroup = 64;                        // tiles whose digit counts are also added up
 constexpr int kTreeTile = 1024;                       // bodies per block in the tree build
-constexpr int kSpare = 4;                             // zero-mass bodies after the sorted bodies
 constexpr int kLevels = kMaxLevel + 1;                // levels a node can have
 constexpr int kCostBuckets = 64;  // half-octaves of estimated record time
 // Whether the Barnes-Hut build pairs sibling ranges (and the traversal orders
@@ -123,7 +122,7 @@ constexpr nb_bh_layout nb_bh_layout_for(int64_t n) {
   bytes[kBhKey0] = bytes[kBhKey1] = bytes[kBhVal0] = bytes[kBhVal1] = bytes[kBhCodes] = 4 * n;
   bytes[kBhHist] = 4 * 256 * sort_blocks;
   bytes[kBhGroupHist] = 4 * 4 * 256 * groups;
-  bytes[kBhPms] = 16 * (n + kSpare);
+  bytes[kBhPms] = 16 * n;
   bytes[kBhPrefix] = 32 * (n + 1);
   bytes[kBhScanPart] = 32 * ((n + kTreeTile - 1) / kTreeTile + 1);
   bytes[kBhNode] = 32 * bound;

@@ -84,10 +84,7 @@ extern "C" int nb_bh_forces_noalloc(const float* pm4, int64_t n, float eps2, flo
   nb_bh_carve(&c, base, kBhBufCount);
   c.flags = status ? status : reinterpret_cast<int*>(base + nb_bh_layout_for(n).off[kBhFlags]);
 
-  // What must start at zero: the status word, and the zero-mass bodies after
-  // the sorted ones (read by the batched leaf loop). Fill kernels, no memset.
-  NB_HIP(nb_launch_fill_i32(c.flags, 0, 1, c.stream));
-  NB_HIP(nb_launch_fill_i32(reinterpret_cast<int*>(c.bh.pms + n), 0, 4 * kSpare, c.stream));
+  NB_HIP(nb_launch_fill_i32(c.flags, 0, 1, c.stream));  // no memset: a caller may capture this
   NB_HIP(nb_bh_build(&c));
   NB_HIP(nb_bh_traverse(&c, false));
   c.bh = nb_bh_state{};  // views only: nothing to free
