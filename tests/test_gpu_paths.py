@@ -411,6 +411,23 @@ def test_build_time_stays_linear(nb):
     assert cost[1] < 1.25 * cost[0]
 
 
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 129, 4097, 16384, 16385, 20011])
+def test_energy_of_unequal_masses(nb, ora, n):
+    """Rows of 64 targets folded two by two against chunks of 64 sources, of 256 above
+    16,384 bodies: every pair once, at the edges of rows and chunks."""
+    rng = np.random.default_rng(n)
+    pos, vel = rng.normal(0, 50, (n, 3)), rng.normal(0, 3, (n, 3))
+    m = rng.uniform(0.1, 10, n).astype(np.float32)
+    with nb.Simulation(n, EPS2, DT, G=1.5) as sim:
+        sim.upload(pos, vel, m)
+        ek, ep, p = sim.energy()
+    rk, rp, q = ora.energy_f64(pos, vel, m.astype(np.float64), EPS2, 1.5)
+    # FP64 sums of one sign: at most 2 n roundings in a row on either side
+    tol = (4 * n + 16) * 2.0 ** -53
+    assert abs(ek - rk) <= tol * rk and abs(ep - rp) <= tol * abs(rp)
+    assert np.abs(p - q).max() <= tol * (m.astype(np.float64)[:, None] * np.abs(vel)).sum(0).max()
+
+
 @pytest.mark.parametrize("n", [300, 3000, 8000])
 def test_small_sizes_use_what_the_tuner_reports(nb, n):
     """Shape 0, 0 is the kernel that takes a step in one launch. Last in the file: a shape
