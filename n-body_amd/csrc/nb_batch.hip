@@ -97,12 +97,15 @@ constexpr int kUnlimited = NB_BATCH_UNLIMITED;
 // bodies 111 / 101, four of 8000 109 / 101, 24 of 256 to 16,384 203 / 197, 256 of 256
 // to 8192 671 / 655, 512 of 256 to 32,768 12,152 / 12,330; 24 served jobs 9.16 / 7.34 ms.
 // The sums of the parts past the first lie where the force array has no bodies: in the
-// pool's free segments and, in a batch of its own, in kSpareBodies entries behind the
-// pool. Parts help while the clusters do not fill the chip, so that is room enough; a
-// cluster that finds none has an item sum its parts one after the other, with the same
-// bits. The parts thus cost a server's pool no memory.
+// pool's free segments and, in a batch of its own, in up to kSpareBodies entries (100 MB)
+// behind the pool; the parts thus cost a server's pool no memory. A cluster that finds
+// no room has an item sum its parts one after the other, with the same bits. That is as
+// fast where an item has eight waves or more, but not below, as its items are longer: 512
+// clusters of 256 to 32,768 bodies with room for a twelfth of their parts / for nearly
+// all, us: 1 x 8 11,426 / 11,411, 2 x 8 11,400 / 11,403, 1 x 4 11,886 / 11,492, 1 x 2
+// 12,584 / 12,125.
 constexpr int kMaxParts = 4;
-constexpr int64_t kSpareBodies = 3 << 17;
+constexpr int64_t kSpareBodies = 1 << 22;
 int batch_parts(int npad) {
   return std::max(1, std::min({kMaxParts, (npad + 4095) / 4096, 1024 / (npad / 64)}));
 }
@@ -156,13 +159,15 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_num_sgpr(80))) void k
     const int ibase = it.ibase + lane;
     const int parts = (it.head >> 4 & 3) + 1, first = it.head >> 2 & 3;
     const int last = it.head & 2 ? parts - 1 : first;
-    const int units = (it.end - it.off + 255) / 256 * 16;  // of 16 sources
+    // of 16 sources; times a slice's number it fits 32 bits: at most 2^26 units are cut
+    // into at most 16 slices, 2048 (clusters in parts) into 64
+    const uint32_t units = (uint32_t)(it.end - it.off + 255) / 256 * 16;
     for (int q = first; q <= last; ++q) {
       nbcore::Targets<B> t;
       nbcore::load_targets<B>(pm, ibase, t);
-      const int slices = K * parts, slice = K * q + wave;
-      const int j0 = it.off + 16 * (int)((int64_t)units * slice / slices);
-      const int j1 = it.off + 16 * (int)((int64_t)units * (slice + 1) / slices);
+      const uint32_t slices = K * parts, slice = K * q + wave;
+      const int j0 = it.off + 16 * (int)(units * slice / slices);
+      const int j1 = it.off + 16 * (int)(units * (slice + 1) / slices);
       if (it.head & 1)
         nbcore::accumulate<B, false, true>(pm, j0, j1, it.eps2, t);
       else if (it.eps2 >= 1e-20f)

@@ -285,7 +285,7 @@ def test_direct_sum_shares_of_unequal_masses(nb, ora, n, bpl, js, eps2):
 def test_batch_parts_with_and_without_room(nb):
     """More clusters in parts than there is room for partial sums: those without it, and a
     batch whose removed clusters make room, give the same forces and steps."""
-    n, clusters = 16000, 12  # four parts each
+    n, clusters = 16000, 90  # four parts each
     pos, vel, m = nb.ic_plummer(9, n, 50.0, 1e4)
     with nb.Batch(clusters * 16128, clusters) as b:
         ids = [b.add(pos, vel, m, EPS2, DT) for _ in range(clusters)]
