@@ -18,7 +18,8 @@
 //                  a stable scatter, whose blocks add up the counts before
 //                  theirs themselves and whose per-wave ranks come from
 //                  64-bit ballots (8 ballots give each lane the mask of lanes
-//                  holding the same digit). Small systems: 3 passes of 10 bits,
+//                  holding the same digit). From 2^22 bodies on a launch between
+//                  the two adds up the counts. Small systems: 3 passes of 10 bits,
 //                  whose blocks count all keys. Stable => sorted by (code, index).
 //   4. mark        gather (x, y, z, m) into sorted order; per body the levels at
 //                  which a node starts there; per tile the node counts of every
